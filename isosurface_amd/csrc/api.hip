@@ -18,6 +18,7 @@
 #include "mc_kernels.h"
 #include "mlp_kernels.h"
 #include "program.h"
+#include "sparse_kernels.h"
 
 namespace {
 
@@ -47,6 +48,7 @@ struct MeshGraphKey {
   const void* ops;
   const float* values;
   int64_t n_prog;
+  int64_t program_kind;  // bounded, stack: which kernel classifies
   iso::McBuffers B;
 };
 
@@ -61,6 +63,8 @@ struct iso_ctx {
   int n_prog = 0;
   bool prog_directed = false;  // the program has a directed form (no smooth union)
   bool prog_hermite = false;   // analytic normals exist (shapes, unions, translations)
+  bool prog_bounded = false;   // interval bounds of the program are sound
+  bool prog_stack = false;     // the program holds values below the running one
 
   // current grid
   DevBuf grid_owned;
@@ -417,6 +421,8 @@ int iso_program_upload(iso_ctx* c, const iso_node* nodes, uint32_t n_nodes) {
                             hipMemcpyHostToDevice, c->stream));
   ISO_HIP(c, hipStreamSynchronize(c->stream));
   c->n_prog = static_cast<int>(ops.size());
+  c->prog_bounded = iso::program_bounded(ops.data(), c->n_prog);
+  c->prog_stack = iso::program_needs_stack(ops.data(), c->n_prog);
   c->prog_directed = true;
   c->prog_hermite = true;
   for (uint32_t i = 0; i < n_nodes; ++i) {
@@ -616,7 +622,10 @@ int classify_and_count(iso_ctx* c, const float* grid, const iso::Lattice& L, con
                      [&] { return iso::launch_signs_grid(grid, L, D, B, c->stream); }));
   } else {
     ISO_HIP(c, timed(c, "mc_signs_program", [&] {
-              return iso::launch_signs_program(ops, c->n_prog, L, D, B, values, c->stream);
+              return iso::sparse_lattice(L, c->prog_bounded)
+                         ? iso::launch_signs_sparse(ops, c->n_prog, c->prog_stack, L, D, B, values,
+                                                    c->stream)
+                         : iso::launch_signs_program(ops, c->n_prog, L, D, B, values, c->stream);
             }));
   }
   ISO_HIP(c, timed(c, "mc_count", [&] { return iso::launch_count(L, D, B, c->stream); }));
@@ -815,7 +824,9 @@ int extract_lattice(iso_ctx* c, const iso::Lattice& L, const float* grid, const 
     iso::FusedPlan P;
     if (iso::fused_plan(L, &P)) return extract_fused(c, L, grid, P, out);
   }
-  const iso::McDims D = iso::mc_dims(L);
+  // Program signs are classified sparsely, into row-aligned sign words.
+  const bool sparse = !grid && !signs && iso::sparse_lattice(L, c->prog_bounded);
+  const iso::McDims D = sparse ? iso::mc_dims_pitched(L) : iso::mc_dims(L);
   if (D.n_segs >= (int64_t(1) << 26))
     return fail(c, ISO_ERR_INVALID_ARGUMENT, "lattice has 2^26 or more 64-cell segments");
   iso::McBuffers B{};
@@ -863,6 +874,7 @@ int extract_lattice(iso_ctx* c, const iso::Lattice& L, const float* grid, const 
       k.ops = grid ? nullptr : ops;
       k.values = values;
       k.n_prog = grid ? 0 : c->n_prog;
+      k.program_kind = grid ? 0 : (c->prog_bounded ? 1 : 0) + (c->prog_stack ? 2 : 0);
       k.B = b;
       return k;
     };
@@ -1248,7 +1260,9 @@ int iso_extract_point_cloud(iso_ctx* c, const iso_grid_desc* desc, iso_mesh_out*
   c->kept = false;
   c->band_valid = false;
   ISO_HIP(c, hipSetDevice(c->device));
-  const iso::McDims D = iso::mc_dims(L);
+  const iso::McDims D =
+      !from_grid && iso::sparse_lattice(L, c->prog_bounded) ? iso::mc_dims_pitched(L)
+                                                            : iso::mc_dims(L);
   if (D.n_segs >= (int64_t(1) << 26))
     return fail(c, ISO_ERR_INVALID_ARGUMENT, "lattice has 2^26 or more 64-cell segments");
   iso::McBuffers B{};
@@ -1706,6 +1720,7 @@ int iso_batch_upload(iso_ctx* c, const iso_node* nodes, uint64_t n_nodes,
       C.spacing[k] = g.spacing[k];
     }
     C.signs = dsigns + sign_off[i];
+    C.sign_pitch = g.nx;
     C.segs_per_row = static_cast<uint32_t>((g.nx - 1 + 63) / 64);
     C.seg_off = seg_start[i];
     C.ops = dops + op_off[i];

@@ -23,6 +23,7 @@ struct McDims {
   int64_t n_segs;        // n_cell_rows * segs_per_row
   int64_t n_blocks;      // count workgroups (kCountBlock segments each)
   int64_t n_cells;       // (nx-1)*(ny-1)*(nz-1)
+  int64_t sign_pitch;    // sign bits from one sample row to the next: nx, or a multiple of 64
 };
 
 constexpr int kCountBlock = 1024;  // threads per count workgroup (16 waves)
@@ -49,6 +50,8 @@ enum : int {
 };
 
 McDims mc_dims(const Lattice& L);
+// The same with row-aligned sign words: every sample row starts a word.
+McDims mc_dims_pitched(const Lattice& L);
 
 // Coordinate of lattice index i along an axis: origin + i * spacing, the
 // reference's `x as f32 * one_over_size` when origin is 0
@@ -67,7 +70,8 @@ struct CellSpace {
   int64_t nx, ny, nz;
   float origin[3];
   float spacing[3];
-  const uint64_t* signs;    // the lattice's flat sign bits
+  const uint64_t* signs;    // the lattice's sign bits, row (y, z) at bit (z ny + y) sign_pitch
+  int64_t sign_pitch;       // nx (flat), or a multiple of 64 (row-aligned)
   uint32_t segs_per_row;
   uint32_t seg_off;         // global index of the lattice's first segment
   const DevOp* ops;         // program source
@@ -76,6 +80,11 @@ struct CellSpace {
   const float* grid;        // dense samples (a batch's stored program samples), or null
   const float* positions;   // per-point vertex positions, or null
 };
+
+// The CellSpace of a single lattice.
+CellSpace single_cell_space(const Lattice& L, const McDims& D, const uint64_t* signs,
+                            const DevOp* ops, int n_ops, const float* grid,
+                            const float* positions);
 
 // Buffers of one extraction.
 struct McBuffers {

@@ -290,6 +290,7 @@ __global__ __launch_bounds__(kCountBlock) void k_count(Space sp, int64_t n_segs,
       const CellSpace& C = sp.at(static_cast<uint32_t>(g), &gg);
       const uint64_t* __restrict__ S = C.signs;
       const int64_t nx = C.nx, ny = C.ny;
+      const int64_t pitch = C.sign_pitch;
       const uint32_t spr = C.segs_per_row;
       const uint32_t cyn = static_cast<uint32_t>(ny - 1);
       const uint32_t row = gg / spr;
@@ -297,12 +298,12 @@ __global__ __launch_bounds__(kCountBlock) void k_count(Space sp, int64_t n_segs,
       const uint32_t cz = row / cyn;
       const uint32_t cy = row - cz * cyn;
       const int64_t f00 =
-          (static_cast<int64_t>(cz) * ny + cy) * nx + 64 * static_cast<int64_t>(w);
+          (static_cast<int64_t>(cz) * ny + cy) * pitch + 64 * static_cast<int64_t>(w);
       uint64_t n00, n10, n01, n11;
       const uint64_t w00 = row_word(S, f00, &n00);
-      const uint64_t w10 = row_word(S, f00 + nx, &n10);
-      const uint64_t w01 = row_word(S, f00 + nx * ny, &n01);
-      const uint64_t w11 = row_word(S, f00 + nx * ny + nx, &n11);
+      const uint64_t w10 = row_word(S, f00 + pitch, &n10);
+      const uint64_t w01 = row_word(S, f00 + pitch * ny, &n01);
+      const uint64_t w11 = row_word(S, f00 + pitch * ny + pitch, &n11);
       const SegWords sw = seg_words(w00, n00, w10, n10, w01, n01, w11, n11);
       const uint64_t valid = seg_valid(nx, w);
       uint64_t vp[4];
@@ -661,13 +662,16 @@ __global__ __launch_bounds__(kEmitThreads) void k_emit(EmitArgs A, Space sp) {
     // x-1, x, x+1, read straight from the flat sign array (the guard words
     // cover x-1 at the array's start; bits of rows or columns outside the
     // lattice are never used).
+    const int64_t pitch = C.sign_pitch;
+    const int64_t fs = (static_cast<int64_t>(cz) * ny + cy) * pitch + cx;
     uint32_t cube = 0;
 #pragma unroll
     for (int dz = 0; dz < 3; ++dz) {
 #pragma unroll
       for (int dy = 0; dy < 3; ++dy) {
         if (cy - 1 + dy >= 0 && cz - 1 + dz >= 0) {
-          const int64_t q = fc - 1 + (dy - 1) * nx + (dz - 1) * nxy;  // sample x-1 (>= -1)
+          // bit of sample x-1 (>= -1)
+          const int64_t q = fs - 1 + (dy - 1) * pitch + (dz - 1) * (pitch * ny);
           // The three bits q..q+2 lie in the 64 bits that start at q's
           // 32-bit word: one 8-byte load (4-byte aligned) per row.
           uint64_t v;
@@ -960,7 +964,38 @@ McDims mc_dims(const Lattice& L) {
   D.n_segs = D.n_cell_rows * D.segs_per_row;
   D.n_blocks = (D.n_segs + kCountSegs - 1) / kCountSegs;
   D.n_cells = (L.nx - 1) * (L.ny - 1) * (L.nz - 1);
+  D.sign_pitch = L.nx;
   return D;
+}
+
+McDims mc_dims_pitched(const Lattice& L) {
+  McDims D = mc_dims(L);
+  D.sign_pitch = (L.nx + 63) / 64 * 64;
+  D.n_sign_words = D.sign_pitch / 64 * L.ny * L.nz;
+  return D;
+}
+
+CellSpace single_cell_space(const Lattice& L, const McDims& D, const uint64_t* signs,
+                            const DevOp* ops, int n_ops, const float* grid,
+                            const float* positions) {
+  CellSpace C;
+  C.nx = L.nx;
+  C.ny = L.ny;
+  C.nz = L.nz;
+  for (int i = 0; i < 3; ++i) {
+    C.origin[i] = L.origin[i];
+    C.spacing[i] = L.spacing[i];
+  }
+  C.signs = signs;
+  C.sign_pitch = D.sign_pitch;
+  C.segs_per_row = static_cast<uint32_t>(D.segs_per_row);
+  C.seg_off = 0;
+  C.ops = ops;
+  C.n_ops = n_ops;
+  C.reserved = 0;
+  C.grid = grid;
+  C.positions = positions;
+  return C;
 }
 
 namespace {
@@ -1029,23 +1064,7 @@ namespace {
 SingleSpace single_space(const Lattice& L, const McDims& D, const uint64_t* signs,
                          const DevOp* ops, int n_ops, const float* grid,
                          const float* positions) {
-  SingleSpace sp;
-  sp.C.nx = L.nx;
-  sp.C.ny = L.ny;
-  sp.C.nz = L.nz;
-  for (int i = 0; i < 3; ++i) {
-    sp.C.origin[i] = L.origin[i];
-    sp.C.spacing[i] = L.spacing[i];
-  }
-  sp.C.signs = signs;
-  sp.C.segs_per_row = static_cast<uint32_t>(D.segs_per_row);
-  sp.C.seg_off = 0;
-  sp.C.ops = ops;
-  sp.C.n_ops = n_ops;
-  sp.C.reserved = 0;
-  sp.C.grid = grid;
-  sp.C.positions = positions;
-  return sp;
+  return SingleSpace{single_cell_space(L, D, signs, ops, n_ops, grid, positions)};
 }
 
 EmitArgs emit_args(const McBuffers& B) {

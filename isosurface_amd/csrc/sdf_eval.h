@@ -20,6 +20,31 @@ __device__ __forceinline__ float f_len3(float x, float y, float z) {
   return __builtin_sqrtf((x * x + y * y) + z * z);
 }
 
+// Correctly rounded square roots of K nonnegative values, bit for bit
+// __builtin_sqrtf's: the hardware's reciprocal square root and one Markstein
+// correction (six instructions; the compiler's sequence for any operand takes
+// sixteen).  Compared with __builtin_sqrtf at every float from 2^-96 to 2^120
+// and at zero; other operands take the compiler's sequence, in a branch that a
+// wavefront shares.
+template <int K>
+__device__ __forceinline__ void f_sqrt(const float (&x)[K], float (&r)[K]) {
+  constexpr uint32_t kLow = 0x0F800000u, kHigh = 0x7B800000u;  // 2^-96, 2^120
+  uint32_t least = ~0u, most = 0u;  // of bits(x) - 1 (zero wraps to the top), and of bits(x)
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const uint32_t b = __builtin_bit_cast(uint32_t, x[k]);
+    least = b - 1u < least ? b - 1u : least;
+    most = b > most ? b : most;
+    const float y = __builtin_amdgcn_rsqf(fmaxf(x[k], 1.2621774e-29f));  // 2^-96
+    const float s = x[k] * y;
+    r[k] = __builtin_fmaf(__builtin_fmaf(-s, s, x[k]), 0.5f * y, s);
+  }
+  if (__builtin_expect(__ballot(least < kLow - 1u || most >= kHigh) != 0ull, 0)) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) r[k] = __builtin_sqrtf(x[k]);
+  }
+}
+
 __device__ __forceinline__ float prim_value(uint32_t code, const float* prm, float x, float y,
                                             float z) {
   if (code == kSphere) {
@@ -40,6 +65,63 @@ __device__ __forceinline__ float prim_value(uint32_t code, const float* prm, flo
     const float qz = __builtin_fabsf(z) - prm[1];
     const float dx = fmaxf(qx, 0.0f), dy = fmaxf(qz, 0.0f);
     return fminf(fmaxf(qx, qz), 0.0f) + f_len3(dx, dy, 0.0f);
+  }
+}
+
+// prim_value at K points (q[k] after the primitive's translation).
+template <int K>
+__device__ __forceinline__ void prim_values(uint32_t code, const float* prm,
+                                            const float (&q)[K][3], float (&v)[K]) {
+  float s[K], r[K];
+  if (code == kSphere) {
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+      s[k] = (q[k][0] * q[k][0] + q[k][1] * q[k][1]) + q[k][2] * q[k][2];
+    f_sqrt(s, r);
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] = r[k] - prm[0];
+  } else if (code == kBox) {
+    float in[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const float qx = __builtin_fabsf(q[k][0]) - prm[0];
+      const float qy = __builtin_fabsf(q[k][1]) - prm[1];
+      const float qz = __builtin_fabsf(q[k][2]) - prm[2];
+      const float mx = fmaxf(qx, 0.0f), my = fmaxf(qy, 0.0f), mz = fmaxf(qz, 0.0f);
+      in[k] = fminf(fmaxf(qx, fmaxf(qy, qz)), 0.0f);
+      s[k] = (mx * mx + my * my) + mz * mz;
+    }
+    f_sqrt(s, r);
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] = r[k] + in[k];
+  } else if (code == kTorus) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) s[k] = q[k][0] * q[k][0] + q[k][1] * q[k][1];
+    f_sqrt(s, r);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const float qx = __builtin_fabsf(r[k]) - prm[0];
+      s[k] = qx * qx + q[k][2] * q[k][2];
+    }
+    f_sqrt(s, r);
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] = r[k] - prm[1];
+  } else {  // kCylinder
+    float in[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) s[k] = q[k][0] * q[k][0] + q[k][1] * q[k][1];
+    f_sqrt(s, r);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const float qx = __builtin_fabsf(r[k]) - prm[0];
+      const float qz = __builtin_fabsf(q[k][2]) - prm[1];
+      const float dx = fmaxf(qx, 0.0f), dy = fmaxf(qz, 0.0f);
+      in[k] = fminf(fmaxf(qx, qz), 0.0f);
+      s[k] = (dx * dx + dy * dy) + 0.0f * 0.0f;
+    }
+    f_sqrt(s, r);
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] = in[k] + r[k];
   }
 }
 

@@ -1,0 +1,548 @@
+// Interval evaluation and list evaluation of lowered SDF programs for a
+// wavefront that works on one tile of a lattice (see sparse_kernels.hip).
+//
+// Intervals: every operation of a program's f32 evaluation is monotone in
+// each |coordinate difference| or operand (a correctly rounded operation is
+// monotone because the exact one is), so evaluating the same operations at
+// the least and the greatest |q_c| of a box gives bounds that no f32
+// evaluation at a point of the box leaves.  Two operations take an allowance:
+// square roots, which the bounds take from the hardware's approximation, and
+// the polynomial smooth minimum, monotone only in exact arithmetic.
+//
+// The bounds hold for finite parameters and coordinates of ordinary
+// magnitude (no overflow of a square): the host checks that (program_bounded
+// and lattice_bounded, sparse_kernels.h), and programs or lattices beyond it
+// are evaluated densely.
+//
+// kStack: the program holds values below the running one (a push after the
+// first).  Most programs do not, and the interpreters without a stack carry a
+// third of the state through their branches.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "sdf_eval.h"
+#include "sdf_program.h"
+
+namespace iso {
+
+// A program in the constant address space: an operation read at a uniform
+// index is then a scalar load into scalar registers, whatever else the kernel
+// stores to (through an ordinary pointer that came from memory or a struct the
+// compiler must assume that a store may change it, and loads it per lane: 185
+// us instead of SPARSE_US for the 257^3 signs of 64 spheres minus a torus).
+using OpsPtr = const DevOp __attribute__((address_space(4)))*;
+__device__ __forceinline__ OpsPtr as_constant(const DevOp* ops) {
+  return (OpsPtr)(reinterpret_cast<uintptr_t>(ops));
+}
+__device__ __forceinline__ DevOp load_op(OpsPtr ops, int i) {
+  DevOp o;
+  o.code = ops[i].code;
+  o.combine = ops[i].combine;
+  o.translated = ops[i].translated;
+  o.k = ops[i].k;
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    o.prm[a] = ops[i].prm[a];
+    o.off[a] = ops[i].off[a];
+  }
+  return o;
+}
+
+// A value stack of registers: pushes and pops move the entries, so no entry
+// is addressed by a run-time index (a program seldom pushes).
+struct ShiftStack {
+  float v[kMaxValueStack];
+  __device__ __forceinline__ void push(float x) {
+#pragma unroll
+    for (int i = kMaxValueStack - 1; i > 0; --i) v[i] = v[i - 1];
+    v[0] = x;
+  }
+  __device__ __forceinline__ float pop() {
+    const float x = v[0];
+#pragma unroll
+    for (int i = 0; i + 1 < kMaxValueStack; ++i) v[i] = v[i + 1];
+    return x;
+  }
+};
+
+// The open translation scopes, innermost in the low bits: op indices of
+// their kPushTranslate, 16 bits each (a program has at most 8192 ops and
+// kMaxPointStack nested scopes).  Leaving a scope re-applies the remaining
+// ones to the base point, outermost first.
+struct ScopeStack {
+  uint64_t ops = 0;
+  int depth = 0;
+  __device__ __forceinline__ void push(int op) {
+    ops = (ops << 16) | static_cast<uint64_t>(op);
+    ++depth;
+  }
+  __device__ __forceinline__ void pop() {
+    ops >>= 16;
+    --depth;
+  }
+  __device__ __forceinline__ int at(int level) const {  // level 0: outermost
+    return static_cast<int>((ops >> (16 * (depth - 1 - level))) & 0xFFFFull);
+  }
+};
+static_assert(kMaxPointStack <= 4 && kMaxProgramOps <= 65536, "ScopeStack packs four op indices");
+
+// Bounds of the correctly rounded square root by the hardware's, which is
+// within one ulp of it (two for certain: four are allowed), and within 2^-62
+// of it where its operand is too small to be normal.
+__device__ __forceinline__ float sqrt_below(float x) {
+  return __builtin_amdgcn_sqrtf(x) * 0.99999976f;  // 1 - 2^-22
+}
+__device__ __forceinline__ float sqrt_above(float x) {
+  return __builtin_fmaf(__builtin_amdgcn_sqrtf(x), 1.00000024f, 1.0e-18f);  // 1 + 2^-22
+}
+
+// Bounds of a primitive's f32 value over the points of the box [lo, hi]
+// (after the primitive's own translation).
+__device__ __forceinline__ void prim_interval(uint32_t code, const float* prm, const float* lo,
+                                              const float* hi, float* vlo, float* vhi) {
+  float an[3], af[3];  // least and greatest |q_c|
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    an[a] = fmaxf(fmaxf(lo[a], -hi[a]), 0.0f);
+    af[a] = fmaxf(-lo[a], hi[a]);
+  }
+  // All but the torus are nondecreasing in each |q_c|.
+  if (code == kSphere) {
+    *vlo = sqrt_below((an[0] * an[0] + an[1] * an[1]) + an[2] * an[2]) - prm[0];
+    *vhi = sqrt_above((af[0] * af[0] + af[1] * af[1]) + af[2] * af[2]) - prm[0];
+  } else if (code == kBox) {
+    float n[3], f[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      an[a] = an[a] - prm[a];
+      af[a] = af[a] - prm[a];
+      n[a] = fmaxf(an[a], 0.0f);
+      f[a] = fmaxf(af[a], 0.0f);
+    }
+    *vlo = sqrt_below((n[0] * n[0] + n[1] * n[1]) + n[2] * n[2]) +
+           fminf(fmaxf(an[0], fmaxf(an[1], an[2])), 0.0f);
+    *vhi = sqrt_above((f[0] * f[0] + f[1] * f[1]) + f[2] * f[2]) +
+           fminf(fmaxf(af[0], fmaxf(af[1], af[2])), 0.0f);
+  } else {
+    // distance to the axis circle or surface
+    const float q0 = sqrt_below(an[0] * an[0] + an[1] * an[1]) - prm[0];
+    const float q1 = sqrt_above(af[0] * af[0] + af[1] * af[1]) - prm[0];
+    if (code == kTorus) {  // nondecreasing in |q| and |z|
+      const float qn = fmaxf(fmaxf(q0, -q1), 0.0f), qf = fmaxf(-q0, q1);
+      *vlo = sqrt_below(qn * qn + an[2] * an[2]) - prm[1];
+      *vhi = sqrt_above(qf * qf + af[2] * af[2]) - prm[1];
+    } else {  // kCylinder
+      const float z0 = an[2] - prm[1], z1 = af[2] - prm[1];
+      const float dx0 = fmaxf(q0, 0.0f), dz0 = fmaxf(z0, 0.0f);
+      const float dx1 = fmaxf(q1, 0.0f), dz1 = fmaxf(z1, 0.0f);
+      *vlo = fminf(fmaxf(q0, z0), 0.0f) + sqrt_below(dx0 * dx0 + dz0 * dz0);
+      *vhi = fminf(fmaxf(q1, z1), 0.0f) + sqrt_above(dx1 * dx1 + dz1 * dz1);
+    }
+  }
+}
+
+// Wave-wide minima by data-parallel primitives: a register move each, where a
+// shuffle goes through the LDS unit and takes about a hundred cycles.
+constexpr float kNoBound = 3.0e38f;
+
+template <int kCtrl, int kRows>
+__device__ __forceinline__ float dpp_min(float v) {
+  const int t = __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, kNoBound),
+                                            __builtin_bit_cast(int, v), kCtrl, kRows, 0xf, false);
+  return fminf(v, __builtin_bit_cast(float, t));
+}
+// Inclusive prefix minimum over the lanes (values at most kNoBound).
+__device__ __forceinline__ float wave_min_upto(float v) {
+  v = dpp_min<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8: within rows of 16 lanes
+  v = dpp_min<0x112, 0xf>(v);
+  v = dpp_min<0x114, 0xf>(v);
+  v = dpp_min<0x118, 0xf>(v);
+  v = dpp_min<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+  v = dpp_min<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+// The minimum over all lanes, in every lane.
+__device__ __forceinline__ float wave_min(float v) {
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wave_min_upto(v)), 63));
+}
+// The minimum over the lanes below this one.
+__device__ __forceinline__ float wave_min_before(float v) {
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, kNoBound),
+                                         __builtin_bit_cast(int, wave_min_upto(v)), 0x138, 0xf, 0xf,
+                                         false));  // wave_shr:1
+}
+
+// Whether an operand of a smooth minimum that is at least `gap` above the
+// running value leaves it unchanged (the blend weight is then exactly 0).
+__device__ __forceinline__ bool smooth_inactive(float gap, float k) {
+  constexpr float u = 5.9604645e-08f;  // 2^-24
+  return gap * (1.0f - 4.0f * u) >= k * (1.0f + 4.0f * u);
+}
+
+// Bounds of smooth_min over operands in [alo, ahi] and [blo, bhi].
+__device__ __forceinline__ void smooth_interval(float alo, float ahi, float blo, float bhi, float k,
+                                                float* lo, float* hi) {
+  constexpr float u = 5.9604645e-08f;
+  const float mag = fmaxf(fmaxf(__builtin_fabsf(alo), __builtin_fabsf(ahi)),
+                          fmaxf(__builtin_fabsf(blo), __builtin_fabsf(bhi)));
+  const float slack = 32.0f * u * (k + mag);
+  *lo = smooth_min(alo, blo, k) - slack;
+  *hi = smooth_min(ahi, bhi, k) + slack;
+}
+
+// The running bounds of a program's evaluation.
+template <bool kStack>
+struct Bounds {
+  // Before the first value: neutral to min, as the first push is read.
+  float lo = kNoBound, hi = kNoBound;
+  bool have_top = false;
+  ShiftStack slo, shi;
+  __device__ __forceinline__ Bounds() {
+#pragma unroll
+    for (int i = 0; i < kMaxValueStack; ++i) slo.v[i] = shi.v[i] = 0.0f;
+  }
+  // Joins a primitive bounded by [vlo, vhi]; returns false, with the bounds as
+  // they were, when for every lane with `active` the operand leaves the
+  // running value bit for bit as it is at every point of the lane's box:
+  //   min:         its lower bound exceeds the running upper bound,
+  //   smooth min:  it does by the blend width (the weight is then exactly 0),
+  //   max, max of the negated operand: its upper bound is below the running
+  //                lower bound.
+  // *matters: the lanes for which it does not.
+  __device__ __forceinline__ bool join(uint32_t mode, float k, float vlo, float vhi, bool active,
+                                       uint64_t* matters) {
+    if (kStack && mode == kPush) {
+      if (have_top) {
+        slo.push(lo);
+        shi.push(hi);
+      }
+      have_top = true;
+      lo = vlo;
+      hi = vhi;
+      *matters = ~0ull;
+      return true;
+    }
+    bool idle;
+    float nlo, nhi;
+    if (mode == kMin || (!kStack && mode == kPush)) {
+      idle = vlo > hi;
+      nlo = fminf(lo, vlo);
+      nhi = fminf(hi, vhi);
+    } else if (mode == kSmooth) {
+      idle = smooth_inactive(vlo - hi, k);
+      smooth_interval(lo, hi, vlo, vhi, k, &nlo, &nhi);
+    } else {
+      // max(top, v), max(v, -top) or max(top, -v)
+      const float al = mode == kDiff ? -hi : lo, ah = mode == kDiff ? -lo : hi;
+      const float bl = mode == kDiffRev ? -vhi : vlo, bh = mode == kDiffRev ? -vlo : vhi;
+      idle = mode != kDiff && bh < al;
+      nlo = fmaxf(al, bl);
+      nhi = fmaxf(ah, bh);
+    }
+    *matters = __ballot(active && !idle);
+    if (*matters == 0ull) return false;
+    lo = nlo;
+    hi = nhi;
+    return true;
+  }
+  // A binary operator on (below, top).
+  __device__ __forceinline__ void operate(uint32_t code, float k) {
+    const float tl = lo, th = hi;
+    const float wl = slo.pop(), wh = shi.pop();
+    if (code == kUnion) {
+      lo = fminf(wl, tl);
+      hi = fminf(wh, th);
+    } else if (code == kSmoothUnion) {
+      smooth_interval(wl, wh, tl, th, k, &lo, &hi);
+    } else {
+      // max(w, t), max(t, -w) or max(w, -t)
+      const bool nw = code == kDifference, nt = code == kDifferenceRev;
+      lo = fmaxf(nw ? -wh : wl, nt ? -th : tl);
+      hi = fmaxf(nw ? -wl : wh, nt ? -tl : th);
+    }
+  }
+};
+
+// Moves a box into or out of a translation scope: [cl, ch] is the base box
+// [bl, bh] less the offsets of the open scopes, outermost first.
+__device__ __forceinline__ void enter_scope(OpsPtr ops, int op, float* cl, float* ch) {
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    cl[a] = cl[a] - ops[op].off[a];
+    ch[a] = ch[a] - ops[op].off[a];
+  }
+}
+__device__ __forceinline__ void restore_scopes(OpsPtr ops, const ScopeStack& scopes,
+                                               const float* bl, const float* bh, float* cl,
+                                               float* ch) {
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    cl[a] = bl[a];
+    ch[a] = bh[a];
+  }
+  for (int s = 0; s < scopes.depth; ++s) enter_scope(ops, scopes.at(s), cl, ch);
+}
+
+__device__ __forceinline__ void op_interval(const DevOp& op, const float* cl, const float* ch,
+                                            float* vlo, float* vhi) {
+  float ql[3], qh[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {  // (an untranslated primitive's offset is 0, and x - 0 is x)
+    ql[a] = cl[a] - op.off[a];
+    qh[a] = ch[a] - op.off[a];
+  }
+  prim_interval(op.code, op.prm, ql, qh, vlo, vhi);
+}
+
+// Scopes that hold the whole program (a recentring wrapper): as many as open
+// it and close it together.  The callers give boxes and points inside them,
+// and walk the operations after their openings, with them already open.
+__device__ __forceinline__ int leading_scopes(OpsPtr ops, int n) {
+  int s = 0;
+  while (2 * s < n && ops[s].code == kPushTranslate && ops[n - 1 - s].code == kPopTranslate) ++s;
+  return s;
+}
+
+// Bounds of the operations [first, n) over one box [tlo, thi], the same for
+// every lane of the wavefront, and those that can change a value in it: their
+// indices go to `list` (LDS, ascending), and their number is returned (above
+// `cap`: they do not fit, and the list is not usable).  Runs of min and
+// smooth-min operands are bounded 64 at a time, one a lane, each against the
+// running upper bound before it.
+template <bool kStack>
+__device__ __forceinline__ int bound_box(OpsPtr ops, int first, int n, const float* tlo,
+                                         const float* thi, uint16_t* list, int cap, float* out_lo,
+                                         float* out_hi) {
+  const int lane = __lane_id();
+  Bounds<kStack> B;
+  ScopeStack scopes;
+  float cl[3] = {tlo[0], tlo[1], tlo[2]}, ch[3] = {thi[0], thi[1], thi[2]};
+  int count = 0;
+  for (int base = first; base < n; base += 64) {
+    // One operation a lane (the last one again past the end).
+    const int j = base + lane < n ? base + lane : n - 1;
+    const DevOp mine = load_op(ops, j);
+    const int e = n - base < 64 ? n - base : 64;
+    const uint64_t run = __ballot(base + lane < n && mine.code <= kCylinder &&
+                                  (mine.combine == kMin || mine.combine == kSmooth));
+    int p = 0;
+    while (p < e) {
+      const uint64_t from = run >> p;
+      if (from & 1ull) {
+        const int m = ~from ? static_cast<int>(__builtin_ctzll(~from)) : 64;
+        const bool in = lane >= p && lane < p + m;
+        float vlo = kNoBound, vhi = kNoBound;
+        if (in) op_interval(mine, cl, ch, &vlo, &vhi);
+        const bool smooth = mine.combine == kSmooth;
+        const float T = fminf(B.hi, wave_min_before(vhi));
+        const bool kept = in && !(smooth ? smooth_inactive(vlo - T, mine.k) : vlo > T);
+        const uint64_t keep = __ballot(kept);
+        if (kept) {
+          const int at = count + static_cast<int>(__popcll(keep & ((1ull << lane) - 1ull)));
+          if (at < cap) list[at] = static_cast<uint16_t>(j);
+        }
+        count += static_cast<int>(__popcll(keep));
+        B.hi = fminf(B.hi, wave_min(vhi));
+        B.lo = fminf(B.lo, wave_min(kept ? vlo : kNoBound));
+        // A chain of smooth minima of values that are at least x stays above
+        // x less the largest blend width: a step from x - d takes off
+        // (k - d)^2 / 4k, less than the k - d that is left.
+        if (__ballot(kept && smooth)) {
+          const float kmax = -wave_min(kept && smooth ? -mine.k : 0.0f);
+          B.lo -= kmax + 1.0e-4f * (kmax + fmaxf(__builtin_fabsf(B.lo), __builtin_fabsf(B.hi)));
+        }
+        p += m;
+        continue;
+      }
+      const int i = base + p;
+      const DevOp op = load_op(ops, i);
+      ++p;
+      if (op.code <= kCylinder) {
+        float vlo, vhi;
+        uint64_t matters;
+        op_interval(op, cl, ch, &vlo, &vhi);
+        if (!B.join(op.combine, op.k, vlo, vhi, true, &matters)) continue;
+      } else if (op.code == kPushTranslate) {
+        scopes.push(i);
+        enter_scope(ops, i, cl, ch);
+      } else if (op.code == kPopTranslate) {
+        if (scopes.depth == 0) continue;  // a leading scope's end, at the program's end
+        scopes.pop();
+        restore_scopes(ops, scopes, tlo, thi, cl, ch);
+      } else if (kStack) {
+        B.operate(op.code, op.k);
+      }
+      if (lane == 0 && count < cap) list[count] = static_cast<uint16_t>(i);
+      ++count;
+    }
+  }
+  *out_lo = B.lo;
+  *out_hi = B.hi;
+  return count;
+}
+
+// Bounds of the program over each lane's own box [blo, bhi] (`active` false:
+// the lane has none), walking the m operations of `list` (null: the operations
+// [first, first + m)).  With a list, the operations that matter to no lane are
+// taken out of it, and mask[j] names the lanes that the j-th remaining one
+// matters to.  Returns the number of operations left.
+template <bool kStack>
+__device__ __forceinline__ int bound_lanes(OpsPtr ops, int first, int m, const float* blo,
+                                           const float* bhi, bool active, uint16_t* list,
+                                           uint64_t* mask, float* out_lo, float* out_hi) {
+  const int lane = __lane_id();
+  Bounds<kStack> B;
+  ScopeStack scopes;
+  float cl[3] = {blo[0], blo[1], blo[2]}, ch[3] = {bhi[0], bhi[1], bhi[2]};
+  // The list is rewritten 64 entries at a time, from registers, one entry a
+  // lane: behind the entries read so far, which `mine` holds.
+  int count = 0, mine = 0, my_op = 0;
+  uint64_t my_mask = 0;
+  for (int j = 0; j < m; ++j) {
+    if ((j & 63) == 0) mine = list ? (j + lane < m ? list[j + lane] : 0) : first + j + lane;
+    const int i = __builtin_amdgcn_readlane(mine, j & 63);
+    const DevOp op = load_op(ops, i);
+    uint64_t matters = ~0ull;
+    if (op.code <= kCylinder) {
+      float vlo, vhi;
+      op_interval(op, cl, ch, &vlo, &vhi);
+      if (!B.join(op.combine, op.k, vlo, vhi, active, &matters)) continue;
+    } else if (op.code == kPushTranslate) {
+      scopes.push(i);
+      enter_scope(ops, i, cl, ch);
+    } else if (op.code == kPopTranslate) {
+      if (scopes.depth == 0) continue;
+      scopes.pop();
+      restore_scopes(ops, scopes, blo, bhi, cl, ch);
+    } else if (kStack) {
+      B.operate(op.code, op.k);
+    }
+    if (lane == (count & 63)) {
+      my_op = i;
+      my_mask = matters;
+    }
+    ++count;
+    if (list && (count & 63) == 0) {
+      list[count - 64 + lane] = static_cast<uint16_t>(my_op);
+      mask[count - 64 + lane] = my_mask;
+    }
+  }
+  if (list && lane < (count & 63)) {
+    list[(count & ~63) + lane] = static_cast<uint16_t>(my_op);
+    mask[(count & ~63) + lane] = my_mask;
+  }
+  *out_lo = B.lo;
+  *out_hi = B.hi;
+  return count;
+}
+
+__device__ __forceinline__ float flip_sign(float x, uint32_t bit) {
+  return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) ^ bit);
+}
+
+// sdf_eval at K points a lane (inside the leading scopes) over the operations
+// named by `list` (m of them; list null: the operations [first, first + m)),
+// without those whose mask has none of the bits of `bricks`.  All arguments
+// but the points are the same for every lane.  The K points share each
+// operation's load and dispatch, whose scalar work and latency are otherwise
+// as long as one point's arithmetic.
+template <int K, bool kStack>
+__device__ __forceinline__ void sdf_eval_list(OpsPtr ops, int first, const uint16_t* list,
+                                              const uint64_t* mask, uint64_t bricks, int m,
+                                              const float (&p)[K][3], float (&top)[K]) {
+  const int lane = __lane_id();
+  ShiftStack st[K];
+  float c[K][3];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    top[k] = kNoBound;  // min(kNoBound, v) is v: the first push is read as a min
+#pragma unroll
+    for (int i = 0; i < kMaxValueStack; ++i) st[k].v[i] = 0.0f;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) c[k][a] = p[k][a];
+  }
+  ScopeStack scopes;
+  bool have_top = false;
+  for (int base = 0; base < m; base += 64) {
+    int mine = first + base + lane;
+    bool use = base + lane < m;
+    if (list && use) {
+      mine = list[base + lane];
+      use = (mask[base + lane] & bricks) != 0ull;
+    }
+    uint64_t todo = __ballot(use);
+    while (todo) {
+      const int i = __builtin_amdgcn_readlane(mine, static_cast<int>(__builtin_ctzll(todo)));
+      todo &= todo - 1;
+      const DevOp op = load_op(ops, i);
+      const uint32_t code = op.code;
+      if (code <= kCylinder) {
+        float q[K][3], v[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+#pragma unroll
+          for (int a = 0; a < 3; ++a) q[k][a] = c[k][a] - op.off[a];  // (x - 0 is x)
+        prim_values(code, op.prm, q, v);
+        const uint32_t mode = op.combine;
+        if (kStack && mode == kPush) {
+#pragma unroll
+          for (int k = 0; k < K; ++k) {
+            if (have_top) st[k].push(top[k]);
+            top[k] = v[k];
+          }
+          have_top = true;
+        } else if (mode == kMin || (!kStack && mode == kPush)) {
+#pragma unroll
+          for (int k = 0; k < K; ++k) top[k] = fminf(top[k], v[k]);
+        } else if (mode == kSmooth) {
+#pragma unroll
+          for (int k = 0; k < K; ++k) top[k] = smooth_min(top[k], v[k], op.k);
+        } else {
+          // max(top, v), max(v, -top) or max(top, -v)
+          const uint32_t nt = mode == kDiff ? 0x80000000u : 0u;
+          const uint32_t nv = mode == kDiffRev ? 0x80000000u : 0u;
+#pragma unroll
+          for (int k = 0; k < K; ++k)
+            top[k] = fmaxf(flip_sign(top[k], nt), flip_sign(v[k], nv));
+        }
+      } else if (code == kPushTranslate) {
+        scopes.push(i);
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+#pragma unroll
+          for (int a = 0; a < 3; ++a) c[k][a] = c[k][a] - op.off[a];
+      } else if (code == kPopTranslate) {
+        if (scopes.depth == 0) continue;
+        scopes.pop();
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+#pragma unroll
+          for (int a = 0; a < 3; ++a) c[k][a] = p[k][a];
+        for (int s = 0; s < scopes.depth; ++s) {
+          const int o = scopes.at(s);
+#pragma unroll
+          for (int k = 0; k < K; ++k)
+#pragma unroll
+            for (int a = 0; a < 3; ++a) c[k][a] = c[k][a] - ops[o].off[a];
+        }
+      } else if (kStack) {
+        const uint32_t nw = code == kDifference ? 0x80000000u : 0u;
+        const uint32_t nt = code == kDifferenceRev ? 0x80000000u : 0u;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          const float w = st[k].pop();
+          if (code == kUnion)
+            top[k] = fminf(w, top[k]);
+          else if (code == kSmoothUnion)
+            top[k] = smooth_min(w, top[k], op.k);
+          else  // max(w, t), max(t, -w) or max(w, -t)
+            top[k] = fmaxf(flip_sign(w, nw), flip_sign(top[k], nt));
+        }
+      }
+    }
+  }
+}
+
+}  // namespace iso

@@ -1,0 +1,47 @@
+// Launch interface of sparse program classification (sparse_kernels.hip).
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "mc_kernels.h"
+#include "sdf_program.h"
+
+namespace iso {
+
+// A tile: 16^3 samples, in 64 bricks of 4^3.
+constexpr int kTileShift = 4;
+constexpr int kTileSide = 1 << kTileShift;
+
+// Whether interval bounds of the program over this lattice are sound: every
+// parameter and coordinate is finite and far from overflowing a square.
+bool program_bounded(const DevOp* ops, int n_ops);
+bool lattice_bounded(const Lattice& L);
+// Whether the program holds values below the running one.
+bool program_needs_stack(const DevOp* ops, int n_ops);
+
+// Whether a program lattice is classified sparsely: sound bounds, rows of at
+// least one tile (narrower ones would leave most of a tile and of a sign word
+// empty), and enough samples.  On a small lattice a tile spans many operands
+// and few tiles run, so the dense pass is the faster one: whole extractions,
+// dense / sparse, of 64 spheres minus a torus take 68 / 94 us at 65^3, 83 / 83
+// at 81^3, 102 / 77 at 97^3 and 158 / 74 at 129^3, and of a torus alone 36 /
+// 38, 39 / 44, 41 / 41 and 46 / 42.
+constexpr int64_t kSparseMinPoints = 786432;  // 92^3
+inline bool sparse_lattice(const Lattice& L, bool program_is_bounded) {
+  return L.nx >= kTileSide && L.nx * L.ny * L.nz >= kSparseMinPoints && program_is_bounded &&
+         lattice_bounded(L);
+}
+
+// Tiles of a lattice.
+int64_t tile_count(int64_t nx, int64_t ny, int64_t nz);
+
+// Program signs like launch_signs_program, from dims of mc_dims_pitched:
+// bounds prove the sign of whole 4^3 bricks of samples, and only the bricks
+// they cannot prove are evaluated (their samples go to `values` when it is
+// not null).  Every lattice edge that crosses the surface has both its ends
+// in evaluated bricks, and every sign is the evaluated program's.
+// Program and lattice must be bounded; `stack`: program_needs_stack.
+hipError_t launch_signs_sparse(const DevOp* ops, int n_ops, bool stack, const Lattice& L,
+                               const McDims& D, const McBuffers& B, float* values, hipStream_t s);
+
+}  // namespace iso

@@ -1,0 +1,322 @@
+// Sparse classification of program sources for gfx950 (MI355X).
+//
+// Marching cubes reads a sample's value only at the ends of an edge that
+// crosses the surface, and everywhere else only its sign.  A wavefront takes
+// a tile of 16^3 samples, one lane for each of its 64 bricks of 4^3, and
+// bounds the program over each brick's samples and their lattice neighbours
+// (the box one sample wider on every side): where the bounds exclude zero,
+// the sign of all of them is proven.  A crossing edge joins two neighbouring
+// samples of different sign, so neither of them lies in a proven brick: the
+// evaluated bricks hold every value that is read.  The same pass lists the
+// operations that can change the program's value anywhere in the tile
+// (sparse_eval.h), and the unproven bricks are evaluated over that list, 64
+// samples a wavefront.  Signs and values are the dense evaluation's, bit for
+// bit.
+//
+// The sign words are row-aligned (each sample row starts a new word), so a
+// tile's 16 samples of a row are one 16-bit store and no two tiles share a
+// piece; the count and emit kernels take the row pitch from the CellSpace.
+//
+// Bound by instruction issue and the latency of one tile's chain (bounds of the
+// tile, of its bricks, then its bricks' samples), not by memory: 64 spheres
+// minus a torus at 257^3 evaluate 25,437 of 274,625 bricks over 8 operations
+// each and take 44 us, where evaluating every sample took 617 us.
+#include <hip/hip_ext.h>
+#include <hip/hip_runtime.h>
+
+#include <cmath>
+
+#include "mc_device.h"
+#include "mc_kernels.h"
+#include "sparse_eval.h"
+#include "sparse_kernels.h"
+
+namespace iso {
+
+namespace {
+
+using namespace mcd;
+
+constexpr int kBricks = 64;      // bricks of a tile: 4 x 4 x 4
+constexpr int kTileCoords = kTileSide + 2;  // coordinates along an axis, neighbours included
+constexpr int kListCap = 512;    // operations of a tile's list; a longer one is not kept
+constexpr uint32_t kSparseXcds = 8;
+
+// A barrier for what the tile's wavefronts exchange in LDS: __syncthreads
+// would also wait for the samples on their way to memory (two microseconds a
+// tile).
+template <int W>
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  if (W > 1) __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// One lattice: its tiles x fastest.
+struct SingleTiles {
+  CellSpace C;
+  __device__ __forceinline__ const CellSpace& at(uint32_t tile, uint32_t* local) const {
+    *local = tile;
+    return C;
+  }
+};
+
+// W wavefronts per tile: one where tiles alone fill the chip, four where a
+// small lattice leaves it idle (the bricks of a tile are then spread over
+// four SIMDs; the bounds are one wavefront's work either way).
+template <class Tiles, int W, bool kStack>
+__global__ __launch_bounds__(64 * W) void k_signs_sparse(Tiles tiles, uint32_t n_tiles,
+                                                         uint32_t group, ResetArgs R) {
+  __shared__ uint64_t s_sign[kBricks];  // sign bits of a brick's samples, x fastest
+  __shared__ uint16_t s_list[kListCap];  // operations that matter in the tile
+  __shared__ uint64_t s_mask[kListCap];  // and the bricks each of them matters in
+  __shared__ float s_coord[3 * kTileCoords];
+  __shared__ int s_len;
+  __shared__ uint64_t s_todo;
+  reset_state(R);
+  // Groups of consecutive tiles (a row's neighbours share lines of sign words
+  // and values) go to one XCD, the groups round robin.
+  const uint32_t q = blockIdx.x / kSparseXcds;
+  const uint32_t tile =
+      ((q / group) * kSparseXcds + blockIdx.x % kSparseXcds) * group + q % group;
+  if (tile >= n_tiles) return;
+  uint32_t local;
+  const CellSpace& C = tiles.at(tile, &local);
+  const int32_t nx = static_cast<int32_t>(C.nx), ny = static_cast<int32_t>(C.ny),
+                nz = static_cast<int32_t>(C.nz);
+  const int32_t n[3] = {nx, ny, nz};
+  const uint32_t ntx = static_cast<uint32_t>(nx + kTileSide - 1) >> kTileShift;
+  const uint32_t nty = static_cast<uint32_t>(ny + kTileSide - 1) >> kTileShift;
+  const uint32_t tz = local / (ntx * nty);
+  const uint32_t tr = local - tz * (ntx * nty);
+  const uint32_t ty = tr / ntx;
+  const uint32_t tx = tr - ty * ntx;
+  const int32_t s0[3] = {static_cast<int32_t>(tx << kTileShift),
+                         static_cast<int32_t>(ty << kTileShift),
+                         static_cast<int32_t>(tz << kTileShift)};
+  const OpsPtr ops = as_constant(C.ops);
+  const int n_ops = C.n_ops;
+  const int lane = __lane_id();
+  const int wv = W == 1 ? 0 : static_cast<int>(threadIdx.x >> 6);
+  const int first = leading_scopes(ops, n_ops);
+
+  if (wv == 0) {
+    // Coordinates of the tile's samples and its neighbours' along each axis,
+    // inside the program's leading scopes (past the lattice: the last sample's).
+    if (lane < 3 * kTileCoords) {
+      const int a = lane / kTileCoords;
+      const int32_t na = a == 0 ? nx : a == 1 ? ny : nz;
+      int32_t i = (a == 0 ? s0[0] : a == 1 ? s0[1] : s0[2]) + lane - kTileCoords * a - 1;
+      i = i < 0 ? 0 : i < na ? i : na - 1;
+      const float o = a == 0 ? C.origin[0] : a == 1 ? C.origin[1] : C.origin[2];
+      const float d = a == 0 ? C.spacing[0] : a == 1 ? C.spacing[1] : C.spacing[2];
+      float x = o + static_cast<float>(i) * d;  // as the dense kernels compute it
+      for (int s = 0; s < first; ++s)
+        x = x - (a == 0 ? ops[s].off[0] : a == 1 ? ops[s].off[1] : ops[s].off[2]);
+      s_coord[lane] = x;
+    }
+    lds_barrier<1>();
+    // The tile's bounds first: most tiles are proven here.
+    float blo[3], bhi[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const float c0 = s_coord[kTileCoords * a], c1 = s_coord[kTileCoords * a + kTileCoords - 1];
+      blo[a] = fminf(c0, c1);
+      bhi[a] = fmaxf(c0, c1);
+    }
+    float lo, hi;
+    int len = bound_box<kStack>(ops, first, n_ops, blo, bhi, s_list, kListCap, &lo, &hi);
+    bool outside = lo > 0.0f, inside = hi <= 0.0f;
+    bool active = true;
+    if (!outside && !inside) {
+      // Then its bricks', each with its samples' neighbours.
+      const int b[3] = {lane & 3, (lane >> 2) & 3, lane >> 4};
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        active = active && s0[a] + 4 * b[a] < n[a];
+        const float c0 = s_coord[kTileCoords * a + 4 * b[a]];
+        const float c1 = s_coord[kTileCoords * a + 4 * b[a] + 5];
+        blo[a] = fminf(c0, c1);
+        bhi[a] = fmaxf(c0, c1);
+      }
+      lds_barrier<1>();
+      const bool fits = len <= kListCap;
+      const int left = bound_lanes<kStack>(ops, first, fits ? len : n_ops - first, blo, bhi,
+                                           active, fits ? s_list : nullptr, s_mask, &lo, &hi);
+      if (fits) len = left;
+      outside = lo > 0.0f;
+      inside = hi <= 0.0f;
+    }
+    s_sign[lane] = inside ? ~0ull : 0ull;
+    const uint64_t todo = __ballot(active && !outside && !inside);
+    if (lane == 0) {
+      s_len = len;
+      s_todo = todo;
+    }
+  }
+  lds_barrier<W>();
+  const int len = __builtin_amdgcn_readfirstlane(s_len);
+  uint64_t todo;
+  {
+    const uint64_t t = s_todo;
+    todo = static_cast<uint64_t>(static_cast<uint32_t>(
+               __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(t)))) |
+           (static_cast<uint64_t>(static_cast<uint32_t>(
+                __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(t >> 32))))
+            << 32);
+  }
+  const uint16_t* list = len <= kListCap ? s_list : nullptr;
+  const int m = len <= kListCap ? len : n_ops - first;
+  const int lx = lane & 3, ly = (lane >> 2) & 3, lz = lane >> 4;
+  const bool full = s0[0] + kTileSide <= nx && s0[1] + kTileSide <= ny && s0[2] + kTileSide <= nz;
+  // A lane's sample within its brick (lattices have less than 2^32 samples).
+  const uint32_t within = (static_cast<uint32_t>(lz) * static_cast<uint32_t>(ny) +
+                           static_cast<uint32_t>(ly)) * static_cast<uint32_t>(nx) +
+                          static_cast<uint32_t>(lx);
+  constexpr int kPoints = kStack ? 2 : 4;
+  // kPoints bricks a round, the wavefronts' rounds interleaved.
+  for (int k = 0; todo; ++k) {
+    int brick[kPoints];
+    uint32_t have = 0;
+    uint64_t bricks = 0;
+#pragma unroll
+    for (int j = 0; j < kPoints; ++j) {
+      brick[j] = j ? brick[0] : 0;
+      if (todo) {
+        brick[j] = static_cast<int>(__builtin_ctzll(todo));
+        bricks |= todo & (0ull - todo);
+        todo &= todo - 1;
+        have |= 1u << j;
+      }
+    }
+    if (W > 1 && (k & (W - 1)) != wv) continue;
+    float p[kPoints][3], v[kPoints];
+#pragma unroll
+    for (int j = 0; j < kPoints; ++j) {
+      const int b = brick[j];
+      p[j][0] = s_coord[1 + 4 * (b & 3) + lx];
+      p[j][1] = s_coord[kTileCoords + 1 + (b & 12) + ly];
+      p[j][2] = s_coord[2 * kTileCoords + 1 + 4 * (b >> 4) + lz];
+    }
+    sdf_eval_list<kPoints, kStack>(ops, first, list, s_mask, bricks, m, p, v);
+    uint64_t mine = 0;
+#pragma unroll
+    for (int j = 0; j < kPoints; ++j) {
+      const int b = brick[j];
+      const int32_t x0 = s0[0] + 4 * (b & 3), y0 = s0[1] + (b & 12), z0 = s0[2] + 4 * (b >> 4);
+      const bool valid = full || (x0 + lx < nx && y0 + ly < ny && z0 + lz < nz);
+      if (C.grid && valid && ((have >> j) & 1u)) {
+        float* at = const_cast<float*>(C.grid) + (static_cast<int64_t>(z0) * ny + y0) * nx + x0;
+        at[within] = v[j];
+      }
+      // classify_corners, distance.rs:52-54
+      const uint64_t in = __ballot(valid && !(v[j] > 0.0f));
+      if (lane == j) mine = in;
+    }
+    // (a spare point repeats the first brick)
+    int slot = brick[0];
+#pragma unroll
+    for (int j = 1; j < kPoints; ++j) slot = lane == j ? brick[j] : slot;
+    if (lane < kPoints) s_sign[slot] = mine;
+  }
+  lds_barrier<W>();
+  // The tile's rows: 16 bits of row (y, z), four from each brick along x.
+  uint16_t* S = reinterpret_cast<uint16_t*>(const_cast<uint64_t*>(C.signs));
+  for (int r = threadIdx.x; r < kTileSide * kTileSide; r += 64 * W) {
+    const int ry = r & (kTileSide - 1), rz = r >> kTileShift;
+    const int32_t y = s0[1] + ry, z = s0[2] + rz;
+    if (y >= ny || z >= nz) continue;
+    const int b0 = (rz >> 2) * 16 + (ry >> 2) * 4;
+    const int sh = 16 * (rz & 3) + 4 * (ry & 3);
+    uint32_t bits = 0;
+#pragma unroll
+    for (int bx = 0; bx < 4; ++bx)
+      bits |= static_cast<uint32_t>((s_sign[b0 + bx] >> sh) & 0xFull) << (4 * bx);
+    S[(static_cast<int64_t>(z) * ny + y) * (C.sign_pitch >> 4) + tx] = static_cast<uint16_t>(bits);
+  }
+}
+
+// Blocks that cover n tiles in groups dealt to the XCDs round robin.
+uint64_t sparse_blocks(uint64_t n_tiles, uint64_t group) {
+  const uint64_t per = kSparseXcds * group;
+  return (n_tiles + per - 1) / per * per;
+}
+
+template <class Kernel, class Tiles>
+hipError_t launch_tiles(Kernel kernel, int threads, const Tiles& tiles, int64_t n_tiles,
+                        int64_t group, const ResetArgs& R, hipStream_t s) {
+  const uint64_t blocks = sparse_blocks(static_cast<uint64_t>(n_tiles), static_cast<uint64_t>(group));
+  if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
+  hipEvent_t a, z;
+  if (take_launch_events(&a, &z))
+    hipExtLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)),
+                          dim3(static_cast<unsigned>(threads)), 0, s, a, z, 0, tiles,
+                          static_cast<uint32_t>(n_tiles), static_cast<uint32_t>(group), R);
+  else
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)),
+                       dim3(static_cast<unsigned>(threads)), 0, s, tiles,
+                       static_cast<uint32_t>(n_tiles), static_cast<uint32_t>(group), R);
+  return hipGetLastError();
+}
+
+// Tiles from which one wavefront each is the better split.  Kernel times with
+// one / four wavefronts a tile, 64 spheres minus a torus: 75 / 44 us at 257^3
+// (4913 tiles), 87 / 83 at 385^3 (15625), 119 / 151 at 513^3 (35937).
+constexpr int64_t kManyTiles = 16384;
+
+// Parameters and coordinates below this: no square or sum of squares of a
+// primitive's operands overflows.
+constexpr float kBoundedMagnitude = 1.0e15f;
+
+bool small(float v) { return std::fabs(v) < kBoundedMagnitude; }  // false for NaN
+
+}  // namespace
+
+bool program_bounded(const DevOp* ops, int n_ops) {
+  for (int i = 0; i < n_ops; ++i) {
+    if (!small(ops[i].k)) return false;
+    for (int j = 0; j < 4; ++j)
+      if (!small(ops[i].prm[j]) || !small(ops[i].off[j])) return false;
+  }
+  return true;
+}
+
+bool lattice_bounded(const Lattice& L) {
+  const int64_t n[3] = {L.nx, L.ny, L.nz};
+  for (int a = 0; a < 3; ++a)
+    if (!small(L.origin[a]) || !small(L.spacing[a] * static_cast<float>(n[a]))) return false;
+  return true;
+}
+
+int64_t tile_count(int64_t nx, int64_t ny, int64_t nz) {
+  return ((nx + kTileSide - 1) >> kTileShift) * ((ny + kTileSide - 1) >> kTileShift) *
+         ((nz + kTileSide - 1) >> kTileShift);
+}
+
+bool program_needs_stack(const DevOp* ops, int n_ops) {
+  int pushes = 0;
+  for (int i = 0; i < n_ops; ++i) pushes += ops[i].code <= kCylinder && ops[i].combine == kPush;
+  return pushes > 1;
+}
+
+hipError_t launch_signs_sparse(const DevOp* ops, int n_ops, bool stack, const Lattice& L,
+                               const McDims& D, const McBuffers& B, float* values, hipStream_t s) {
+  if (!ops || !B.signs || (D.sign_pitch & 63)) return hipErrorInvalidValue;
+  const SingleTiles t{single_cell_space(L, D, B.signs, ops, n_ops, values, nullptr)};
+  ResetArgs R;
+  R.signs = B.signs;
+  R.n_words = D.n_sign_words;
+  R.agg = B.agg;
+  R.incl = B.incl;
+  R.n_blocks = D.n_blocks;
+  R.totals = B.totals;
+  const int64_t n = tile_count(L.nx, L.ny, L.nz);
+  const int64_t group = (L.nx + kTileSide - 1) >> kTileShift;
+  if (n >= kManyTiles)
+    return stack ? launch_tiles(k_signs_sparse<SingleTiles, 1, true>, 64, t, n, group, R, s)
+                 : launch_tiles(k_signs_sparse<SingleTiles, 1, false>, 64, t, n, group, R, s);
+  return stack ? launch_tiles(k_signs_sparse<SingleTiles, 4, true>, 256, t, n, group, R, s)
+               : launch_tiles(k_signs_sparse<SingleTiles, 4, false>, 256, t, n, group, R, s);
+}
+
+}  // namespace iso
