@@ -93,7 +93,7 @@ struct iso_ctx {
   unsigned long long* h_stage = nullptr;  // pinned, 8 words
 
   // batched chunks: lowered programs, chunk table, sign words, offsets
-  DevBuf b_ops, b_chunks, b_segstart, b_wordstart, b_signs, b_voff, b_ioff, b_values;
+  DevBuf b_ops, b_chunks, b_segstart, b_wordstart, b_tilestart, b_signs, b_voff, b_ioff, b_values;
   iso::BatchPlan plan{};
   uint64_t b_cells = 0;
   bool b_ready = false;
@@ -370,7 +370,7 @@ int iso_ctx_destroy(iso_ctx* c) {
                     &c->oc_plevel,  &c->oc_corner,  &c->oc_case,   &c->oc_base,  &c->oc_tkeys,
                     &c->oc_towner,  &c->oc_tid,     &c->sc_slot,   &c->sc_ctl,
                     &c->oc_pkeys,   &c->oc_plevels, &c->oc_skeys,  &c->oc_slevels, &c->oc_sort,
-                    &c->b_ops,      &c->b_chunks,   &c->b_segstart, &c->b_wordstart,
+                    &c->b_ops,      &c->b_chunks,   &c->b_segstart, &c->b_wordstart, &c->b_tilestart,
                     &c->b_signs,    &c->b_voff,     &c->b_ioff,    &c->b_values,
                     &c->nn_theta,   &c->nn_m,
                     &c->nn_v,       &c->nn_grad,    &c->nn_frags,  &c->nn_loss,  &c->nn_x,
@@ -1660,9 +1660,10 @@ int iso_batch_upload(iso_ctx* c, const iso_node* nodes, uint64_t n_nodes,
     c->b_graph = nullptr;
   }
   std::vector<iso::DevOp> ops;
-  std::vector<uint32_t> op_off(n_chunks), seg_start(n_chunks + 1);
-  std::vector<uint64_t> word_start(n_chunks + 1), sign_off(n_chunks);
-  uint64_t segs = 0, words = 0, sign_words = 0, cells = 0;
+  std::vector<uint32_t> op_off(n_chunks), seg_start(n_chunks + 1), tile_start(n_chunks + 1);
+  std::vector<uint64_t> word_start(n_chunks + 1), sign_off(n_chunks), row_off(n_chunks);
+  uint64_t segs = 0, words = 0, sign_words = 0, row_words = 0, tiles = 0, cells = 0;
+  bool bounded = true, stack = false;
   for (uint32_t i = 0; i < n_chunks; ++i) {
     const iso_chunk_desc& ch = chunks[i];
     iso::Lattice L;
@@ -1680,19 +1681,36 @@ int iso_batch_upload(iso_ctx* c, const iso_node* nodes, uint64_t n_nodes,
     op_off[i] = static_cast<uint32_t>(ops.size());
     ops.insert(ops.end(), part.begin(), part.end());
     const iso::McDims D = iso::mc_dims(L);
+    const int n_part = static_cast<int>(part.size());
+    bounded = bounded && iso::program_bounded(part.data(), n_part) && iso::lattice_bounded(L);
+    stack = stack || iso::program_needs_stack(part.data(), n_part);
     seg_start[i] = static_cast<uint32_t>(segs);
     word_start[i] = words;
-    sign_off[i] = sign_words + 1;  // one guard word before, two after
+    tile_start[i] = static_cast<uint32_t>(tiles);
+    // one guard word before, two after
+    sign_off[i] = sign_words + 1;
+    row_off[i] = row_words + 1;
     segs += static_cast<uint64_t>(D.n_segs);
     words += static_cast<uint64_t>(D.n_sign_words);
     sign_words += static_cast<uint64_t>(D.n_sign_words) + 3;
+    row_words += static_cast<uint64_t>(iso::mc_dims_pitched(L).n_sign_words) + 3;
+    tiles += static_cast<uint64_t>(iso::tile_count(L.nx, L.ny, L.nz));
     cells += static_cast<uint64_t>(D.n_cells);
     if (segs >= (1ull << 26))
       return fail(c, ISO_ERR_INVALID_ARGUMENT, "batch has 2^26 or more 64-cell segments");
   }
   seg_start[n_chunks] = static_cast<uint32_t>(segs);
   word_start[n_chunks] = words;
+  tile_start[n_chunks] = static_cast<uint32_t>(tiles);
+  // Sparse classification unless bounds are not sound somewhere, or the rows
+  // are so narrow that row-aligned words would be mostly padding.
+  const bool sparse = bounded && row_words <= 8 * sign_words && tiles < (1ull << 30);
+  if (sparse) {
+    sign_words = row_words;
+    sign_off = row_off;
+  }
   ISO_HIP(c, ensure(&c->b_ops, ops.size() * sizeof(iso::DevOp)));
+  ISO_HIP(c, ensure(&c->b_tilestart, (n_chunks + 1) * sizeof(uint32_t)));
   ISO_HIP(c, ensure(&c->b_signs, sign_words * sizeof(uint64_t)));
   ISO_HIP(c, ensure(&c->b_chunks, n_chunks * sizeof(iso::CellSpace)));
   ISO_HIP(c, ensure(&c->b_segstart, (n_chunks + 1) * sizeof(uint32_t)));
@@ -1720,7 +1738,7 @@ int iso_batch_upload(iso_ctx* c, const iso_node* nodes, uint64_t n_nodes,
       C.spacing[k] = g.spacing[k];
     }
     C.signs = dsigns + sign_off[i];
-    C.sign_pitch = g.nx;
+    C.sign_pitch = sparse ? (g.nx + 63) / 64 * 64 : g.nx;
     C.segs_per_row = static_cast<uint32_t>((g.nx - 1 + 63) / 64);
     C.seg_off = seg_start[i];
     C.ops = dops + op_off[i];
@@ -1735,7 +1753,13 @@ int iso_batch_upload(iso_ctx* c, const iso_node* nodes, uint64_t n_nodes,
                             hipMemcpyHostToDevice, c->stream));
   ISO_HIP(c, hipMemcpyAsync(c->b_wordstart.ptr, word_start.data(),
                             (n_chunks + 1) * sizeof(uint64_t), hipMemcpyHostToDevice, c->stream));
+  ISO_HIP(c, hipMemcpyAsync(c->b_tilestart.ptr, tile_start.data(),
+                            (n_chunks + 1) * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
   ISO_HIP(c, hipStreamSynchronize(c->stream));
+  c->plan.sparse = sparse;
+  c->plan.stack = stack;
+  c->plan.tile_start = static_cast<const uint32_t*>(c->b_tilestart.ptr);
+  c->plan.n_tiles = static_cast<int64_t>(tiles);
   c->plan.chunks = static_cast<const iso::CellSpace*>(c->b_chunks.ptr);
   c->plan.seg_start = static_cast<const uint32_t*>(c->b_segstart.ptr);
   c->plan.word_start = static_cast<const uint64_t*>(c->b_wordstart.ptr);
@@ -1808,7 +1832,7 @@ int autotune_batch(iso_ctx* c, const iso::McBuffers& B) {
   }
   c->b_rounds = br;
   for (int w : wpw) {
-    if (st != ISO_OK) break;
+    if (st != ISO_OK || c->plan.sparse) break;  // the sparse pass has no such shape
     c->b_words_per_wave = w;
     float ms;
     if ((st = measure(&ms)) != ISO_OK) break;

@@ -81,6 +81,30 @@ struct CellSpace {
   const float* positions;   // per-point vertex positions, or null
 };
 
+// Entry i (the same for every lane) of a chunk table, by scalar loads.
+__device__ __forceinline__ CellSpace load_space(const CellSpace* table, uint32_t i) {
+  using Space = const CellSpace __attribute__((address_space(4)))*;
+  const Space t = (Space)(reinterpret_cast<uintptr_t>(table)) + i;
+  CellSpace C;
+  C.nx = t->nx;
+  C.ny = t->ny;
+  C.nz = t->nz;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    C.origin[a] = t->origin[a];
+    C.spacing[a] = t->spacing[a];
+  }
+  C.signs = t->signs;
+  C.sign_pitch = t->sign_pitch;
+  C.segs_per_row = t->segs_per_row;
+  C.seg_off = t->seg_off;
+  C.ops = t->ops;
+  C.n_ops = t->n_ops;
+  C.reserved = t->reserved;
+  C.grid = t->grid;
+  C.positions = t->positions;
+  return C;
+}
 // The CellSpace of a single lattice.
 CellSpace single_cell_space(const Lattice& L, const McDims& D, const uint64_t* signs,
                             const DevOp* ops, int n_ops, const float* grid,
@@ -169,6 +193,13 @@ struct BatchPlan {
   // program's samples there and emit reads them.  False: no such buffer,
   // emit evaluates the programs at the edge endpoints.
   bool stored_values;
+  // Sparse classification (sparse_kernels.hip): the chunks' sign words are
+  // row-aligned and their programs and lattices bounded; otherwise the flat
+  // words of every sample.
+  bool sparse;
+  bool stack;                  // a chunk's program needs a value stack
+  const uint32_t* tile_start;  // device, n_chunks + 1: first tile of each chunk
+  int64_t n_tiles;
 };
 
 // Count workgroups of a batch at `rounds` segments per thread (1 or 2).

@@ -34,6 +34,7 @@
 #include "mc_kernels.h"
 #include "mc_tables.h"
 #include "sdf_eval.h"
+#include "sparse_kernels.h"
 
 namespace iso {
 
@@ -242,19 +243,30 @@ struct SingleSpace {
   }
 };
 
-// A batch: the chunk owning global segment g is found by binary search over
-// the chunks' first segments.
+// A batch: the chunk owning global segment g.  A wavefront's segments ascend
+// with the lane and mostly lie in one chunk: the first lane's chunk is found by
+// a binary search in scalar loads, the others step on from it, and one chunk's
+// record is read by scalar loads too.
 struct BatchSpace {
   const CellSpace* chunks;
   const uint32_t* seg_start;  // n_chunks + 1 ascending first segments
   uint32_t n_chunks;
   __device__ __forceinline__ CellSpace at(uint32_t g, uint32_t* local) const {
-    uint32_t lo = 0, hi = n_chunks;  // last chunk with seg_start <= g
-    while (hi - lo > 1) {
-      const uint32_t mid = (lo + hi) >> 1;
-      if (seg_start[mid] <= g) lo = mid;
+    using U32 = const uint32_t __attribute__((address_space(4)))*;
+    const U32 first = (U32)(reinterpret_cast<uintptr_t>(seg_start));
+    const uint32_t g0 = __builtin_amdgcn_readfirstlane(g);
+    uint32_t lo0 = 0, hi = n_chunks;  // last chunk whose first segment <= g0
+    while (hi - lo0 > 1) {
+      const uint32_t mid = (lo0 + hi) >> 1;
+      if (first[mid] <= g0) lo0 = mid;
       else hi = mid;
     }
+    if (__ballot(lo0 + 1 < n_chunks && first[lo0 + 1] <= g) == 0ull) {
+      *local = g - first[lo0];
+      return load_space(chunks, lo0);
+    }
+    uint32_t lo = lo0;
+    while (lo + 1 < n_chunks && seg_start[lo + 1] <= g) ++lo;
     *local = g - seg_start[lo];
     return chunks[lo];
   }
@@ -1191,6 +1203,7 @@ hipError_t launch_batch_signs(const BatchPlan& P, const McBuffers& B, int words_
                               hipStream_t s) {
   // The state reset covers the look-back words of the finest count tile.
   const int64_t n_blocks = batch_count_blocks(P, 1);
+  if (P.sparse) return launch_batch_signs_sparse(P, B, n_blocks, s);
   ResetArgs R;
   R.signs = nullptr;
   R.n_words = 0;

@@ -44,4 +44,9 @@ int64_t tile_count(int64_t nx, int64_t ny, int64_t nz);
 hipError_t launch_signs_sparse(const DevOp* ops, int n_ops, bool stack, const Lattice& L,
                                const McDims& D, const McBuffers& B, float* values, hipStream_t s);
 
+// The same for every chunk of a batch (P.sparse), and the extraction's state
+// reset for n_blocks look-back words.
+hipError_t launch_batch_signs_sparse(const BatchPlan& P, const McBuffers& B, int64_t n_blocks,
+                                     hipStream_t s);
+
 }  // namespace iso

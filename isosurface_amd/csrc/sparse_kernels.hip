@@ -61,6 +61,27 @@ struct SingleTiles {
   }
 };
 
+// A batch: the chunk that holds a tile is found by binary search of the
+// chunks' first tiles.  The table is read through the constant address space:
+// scalar loads, as the index is the same for the whole workgroup.
+struct BatchTiles {
+  const CellSpace* chunks;
+  const uint32_t* tile_start;
+  uint32_t n_chunks;
+  __device__ __forceinline__ CellSpace at(uint32_t tile, uint32_t* local) const {
+    using U32 = const uint32_t __attribute__((address_space(4)))*;
+    const U32 first = (U32)(reinterpret_cast<uintptr_t>(tile_start));
+    uint32_t lo = 0, hi = n_chunks;  // last chunk whose first tile <= tile
+    while (hi - lo > 1) {
+      const uint32_t mid = (lo + hi) >> 1;
+      if (first[mid] <= tile) lo = mid;
+      else hi = mid;
+    }
+    *local = tile - first[lo];
+    return load_space(chunks, lo);
+  }
+};
+
 // W wavefronts per tile: one where tiles alone fill the chip, four where a
 // small lattice leaves it idle (the bricks of a tile are then spread over
 // four SIMDs; the bounds are one wavefront's work either way).
@@ -81,7 +102,7 @@ __global__ __launch_bounds__(64 * W) void k_signs_sparse(Tiles tiles, uint32_t n
       ((q / group) * kSparseXcds + blockIdx.x % kSparseXcds) * group + q % group;
   if (tile >= n_tiles) return;
   uint32_t local;
-  const CellSpace& C = tiles.at(tile, &local);
+  const auto& C = tiles.at(tile, &local);
   const int32_t nx = static_cast<int32_t>(C.nx), ny = static_cast<int32_t>(C.ny),
                 nz = static_cast<int32_t>(C.nz);
   const int32_t n[3] = {nx, ny, nz};
@@ -317,6 +338,25 @@ hipError_t launch_signs_sparse(const DevOp* ops, int n_ops, bool stack, const La
                  : launch_tiles(k_signs_sparse<SingleTiles, 1, false>, 64, t, n, group, R, s);
   return stack ? launch_tiles(k_signs_sparse<SingleTiles, 4, true>, 256, t, n, group, R, s)
                : launch_tiles(k_signs_sparse<SingleTiles, 4, false>, 256, t, n, group, R, s);
+}
+
+hipError_t launch_batch_signs_sparse(const BatchPlan& P, const McBuffers& B, int64_t n_blocks,
+                                     hipStream_t s) {
+  if (!P.sparse || !P.chunks || !P.tile_start) return hipErrorInvalidValue;
+  const BatchTiles t{P.chunks, P.tile_start, P.n_chunks};
+  ResetArgs R;
+  R.signs = nullptr;
+  R.n_words = 0;
+  R.agg = B.agg;
+  R.incl = B.incl;
+  R.n_blocks = n_blocks;
+  R.totals = B.totals;
+  constexpr int64_t kGroup = 4;  // about a row of a chunk's tiles
+  if (P.n_tiles >= kManyTiles)
+    return P.stack ? launch_tiles(k_signs_sparse<BatchTiles, 1, true>, 64, t, P.n_tiles, kGroup, R, s)
+                   : launch_tiles(k_signs_sparse<BatchTiles, 1, false>, 64, t, P.n_tiles, kGroup, R, s);
+  return P.stack ? launch_tiles(k_signs_sparse<BatchTiles, 4, true>, 256, t, P.n_tiles, kGroup, R, s)
+                 : launch_tiles(k_signs_sparse<BatchTiles, 4, false>, 256, t, P.n_tiles, kGroup, R, s);
 }
 
 }  // namespace iso

@@ -151,3 +151,19 @@ def device_mesh(ctx, d, flags, nv, ni):
         ctx.lib.iso_device_free(ctx.handle, v)
         ctx.lib.iso_device_free(ctx.handle, i)
     return hv, hi
+
+
+@pytest.mark.parametrize("unbounded", [False, True])
+def test_batches(ctx, unbounded):
+    """Chunks of every size class over trees with a value stack; one program
+    without sound bounds takes the whole batch to the dense pass."""
+    from isosurface_amd import BatchedMarchingCubes, chunk_desc
+    sizes = [15, 16, 2, 17, 31, 32, 3, 33, 48, 63, 64, 65, 1]
+    chunks = [(tree(20 + i, 5 + i % 4), chunk_desc(s)) for i, s in enumerate(sizes)]
+    if unbounded:
+        chunks[4] = (DemoSource(Intersection(Sphere(float("inf")), Sphere(0.4))), chunks[4][1])
+    meshes = BatchedMarchingCubes(ctx).extract_meshes(chunks)
+    for (src, d), m in zip(chunks, meshes):
+        ref = O.extract_mc(src.program(), desc=O.as_desc(d))
+        assert np.array_equal(m.indices, ref.indices)
+        assert m.vertices.tobytes() == ref.vertices.tobytes()
