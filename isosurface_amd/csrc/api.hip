@@ -63,8 +63,7 @@ struct iso_ctx {
   int n_prog = 0;
   bool prog_directed = false;  // the program has a directed form (no smooth union)
   bool prog_hermite = false;   // analytic normals exist (shapes, unions, translations)
-  bool prog_bounded = false;   // interval bounds of the program are sound
-  bool prog_stack = false;     // the program holds values below the running one
+  iso::ProgramKind prog_kind;  // what the sparse kernels ask of it
 
   // current grid
   DevBuf grid_owned;
@@ -102,7 +101,7 @@ struct iso_ctx {
   bool b_tuned = false;
   // learned narrow band: network, training batch, brick buffers, counters
   DevBuf nn_theta, nn_m, nn_v, nn_grad, nn_frags, nn_loss, nn_x, nn_h, nn_dz, nn_g, nn_pts, nn_t,
-      nn_w, nn_out, br_centres, br_hd, br_pred, br_flags, br_list, br_count, br_coarse, br_proof;
+      nn_w, nn_out, br_centres, br_hd, br_pred, br_flags, br_count, br_coarse, br_proof;
   bool nn_ready = false;
   uint32_t nn_step = 0;  // Adam steps taken
   int64_t nn_batch = 0;  // batch the activation buffers are sized for
@@ -376,7 +375,7 @@ int iso_ctx_destroy(iso_ctx* c) {
                     &c->nn_v,       &c->nn_grad,    &c->nn_frags,  &c->nn_loss,  &c->nn_x,
                     &c->nn_h,       &c->nn_dz,      &c->nn_g,      &c->nn_pts,   &c->nn_t,
                     &c->nn_w,       &c->nn_out,     &c->br_centres, &c->br_hd,   &c->br_pred,
-                    &c->br_flags,   &c->br_list,    &c->br_count,  &c->pvals,  &c->dense_check,  &c->nrm,
+                    &c->br_flags,   &c->br_count,  &c->pvals,  &c->dense_check,  &c->nrm,
                     &c->dgrid,      &c->dvals,      &c->emc_cells, &c->emc_first, &c->emc_cross,
                     &c->emc_flips,  &c->emc_ctr,    &c->br_coarse, &c->br_proof,
                     &c->f_signs,    &c->f_flags,    &c->f_slots,   &c->f_rowbase, &c->f_ctl};
@@ -421,8 +420,7 @@ int iso_program_upload(iso_ctx* c, const iso_node* nodes, uint32_t n_nodes) {
                             hipMemcpyHostToDevice, c->stream));
   ISO_HIP(c, hipStreamSynchronize(c->stream));
   c->n_prog = static_cast<int>(ops.size());
-  c->prog_bounded = iso::program_bounded(ops.data(), c->n_prog);
-  c->prog_stack = iso::program_needs_stack(ops.data(), c->n_prog);
+  c->prog_kind = iso::program_kind(ops.data(), c->n_prog);
   c->prog_directed = true;
   c->prog_hermite = true;
   for (uint32_t i = 0; i < n_nodes; ++i) {
@@ -622,8 +620,8 @@ int classify_and_count(iso_ctx* c, const float* grid, const iso::Lattice& L, con
                      [&] { return iso::launch_signs_grid(grid, L, D, B, c->stream); }));
   } else {
     ISO_HIP(c, timed(c, "mc_signs_program", [&] {
-              return iso::sparse_lattice(L, c->prog_bounded)
-                         ? iso::launch_signs_sparse(ops, c->n_prog, c->prog_stack, L, D, B, values,
+              return iso::sparse_lattice(L, c->prog_kind.bounded)
+                         ? iso::launch_signs_sparse(ops, c->n_prog, c->prog_kind.stack, L, D, B, values,
                                                     c->stream)
                          : iso::launch_signs_program(ops, c->n_prog, L, D, B, values, c->stream);
             }));
@@ -824,8 +822,10 @@ int extract_lattice(iso_ctx* c, const iso::Lattice& L, const float* grid, const 
     iso::FusedPlan P;
     if (iso::fused_plan(L, &P)) return extract_fused(c, L, grid, P, out);
   }
-  // Program signs are classified sparsely, into row-aligned sign words.
-  const bool sparse = !grid && !signs && iso::sparse_lattice(L, c->prog_bounded);
+  // Program signs are classified sparsely and a band's by tiles, into
+  // row-aligned sign words.
+  const bool sparse =
+      band || (!grid && !signs && iso::sparse_lattice(L, c->prog_kind.bounded));
   const iso::McDims D = sparse ? iso::mc_dims_pitched(L) : iso::mc_dims(L);
   if (D.n_segs >= (int64_t(1) << 26))
     return fail(c, ISO_ERR_INVALID_ARGUMENT, "lattice has 2^26 or more 64-cell segments");
@@ -874,7 +874,7 @@ int extract_lattice(iso_ctx* c, const iso::Lattice& L, const float* grid, const 
       k.ops = grid ? nullptr : ops;
       k.values = values;
       k.n_prog = grid ? 0 : c->n_prog;
-      k.program_kind = grid ? 0 : (c->prog_bounded ? 1 : 0) + (c->prog_stack ? 2 : 0);
+      k.program_kind = grid ? 0 : (c->prog_kind.bounded ? 1 : 0) + (c->prog_kind.stack ? 2 : 0);
       k.B = b;
       return k;
     };
@@ -1261,7 +1261,7 @@ int iso_extract_point_cloud(iso_ctx* c, const iso_grid_desc* desc, iso_mesh_out*
   c->band_valid = false;
   ISO_HIP(c, hipSetDevice(c->device));
   const iso::McDims D =
-      !from_grid && iso::sparse_lattice(L, c->prog_bounded) ? iso::mc_dims_pitched(L)
+      !from_grid && iso::sparse_lattice(L, c->prog_kind.bounded) ? iso::mc_dims_pitched(L)
                                                             : iso::mc_dims(L);
   if (D.n_segs >= (int64_t(1) << 26))
     return fail(c, ISO_ERR_INVALID_ARGUMENT, "lattice has 2^26 or more 64-cell segments");
@@ -2255,6 +2255,14 @@ int iso_band_predict(iso_ctx* c, const float* points, uint64_t n, float* out, in
   return ISO_OK;
 }
 
+// Words of the band's counters: bricks in the band, network culls overturned,
+// cells that differ from the dense classification; then the spread counters
+// of exact samples and of certificate centres.
+constexpr int kBandBricks = 0, kBandOverturned = 1, kBandDiffering = 2;
+constexpr int kBandSpread = iso::kCounterLines * iso::kCounterStride;
+constexpr int kBandExact = iso::kCounterStride, kBandCentre = kBandExact + kBandSpread;
+constexpr int kBandCounters = kBandCentre + kBandSpread;
+
 int iso_extract_mc_band(iso_ctx* c, const iso_grid_desc* desc, float margin, uint32_t flags,
                         iso_mesh_out* out, iso_band_stats* stats) {
   if (!c || !out) return fail(c, ISO_ERR_INVALID_ARGUMENT, "null argument");
@@ -2284,53 +2292,45 @@ int iso_extract_mc_band(iso_ctx* c, const iso_grid_desc* desc, float margin, uin
   ISO_HIP(c, ensure(&c->br_hd, nb * sizeof(float)));
   ISO_HIP(c, ensure(&c->br_pred, nb * sizeof(float)));
   ISO_HIP(c, ensure(&c->br_flags, nb));
-  ISO_HIP(c, ensure(&c->br_list, nb * sizeof(uint32_t)));
-  ISO_HIP(c, ensure(&c->br_count, 4 * sizeof(unsigned long long)));
+  ISO_HIP(c, ensure(&c->br_count, kBandCounters * sizeof(unsigned long long)));
   ISO_HIP(c, ensure(&c->br_coarse, static_cast<size_t>(G.nc)));
   ISO_HIP(c, ensure(&c->br_proof, nb));
   float* centres = static_cast<float*>(c->br_centres.ptr);
   float* hd = static_cast<float*>(c->br_hd.ptr);
   float* pred = static_cast<float*>(c->br_pred.ptr);
   uint8_t* bflags = static_cast<uint8_t*>(c->br_flags.ptr);
-  uint32_t* list = static_cast<uint32_t*>(c->br_list.ptr);
   uint8_t* coarse = static_cast<uint8_t*>(c->br_coarse.ptr);
   uint8_t* proof = static_cast<uint8_t*>(c->br_proof.ptr);
-  // counters: exact samples, (the dense check's), centre samples, overturned culls
   unsigned long long* counters = static_cast<unsigned long long*>(c->br_count.ptr);
-  iso::scan::State S{};
-  if ((st = prepare_scan(c, nb, &S)) != ISO_OK) return st;
-  ISO_HIP(c, iso::launch_fill_u32(reinterpret_cast<uint32_t*>(S.err), 2, 0u, c->stream));
-  ISO_HIP(c, iso::launch_fill_u32(reinterpret_cast<uint32_t*>(counters), 8, 0u, c->stream));
+  ISO_HIP(c, iso::launch_fill_u32(reinterpret_cast<uint32_t*>(counters), 2 * kBandCounters, 0u,
+                                  c->stream));
   const iso::DevOp* ops = static_cast<const iso::DevOp*>(c->prog.ptr);
   ISO_HIP(c, timed(c, "band_bricks", [&] {
             hipError_t e = iso::launch_brick_centres(L, G, centres, hd, c->stream);
             if (e == hipSuccess && use_network)
               e = iso::mlp::launch_forward(M, centres, static_cast<int64_t>(nb), pred, c->stream);
             if (e == hipSuccess && certify)
-              e = iso::launch_coarse_certify(ops, c->n_prog, L, G, coarse, counters + 2,
+              e = iso::launch_coarse_certify(ops, c->n_prog, L, G, coarse, counters + kBandCentre,
                                              c->stream);
             if (e == hipSuccess && certify)
-              e = iso::launch_brick_certify(ops, c->n_prog, L, G, coarse, centres, hd, proof,
-                                            counters + 2, c->stream);
+              e = iso::launch_brick_certify(ops, c->n_prog, c->prog_kind, L, G, coarse, centres, hd,
+                                            proof, counters + kBandCentre, c->stream);
             if (e == hipSuccess)
               e = iso::launch_brick_flags(G, use_network ? pred : nullptr, hd,
-                                          certify ? proof : nullptr, margin, bflags, list,
-                                          counters + 3, S, c->stream);
+                                          certify ? proof : nullptr, margin, bflags,
+                                          counters + kBandBricks, counters + kBandOverturned,
+                                          c->stream);
             return e;
           }));
-  if ((st = read_ctl(c, S, "band brick selection")) != ISO_OK) return st;
-  const uint64_t n_band = c->h_stage[1];
-  const iso::McDims D = iso::mc_dims(L);
+  const iso::McDims D = iso::mc_dims_pitched(L);
   SignsStage signs = [&](const iso::McBuffers& B, float* values) -> int {
-    ISO_HIP(c, timed(c, "band_background", [&] {
-              return iso::launch_band_background(L, D, G, bflags, B, c->stream);
-            }));
     // The stage reruns when the active-cell list grows: count the exact
     // samples of this run only.
-    ISO_HIP(c, iso::launch_fill_u32(reinterpret_cast<uint32_t*>(counters), 2, 0u, c->stream));
+    ISO_HIP(c, iso::launch_fill_u32(reinterpret_cast<uint32_t*>(counters + kBandExact),
+                                    2 * kBandSpread, 0u, c->stream));
     ISO_HIP(c, timed(c, "band_exact", [&] {
-              return iso::launch_band_exact(ops, c->n_prog, L, G, bflags, list, n_band, B, values,
-                                            counters, c->stream);
+              return iso::launch_band_tiles(ops, c->n_prog, c->prog_kind, L, D, G, bflags, B,
+                                            values, counters + kBandExact, c->stream);
             }));
     return ISO_OK;
   };
@@ -2341,14 +2341,20 @@ int iso_extract_mc_band(iso_ctx* c, const iso_grid_desc* desc, float margin, uin
   c->band_desc = *desc;
   c->band_valid = true;
   if (stats) {
-    ISO_HIP(c, hipMemcpyAsync(c->h_stage + 4, counters, 4 * sizeof(unsigned long long),
+    std::vector<unsigned long long> h(kBandCounters);
+    ISO_HIP(c, hipMemcpyAsync(h.data(), counters, kBandCounters * sizeof(unsigned long long),
                               hipMemcpyDeviceToHost, c->stream));
     ISO_HIP(c, hipStreamSynchronize(c->stream));
+    auto spread = [&](int at) {
+      unsigned long long sum = 0;
+      for (int i = 0; i < iso::kCounterLines; ++i) sum += h[at + i * iso::kCounterStride];
+      return sum;
+    };
     stats->bricks = nb;
-    stats->band_bricks = n_band;
-    stats->exact_samples = c->h_stage[4];
-    stats->centre_samples = c->h_stage[6];
-    stats->overturned_culls = c->h_stage[7];
+    stats->band_bricks = h[kBandBricks];
+    stats->exact_samples = spread(kBandExact);
+    stats->centre_samples = spread(kBandCentre);
+    stats->overturned_culls = h[kBandOverturned];
   }
   return st;
 }
@@ -2371,10 +2377,12 @@ int iso_band_missed_cells(iso_ctx* c, const iso_grid_desc* desc, uint64_t* misse
   J.signs = static_cast<uint64_t*>(c->dense_check.ptr) + 1;
   const iso::DevOp* ops = static_cast<const iso::DevOp*>(c->prog.ptr);
   ISO_HIP(c, iso::launch_signs_program(ops, c->n_prog, L, D, J, nullptr, c->stream));
-  unsigned long long* counters = static_cast<unsigned long long*>(c->br_count.ptr);
-  ISO_HIP(c, iso::launch_fill_u32(reinterpret_cast<uint32_t*>(counters + 1), 2, 0u, c->stream));
-  ISO_HIP(c, iso::launch_band_diff(L, D, B.signs, J.signs, counters + 1, c->stream));
-  ISO_HIP(c, hipMemcpyAsync(c->h_stage + 4, counters + 1, sizeof(unsigned long long),
+  unsigned long long* differing =
+      static_cast<unsigned long long*>(c->br_count.ptr) + kBandDiffering;
+  ISO_HIP(c, iso::launch_fill_u32(reinterpret_cast<uint32_t*>(differing), 2, 0u, c->stream));
+  ISO_HIP(c, iso::launch_band_diff(L, D, iso::mc_dims_pitched(L).sign_pitch, B.signs, J.signs,
+                                   differing, c->stream));
+  ISO_HIP(c, hipMemcpyAsync(c->h_stage + 4, differing, sizeof(unsigned long long),
                             hipMemcpyDeviceToHost, c->stream));
   ISO_HIP(c, hipStreamSynchronize(c->stream));
   *missed = c->h_stage[4];

@@ -14,8 +14,8 @@
 
 #include "mc_kernels.h"
 #include "mlp_kernels.h"
-#include "scan.h"
 #include "sdf_program.h"
+#include "sparse_kernels.h"
 
 namespace iso {
 
@@ -63,13 +63,17 @@ hipError_t launch_coarse_certify(const DevOp* ops, int n_ops, const Lattice& L,
                                  const BrickGrid& G, uint8_t* coarse,
                                  unsigned long long* certified, hipStream_t s);
 
+// A counter that many wavefronts add to is spread over lines of its own;
+// its value is the sum of its kCounterLines words, kCounterStride apart.
+constexpr int kCounterLines = 64;
+constexpr int kCounterStride = 16;
+
 // Brick proofs: proof[b] = its super-brick's flag when that proves the
 // sign, else the same test at brick b's own centre (against half_diag[b];
-// evaluations added to *certified).
-hipError_t launch_brick_certify(const DevOp* ops, int n_ops, const Lattice& L,
-                                const BrickGrid& G,
-                                const uint8_t* coarse, const float* centres,
-                                const float* half_diag, uint8_t* proof,
+// evaluations added to the spread counter *certified).
+hipError_t launch_brick_certify(const DevOp* ops, int n_ops, const ProgramKind& kind,
+                                const Lattice& L, const BrickGrid& G, const uint8_t* coarse,
+                                const float* centres, const float* half_diag, uint8_t* proof,
                                 unsigned long long* certified, hipStream_t s);
 
 // Band / inside flags.  With predictions alone, a brick is in the band if
@@ -77,27 +81,25 @@ hipError_t launch_brick_certify(const DevOp* ops, int n_ops, const Lattice& L,
 // `proof` (launch_brick_certify's flags), a brick leaves the band only when
 // its proof allows it, whatever the network predicted, and a brick the
 // network culled that its proof does not allow is counted in *overturned.
-// The list of band bricks (ascending) and its length go to st.ctl[1].
+// *n_band receives the number of band bricks (both are added to).
 hipError_t launch_brick_flags(const BrickGrid& G, const float* pred, const float* half_diag,
                               const uint8_t* proof, float margin, uint8_t* flags,
-                              uint32_t* band_list, unsigned long long* overturned,
-                              const scan::State& st, hipStream_t s);
-// Sign bits of the whole lattice from the bricks' predicted signs (and the
-// extraction's state reset, like the other signs launchers).
-hipError_t launch_band_background(const Lattice& L, const McDims& D, const BrickGrid& G,
-                                  const uint8_t* flags, const McBuffers& B, hipStream_t s);
-// Exact sign bits of every sample of the band bricks' closed sample boxes,
-// each sample evaluated once (by the band brick latest in brick order among
-// those holding it); values[f] receives the sample when values is not null.
-// n_band bricks from band_list; *evaluated receives the sample count.
-hipError_t launch_band_exact(const DevOp* ops, int n_ops, const Lattice& L, const BrickGrid& G,
-                             const uint8_t* flags, const uint32_t* band_list, uint64_t n_band,
-                             const McBuffers& B, float* values, unsigned long long* evaluated,
-                             hipStream_t s);
+                              unsigned long long* n_band, unsigned long long* overturned,
+                              hipStream_t s);
+// Row-aligned sign words of the whole lattice (dims of mc_dims_pitched) and
+// the extraction's state reset: exact signs for the samples of the band
+// bricks' closed sample boxes, whose values go to `values` when it is not
+// null, the bricks' predicted signs elsewhere.  The number of exact samples is
+// added to the spread counter *evaluated.
+hipError_t launch_band_tiles(const DevOp* ops, int n_ops, const ProgramKind& kind,
+                             const Lattice& L, const McDims& D, const BrickGrid& G,
+                             const uint8_t* flags, const McBuffers& B, float* values,
+                             unsigned long long* evaluated, hipStream_t s);
 // Cells of lattice L whose marching-cubes case differs between the sign
-// arrays signs_a and signs_b (each with the extraction's guard words); the
-// count is added to *differing.
-hipError_t launch_band_diff(const Lattice& L, const McDims& D, const uint64_t* signs_a,
+// arrays signs_a (rows pitch_a bits apart) and signs_b (flat), each with the
+// extraction's guard words; the count is added to *differing.
+hipError_t launch_band_diff(const Lattice& L, const McDims& D, int64_t pitch_a,
+                            const uint64_t* signs_a,
                             const uint64_t* signs_b, unsigned long long* differing,
                             hipStream_t s);
 

@@ -8,12 +8,16 @@
 #include <type_traits>
 
 #include "sdf_eval.h"
+#include "sparse_eval.h"
+#include "sparse_kernels.h"
 
 namespace iso {
 
 namespace {
 
 using namespace mcd;
+
+constexpr int kCertifyListCap = 512;
 
 struct BrickBox {
   int64_t lo[3], hi[3];  // sample range [lo, hi] per axis
@@ -140,14 +144,79 @@ __global__ __launch_bounds__(256) void k_brick_certify(const DevOp* __restrict__
   if (live) proof[b] = out;
 }
 
-struct FlagLoad {
-  const float* pred;       // network predictions; null: no network
-  const float* half_diag;
-  const uint8_t* proof;    // non-null: a brick leaves the band only by its proof
-  float margin;
-  uint8_t* flags;
-  unsigned long long* overturned;  // network culls no proof allows
-  __device__ unsigned long long operator()(uint64_t i) const {
+// k_brick_certify for bounded programs.  A wavefront evaluates its bricks'
+// centres over the operations that matter in the box of the centres: the
+// values are the whole program's, and so are the proofs.  The operations left
+// out enter an evaluation's error bound only as one more operand of its
+// maximum, so the bound lies between the one of the listed operations alone
+// and the one that starts from the greatest bound of any operation in the box;
+// where the two decide a brick differently, the wavefront evaluates the whole
+// program after all.
+template <bool kStack>
+__global__ __launch_bounds__(256) void k_brick_certify_listed(
+    const DevOp* __restrict__ dops, int n_ops, BrickGrid G, const uint8_t* __restrict__ coarse,
+    const float* __restrict__ centres, const float* __restrict__ half_diag,
+    uint8_t* __restrict__ proof, unsigned long long* certified, float pos_slack, float mag) {
+  __shared__ uint16_t s_list[4][kCertifyListCap];
+  const int lane = __lane_id();
+  const int wv = static_cast<int>(threadIdx.x >> 6);
+  const int64_t s = static_cast<int64_t>(blockIdx.x) * 4 + wv;
+  if (s >= G.nc) return;  // uniform per wave
+  const int64_t sx = s % G.ncx;
+  const int64_t r = s / G.ncx;
+  const int64_t bx = kCoarse * sx + lane % kCoarse;
+  const int64_t by = kCoarse * (r % G.ncy) + (lane / kCoarse) % kCoarse;
+  const int64_t bz = kCoarse * (r / G.ncy) + lane / (kCoarse * kCoarse);
+  const bool live = bx < G.nbx && by < G.nby && bz < G.nbz;
+  const int64_t b = (bz * G.nby + by) * G.nbx + bx;
+  const uint8_t cf = coarse[s];
+  if (cf & kBrickProven) {
+    if (live) proof[b] = cf;
+    return;
+  }
+  const uint64_t lives = __ballot(live);
+  if (lane == 0)
+    atomicAdd(certified + kCounterStride * (s % kCounterLines),
+              static_cast<unsigned long long>(__popcll(lives)));
+  const OpsPtr ops = as_constant(dops);
+  float p[3], lo[3], hi[3], widen = 0.0f;
+  if (live) widen = half_diag[b] * (1.0f + kCertifyRelSlack) + pos_slack;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    p[a] = live ? centres[3 * b + a] : 0.0f;
+    lo[a] = wave_min(live ? p[a] : kNoBound);
+    hi[a] = -wave_min(live ? -p[a] : kNoBound);
+  }
+  const float wide = -wave_min(-widen);
+  float floor_e;
+  const int len = certify_list(ops, n_ops, lo, hi, wide, mag, s_list[wv], kCertifyListCap, &floor_e);
+  lds_barrier<1>();
+  uint8_t out = 0;
+  bool unsure = true;
+  if (len <= kCertifyListCap) {
+    float e0, e1;
+    const float v =
+        eval_bound_list<kStack>(ops, s_list[wv], len, p[0], p[1], p[2], widen, floor_e, &e0, &e1);
+    const bool p0 = fabsf(v) > widen + 2.0f * e0 + kCertifyAbsSlack;
+    const bool p1 = fabsf(v) > widen + 2.0f * e1 + kCertifyAbsSlack;
+    unsure = p0 != p1;
+    out = p1 ? static_cast<uint8_t>(kBrickProven | (!(v > 0.0f) ? kBrickInside : 0)) : uint8_t{0};
+  }
+  if (__ballot(live && unsure) && live)
+    out = certify_at(dops, n_ops, p[0], p[1], p[2], half_diag[b], pos_slack);
+  if (live) proof[b] = out;
+}
+
+// The bricks' band and inside flags, with the numbers of band bricks and of
+// network culls that no proof allows.
+__global__ __launch_bounds__(256) void k_brick_flags(
+    uint64_t n, const float* __restrict__ pred, const float* __restrict__ half_diag,
+    const uint8_t* __restrict__ proof, float margin, uint8_t* __restrict__ flags,
+    unsigned long long* n_band, unsigned long long* overturned) {
+  uint32_t bands = 0, turned = 0;
+  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
+  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
+       i += stride) {
     bool band = true, inside = false;
     if (pred) {
       const float p = pred[i];
@@ -158,266 +227,239 @@ struct FlagLoad {
     if (proof) {
       const uint8_t pf = proof[i];
       const bool proven = (pf & kBrickProven) != 0;
-      count_lanes(pred != nullptr && !band && !proven, overturned);
+      turned += pred != nullptr && !band && !proven;
       band = !proven;
       inside = proven && (pf & kBrickInside) != 0;
     }
     flags[i] = static_cast<uint8_t>((band ? kBrickBand : 0) | (inside ? kBrickInside : 0));
-    return band ? 1ull : 0ull;
+    bands += band;
   }
-};
-
-struct FlagSink {
-  uint32_t* list;
-  __device__ void operator()(uint64_t i, unsigned long long v, unsigned long long ex) const {
-    if (v) list[ex] = static_cast<uint32_t>(i);
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) {
+    bands += __shfl_xor(bands, d, 64);
+    turned += __shfl_xor(turned, d, 64);
   }
-};
-
-__device__ __forceinline__ int64_t brick_of(int64_t c, int shift, int64_t nb) {
-  const int64_t b = c >> shift;
-  return b < nb ? b : nb - 1;
+  if (__lane_id() == 0) {
+    if (bands) atomicAdd(n_band, static_cast<unsigned long long>(bands));
+    if (turned) atomicAdd(overturned, static_cast<unsigned long long>(turned));
+  }
 }
 
-// Background signs: the predicted sign of each sample's brick (the brick
-// holding the sample's cell-space position, clamped at the far faces).
-__global__ __launch_bounds__(256) void k_band_background(Lattice L, BrickGrid G,
-                                                         const uint8_t* __restrict__ flags,
-                                                         int64_t n_points, int64_t n_words,
-                                                         uint64_t* __restrict__ S,
-                                                         ResetArgs R) {
+// Signs and exact samples of one 16^3-sample tile (sparse_kernels.h) of the
+// band's lattice.  A sample is exact when a band brick's closed sample box
+// holds it (up to eight bricks do); every other one takes its own brick's
+// predicted sign.  The tile's exact samples are queued in LDS, the samples of
+// a 4^3 block of samples together, so that whole wavefronts evaluate 256 of
+// them at a time however few each block has; with sound bounds they are
+// evaluated over the operations that matter in the tile and, of those, in the
+// blocks that the 256 come from.  Row-aligned sign words, one 16-bit store a
+// row.  Bound by instruction issue: 98.4 M samples of 1024 smoothly joined
+// spheres at 1025^3 take BAND_EXACT_US, where the flat background pass and a
+// culled evaluation of the whole program took 19.2 ms.
+constexpr int kTileBlocks = 64;
+constexpr int kTileSamples = kTileSide * kTileSide * kTileSide;
+constexpr int kBandListCap = 512;
+constexpr int kBandCoords = kTileSide + 2;
+constexpr int kBandWaves = 4;
+
+template <bool kStack>
+__global__ __launch_bounds__(64 * kBandWaves) void k_band_tiles(
+    CellSpace C, BrickGrid G, int bounded, const uint8_t* __restrict__ flags, uint32_t n_tiles,
+    unsigned long long* evaluated, ResetArgs R) {
+  __shared__ uint64_t s_sign[kTileBlocks];
+  __shared__ uint64_t s_mask[kBandListCap];
+  __shared__ uint64_t s_from[kTileSamples / 64];  // blocks that each 64 queue entries come from
+  __shared__ uint16_t s_queue[kTileSamples];
+  __shared__ uint16_t s_list[kBandListCap];
+  __shared__ float s_coord[3 * kBandCoords];
+  __shared__ uint8_t s_flag[125];
+  __shared__ uint32_t s_n;
+  __shared__ int s_len;
   reset_state(R);
+  const uint32_t tile = blockIdx.x;
+  if (tile >= n_tiles) return;
+  const int32_t n[3] = {static_cast<int32_t>(C.nx), static_cast<int32_t>(C.ny),
+                        static_cast<int32_t>(C.nz)};
+  const int32_t nb[3] = {static_cast<int32_t>(G.nbx), static_cast<int32_t>(G.nby),
+                         static_cast<int32_t>(G.nbz)};
+  const uint32_t ntx = static_cast<uint32_t>(n[0] + kTileSide - 1) >> kTileShift;
+  const uint32_t nty = static_cast<uint32_t>(n[1] + kTileSide - 1) >> kTileShift;
+  const uint32_t tz = tile / (ntx * nty);
+  const uint32_t tr = tile - tz * (ntx * nty);
+  const uint32_t ty = tr / ntx;
+  const uint32_t tx = tr - ty * ntx;
+  const int32_t s0[3] = {static_cast<int32_t>(tx << kTileShift),
+                         static_cast<int32_t>(ty << kTileShift),
+                         static_cast<int32_t>(tz << kTileShift)};
   const int lane = __lane_id();
-  const int64_t wave = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  const int64_t n_waves = static_cast<int64_t>(gridDim.x) * 4;
-  const uint32_t nx = static_cast<uint32_t>(L.nx);
-  const uint32_t nxy = static_cast<uint32_t>(L.nx * L.ny);
-  for (int64_t w = wave; w < n_words; w += n_waves) {
-    const int64_t f = w * 64 + lane;
-    bool inside = false;
-    if (f < n_points) {
-      const uint32_t ff = static_cast<uint32_t>(f);
-      const uint32_t z = ff / nxy;
-      const uint32_t r = ff - z * nxy;
-      const uint32_t y = r / nx;
-      const uint32_t x = r - y * nx;
-      const int64_t b =
-          (brick_of(z, G.shift, G.nbz) * G.nby + brick_of(y, G.shift, G.nby)) * G.nbx +
-          brick_of(x, G.shift, G.nbx);
-      inside = (flags[b] & kBrickInside) != 0;
+  const int wv = static_cast<int>(threadIdx.x >> 6);
+  // Flags of the tile's bricks and the ones below them: at most 5 per axis,
+  // entry 0 the brick below the tile's first.
+  const int per = (kTileSide >> G.shift) + 1;
+  bool any = false;
+  if (static_cast<int>(threadIdx.x) < per * per * per) {
+    const int q[3] = {static_cast<int>(threadIdx.x) % per,
+                      static_cast<int>(threadIdx.x) / per % per,
+                      static_cast<int>(threadIdx.x) / (per * per)};
+    int32_t b[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      b[a] = (s0[a] >> G.shift) - 1 + q[a];
+      b[a] = b[a] < 0 ? 0 : b[a] < nb[a] ? b[a] : nb[a] - 1;
     }
-    const uint64_t m = __ballot(inside);
-    if (lane == 0) S[w] = m;
+    const uint8_t f = flags[(static_cast<int64_t>(b[2]) * G.nby + b[1]) * G.nbx + b[0]];
+    s_flag[threadIdx.x] = f;
+    any = (f & kBrickBand) != 0;
   }
-}
+  if (threadIdx.x == 0) s_n = 0;
+  if (threadIdx.x < kTileSamples / 64) s_from[threadIdx.x] = 0ull;
+  const bool work = __syncthreads_or(any) != 0;
 
-// Neighbour bricks (bit (dz+1)*9 + (dy+1)*3 + dx+1) that also hold a sample
-// of class (cx, cy, cz) — per axis 0: on the brick's low face, 1: inside,
-// 2: on its high face — and come later in brick order.  The band brick
-// latest in brick order among those holding a sample evaluates it, so each
-// exact sample is evaluated once.
-__device__ __forceinline__ uint32_t later_holders(int cx, int cy, int cz) {
-  uint32_t m = 0;
-  for (int dz = cz == 0 ? -1 : 0; dz <= (cz == 2 ? 1 : 0); ++dz)
-    for (int dy = cy == 0 ? -1 : 0; dy <= (cy == 2 ? 1 : 0); ++dy)
-      for (int dx = cx == 0 ? -1 : 0; dx <= (cx == 2 ? 1 : 0); ++dx)
-        if (dz > 0 || (dz == 0 && (dy > 0 || (dy == 0 && dx > 0))))
-          m |= 1u << ((dz + 1) * 9 + (dy + 1) * 3 + dx + 1);
-  return m;
-}
-
-constexpr int kExactThreads = 256;
-
-// Sizes of the exact-sample kernel for bricks of 2^kShift cells per edge.
-// Eight-cell bricks take fewer bricks per workgroup pass, so a workgroup's
-// LDS stays near 17 KB and eight workgroups still fit a CU.
-template <int kShift>
-struct ExactShape {
-  static constexpr int kBrick = 1 << kShift;              // cells per brick edge
-  static constexpr int kSide = kBrick + 1;                 // samples per edge of a brick box
-  static constexpr int kBoxRows = kSide * kSide;           // x rows of a brick's sample box
-  static constexpr int kBoxSamples = kBoxRows * kSide;
-  static constexpr int kGroupBricks = kShift == 2 ? 32 : 8;  // band bricks per workgroup pass
-  static constexpr int kBricksPerWave = kGroupBricks / (kExactThreads / 64);
-  // box position lx + kSide (ly + kSide lz)
-  using Pos = typename std::conditional<(kBoxSamples <= 256), uint8_t, uint16_t>::type;
-  static_assert(kSide <= 32, "a box row is one 32-bit mask");
-};
-
-// Thirty-two band bricks (of 4^3 cells; eight of 8^3) per workgroup pass.
-// Each wavefront takes a quarter of them: it reads a brick's and its 26 neighbours' band flags, walks the brick's
-// closed sample box (x fastest) and appends the samples the brick owns to
-// the brick's list in LDS.  Then all 256 lanes evaluate the 32 lists
-// as one queue (a lane's brick by binary search of the lists' offsets), so
-// lanes stay busy however few samples each brick owns, store the values,
-// and gather sign bits per x row in LDS; last, one lane per row merges the
-// row into the sign words (at most two words, OR for inside, AND-NOT for
-// outside, over the background the bricks' flags wrote).
-template <int kShift>
-__global__ __launch_bounds__(kExactThreads) void
-k_band_exact(
-    const DevOp* __restrict__ ops, int n_ops, Lattice L, BrickGrid G,
-    const uint8_t* __restrict__ flags, const uint32_t* __restrict__ band_list, uint64_t n_band,
-    uint64_t* __restrict__ S, float* __restrict__ values, unsigned long long* evaluated) {
-  using X = ExactShape<kShift>;
-  constexpr int kBrick = X::kBrick, kSide = X::kSide, kBoxRows = X::kBoxRows;
-  constexpr int kGroupBricks = X::kGroupBricks, kBricksPerWave = X::kBricksPerWave;
-  __shared__ uint32_t s_in[kGroupBricks][kBoxRows];
-  __shared__ uint32_t s_own[kGroupBricks][kBoxRows];
-  __shared__ typename X::Pos s_pos[kGroupBricks][X::kBoxSamples];
-  __shared__ uint32_t s_lo[kGroupBricks][3];
-  __shared__ uint32_t s_n[kGroupBricks];
-  __shared__ uint32_t s_pre[kGroupBricks + 1];
-  const int lane = __lane_id();
-  const int wv = threadIdx.x >> 6;
-  uint32_t count = 0;
-  for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * kGroupBricks; base < n_band;
-       base += static_cast<uint64_t>(gridDim.x) * kGroupBricks) {
-    for (int r = threadIdx.x; r < kGroupBricks * kBoxRows; r += kExactThreads) {
-      (&s_in[0][0])[r] = 0;
-      (&s_own[0][0])[r] = 0;
+  // Each block of 4^3 samples, a wavefront at a time: signs of the samples
+  // that are not exact, the others queued.
+  const int l[3] = {lane & 3, (lane >> 2) & 3, lane >> 4};
+  for (int blk = wv; blk < kTileBlocks; blk += kBandWaves) {
+    const int o[3] = {4 * (blk & 3), blk & 12, 4 * (blk >> 4)};
+    int hi[3], lo[3];
+    bool valid = true;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const int32_t s = s0[a] + o[a] + l[a];
+      valid = valid && s < n[a];
+      const int32_t own = s >> G.shift;
+      const int32_t first = (s0[a] >> G.shift) - 1;
+      hi[a] = (own < nb[a] ? own : nb[a] - 1) - first;
+      lo[a] = (s & (G.brick - 1)) == 0 && s > 0 ? own - 1 - first : hi[a];
+      if (!valid) hi[a] = lo[a] = 0;
     }
-    __syncthreads();
-#pragma unroll 1
-    for (int q = 0; q < kBricksPerWave; ++q) {
-      const int j = wv * kBricksPerWave + q;
-      const uint64_t item = base + j;
-      uint32_t n_own = 0;
-      if (item < n_band) {  // uniform per wave
-        const int64_t b = band_list[item];
-        const int64_t bc[3] = {b % G.nbx, (b / G.nbx) % G.nby, b / (G.nbx * G.nby)};
-        const int64_t nbk[3] = {G.nbx, G.nby, G.nbz};
-        const int64_t n[3] = {L.nx, L.ny, L.nz};
-        // Band flags of the 26 neighbours (and the brick itself, bit 13).
-        bool band = false;
-        if (lane < 27) {
-          const int64_t nq[3] = {bc[0] + lane % 3 - 1, bc[1] + (lane / 3) % 3 - 1,
-                                 bc[2] + lane / 9 - 1};
-          if (nq[0] >= 0 && nq[1] >= 0 && nq[2] >= 0 && nq[0] < nbk[0] && nq[1] < nbk[1] &&
-              nq[2] < nbk[2])
-            band = (flags[(nq[2] * G.nby + nq[1]) * G.nbx + nq[0]] & kBrickBand) != 0;
-        }
-        const uint32_t nb = static_cast<uint32_t>(__ballot(band));
-        int64_t lo[3];
-        int ext[3];
+    const uint8_t mine = s_flag[(hi[2] * per + hi[1]) * per + hi[0]];
+    bool exact = false;
+    if (work) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        exact |= (s_flag[((k & 4 ? lo[2] : hi[2]) * per + (k & 2 ? lo[1] : hi[1])) * per +
+                         (k & 1 ? lo[0] : hi[0])] &
+                  kBrickBand) != 0;
+      exact = exact && valid;
+    }
+    const uint64_t in = __ballot(valid && !exact && (mine & kBrickInside));
+    const uint64_t m = __ballot(exact);
+    uint32_t at = 0;
+    if (lane == 0) {
+      s_sign[blk] = in;
+      if (m) {
+        const uint32_t cnt = static_cast<uint32_t>(__popcll(m));
+        at = atomicAdd(&s_n, cnt);
+        atomicOr(reinterpret_cast<unsigned long long*>(&s_from[at >> 6]), 1ull << blk);
+        atomicOr(reinterpret_cast<unsigned long long*>(&s_from[(at + cnt - 1) >> 6]), 1ull << blk);
+      }
+    }
+    at = __builtin_amdgcn_readfirstlane(at);
+    if (exact)
+      s_queue[at + static_cast<uint32_t>(__popcll(m & ((1ull << lane) - 1ull)))] =
+          static_cast<uint16_t>(blk * 64 + lane);
+  }
+  __syncthreads();
+  const uint32_t total = __builtin_amdgcn_readfirstlane(s_n);
+  if (total) {
+    const OpsPtr ops = as_constant(C.ops);
+    const int n_ops = C.n_ops;
+    const int first = leading_scopes(ops, n_ops);
+    if (wv == 0) {
+      if (lane < 3 * kBandCoords) {
+        const int a = lane / kBandCoords;
+        const int32_t na = a == 0 ? n[0] : a == 1 ? n[1] : n[2];
+        int32_t i = (a == 0 ? s0[0] : a == 1 ? s0[1] : s0[2]) + lane - kBandCoords * a - 1;
+        i = i < 0 ? 0 : i < na ? i : na - 1;
+        const float org = a == 0 ? C.origin[0] : a == 1 ? C.origin[1] : C.origin[2];
+        const float d = a == 0 ? C.spacing[0] : a == 1 ? C.spacing[1] : C.spacing[2];
+        float x = org + static_cast<float>(i) * d;
+        for (int s = 0; s < first; ++s)
+          x = x - (a == 0 ? ops[s].off[0] : a == 1 ? ops[s].off[1] : ops[s].off[2]);
+        s_coord[lane] = x;
+      }
+      lds_barrier<1>();
+      int len = kBandListCap + 1;
+      if (bounded) {
+        float blo[3], bhi[3], vlo, vhi;
+#pragma unroll
         for (int a = 0; a < 3; ++a) {
-          lo[a] = kBrick * bc[a];
-          int64_t hi = lo[a] + kBrick < n[a] - 1 ? lo[a] + kBrick : n[a] - 1;
-          // the high face goes to the next brick along the axis when it is in the band
-          const int up = a == 0 ? 14 : a == 1 ? 16 : 22;
-          if (hi == lo[a] + kBrick && (nb >> up) & 1u) hi -= 1;
-          ext[a] = static_cast<int>(hi - lo[a] + 1);
+          const float c0 = s_coord[kBandCoords * a + 1], c1 = s_coord[kBandCoords * a + kTileSide];
+          blo[a] = fminf(c0, c1);
+          bhi[a] = fmaxf(c0, c1);
         }
-        const int exy = ext[0] * ext[1];
-        const int total = exy * ext[2];
-#pragma unroll 1
-        for (int t0 = 0; t0 < total; t0 += 64) {  // uniform trip count
-          const int t = t0 + lane;
-          bool own = false;
-          int lx = 0, ly = 0, lz = 0;
-          if (t < total) {
-            lz = t / exy;
-            const int rem = t - lz * exy;
-            ly = rem / ext[0];
-            lx = rem - ly * ext[0];
-            const int cx = lx == 0 ? 0 : lx == kBrick ? 2 : 1;
-            const int cy = ly == 0 ? 0 : ly == kBrick ? 2 : 1;
-            const int cz = lz == 0 ? 0 : lz == kBrick ? 2 : 1;
-            own = !(later_holders(cx, cy, cz) & nb);
-          }
-          const uint64_t m = __ballot(own);
-          if (own) {
-            const uint32_t k = n_own + static_cast<uint32_t>(__popcll(m & ((1ull << lane) - 1)));
-            s_pos[j][k] = static_cast<typename X::Pos>(lx + kSide * (ly + kSide * lz));
-            atomicOr(&s_own[j][ly + kSide * lz], 1u << lx);
-          }
-          n_own += static_cast<uint32_t>(__popcll(m));
-        }
-        if (lane == 0) {
-          s_lo[j][0] = static_cast<uint32_t>(lo[0]);
-          s_lo[j][1] = static_cast<uint32_t>(lo[1]);
-          s_lo[j][2] = static_cast<uint32_t>(lo[2]);
-        }
-      }
-      if (lane == 0) s_n[j] = n_own;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      uint32_t a = 0;
-      for (int j = 0; j < kGroupBricks; ++j) {
-        s_pre[j] = a;
-        a += s_n[j];
-      }
-      s_pre[kGroupBricks] = a;
-    }
-    __syncthreads();
-    const uint32_t T = s_pre[kGroupBricks];
-    // Whole wavefronts step through the queue (the culled evaluator works on
-    // all 64 lanes); lanes past its end repeat its last entry and drop it.
-#pragma unroll 1
-    for (uint32_t t0 = threadIdx.x & ~63u; t0 < T; t0 += kExactThreads) {
-      const bool valid = t0 + (threadIdx.x & 63u) < T;
-      const uint32_t t = valid ? t0 + (threadIdx.x & 63u) : T - 1;
-      int j = 0;  // the brick whose list holds queue entry t: s_pre[j] <= t < s_pre[j + 1]
+        len = bound_box<kStack>(ops, first, n_ops, blo, bhi, s_list, kBandListCap, &vlo, &vhi);
+        if (len <= kBandListCap) {
+          const int b[3] = {lane & 3, (lane >> 2) & 3, lane >> 4};
+          bool active = true;
 #pragma unroll
-      for (int step = kGroupBricks / 2; step >= 1; step >>= 1)
-        if (s_pre[j + step] <= t) j += step;
-      const int pos = s_pos[j][t - s_pre[j]];
-      const int lz = pos / kBoxRows;
-      const int ly = (pos - lz * kBoxRows) / kSide;
-      const int lx = pos - lz * kBoxRows - ly * kSide;
-      const int64_t x = static_cast<int64_t>(s_lo[j][0]) + lx;
-      const int64_t y = static_cast<int64_t>(s_lo[j][1]) + ly;
-      const int64_t z = static_cast<int64_t>(s_lo[j][2]) + lz;
-      const float v =
-          sdf_eval_culled(ops, n_ops, L.origin[0] + static_cast<float>(x) * L.spacing[0],
-                          L.origin[1] + static_cast<float>(y) * L.spacing[1],
-                          L.origin[2] + static_cast<float>(z) * L.spacing[2]);
-      if (!valid) continue;
-      if (values) values[(z * L.ny + y) * L.nx + x] = v;
-      // classify_corners, distance.rs:52-54
-      if (!(v > 0.0f)) atomicOr(&s_in[j][ly + kSide * lz], 1u << lx);
-      ++count;
+          for (int a = 0; a < 3; ++a) {
+            active = active && s0[a] + 4 * b[a] < n[a];
+            const float c0 = s_coord[kBandCoords * a + 1 + 4 * b[a]];
+            const float c1 = s_coord[kBandCoords * a + 4 + 4 * b[a]];
+            blo[a] = fminf(c0, c1);
+            bhi[a] = fmaxf(c0, c1);
+          }
+          lds_barrier<1>();
+          len = bound_lanes<kStack>(ops, first, len, blo, bhi, active, s_list, s_mask, &vlo, &vhi);
+        }
+      }
+      if (lane == 0) s_len = len;
     }
     __syncthreads();
-    for (int r = threadIdx.x; r < kGroupBricks * kBoxRows; r += kExactThreads) {
-      const int j = r / kBoxRows;
-      const int row = r - j * kBoxRows;
-      const uint64_t own = s_own[j][row];
-      if (!own) continue;
-      const uint64_t in = s_in[j][row] & own;
-      const uint64_t out = own & ~in;
-      const int ly = row % kSide, lz = row / kSide;
-      const int64_t f0 = ((static_cast<int64_t>(s_lo[j][2]) + lz) * L.ny +
-                          static_cast<int64_t>(s_lo[j][1]) + ly) * L.nx +
-                         static_cast<int64_t>(s_lo[j][0]);
-      const int64_t w0 = f0 >> 6;
-      const int sh = static_cast<int>(f0 & 63);
-      unsigned long long* W = reinterpret_cast<unsigned long long*>(S);
-      if (in << sh) atomicOr(&W[w0], in << sh);
-      if (out << sh) atomicAnd(&W[w0], ~(out << sh));
-      if (sh) {
-        const uint64_t in1 = in >> (64 - sh), out1 = out >> (64 - sh);
-        if (in1) atomicOr(&W[w0 + 1], in1);
-        if (out1) atomicAnd(&W[w0 + 1], ~out1);
+    const int len = __builtin_amdgcn_readfirstlane(s_len);
+    const uint16_t* list = len <= kBandListCap ? s_list : nullptr;
+    const int m = len <= kBandListCap ? len : n_ops - first;
+    constexpr int kPoints = kStack ? 2 : 4;
+    const int64_t base = (static_cast<int64_t>(s0[2]) * n[1] + s0[1]) * n[0] + s0[0];
+    for (uint32_t q0 = static_cast<uint32_t>(wv) * 64 * kPoints; q0 < total;
+         q0 += 64 * kPoints * kBandWaves) {
+      float p[kPoints][3], v[kPoints];
+      int id[kPoints];
+      uint64_t from = 0;
+#pragma unroll
+      for (int j = 0; j < kPoints; ++j) {
+        const uint32_t q = q0 + 64 * j + lane;
+        id[j] = s_queue[q < total ? q : total - 1];
+        if (q0 + 64 * j < total) from |= s_from[(q0 >> 6) + j];
+        const int blk = id[j] >> 6;
+        p[j][0] = s_coord[1 + 4 * (blk & 3) + (id[j] & 3)];
+        p[j][1] = s_coord[kBandCoords + 1 + (blk & 12) + ((id[j] >> 2) & 3)];
+        p[j][2] = s_coord[2 * kBandCoords + 1 + 4 * (blk >> 4) + ((id[j] >> 4) & 3)];
+      }
+      // (spare points repeat the queue's last entry)
+      from |= s_from[(total - 1) >> 6];
+      sdf_eval_list<kPoints, kStack>(ops, first, list, s_mask, from, m, p, v);
+#pragma unroll
+      for (int j = 0; j < kPoints; ++j) {
+        if (q0 + 64 * j + lane >= total) continue;
+        const int blk = id[j] >> 6;
+        const uint32_t x = 4 * (blk & 3) + (id[j] & 3), y = (blk & 12) + ((id[j] >> 2) & 3),
+                       z = 4 * (blk >> 4) + ((id[j] >> 4) & 3);
+        if (C.grid)
+          (const_cast<float*>(C.grid) + base)[(z * static_cast<uint32_t>(n[1]) + y) *
+                                                  static_cast<uint32_t>(n[0]) + x] = v[j];
+        // classify_corners, distance.rs:52-54
+        if (!(v[j] > 0.0f))
+          atomicOr(reinterpret_cast<unsigned long long*>(&s_sign[blk]), 1ull << (id[j] & 63));
       }
     }
     __syncthreads();
+    // One counter line for every 64 tiles: thousands of tiles adding to one
+    // word would wait for each other.
+    if (threadIdx.x == 0) atomicAdd(evaluated + kCounterStride * (tile % kCounterLines), total);
   }
-  unsigned long long c = count;
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) c += __shfl_xor(c, d, 64);
-  if (__lane_id() == 0 && c) atomicAdd(evaluated, c);
+  store_tile_signs(C, s_sign, s0, tx, threadIdx.x, 64 * kBandWaves);
 }
 
 // Cells whose marching-cubes case differs between two sign arrays of the
 // same lattice (a band extraction's and the dense one's): a cell differs
 // when any of its eight corner bits does.  One thread per 64-cell segment.
-__global__ __launch_bounds__(256) void k_band_diff(Lattice L, McDims D,
+__global__ __launch_bounds__(256) void k_band_diff(Lattice L, McDims D, int64_t pitch_a,
                                                    const uint64_t* __restrict__ Sa,
                                                    const uint64_t* __restrict__ Sb,
                                                    unsigned long long* differing) {
-  const int64_t nx = L.nx, nxy = L.nx * L.ny;
+  const int64_t nx = L.nx;
   const int64_t spr = D.segs_per_row;
   const int64_t cyn = L.ny - 1;
   uint32_t count = 0;
@@ -425,14 +467,13 @@ __global__ __launch_bounds__(256) void k_band_diff(Lattice L, McDims D,
        g += static_cast<int64_t>(gridDim.x) * blockDim.x) {
     const int64_t row = g / spr, w = g - (g / spr) * spr;
     const int64_t cz = row / cyn, cy = row - (row / cyn) * cyn;
-    const int64_t f00 = cz * nxy + cy * nx + 64 * w;
     uint64_t m = 0, n = 0;
-    const int64_t offs[4] = {0, nx, nxy, nxy + nx};
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
+      const int64_t row_k = (cz + (k >> 1)) * L.ny + cy + (k & 1);
       uint64_t na, nb;
-      const uint64_t a = row_word(Sa, f00 + offs[k], &na);
-      const uint64_t b = row_word(Sb, f00 + offs[k], &nb);
+      const uint64_t a = row_word(Sa, row_k * pitch_a + 64 * w, &na);
+      const uint64_t b = row_word(Sb, row_k * nx + 64 * w, &nb);
       m |= a ^ b;
       n |= na ^ nb;
     }
@@ -503,33 +544,54 @@ float certify_position_slack(const Lattice& L) {
   return static_cast<float>(2.0 * std::sqrt(3.0) * std::ldexp(m, -23) * 1.01);
 }
 
-hipError_t launch_brick_certify(const DevOp* ops, int n_ops, const Lattice& L,
-                                const BrickGrid& G, const uint8_t* coarse, const float* centres,
-                                const float* half_diag, uint8_t* proof,
+hipError_t launch_brick_certify(const DevOp* ops, int n_ops, const ProgramKind& kind,
+                                const Lattice& L, const BrickGrid& G, const uint8_t* coarse,
+                                const float* centres, const float* half_diag, uint8_t* proof,
                                 unsigned long long* certified, hipStream_t s) {
   if (!ops || !coarse || !centres || !half_diag || !proof || !certified)
     return hipErrorInvalidValue;
   const uint64_t blocks = (static_cast<uint64_t>(G.nc) + 3) / 4;
   if (blocks > 0x7fffffffu) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_brick_certify, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, ops,
-                     n_ops, G, coarse, centres, half_diag, proof, certified,
-                     certify_position_slack(L));
+  const dim3 grid(static_cast<unsigned>(blocks)), block(256);
+  const float slack = certify_position_slack(L);
+  if (!kind.bounded || !lattice_bounded(L)) {
+    hipLaunchKernelGGL(k_brick_certify, grid, block, 0, s, ops, n_ops, G, coarse, centres,
+                       half_diag, proof, certified, slack);
+  } else {
+    double m = kind.magnitude;
+    const int64_t n[3] = {L.nx, L.ny, L.nz};
+    for (int a = 0; a < 3; ++a)
+      m = std::fmax(m, kind.magnitude + std::fabs(static_cast<double>(L.origin[a])) +
+                           static_cast<double>(n[a]) * std::fabs(static_cast<double>(L.spacing[a])));
+    const float mag = static_cast<float>(m * 1.001);
+    if (kind.stack)
+      hipLaunchKernelGGL(k_brick_certify_listed<true>, grid, block, 0, s, ops, n_ops, G, coarse,
+                         centres, half_diag, proof, certified, slack, mag);
+    else
+      hipLaunchKernelGGL(k_brick_certify_listed<false>, grid, block, 0, s, ops, n_ops, G, coarse,
+                         centres, half_diag, proof, certified, slack, mag);
+  }
   return hipGetLastError();
 }
 
 hipError_t launch_brick_flags(const BrickGrid& G, const float* pred, const float* half_diag,
                               const uint8_t* proof, float margin, uint8_t* flags,
-                              uint32_t* band_list, unsigned long long* overturned,
-                              const scan::State& st, hipStream_t s) {
-  if (!pred && !proof) return hipErrorInvalidValue;
-  if (proof && !overturned) return hipErrorInvalidValue;
-  FlagLoad load{pred, half_diag, proof, margin, flags, overturned};
-  FlagSink sink{band_list};
-  return scan::launch<scan::kItems>(static_cast<uint64_t>(G.n), load, sink, st, s);
+                              unsigned long long* n_band, unsigned long long* overturned,
+                              hipStream_t s) {
+  if ((!pred && !proof) || !flags || !n_band || !overturned) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_brick_flags, dim3(grid_of(static_cast<uint64_t>(G.n), 2048)), dim3(256), 0,
+                     s, static_cast<uint64_t>(G.n), pred, half_diag, proof, margin, flags, n_band,
+                     overturned);
+  return hipGetLastError();
 }
 
-hipError_t launch_band_background(const Lattice& L, const McDims& D, const BrickGrid& G,
-                                  const uint8_t* flags, const McBuffers& B, hipStream_t s) {
+hipError_t launch_band_tiles(const DevOp* ops, int n_ops, const ProgramKind& kind,
+                             const Lattice& L, const McDims& D, const BrickGrid& G,
+                             const uint8_t* flags, const McBuffers& B, float* values,
+                             unsigned long long* evaluated, hipStream_t s) {
+  if (!ops || !flags || !B.signs || !evaluated || (D.sign_pitch & 63)) return hipErrorInvalidValue;
+  const int64_t n_tiles = tile_count(L.nx, L.ny, L.nz);
+  if (n_tiles > 0x7fffffff) return hipErrorInvalidValue;
   ResetArgs R;
   R.signs = B.signs;
   R.n_words = D.n_sign_words;
@@ -537,40 +599,27 @@ hipError_t launch_band_background(const Lattice& L, const McDims& D, const Brick
   R.incl = B.incl;
   R.n_blocks = D.n_blocks;
   R.totals = B.totals;
-  int64_t blocks = (D.n_sign_words + 3) / 4;
-  const int64_t min_blocks = (D.n_blocks + 255) / 256;
-  if (blocks > 16384) blocks = 16384;
-  if (blocks < min_blocks) blocks = min_blocks;
-  if (blocks < 1) blocks = 1;
-  hipLaunchKernelGGL(k_band_background, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, L,
-                     G, flags, D.n_points, D.n_sign_words, B.signs, R);
+  const CellSpace C = single_cell_space(L, D, B.signs, ops, n_ops, values, nullptr);
+  const int bounded = kind.bounded && lattice_bounded(L) ? 1 : 0;
+  const dim3 grid(static_cast<unsigned>(n_tiles)), block(64 * kBandWaves);
+  // (without sound bounds the first push must be kept as it is: no shortcut
+  // for it, as the interpreter without a stack takes)
+  if (kind.stack || !bounded)
+    hipLaunchKernelGGL(k_band_tiles<true>, grid, block, 0, s, C, G, bounded, flags,
+                       static_cast<uint32_t>(n_tiles), evaluated, R);
+  else
+    hipLaunchKernelGGL(k_band_tiles<false>, grid, block, 0, s, C, G, bounded, flags,
+                       static_cast<uint32_t>(n_tiles), evaluated, R);
   return hipGetLastError();
 }
 
-hipError_t launch_band_exact(const DevOp* ops, int n_ops, const Lattice& L, const BrickGrid& G,
-                             const uint8_t* flags, const uint32_t* band_list, uint64_t n_band,
-                             const McBuffers& B, float* values, unsigned long long* evaluated,
-                             hipStream_t s) {
-  if (n_band == 0) return hipSuccess;
-  if (!ops || !flags || !band_list || !B.signs || !evaluated) return hipErrorInvalidValue;
-  auto launch = [&](auto kernel, uint64_t group) {
-    uint64_t blocks = (n_band + group - 1) / group;
-    if (blocks > (1u << 20)) blocks = 1u << 20;
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(kExactThreads), 0, s, ops,
-                       n_ops, L, G, flags, band_list, n_band, B.signs, values, evaluated);
-    return hipGetLastError();
-  };
-  if (G.shift == 2) return launch(k_band_exact<2>, ExactShape<2>::kGroupBricks);
-  if (G.shift == 3) return launch(k_band_exact<3>, ExactShape<3>::kGroupBricks);
-  return hipErrorInvalidValue;
-}
-
-hipError_t launch_band_diff(const Lattice& L, const McDims& D, const uint64_t* signs_a,
+hipError_t launch_band_diff(const Lattice& L, const McDims& D, int64_t pitch_a,
+                            const uint64_t* signs_a,
                             const uint64_t* signs_b, unsigned long long* differing,
                             hipStream_t s) {
   if (!signs_a || !signs_b || !differing) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_band_diff, dim3(grid_of(static_cast<uint64_t>(D.n_segs), 16384)),
-                     dim3(256), 0, s, L, D, signs_a, signs_b, differing);
+                     dim3(256), 0, s, L, D, pitch_a, signs_a, signs_b, differing);
   return hipGetLastError();
 }
 

@@ -20,6 +20,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "mc_kernels.h"
 #include "sdf_eval.h"
 #include "sdf_program.h"
 
@@ -543,6 +544,259 @@ __device__ __forceinline__ void sdf_eval_list(OpsPtr ops, int first, const uint1
       }
     }
   }
+}
+
+// A barrier for what the tile's wavefronts exchange in LDS: __syncthreads
+// would also wait for the samples on their way to memory (two microseconds a
+// tile).
+template <int W>
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  if (W > 1) __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Stores the sign words of a 16^3-sample tile at sample s0 (tile tx along x)
+// from its 64 blocks' bits (4^3 samples each, x fastest): 16 bits of each row,
+// four from each block along x.
+__device__ __forceinline__ void store_tile_signs(const CellSpace& C, const uint64_t* s_sign,
+                                                 const int32_t* s0, uint32_t tx, int thread,
+                                                 int threads) {
+  const int32_t ny = static_cast<int32_t>(C.ny), nz = static_cast<int32_t>(C.nz);
+  uint16_t* S = reinterpret_cast<uint16_t*>(const_cast<uint64_t*>(C.signs));
+  for (int r = thread; r < 256; r += threads) {
+    const int ry = r & 15, rz = r >> 4;
+    const int32_t y = s0[1] + ry, z = s0[2] + rz;
+    if (y >= ny || z >= nz) continue;
+    const int b0 = (rz >> 2) * 16 + (ry >> 2) * 4;
+    const int sh = 16 * (rz & 3) + 4 * (ry & 3);
+    uint32_t bits = 0;
+#pragma unroll
+    for (int bx = 0; bx < 4; ++bx)
+      bits |= static_cast<uint32_t>((s_sign[b0 + bx] >> sh) & 0xFull) << (4 * bx);
+    S[(static_cast<int64_t>(z) * ny + y) * (C.sign_pitch >> 4) + tx] = static_cast<uint16_t>(bits);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Evaluation with an error bound (sdf_eval_bound) over a list of operations.
+// ---------------------------------------------------------------------------
+
+// The operations of a bounded program that matter to sdf_eval_bound at points
+// of the box [blo, bhi], for balls of radius `widen` at most: bound_box's, and
+// also the smooth-min operands whose blend its error bound might count (within
+// the blend width, the ball and the errors of either operand, which `mag`, a
+// bound of every coordinate and parameter, bounds in turn).  Returns their
+// number (above `cap`: they do not fit).  *floor_e receives the greatest error
+// bound of any primitive at a point of the box.
+__device__ __forceinline__ int certify_list(OpsPtr ops, int n, const float* blo, const float* bhi,
+                                            float widen, float mag, uint16_t* list, int cap,
+                                            float* floor_e) {
+  constexpr float u = 5.9604645e-08f;  // 2^-24
+  const int lane = __lane_id();
+  ScopeStack scopes;
+  float cl[3] = {blo[0], blo[1], blo[2]}, ch[3] = {bhi[0], bhi[1], bhi[2]};
+  float pe = 0.0f;  // bound of the rounding of the box's translated points
+  float top = kNoBound;  // upper bound of the running value of the current run
+  float worst = 0.0f;
+  int count = 0;
+  // Twice the errors of two operands, a primitive's being at most 64 u (mag +
+  // 2 widen) and each blend adding at most u (10 k + 4 (mag + 2 widen)) to the
+  // running one, and the rounding of the operands' difference.
+  auto room = [&](float k) {
+    const float w = mag + 2.0f * widen;
+    return 2.0f * u * (128.0f * w + static_cast<float>(n) * (10.0f * k + 4.0f * w)) + 16.0f * u * w;
+  };
+  auto far_of = [&](const DevOp& op) {  // greatest |q_c| over the box, and the primitive's error
+    float q = 0.0f;
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+      q = fmaxf(q, fmaxf(-(cl[a] - op.off[a]), ch[a] - op.off[a]));
+    const float qe = op.translated ? pe + u * (q + widen + pe) : pe;
+    const float qmax = q + widen + qe;
+    const float pm = __builtin_fabsf(op.prm[0]) + __builtin_fabsf(op.prm[1]) +
+                     __builtin_fabsf(op.prm[2]) + __builtin_fabsf(op.prm[3]);
+    return 1.7320509f * qe + 16.0f * u * (1.7320509f * qmax + pm);
+  };
+  for (int base = 0; base < n; base += 64) {
+    const int j = base + lane < n ? base + lane : n - 1;
+    const DevOp mine = load_op(ops, j);
+    const int e = n - base < 64 ? n - base : 64;
+    const uint64_t run = __ballot(base + lane < n && mine.code <= kCylinder &&
+                                  (mine.combine == kMin || mine.combine == kSmooth));
+    int p = 0;
+    while (p < e) {
+      const uint64_t from = run >> p;
+      if (from & 1ull) {
+        const int m = ~from ? static_cast<int>(__builtin_ctzll(~from)) : 64;
+        const bool in = lane >= p && lane < p + m;
+        float vlo = kNoBound, vhi = kNoBound, err = 0.0f;
+        if (in) {
+          op_interval(mine, cl, ch, &vlo, &vhi);
+          err = far_of(mine);
+        }
+        const float T = fminf(top, wave_min_before(vhi));
+        const float gap = (vlo - T) * (1.0f - 8.0f * u);
+        const bool idle = mine.combine == kSmooth
+                              ? gap >= (mine.k + 2.0f * widen + room(mine.k)) * (1.0f + 8.0f * u)
+                              : vlo > T;
+        const bool kept = in && !idle;
+        const uint64_t keep = __ballot(kept);
+        if (kept) {
+          const int at = count + static_cast<int>(__popcll(keep & ((1ull << lane) - 1ull)));
+          if (at < cap) list[at] = static_cast<uint16_t>(j);
+        }
+        count += static_cast<int>(__popcll(keep));
+        top = fminf(top, wave_min(vhi));
+        worst = fmaxf(worst, -wave_min(-err));
+        p += m;
+        continue;
+      }
+      const int i = base + p;
+      const DevOp op = load_op(ops, i);
+      ++p;
+      if (op.code <= kCylinder) {
+        float vlo, vhi;
+        op_interval(op, cl, ch, &vlo, &vhi);
+        worst = fmaxf(worst, far_of(op));
+        top = op.combine == kPush ? vhi : kNoBound;  // (after a max: not bounded here)
+      } else if (op.code == kPushTranslate) {
+        scopes.push(i);
+        enter_scope(ops, i, cl, ch);
+        float q = 0.0f;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) q = fmaxf(q, fmaxf(-cl[a], ch[a]));
+        pe = pe + u * (q + widen + pe);
+      } else if (op.code == kPopTranslate) {
+        scopes.pop();
+        restore_scopes(ops, scopes, blo, bhi, cl, ch);
+        // (pe stays at the inner scope's, which is no smaller)
+      } else {
+        top = kNoBound;  // a binary operator's value: not bounded here
+      }
+      if (lane == 0 && count < cap) list[count] = static_cast<uint16_t>(i);
+      ++count;
+    }
+  }
+  *floor_e = worst;
+  return count;
+}
+
+// sdf_eval_bound over the m operations of `list` (certify_list's): its value,
+// and two bounds of its error bound, from the listed operations alone (*e0) and
+// with every operand's error at least floor_e (*e1).
+template <bool kStack>
+__device__ __forceinline__ float eval_bound_list(OpsPtr ops, const uint16_t* list, int m, float px,
+                                                 float py, float pz, float widen, float floor_e,
+                                                 float* e0, float* e1) {
+  constexpr float u = 5.9604645e-08f;  // 2^-24
+  const int lane = __lane_id();
+  float top = 0.0f, a0 = 0.0f, a1 = 0.0f;
+  ShiftStack st, s0, s1;
+#pragma unroll
+  for (int i = 0; i < kMaxValueStack; ++i) st.v[i] = s0.v[i] = s1.v[i] = 0.0f;
+  float c[3] = {px, py, pz}, pe = 0.0f;
+  ScopeStack scopes;
+  bool have_top = false;
+  auto moved = [&](const float* q, float e) {
+    return e + u * (bound_max3(__builtin_fabsf(q[0]), __builtin_fabsf(q[1]), __builtin_fabsf(q[2])) +
+                    widen + e);
+  };
+  auto blend = [&](float a, float ea, float b, float eb, float k) {
+    float e = fmaxf(ea, eb);
+    if (__builtin_fabsf(a - b) < k + 2.0f * widen + 2.0f * (ea + eb) +
+                                     u * (__builtin_fabsf(a) + __builtin_fabsf(b))) {
+      const float mg = fminf(__builtin_fabsf(a), __builtin_fabsf(b)) + widen + e;
+      e += 8.0f * u * k + 2.0f * u * (mg + k);
+    }
+    return e;
+  };
+  for (int base = 0; base < m; base += 64) {
+    const int mine = base + lane < m ? list[base + lane] : 0;
+    const int e = m - base < 64 ? m - base : 64;
+    for (int j = 0; j < e; ++j) {
+      const int i = __builtin_amdgcn_readlane(mine, j);
+      const DevOp op = load_op(ops, i);
+      if (op.code <= kCylinder) {
+        float q[1][3], v[1];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) q[0][a] = c[a] - op.off[a];
+        const float qe = op.translated ? moved(q[0], pe) : pe;
+        prim_values(op.code, op.prm, q, v);
+        const float qmax =
+            bound_max3(__builtin_fabsf(q[0][0]), __builtin_fabsf(q[0][1]),
+                       __builtin_fabsf(q[0][2])) + widen + qe;
+        const float pm = __builtin_fabsf(op.prm[0]) + __builtin_fabsf(op.prm[1]) +
+                         __builtin_fabsf(op.prm[2]) + __builtin_fabsf(op.prm[3]);
+        const float ev = 1.7320509f * qe + 16.0f * u * (1.7320509f * qmax + pm);
+        const float ev1 = fmaxf(ev, floor_e);
+        if (op.combine == kPush) {
+          if (kStack && have_top) {
+            st.push(top);
+            s0.push(a0);
+            s1.push(a1);
+          }
+          top = v[0];
+          a0 = ev;
+          a1 = ev1;
+          have_top = true;
+        } else if (op.combine == kSmooth) {
+          a0 = blend(top, a0, v[0], ev, op.k);
+          a1 = blend(top, a1, v[0], ev1, op.k);
+          top = smooth_min(top, v[0], op.k);
+        } else {
+          if (op.combine == kMin)
+            top = fminf(top, v[0]);
+          else if (op.combine == kMax)
+            top = fmaxf(top, v[0]);
+          else if (op.combine == kDiff)
+            top = fmaxf(v[0], -top);
+          else
+            top = fmaxf(top, -v[0]);
+          a0 = fmaxf(a0, ev);
+          a1 = fmaxf(a1, ev1);
+        }
+      } else if (op.code == kPushTranslate) {
+        scopes.push(i);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) c[a] = c[a] - op.off[a];
+        pe = moved(c, pe);
+      } else if (op.code == kPopTranslate) {
+        scopes.pop();
+        c[0] = px;
+        c[1] = py;
+        c[2] = pz;
+        pe = 0.0f;
+        for (int s = 0; s < scopes.depth; ++s) {
+          const int o = scopes.at(s);
+#pragma unroll
+          for (int a = 0; a < 3; ++a) c[a] = c[a] - ops[o].off[a];
+          pe = moved(c, pe);
+        }
+      } else if (kStack) {
+        const float w = st.pop(), w0 = s0.pop(), w1 = s1.pop();
+        if (op.code == kSmoothUnion) {
+          a0 = blend(w, w0, top, a0, op.k);
+          a1 = blend(w, w1, top, a1, op.k);
+          top = smooth_min(w, top, op.k);
+        } else {
+          if (op.code == kUnion)
+            top = fminf(w, top);
+          else if (op.code == kIntersection)
+            top = fmaxf(w, top);
+          else if (op.code == kDifference)
+            top = fmaxf(top, -w);
+          else
+            top = fmaxf(w, -top);
+          a0 = fmaxf(w0, a0);
+          a1 = fmaxf(w1, a1);
+        }
+      }
+    }
+  }
+  *e0 = a0 * 1.001f;
+  *e1 = a1 * 1.001f;
+  return top;
 }
 
 }  // namespace iso

@@ -19,6 +19,14 @@ bool lattice_bounded(const Lattice& L);
 // Whether the program holds values below the running one.
 bool program_needs_stack(const DevOp* ops, int n_ops);
 
+// What the kernels ask of a program.
+struct ProgramKind {
+  bool bounded = false;    // program_bounded
+  bool stack = false;      // program_needs_stack
+  float magnitude = 0.0f;  // bounds the offsets of its nested scopes, its parameters and widths
+};
+ProgramKind program_kind(const DevOp* ops, int n_ops);
+
 // Whether a program lattice is classified sparsely: sound bounds, rows of at
 // least one tile (narrower ones would leave most of a tile and of a sign word
 // empty), and enough samples.  On a small lattice a tile spans many operands

@@ -42,16 +42,6 @@ constexpr int kTileCoords = kTileSide + 2;  // coordinates along an axis, neighb
 constexpr int kListCap = 512;    // operations of a tile's list; a longer one is not kept
 constexpr uint32_t kSparseXcds = 8;
 
-// A barrier for what the tile's wavefronts exchange in LDS: __syncthreads
-// would also wait for the samples on their way to memory (two microseconds a
-// tile).
-template <int W>
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  if (W > 1) __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // One lattice: its tiles x fastest.
 struct SingleTiles {
   CellSpace C;
@@ -241,20 +231,7 @@ __global__ __launch_bounds__(64 * W) void k_signs_sparse(Tiles tiles, uint32_t n
     if (lane < kPoints) s_sign[slot] = mine;
   }
   lds_barrier<W>();
-  // The tile's rows: 16 bits of row (y, z), four from each brick along x.
-  uint16_t* S = reinterpret_cast<uint16_t*>(const_cast<uint64_t*>(C.signs));
-  for (int r = threadIdx.x; r < kTileSide * kTileSide; r += 64 * W) {
-    const int ry = r & (kTileSide - 1), rz = r >> kTileShift;
-    const int32_t y = s0[1] + ry, z = s0[2] + rz;
-    if (y >= ny || z >= nz) continue;
-    const int b0 = (rz >> 2) * 16 + (ry >> 2) * 4;
-    const int sh = 16 * (rz & 3) + 4 * (ry & 3);
-    uint32_t bits = 0;
-#pragma unroll
-    for (int bx = 0; bx < 4; ++bx)
-      bits |= static_cast<uint32_t>((s_sign[b0 + bx] >> sh) & 0xFull) << (4 * bx);
-    S[(static_cast<int64_t>(z) * ny + y) * (C.sign_pitch >> 4) + tx] = static_cast<uint16_t>(bits);
-  }
+  store_tile_signs(C, s_sign, s0, tx, threadIdx.x, 64 * W);
 }
 
 // Blocks that cover n tiles in groups dealt to the XCDs round robin.
@@ -318,6 +295,22 @@ bool program_needs_stack(const DevOp* ops, int n_ops) {
   int pushes = 0;
   for (int i = 0; i < n_ops; ++i) pushes += ops[i].code <= kCylinder && ops[i].combine == kPush;
   return pushes > 1;
+}
+
+ProgramKind program_kind(const DevOp* ops, int n_ops) {
+  ProgramKind K;
+  K.bounded = program_bounded(ops, n_ops);
+  K.stack = program_needs_stack(ops, n_ops);
+  double off = 0.0, prm = 0.0;
+  for (int i = 0; i < n_ops; ++i) {
+    for (int a = 0; a < 3; ++a) off = std::fmax(off, std::fabs(static_cast<double>(ops[i].off[a])));
+    double p = std::fabs(static_cast<double>(ops[i].k));
+    for (int a = 0; a < 4; ++a) p += std::fabs(static_cast<double>(ops[i].prm[a]));
+    prm = std::fmax(prm, p);
+  }
+  // a point moves by the open scopes' offsets and the primitive's own
+  K.magnitude = static_cast<float>((kMaxPointStack + 1) * off + prm);
+  return K;
 }
 
 hipError_t launch_signs_sparse(const DevOp* ops, int n_ops, bool stack, const Lattice& L,
