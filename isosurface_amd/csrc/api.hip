@@ -2255,13 +2255,14 @@ int iso_band_predict(iso_ctx* c, const float* points, uint64_t n, float* out, in
   return ISO_OK;
 }
 
-// Words of the band's counters: bricks in the band, network culls overturned,
-// cells that differ from the dense classification; then the spread counters
-// of exact samples and of certificate centres.
-constexpr int kBandBricks = 0, kBandOverturned = 1, kBandDiffering = 2;
+// Words of the band's counters: cells that differ from the dense
+// classification, then the spread counters of exact samples, certificate
+// centres, bricks in the band and network culls overturned.
+constexpr int kBandDiffering = 0;
 constexpr int kBandSpread = iso::kCounterLines * iso::kCounterStride;
 constexpr int kBandExact = iso::kCounterStride, kBandCentre = kBandExact + kBandSpread;
-constexpr int kBandCounters = kBandCentre + kBandSpread;
+constexpr int kBandBricks = kBandCentre + kBandSpread, kBandOverturned = kBandBricks + kBandSpread;
+constexpr int kBandCounters = kBandOverturned + kBandSpread;
 
 int iso_extract_mc_band(iso_ctx* c, const iso_grid_desc* desc, float margin, uint32_t flags,
                         iso_mesh_out* out, iso_band_stats* stats) {
@@ -2351,10 +2352,10 @@ int iso_extract_mc_band(iso_ctx* c, const iso_grid_desc* desc, float margin, uin
       return sum;
     };
     stats->bricks = nb;
-    stats->band_bricks = h[kBandBricks];
+    stats->band_bricks = spread(kBandBricks);
     stats->exact_samples = spread(kBandExact);
     stats->centre_samples = spread(kBandCentre);
-    stats->overturned_culls = h[kBandOverturned];
+    stats->overturned_culls = spread(kBandOverturned);
   }
   return st;
 }

@@ -81,7 +81,8 @@ hipError_t launch_brick_certify(const DevOp* ops, int n_ops, const ProgramKind& 
 // `proof` (launch_brick_certify's flags), a brick leaves the band only when
 // its proof allows it, whatever the network predicted, and a brick the
 // network culled that its proof does not allow is counted in *overturned.
-// *n_band receives the number of band bricks (both are added to).
+// *n_band receives the number of band bricks (both are spread counters, added
+// to).
 hipError_t launch_brick_flags(const BrickGrid& G, const float* pred, const float* half_diag,
                               const uint8_t* proof, float margin, uint8_t* flags,
                               unsigned long long* n_band, unsigned long long* overturned,

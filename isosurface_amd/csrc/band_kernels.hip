@@ -213,7 +213,10 @@ __global__ __launch_bounds__(256) void k_brick_flags(
     uint64_t n, const float* __restrict__ pred, const float* __restrict__ half_diag,
     const uint8_t* __restrict__ proof, float margin, uint8_t* __restrict__ flags,
     unsigned long long* n_band, unsigned long long* overturned) {
+  __shared__ uint32_t s_sum[2];
   uint32_t bands = 0, turned = 0;
+  if (threadIdx.x < 2) s_sum[threadIdx.x] = 0;
+  __syncthreads();
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
   for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
        i += stride) {
@@ -240,9 +243,14 @@ __global__ __launch_bounds__(256) void k_brick_flags(
     turned += __shfl_xor(turned, d, 64);
   }
   if (__lane_id() == 0) {
-    if (bands) atomicAdd(n_band, static_cast<unsigned long long>(bands));
-    if (turned) atomicAdd(overturned, static_cast<unsigned long long>(turned));
+    atomicAdd(&s_sum[0], bands);
+    atomicAdd(&s_sum[1], turned);
   }
+  __syncthreads();
+  const int line = kCounterStride * (blockIdx.x % kCounterLines);
+  if (threadIdx.x == 0 && s_sum[0]) atomicAdd(n_band + line, static_cast<unsigned long long>(s_sum[0]));
+  if (threadIdx.x == 1 && s_sum[1])
+    atomicAdd(overturned + line, static_cast<unsigned long long>(s_sum[1]));
 }
 
 // Signs and exact samples of one 16^3-sample tile (sparse_kernels.h) of the
@@ -315,38 +323,55 @@ __global__ __launch_bounds__(64 * kBandWaves) void k_band_tiles(
   if (threadIdx.x < kTileSamples / 64) s_from[threadIdx.x] = 0ull;
   const bool work = __syncthreads_or(any) != 0;
 
-  // Each block of 4^3 samples, a wavefront at a time: signs of the samples
-  // that are not exact, the others queued.
-  const int l[3] = {lane & 3, (lane >> 2) & 3, lane >> 4};
-  for (int blk = wv; blk < kTileBlocks; blk += kBandWaves) {
-    const int o[3] = {4 * (blk & 3), blk & 12, 4 * (blk >> 4)};
-    int hi[3], lo[3];
-    bool valid = true;
+  // Lane b looks at block b (4^3 samples): bit k of its word says whether the
+  // brick that holds a sample on the block's low faces along the axes of k is
+  // in the band (bit 0: the block's own brick), bit 8 the own brick's sign.
+  uint32_t around = 0;
+  {
+    int own[3], low[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      const int32_t s = s0[a] + o[a] + l[a];
-      valid = valid && s < n[a];
-      const int32_t own = s >> G.shift;
+      const int32_t s = s0[a] + (a == 0 ? 4 * (lane & 3) : a == 1 ? lane & 12 : 4 * (lane >> 4));
       const int32_t first = (s0[a] >> G.shift) - 1;
-      hi[a] = (own < nb[a] ? own : nb[a] - 1) - first;
-      lo[a] = (s & (G.brick - 1)) == 0 && s > 0 ? own - 1 - first : hi[a];
-      if (!valid) hi[a] = lo[a] = 0;
+      const int32_t b = s >> G.shift;
+      // (blocks past the lattice: any entry)
+      own[a] = (b < nb[a] ? b : nb[a] - 1) - first;
+      if (own[a] < 0) own[a] = 0;
+      low[a] = (s & (G.brick - 1)) == 0 && s > 0 && b <= nb[a] ? b - 1 - first : own[a];
     }
-    const uint8_t mine = s_flag[(hi[2] * per + hi[1]) * per + hi[0]];
-    bool exact = false;
-    if (work) {
 #pragma unroll
-      for (int k = 0; k < 8; ++k)
-        exact |= (s_flag[((k & 4 ? lo[2] : hi[2]) * per + (k & 2 ? lo[1] : hi[1])) * per +
-                         (k & 1 ? lo[0] : hi[0])] &
-                  kBrickBand) != 0;
-      exact = exact && valid;
+    for (int k = 0; k < 8; ++k) {
+      const uint8_t f = s_flag[((k & 4 ? low[2] : own[2]) * per + (k & 2 ? low[1] : own[1])) * per +
+                               (k & 1 ? low[0] : own[0])];
+      around |= (f & kBrickBand ? 1u : 0u) << k;
+      if (k == 0) around |= (f & kBrickInside ? 1u : 0u) << 8;
     }
-    const uint64_t in = __ballot(valid && !exact && (mine & kBrickInside));
+  }
+  if (!work) {
+    if (wv == 0) s_sign[lane] = around & 256u ? ~0ull : 0ull;
+    __syncthreads();
+    store_tile_signs(C, s_sign, s0, tx, threadIdx.x, 64 * kBandWaves);
+    return;
+  }
+  // Each block, a wavefront at a time: signs of the samples that are not
+  // exact, the others queued.
+  const int l[3] = {lane & 3, (lane >> 2) & 3, lane >> 4};
+  uint32_t held = 0;  // the bits of a block's word whose bricks hold this lane's sample
+#pragma unroll
+  for (int k = 0; k < 8; ++k)
+    held |= (!(k & 1) || l[0] == 0) && (!(k & 2) || l[1] == 0) && (!(k & 4) || l[2] == 0) ? 1u << k : 0u;
+  const bool full =
+      s0[0] + kTileSide <= n[0] && s0[1] + kTileSide <= n[1] && s0[2] + kTileSide <= n[2];
+  for (int blk = wv; blk < kTileBlocks; blk += kBandWaves) {
+    const uint32_t w = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(around), blk));
+    const bool valid = full || (s0[0] + 4 * (blk & 3) + l[0] < n[0] &&
+                                s0[1] + (blk & 12) + l[1] < n[1] &&
+                                s0[2] + 4 * (blk >> 4) + l[2] < n[2]);
+    const bool exact = valid && (w & held & 255u) != 0u;
     const uint64_t m = __ballot(exact);
     uint32_t at = 0;
     if (lane == 0) {
-      s_sign[blk] = in;
+      s_sign[blk] = w & 256u ? ~m : 0ull;
       if (m) {
         const uint32_t cnt = static_cast<uint32_t>(__popcll(m));
         at = atomicAdd(&s_n, cnt);
@@ -354,6 +379,7 @@ __global__ __launch_bounds__(64 * kBandWaves) void k_band_tiles(
         atomicOr(reinterpret_cast<unsigned long long*>(&s_from[(at + cnt - 1) >> 6]), 1ull << blk);
       }
     }
+    if (m == 0ull) continue;
     at = __builtin_amdgcn_readfirstlane(at);
     if (exact)
       s_queue[at + static_cast<uint32_t>(__popcll(m & ((1ull << lane) - 1ull)))] =
