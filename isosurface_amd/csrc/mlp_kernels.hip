@@ -5,23 +5,21 @@
 //   A operand: lane l holds A[l % 16][4 (l / 16) + j], j = 0..3
 //   B operand: lane l holds B[4 (l / 16) + j][l % 16]
 //   D result:  lane l holds D[4 (l / 16) + j][l % 16]
-// The inference forward uses gfx950's double-K form
-// (v_mfma_f32_16x16x32_bf16: lane l holds K values 8 (l / 16) + j,
-// j = 0..7) on two adjacent 16-wide K blocks at once: lane l passes its
-// four values of block 2i then its four of block 2i+1, for A and B alike,
-// which the instruction reads as one 32-wide block with its K index
+// gfx950's double-K form (v_mfma_f32_16x16x32_bf16: lane l holds K values
+// 8 (l / 16) + j, j = 0..7) takes two adjacent 16-wide K blocks at once: lane l
+// passes its four values of block 2i then its four of block 2i+1, for A and B
+// alike, which the instruction reads as one 32-wide block with its K index
 // permuted the same way in both operands — the same sum of products.
-// Its features come in another row order than training's (F1I, see
-// mlp_kernels.h): in each K block every lane evaluates the same function
-// (sin or cos of one coordinate) at its own frequencies, c_k = 2^(k / 2) / 2
-// for k = 4 j + g, g = l / 16, i.e. c_g 4^j with c_g a power-of-two multiple
-// of 1/2 or of sqrt(2)/2 — the same f32 multipliers, so the same features.
+// In each K block of features every lane evaluates the same function (sin or
+// cos of one coordinate) at its own frequencies, c_k = 2^(k / 2) / 2 for
+// k = 4 j + g, g = l / 16, i.e. c_g 4^j with c_g a power-of-two multiple of
+// 1/2 or of sqrt(2)/2.
 // A wavefront pushes 16 samples (the N dimension) through the network:
 // layer outputs land in exactly the layout the next layer's B operand
 // needs, so activations stay in registers from the features to the output.
-// The backward-data pass uses the same layout with W^T fragments; weight
-// gradients are products over the batch of hidden-major bf16 activations
-// (split over the batch, accumulated with f32 atomics).
+// The backward-data pass uses the same layout with W^T fragments.  Weight
+// gradients are products over the samples: the workgroup's 64 samples meet in
+// LDS, unit by unit, which is the layout of both their operands.
 #include <hip/hip_runtime.h>
 
 #include "mlp_kernels.h"
@@ -33,14 +31,6 @@ namespace {
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// c_k = 2^(k / 2) / 2 revolutions per unit (2 pi c_k = pi 2^(k / 2)),
-// rounded to f32: powers of two for even k, sqrt(2) scaled for odd k.
-__constant__ float c_rev[kFreq] = {
-    0x1p-1f, 0x1.6a09e6p-1f, 0x1p+0f, 0x1.6a09e6p+0f,
-    0x1p+1f, 0x1.6a09e6p+1f, 0x1p+2f, 0x1.6a09e6p+2f,
-    0x1p+3f, 0x1.6a09e6p+3f, 0x1p+4f, 0x1.6a09e6p+4f,
-    0x1p+5f, 0x1.6a09e6p+5f, 0x1p+6f, 0x1.6a09e6p+6f};
 
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x4v __attribute__((ext_vector_type(4)));
@@ -75,137 +65,82 @@ __device__ __forceinline__ bf16x4 pack4f(float a, float b, float c, float d) {
   return __builtin_bit_cast(bf16x4, __builtin_convertvector(f32x4v{a, b, c, d}, bf16x4v));
 }
 
-__device__ __forceinline__ bf16x4 pack4(uint16_t a, uint16_t b, uint16_t c, uint16_t d) {
-  bf16x4 r;
-  r[0] = static_cast<short>(a);
-  r[1] = static_cast<short>(b);
-  r[2] = static_cast<short>(c);
-  r[3] = static_cast<short>(d);
-  return r;
-}
-
-// Feature fi (0..111) of point p: p_d, sin(2 pi r), cos(2 pi r) with
-// r = c_k p_d in revolutions, zero padding.  v_sin_f32 / v_cos_f32 take
-// revolutions; the fractional part of an f32 r is exact, so reducing r to
-// it first changes nothing and keeps every argument in their input range.
-__device__ __forceinline__ float feature(int fi, float px, float py, float pz) {
-  if (fi < 3) return fi == 0 ? px : (fi == 1 ? py : pz);
-  if (fi >= kFeat) return 0.0f;
-  const int q = fi - 3;
-  const int k = q / 6, r = q - 6 * k;
-  const int d = r < 3 ? r : r - 3;
-  // the fractional part (exact) keeps the argument in the instructions' range
-  const float rev = __builtin_amdgcn_fractf(c_rev[k] * (d == 0 ? px : (d == 1 ? py : pz)));
-  return r < 3 ? __builtin_amdgcn_sinf(rev) : __builtin_amdgcn_cosf(rev);
-}
-
 // Fragments of one 16-row block set, read from LDS: lane's 4 bf16 of block (mb, kb).
 __device__ __forceinline__ bf16x4 frag(const uint16_t* F, int n_kb, int mb, int kb, int lane) {
   const uint16_t* p = F + ((mb * n_kb + kb) * 64 + lane) * 4;
   return *reinterpret_cast<const bf16x4*>(p);
 }
 
-struct Tile {
-  bf16x4 h1[4], h2[4], h3[4];  // activations (B layout of the next layer), bf16
-  float f;                     // output of this lane's sample
-};
-
-// Training forward pass of 16 samples; lane l's sample is l % 16 at
-// (px, py, pz).  sF: fragments F1 F2 F3 in LDS; sB: b1 b2 b3 w4 b4 in LDS.
-// Layer 1 consumes the features one K-block at a time (computed just in
-// time, and stored hidden-major to xdst[row * n + s] when xdst is given).
-__device__ __forceinline__ void forward_tile(const uint16_t* sF, const float* sB, float px,
-                                             float py, float pz, int lane, Tile& T,
-                                             uint16_t* xdst, int64_t n, int64_t s) {
-  const int r0 = 4 * (lane >> 4);
-  const uint16_t* F1 = sF + kFragF1;
-  const uint16_t* F2 = sF + kFragF2;
-  const uint16_t* F3 = sF + kFragF3;
-  const float* b1 = sB;
-  const float* b2 = sB + kHidden;
-  const float* b3 = sB + 2 * kHidden;
-  const float* w4 = sB + 3 * kHidden;
-  const float b4 = sB[4 * kHidden];
-  f32x4 acc1[4];
+// A lane's four features of K block kb for the point q (see the tiling note).
+__device__ __forceinline__ bf16x4 features(const float* q, int kb, int lane) {
+  const int g = lane >> 4;
+  const float cg = __builtin_amdgcn_ldexpf((g & 1) ? 0x1.6a09e6p-1f : 0x1p-1f, g >> 1);
+  float xf[4];
+  if (kb < 6) {
+    const float m = cg * q[kb % 3];  // c_k q for j = 0
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb) acc1[mb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  auto features = [&](int kb) {
-    const int f0 = 16 * kb + r0;
-    uint16_t xb[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) xb[j] = to_bf16(feature(f0 + j, px, py, pz));
-    if (xdst) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) xdst[(f0 + j) * n + s] = xb[j];
+    for (int j = 0; j < 4; ++j) {
+      // c_g 4^j q: a power-of-two scaling of m, exact.  v_sin_f32 / v_cos_f32
+      // take revolutions; the fraction of an f32 is exact, so reducing to it
+      // changes nothing and keeps the argument in their input range.
+      const float rev = __builtin_amdgcn_fractf(m * static_cast<float>(1 << (2 * j)));
+      xf[j] = kb < 3 ? __builtin_amdgcn_sinf(rev) : __builtin_amdgcn_cosf(rev);
     }
-    return pack4(xb[0], xb[1], xb[2], xb[3]);
-  };
-#pragma unroll 1
-  for (int kb = 0; kb < kKB1; ++kb) {
-    const bf16x4 x = features(kb);
+  } else {
 #pragma unroll
-    for (int mb = 0; mb < 4; ++mb) acc1[mb] = mfma(frag(F1, kKB1, mb, kb, lane), x, acc1[mb]);
+    for (int j = 0; j < 4; ++j) xf[j] = g == 0 && j < 3 ? q[j] : 0.0f;
   }
-  // A 64-wide K product: four MFMAs.
-  auto product64 = [&](const uint16_t* F, int mb, const bf16x4* h) {
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) acc = mfma(frag(F, 4, mb, kb, lane), h[kb], acc);
-    return acc;
-  };
-  // Bias, ReLU and the bf16 rounding of a layer's 16 x 16 output block.
-  auto activate = [&](const f32x4& acc, const float* b) {
-    return pack4f(fmaxf(acc[0] + b[r0 + 0], 0.0f), fmaxf(acc[1] + b[r0 + 1], 0.0f),
-                  fmaxf(acc[2] + b[r0 + 2], 0.0f), fmaxf(acc[3] + b[r0 + 3], 0.0f));
-  };
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb) T.h1[mb] = activate(acc1[mb], b1 + 16 * mb);
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb) T.h2[mb] = activate(product64(F2, mb, T.h1), b2 + 16 * mb);
-  float part = 0.0f;
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb) {
-    T.h3[mb] = activate(product64(F3, mb, T.h2), b3 + 16 * mb);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      part += w4[16 * mb + r0 + j] * from_bf16(static_cast<uint16_t>(T.h3[mb][j]));
-  }
-  // The four lanes of a sample (l, l^16, l^32, l^48) hold its 64 terms.
-  part += __shfl_xor(part, 16, 64);
-  part += __shfl_xor(part, 32, 64);
-  T.f = part + b4;
+  return pack4f(xf[0], xf[1], xf[2], xf[3]);
+}
+
+// Bias, ReLU and the bf16 rounding of a layer's 16 x 16 output block (b: the
+// block's bias rows).
+__device__ __forceinline__ bf16x4 activate(const f32x4& acc, const float* b, int r0) {
+  return pack4f(fmaxf(acc[0] + b[r0 + 0], 0.0f), fmaxf(acc[1] + b[r0 + 1], 0.0f),
+                fmaxf(acc[2] + b[r0 + 2], 0.0f), fmaxf(acc[3] + b[r0 + 3], 0.0f));
 }
 
 constexpr int kThreads = 256;
-constexpr int kLdsFrags = kFragT3;  // forward fragments only (F1I F2 F3)
+constexpr int kLdsFrags = kFragT2;  // forward fragments only (F1 F2 F3)
 
-// Loads fragments [0, n_frag) and the bias block into LDS.
-__device__ __forceinline__ void load_model(const Model& M, uint16_t* sF, int n_frag, float* sB) {
-  const uint32_t* src = reinterpret_cast<const uint32_t*>(M.frags);
-  uint32_t* dst = reinterpret_cast<uint32_t*>(sF);
-  for (int i = threadIdx.x; i < n_frag / 2; i += blockDim.x) dst[i] = src[i];
-  for (int i = threadIdx.x; i < 4 * kHidden + 1; i += blockDim.x) {
-    // b1 b2 b3 w4 b4
-    const int which = i / kHidden, k = i - which * kHidden;
-    const int off = which == 0 ? kOffB1 : which == 1 ? kOffB2 : which == 2 ? kOffB3 : kOffW4;
-    sB[i] = i == 4 * kHidden ? M.theta[kOffB4] : M.theta[off + k];
+// Loads the first kN fragments and the bias block into LDS, with kT threads:
+// every load is issued before the first is stored.
+template <int kN, int kT>
+__device__ __forceinline__ void load_model(const Model& M, uint16_t* sF, float* sB) {
+  static_assert(kN % 8 == 0, "16-byte loads");
+  constexpr int n = kN / 8, kRounds = (n + kT - 1) / kT;
+  const uint4* src = reinterpret_cast<const uint4*>(M.frags);
+  uint4* dst = reinterpret_cast<uint4*>(sF);
+  const int t = static_cast<int>(threadIdx.x);
+  uint4 v[kRounds];
+#pragma unroll
+  for (int i = 0; i < kRounds; ++i) {
+    const int at = t + i * kT;
+    v[i] = src[at < n ? at : 0];
   }
+  // b1 b2 b3 w4 b4
+  const int which = (t & 255) >> 6, k = t & 63;
+  const int off = which == 0 ? kOffB1 : which == 1 ? kOffB2 : which == 2 ? kOffB3 : kOffW4;
+  static_assert(kHidden == 64 && kT >= 4 * kHidden, "one bias a thread");
+  const float bias = M.theta[off + k], last = M.theta[kOffB4];
+#pragma unroll
+  for (int i = 0; i < kRounds; ++i) {
+    const int at = t + i * kT;
+    if (at < n) dst[at] = v[i];
+  }
+  if (t < 4 * kHidden) sB[t] = bias;
+  if (t == 0) sB[4 * kHidden] = last;
 }
 
 // Inference forward of kT 16-sample tiles at once: every weight fragment
 // read from LDS feeds all kT tiles' MFMAs, 1/kT of the LDS traffic per
 // sample of one tile at a time.  Pairs of K blocks go through double-K
-// MFMAs.  The features come in the inference order of F1I: block kb < 6
-// holds function kb (sin of x, y, z, then cos) at the lane's four
-// frequencies, block 6 the coordinates (rows 0-2 of lanes 0-15) and
-// padding.  p[t]: this lane's sample of tile t (lane l's sample is l % 16);
+// MFMAs.  p[t]: this lane's sample of tile t (lane l's sample is l % 16);
 // f[t]: its output.
 template <int kT>
 __device__ __forceinline__ void forward_tiles(const uint16_t* sF, const float* sB,
                                               const float (*p)[3], int lane, float* f) {
   const int r0 = 4 * (lane >> 4);
-  const int g = lane >> 4;
-  const float cg = __builtin_amdgcn_ldexpf((g & 1) ? 0x1.6a09e6p-1f : 0x1p-1f, g >> 1);
   const uint16_t* F1 = sF + kFragF1;
   const uint16_t* F2 = sF + kFragF2;
   const uint16_t* F3 = sF + kFragF3;
@@ -214,27 +149,6 @@ __device__ __forceinline__ void forward_tiles(const uint16_t* sF, const float* s
   const float* b3 = sB + 2 * kHidden;
   const float* w4 = sB + 3 * kHidden;
   const float b4 = sB[4 * kHidden];
-  auto feats = [&](const float* q, int kb) {
-    float xf[4];
-    if (kb < 6) {
-      const float m = cg * q[kb % 3];  // c_k q for j = 0
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        // c_g 4^j q: a power-of-two scaling of m, exact
-        const float rev = __builtin_amdgcn_fractf(m * static_cast<float>(1 << (2 * j)));
-        xf[j] = kb < 3 ? __builtin_amdgcn_sinf(rev) : __builtin_amdgcn_cosf(rev);
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) xf[j] = g == 0 && j < 3 ? q[j] : 0.0f;
-    }
-    return pack4f(xf[0], xf[1], xf[2], xf[3]);
-  };
-  // Bias, ReLU and the bf16 rounding of a layer's 16 x 16 output block.
-  auto activate = [&](const f32x4& acc, const float* b) {
-    return pack4f(fmaxf(acc[0] + b[r0 + 0], 0.0f), fmaxf(acc[1] + b[r0 + 1], 0.0f),
-                  fmaxf(acc[2] + b[r0 + 2], 0.0f), fmaxf(acc[3] + b[r0 + 3], 0.0f));
-  };
   f32x4 z[kT][4];
 #pragma unroll
   for (int t = 0; t < kT; ++t)
@@ -245,8 +159,8 @@ __device__ __forceinline__ void forward_tiles(const uint16_t* sF, const float* s
     bf16x4 x0[kT], x1[kT];
 #pragma unroll
     for (int t = 0; t < kT; ++t) {
-      x0[t] = feats(p[t], kb);
-      x1[t] = feats(p[t], kb + 1);
+      x0[t] = features(p[t], kb, lane);
+      x1[t] = features(p[t], kb + 1, lane);
     }
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb) {
@@ -258,7 +172,7 @@ __device__ __forceinline__ void forward_tiles(const uint16_t* sF, const float* s
   if (kKB1 & 1) {
     bf16x4 x[kT];
 #pragma unroll
-    for (int t = 0; t < kT; ++t) x[t] = feats(p[t], kKB1 - 1);
+    for (int t = 0; t < kT; ++t) x[t] = features(p[t], kKB1 - 1, lane);
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb) {
       const bf16x4 w = frag(F1, kKB1, mb, kKB1 - 1, lane);
@@ -270,7 +184,7 @@ __device__ __forceinline__ void forward_tiles(const uint16_t* sF, const float* s
 #pragma unroll
   for (int t = 0; t < kT; ++t)
 #pragma unroll
-    for (int mb = 0; mb < 4; ++mb) h[t][mb] = activate(z[t][mb], b1 + 16 * mb);
+    for (int mb = 0; mb < 4; ++mb) h[t][mb] = activate(z[t][mb], b1 + 16 * mb, r0);
   // Hidden layers 2 and 3 (W2, W3): 64-wide K, two double-K MFMAs a block.
   auto layer = [&](const uint16_t* F, const float* b) {
     bf16x4 y[kT][4];
@@ -286,7 +200,7 @@ __device__ __forceinline__ void forward_tiles(const uint16_t* sF, const float* s
         for (int t = 0; t < kT; ++t) a[t] = mfma2(w0, w1, h[t][kp], h[t][kp + 1], a[t]);
       }
 #pragma unroll
-      for (int t = 0; t < kT; ++t) y[t][mb] = activate(a[t], b + 16 * mb);
+      for (int t = 0; t < kT; ++t) y[t][mb] = activate(a[t], b + 16 * mb, r0);
     }
 #pragma unroll
     for (int t = 0; t < kT; ++t)
@@ -320,15 +234,7 @@ __global__ __launch_bounds__(kFwdThreads) void k_forward(Model M, const float* _
                                                          int64_t n, float* __restrict__ out) {
   __shared__ __align__(16) uint16_t sF[kLdsFrags];
   __shared__ float sB[4 * kHidden + 1];
-  // F1I in F1's place, then F2 F3, and the bias block
-  {
-    const uint32_t* f1 = reinterpret_cast<const uint32_t*>(M.frags + kFragF1I);
-    const uint32_t* f23 = reinterpret_cast<const uint32_t*>(M.frags + kFragF2);
-    uint32_t* dst = reinterpret_cast<uint32_t*>(sF);
-    constexpr int n1 = (kFragF2 - kFragF1) / 2, n = kLdsFrags / 2;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) dst[i] = i < n1 ? f1[i] : f23[i - n1];
-  }
-  load_model(M, sF, 0, sB);
+  load_model<kLdsFrags, kFwdThreads>(M, sF, sB);
   __syncthreads();
   const int lane = __lane_id();
   const int64_t wave = static_cast<int64_t>(blockIdx.x) * (kFwdThreads / 64) + (threadIdx.x >> 6);
@@ -367,187 +273,244 @@ __device__ __forceinline__ uint32_t hash32(uint32_t a, uint32_t b, uint32_t c) {
   return h;
 }
 
-// Forward + backward-data of a batch; writes hidden-major activations and
-// per-sample dL/df, accumulates the loss.
-__global__ __launch_bounds__(kThreads) void k_train_fb(Model M, Batch B, Samples S,
-                                                       uint32_t step) {
-  __shared__ __align__(16) uint16_t sF[kTrainFrags];
+// Forward and backward of one batch.  A workgroup takes kGroup samples at a
+// time: each of its four wavefronts runs 16 of them forward and back through
+// the data path in registers, leaving the bf16 activations and their
+// derivatives in LDS, unit by unit; then wavefront w multiplies rows 16w..16w+15
+// of every layer's derivatives with the layer's inputs over the 64 samples
+// (15 blocks of 16 x 16, accumulated in registers over the workgroup's
+// groups).  Its gradient goes to a row of its own: no atomics, and the same
+// sums on every run.  Bound by the latency of one wavefront's chain on each
+// SIMD (a batch of 16384 is one group a CU): 21 us a step with the Adam
+// kernel, where activations through memory, their re-reading by one wavefront
+// per block and f32 atomics took 73 us.
+constexpr int kPitch = kGroup + 8;  // samples of an LDS row: 16-byte rows, spread over the banks
+constexpr int kRowX = 0, kRowH1 = kRowX + kFeatPad, kRowH2 = kRowH1 + kHidden,
+              kRowH3 = kRowH2 + kHidden, kRowD1 = kRowH3 + kHidden, kRowD2 = kRowD1 + kHidden,
+              kRowD3 = kRowD2 + kHidden, kLdsRows = kRowD3 + kHidden;
+
+__global__ __launch_bounds__(kThreads) void k_train(Model M, Batch B, Samples S, uint32_t step) {
+  __shared__ __align__(16) uint16_t sF[kFrags];
+  __shared__ __align__(16) uint16_t sA[kLdsRows * kPitch];
   __shared__ float sB[4 * kHidden + 1];
-  load_model(M, sF, kTrainFrags, sB);
-  __syncthreads();
+  __shared__ float sG[kGroup];
+  __shared__ float sSum[2][kThreads / 64];
+  load_model<kFrags, kThreads>(M, sF, sB);
   const int lane = __lane_id();
+  const int wv = static_cast<int>(threadIdx.x >> 6);
   const int r0 = 4 * (lane >> 4);
   const int col = lane & 15;
-  const int64_t wave = static_cast<int64_t>(blockIdx.x) * (kThreads / 64) + (threadIdx.x >> 6);
-  const int64_t n_waves = static_cast<int64_t>(gridDim.x) * (kThreads / 64);
   const float* w4 = sB + 3 * kHidden;
   const float inv_n = 1.0f / static_cast<float>(B.n);
-  float loss = 0.0f;
-  for (int64_t t0 = wave * 16; t0 < B.n; t0 += n_waves * 16) {
-    const int64_t s = t0 + col;  // batch sample (B.n is a multiple of 16)
-    const uint64_t src =
-        S.gather ? hash32(S.seed, step, static_cast<uint32_t>(s)) % S.count
-                 : static_cast<uint64_t>(s);
-    const float px = S.points[3 * src], py = S.points[3 * src + 1], pz = S.points[3 * src + 2];
-    const float t = fminf(fmaxf(S.sdf[src], -S.clamp), S.clamp);
-    const float wgt = S.weight ? S.weight[src] : 1.0f;
-    Tile T;
-    forward_tile(sF, sB, px, py, pz, lane, T, B.x, B.n, s);
+  const int64_t n_groups = (B.n + kGroup - 1) / kGroup;
+  // rows first + 4 (lane / 16) + j of an LDS block, this wavefront's sample col
+  auto keep = [&](int first, const bf16x4& v) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      sA[(first + r0 + j) * kPitch + 16 * wv + col] = static_cast<uint16_t>(v[j]);
+  };
+  f32x4 acc1[kKB1], acc2[4], acc3[4];  // rows 16 wv of dW1, dW2, dW3
+#pragma unroll
+  for (int i = 0; i < kKB1; ++i) acc1[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc2[i] = acc3[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  float unit_sum = 0.0f;             // this thread's bias or output weight
+  float loss = 0.0f, g_sum = 0.0f;  // lanes 0..15
+  for (int64_t grp = blockIdx.x; grp < n_groups; grp += gridDim.x) {
+    __syncthreads();  // the fragments are there; the last group's rows are read
+    const int64_t s = grp * kGroup + 16 * wv + col;
+    const bool live = s < B.n;  // (the same for a whole wavefront)
+    float q[3] = {0.0f, 0.0f, 0.0f}, t = 0.0f, wgt = 0.0f;
+    if (live) {
+      uint64_t src = static_cast<uint64_t>(s);
+      if (S.gather) {
+        const uint32_t h = hash32(S.seed, step, static_cast<uint32_t>(s));
+        src = S.count > 0xffffffffull ? h : h % static_cast<uint32_t>(S.count);
+      }
+      q[0] = S.points[3 * src];
+      q[1] = S.points[3 * src + 1];
+      q[2] = S.points[3 * src + 2];
+      t = fminf(fmaxf(S.sdf[src], -S.clamp), S.clamp);
+      wgt = S.weight ? S.weight[src] : 1.0f;
+    }
+    // forward
+    bf16x4 h1[4], h2[4], h3[4];
+    {
+      f32x4 z[4];
+#pragma unroll
+      for (int mb = 0; mb < 4; ++mb) z[mb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int kb = 0; kb + 1 < kKB1; kb += 2) {
+        const bf16x4 x0 = features(q, kb, lane), x1 = features(q, kb + 1, lane);
+        keep(kRowX + 16 * kb, x0);
+        keep(kRowX + 16 * kb + 16, x1);
+#pragma unroll
+        for (int mb = 0; mb < 4; ++mb)
+          z[mb] = mfma2(frag(sF + kFragF1, kKB1, mb, kb, lane),
+                        frag(sF + kFragF1, kKB1, mb, kb + 1, lane), x0, x1, z[mb]);
+      }
+      static_assert(kKB1 & 1, "the last feature block stands alone");
+      const bf16x4 x = features(q, kKB1 - 1, lane);
+      keep(kRowX + 16 * (kKB1 - 1), x);
+#pragma unroll
+      for (int mb = 0; mb < 4; ++mb) {
+        z[mb] = mfma(frag(sF + kFragF1, kKB1, mb, kKB1 - 1, lane), x, z[mb]);
+        h1[mb] = activate(z[mb], sB + 16 * mb, r0);
+        keep(kRowH1 + 16 * mb, h1[mb]);
+      }
+    }
+    // A 64-wide K product with fragment set F.
+    auto product64 = [&](const uint16_t* F, int mb, const bf16x4* h) {
+      f32x4 a = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int kp = 0; kp < 4; kp += 2)
+        a = mfma2(frag(F, 4, mb, kp, lane), frag(F, 4, mb, kp + 1, lane), h[kp], h[kp + 1], a);
+      return a;
+    };
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb) {
+      h2[mb] = activate(product64(sF + kFragF2, mb, h1), sB + kHidden + 16 * mb, r0);
+      keep(kRowH2 + 16 * mb, h2[mb]);
+    }
+    float f = 0.0f;
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb) {
+      h3[mb] = activate(product64(sF + kFragF3, mb, h2), sB + 2 * kHidden + 16 * mb, r0);
+      keep(kRowH3 + 16 * mb, h3[mb]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        f += w4[16 * mb + r0 + j] * from_bf16(static_cast<uint16_t>(h3[mb][j]));
+    }
+    // The four lanes of a sample (l, l^16, l^32, l^48) hold its 64 terms.
+    f += __shfl_xor(f, 16, 64);
+    f += __shfl_xor(f, 32, 64);
+    f += sB[4 * kHidden];
     // Least squares plus (overshoot - 1) e^2, e the part of the error that
     // lies outside the interval between 0 and the target.
-    const float r = T.f - t;
-    const float e = T.f - fminf(fmaxf(T.f, fminf(t, 0.0f)), fmaxf(t, 0.0f));
+    const float r = f - t;
+    const float e = f - fminf(fmaxf(f, fminf(t, 0.0f)), fmaxf(t, 0.0f));
     const float ow = S.overshoot - 1.0f;
-    const float g = wgt * (r + ow * e) * inv_n;
+    const float g = live ? wgt * (r + ow * e) * inv_n : 0.0f;
     if (lane < 16) {
-      loss += wgt * (r * r + ow * e * e);
-      B.g[s] = g;
+      if (live) loss += wgt * (r * r + ow * e * e);
+      g_sum += g;
+      sG[16 * wv + col] = g;
     }
     // dz3 = bf16(g w4 [h3 > 0]), dz2 = bf16((W3^T dz3) [h2 > 0]), dz1 likewise.
-    bf16x4 d3[4], d2[4], d1[4];
+    auto gate = [&](const f32x4& a, const bf16x4& h) {
+      float d[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        d[j] = from_bf16(static_cast<uint16_t>(h[j])) > 0.0f ? a[j] : 0.0f;
+      return pack4f(d[0], d[1], d[2], d[3]);
+    };
+    bf16x4 d3[4], d2[4];
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb) {
-      uint16_t d[4];
+      f32x4 a;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float h = from_bf16(static_cast<uint16_t>(T.h3[mb][j]));
-        d[j] = to_bf16(h > 0.0f ? g * w4[16 * mb + r0 + j] : 0.0f);
-      }
-      d3[mb] = pack4(d[0], d[1], d[2], d[3]);
+      for (int j = 0; j < 4; ++j) a[j] = g * w4[16 * mb + r0 + j];
+      d3[mb] = gate(a, h3[mb]);
+      keep(kRowD3 + 16 * mb, d3[mb]);
     }
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb) {
-      f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb) acc = mfma(frag(sF + kFragT3, 4, mb, kb, lane), d3[kb], acc);
-      uint16_t d[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float h = from_bf16(static_cast<uint16_t>(T.h2[mb][j]));
-        d[j] = to_bf16(h > 0.0f ? acc[j] : 0.0f);
-      }
-      d2[mb] = pack4(d[0], d[1], d[2], d[3]);
+      d2[mb] = gate(product64(sF + kFragT3, mb, d3), h2[mb]);
+      keep(kRowD2 + 16 * mb, d2[mb]);
     }
-#pragma unroll
-    for (int mb = 0; mb < 4; ++mb) {
-      f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb) acc = mfma(frag(sF + kFragT2, 4, mb, kb, lane), d2[kb], acc);
-      uint16_t d[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float h = from_bf16(static_cast<uint16_t>(T.h1[mb][j]));
-        d[j] = to_bf16(h > 0.0f ? acc[j] : 0.0f);
-      }
-      d1[mb] = pack4(d[0], d[1], d[2], d[3]);
-    }
-    // Hidden-major stores: row 16 mb + r0 + j, column s.
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb)
+      keep(kRowD1 + 16 * mb, gate(product64(sF + kFragT2, mb, d2), h1[mb]));
+    __syncthreads();
+
+    // Weight gradients: block rows 16 wv, K = the 64 samples in two halves; lane
+    // l holds row l % 16 at samples 32 half + 8 (l / 16) .. + 7 of either operand.
+    auto operand = [&](int row, int half) {
+      return *reinterpret_cast<const bf16x8*>(sA + (row + col) * kPitch + 32 * half +
+                                              8 * (lane >> 4));
+    };
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int64_t o = (16 * mb + r0 + j) * B.n + s;
-        B.h1[o] = static_cast<uint16_t>(T.h1[mb][j]);
-        B.h2[o] = static_cast<uint16_t>(T.h2[mb][j]);
-        B.h3[o] = static_cast<uint16_t>(T.h3[mb][j]);
-        B.dz1[o] = static_cast<uint16_t>(d1[mb][j]);
-        B.dz2[o] = static_cast<uint16_t>(d2[mb][j]);
-        B.dz3[o] = static_cast<uint16_t>(d3[mb][j]);
+    for (int half = 0; half < 2; ++half) {
+      const bf16x8 a1 = operand(kRowD1 + 16 * wv, half), a2 = operand(kRowD2 + 16 * wv, half),
+                   a3 = operand(kRowD3 + 16 * wv, half);
+#pragma unroll
+      for (int nb = 0; nb < kKB1; ++nb)
+        acc1[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, operand(kRowX + 16 * nb, half),
+                                                           acc1[nb], 0, 0, 0);
+#pragma unroll
+      for (int nb = 0; nb < 4; ++nb) {
+        acc2[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, operand(kRowH1 + 16 * nb, half),
+                                                           acc2[nb], 0, 0, 0);
+        acc3[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a3, operand(kRowH2 + 16 * nb, half),
+                                                           acc3[nb], 0, 0, 0);
       }
-  }
-  // wave sum of the loss terms (lanes 0..15 hold them)
+    }
+    // Thread i: db of unit i (threads 0-191: dz1, dz2, dz3) or dw4 of unit i - 192.
+    {
+      const int i = static_cast<int>(threadIdx.x);
+      const uint16_t* row = sA + (i < 192 ? kRowD1 + i : kRowH3 + i - 192) * kPitch;
 #pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) loss += __shfl_xor(loss, d, 64);
-  if (lane == 0 && loss != 0.0f) atomicAdd(M.loss, loss);
-}
-
-// Weight gradients: block (layer, mb, nb) of dW_l = DZ_l Hprev^T over one
-// chunk of the batch, accumulated into M.grad.  One wavefront per (block,
-// chunk).  Output blocks: layer 1 4x7, layer 2 4x4, layer 3 4x4.
-constexpr int kWgradBlocks = 4 * kKB1 + 16 + 16;
-constexpr int kWgradChunk = 1024;
-
-__global__ __launch_bounds__(kThreads) void k_wgrad(Model M, Batch B) {
-  const int lane = __lane_id();
-  const int64_t wave = static_cast<int64_t>(blockIdx.x) * (kThreads / 64) + (threadIdx.x >> 6);
-  const int64_t n_chunks = (B.n + kWgradChunk - 1) / kWgradChunk;
-  if (wave >= kWgradBlocks * n_chunks) return;
-  const int blk = static_cast<int>(wave % kWgradBlocks);
-  const int64_t chunk = wave / kWgradBlocks;
-  int layer, mb, nb;
-  if (blk < 4 * kKB1) {
-    layer = 1;
-    mb = blk / kKB1;
-    nb = blk % kKB1;
-  } else if (blk < 4 * kKB1 + 16) {
-    layer = 2;
-    mb = (blk - 4 * kKB1) / 4;
-    nb = (blk - 4 * kKB1) % 4;
-  } else {
-    layer = 3;
-    mb = (blk - 4 * kKB1 - 16) / 4;
-    nb = (blk - 4 * kKB1 - 16) % 4;
+      for (int k = 0; k < kGroup; k += 8) {
+        const s16x8 v = *reinterpret_cast<const s16x8*>(row + k);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float x = from_bf16(static_cast<uint16_t>(v[j]));
+          unit_sum += i < 192 ? x : sG[k + j] * x;
+        }
+      }
+    }
   }
-  const uint16_t* dz = layer == 1 ? B.dz1 : layer == 2 ? B.dz2 : B.dz3;
-  const uint16_t* hp = layer == 1 ? B.x : layer == 2 ? B.h1 : B.h2;
-  const int cols = layer == 1 ? kFeatPad : kHidden;
-  const int off = layer == 1 ? kOffW1 : layer == 2 ? kOffW2 : kOffW3;
-  const int r0 = 4 * (lane >> 4), col = lane & 15;
-  const int64_t s_end = (chunk + 1) * kWgradChunk < B.n ? (chunk + 1) * kWgradChunk : B.n;
-  f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int64_t s0 = chunk * kWgradChunk; s0 < s_end; s0 += 16) {
-    const bf16x4 a = *reinterpret_cast<const bf16x4*>(dz + (16 * mb + col) * B.n + s0 + r0);
-    const bf16x4 b = *reinterpret_cast<const bf16x4*>(hp + (16 * nb + col) * B.n + s0 + r0);
-    acc = mfma(a, b, acc);
+  // The workgroup's row: W1's columns stay in the kernels' feature order.
+  float* row = B.rows + static_cast<int64_t>(blockIdx.x) * kGradRow;
+  auto store = [&](int off, int cols, int nb, const f32x4& a) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) row[off + (16 * wv + r0 + j) * cols + 16 * nb + col] = a[j];
+  };
+#pragma unroll
+  for (int nb = 0; nb < kKB1; ++nb) store(kOffW1, kFeatPad, nb, acc1[nb]);
+#pragma unroll
+  for (int nb = 0; nb < 4; ++nb) {
+    store(kOffW2, kHidden, nb, acc2[nb]);
+    store(kOffW3, kHidden, nb, acc3[nb]);
+  }
+  {
+    const int i = static_cast<int>(threadIdx.x);
+    const int off = i < 64 ? kOffB1 : i < 128 ? kOffB2 : i < 192 ? kOffB3 : kOffW4;
+    row[off + (i & 63)] = unit_sum;
   }
 #pragma unroll
-  for (int j = 0; j < 4; ++j) atomicAdd(&M.grad[off + (16 * mb + r0 + j) * cols + 16 * nb + col], acc[j]);
-}
-
-// Bias gradients and the output layer: db_l[i] = sum_s dz_l[i][s],
-// dw4[i] = sum_s g[s] h3[i][s], db4 = sum_s g[s].  One wavefront per
-// (row, chunk of samples): lanes stride over the chunk (coalesced reads of
-// the hidden-major rows), then a wave reduction and one atomic per wave.
-// Rows 0..191 biases, 192..255 w4, 256 b4.
-__global__ __launch_bounds__(kThreads) void k_bgrad(Model M, Batch B) {
-  const int64_t n_chunks = (B.n + kWgradChunk - 1) / kWgradChunk;
-  const int64_t t = (static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x) >> 6;
-  if (t >= 257 * n_chunks) return;  // uniform per wave
-  const int lane = __lane_id();
-  const int row = static_cast<int>(t % 257);
-  const int64_t chunk = t / 257;
-  const int64_t s0 = chunk * kWgradChunk;
-  const int64_t s1 = s0 + kWgradChunk < B.n ? s0 + kWgradChunk : B.n;
-  float acc = 0.0f;
-  int dst;
-  if (row < 192) {
-    const int layer = row / 64, i = row % 64;
-    const uint16_t* dz = (layer == 0 ? B.dz1 : layer == 1 ? B.dz2 : B.dz3) + i * B.n;
-    for (int64_t s = s0 + lane; s < s1; s += 64) acc += from_bf16(dz[s]);
-    dst = (layer == 0 ? kOffB1 : layer == 1 ? kOffB2 : kOffB3) + i;
-  } else if (row < 256) {
-    const uint16_t* h3 = B.h3 + (row - 192) * B.n;
-    for (int64_t s = s0 + lane; s < s1; s += 64) acc += B.g[s] * from_bf16(h3[s]);
-    dst = kOffW4 + row - 192;
-  } else {
-    for (int64_t s = s0 + lane; s < s1; s += 64) acc += B.g[s];
-    dst = kOffB4;
+  for (int d = 8; d >= 1; d >>= 1) {
+    loss += __shfl_xor(loss, d, 64);
+    g_sum += __shfl_xor(g_sum, d, 64);
   }
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) acc += __shfl_xor(acc, d, 64);
-  if (lane == 0) atomicAdd(&M.grad[dst], acc);
+  if (lane == 0) {
+    sSum[0][wv] = g_sum;
+    sSum[1][wv] = loss;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    row[kOffB4] = (sSum[0][0] + sSum[0][1]) + (sSum[0][2] + sSum[0][3]);
+    row[kParams] = (sSum[1][0] + sSum[1][1]) + (sSum[1][2] + sSum[1][3]);
+  }
 }
 
-// Inference feature row of training feature column c (see kFragF1I).
-__device__ __forceinline__ int inference_row(int c) {
+// Feature row in the kernels' order of feature column c of the parameters,
+// and the reverse.
+__device__ __forceinline__ int feature_row(int c) {
   if (c < 3) return 96 + c;       // coordinates
   if (c >= kFeat) return c;       // padding
   const int q = c - 3, k = q / 6, t = q - 6 * k;  // frequency k, function t
   return 16 * t + 4 * (k & 3) + (k >> 2);
 }
+__device__ __forceinline__ int feature_column(int r) {
+  if (r >= kFeat) return r;
+  if (r >= 96) return r - 96;
+  const int t = r >> 4, i = r & 15;
+  return 3 + 6 * ((i >> 2) + 4 * (i & 3)) + t;
+}
 
-// Fragment slot of master weight index p (layers 1-3), and of its transpose
-// (layers 2-3) or its inference-order copy (layer 1).
+// Fragment slot of parameter p (weights of layers 1-3), and of its transpose
+// (layers 2-3).
 __device__ __forceinline__ void frag_slots(int p, int* f, int* ft) {
   *f = -1;
   *ft = -1;
@@ -562,14 +525,11 @@ __device__ __forceinline__ void frag_slots(int p, int* f, int* ft) {
     return;
   }
   const int q = p - base;
-  const int row = q / cols, c = q - row * cols;
+  const int row = q / cols;
+  int c = q - row * cols;
+  if (base == kOffW1) c = feature_row(c);
   // W[row][c] sits in block (row / 16, c / 16) at lane (row % 16) + 16 ((c % 16) / 4), slot c % 4
   *f = fbase + (((row >> 4) * kbn + (c >> 4)) * 64 + (row & 15) + 16 * ((c & 15) >> 2)) * 4 + (c & 3);
-  if (base == kOffW1) {
-    const int ci = inference_row(c);
-    *ft = kFragF1I + (((row >> 4) * kbn + (ci >> 4)) * 64 + (row & 15) + 16 * ((ci & 15) >> 2)) * 4 +
-          (ci & 3);
-  }
   if (tbase >= 0) {
     // W^T[c][row]: block (c / 16, row / 16), lane (c % 16) + 16 ((row % 16) / 4), slot row % 4
     *ft = tbase + (((c >> 4) * 4 + (row >> 4)) * 64 + (c & 15) + 16 * ((row & 15) >> 2)) * 4 +
@@ -587,30 +547,55 @@ __global__ __launch_bounds__(kThreads) void k_pack(Model M) {
   if (ft >= 0) M.frags[ft] = b;
 }
 
-__global__ __launch_bounds__(kThreads) void k_adam(Model M, float lr, float beta1, float beta2,
+// The sum of the batch's rows, and with kStep the Adam step from it.  A
+// workgroup takes 32 neighbouring entries; 32 threads read a row's 128 bytes
+// of them and the 8 sets of threads every eighth row, so the chip reads the
+// 16 MB of a full batch's rows at once.
+constexpr int kSumSlots = 32, kSumParts = kThreads / kSumSlots;
+
+template <bool kStep>
+__global__ __launch_bounds__(kThreads) void k_adam(Model M, const float* __restrict__ rows,
+                                                   int n_rows, float lr, float beta1, float beta2,
                                                    float eps, float c1, float c2) {
-  const int p = blockIdx.x * kThreads + threadIdx.x;
-  if (p >= kParams) return;
-  const float g = M.grad[p];
+  __shared__ float s_part[kSumParts][kSumSlots];
+  const int i = static_cast<int>(threadIdx.x) % kSumSlots, part = threadIdx.x / kSumSlots;
+  const int slot = blockIdx.x * kSumSlots + i;
+  float sum = 0.0f;
+  if (slot <= kParams) {
+#pragma unroll 8
+    for (int r = part; r < n_rows; r += kSumParts)
+      sum += rows[static_cast<int64_t>(r) * kGradRow + slot];
+  }
+  s_part[part][i] = sum;
+  __syncthreads();
+  if (part != 0 || slot > kParams) return;
+#pragma unroll
+  for (int k = 1; k < kSumParts; ++k) sum += s_part[k][i];
+  if (slot == kParams) {
+    M.loss[0] = sum;
+    return;
+  }
+  int p = slot;
+  if (slot < kOffB1) {
+    const int row = slot / kFeatPad;
+    p = row * kFeatPad + feature_column(slot - row * kFeatPad);
+  }
+  if (!kStep) {
+    M.grad[p] = sum;
+    return;
+  }
+  const float g = sum;
   const float m = beta1 * M.m[p] + (1.0f - beta1) * g;
   const float v = beta2 * M.v[p] + (1.0f - beta2) * g * g;
   M.m[p] = m;
   M.v[p] = v;
   const float w = M.theta[p] - lr * (m / c1) / (sqrtf(v / c2) + eps);
   M.theta[p] = w;
-  M.grad[p] = 0.0f;
-  if (p == 0) M.loss[0] = 0.0f;
   int f, ft;
   frag_slots(p, &f, &ft);
   const uint16_t b = to_bf16(w);
   if (f >= 0) M.frags[f] = b;
   if (ft >= 0) M.frags[ft] = b;
-}
-
-__global__ __launch_bounds__(kThreads) void k_zero_grad(Model M) {
-  const int p = blockIdx.x * kThreads + threadIdx.x;
-  if (p < kParams) M.grad[p] = 0.0f;
-  if (p == 0) M.loss[0] = 0.0f;
 }
 
 unsigned blocks_for(int64_t n) { return static_cast<unsigned>((n + kThreads - 1) / kThreads); }
@@ -635,29 +620,29 @@ hipError_t launch_forward(const Model& M, const float* points, int64_t n, float*
 
 hipError_t launch_train_batch(const Model& M, const Batch& B, const Samples& S, uint32_t step,
                               hipStream_t s) {
-  if (B.n <= 0 || (B.n & 15) || S.count == 0) return hipErrorInvalidValue;
-  int64_t blocks = (B.n + 16 * 4 - 1) / (16 * 4);
-  if (blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL(k_train_fb, dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0, s, M, B,
-                     S, step);
-  const int64_t n_chunks = (B.n + kWgradChunk - 1) / kWgradChunk;
-  hipLaunchKernelGGL(k_wgrad, dim3(blocks_for(64 * kWgradBlocks * n_chunks)), dim3(kThreads), 0, s,
-                     M, B);
-  hipLaunchKernelGGL(k_bgrad, dim3(blocks_for(64 * 257 * n_chunks)), dim3(kThreads), 0, s, M, B);
+  if (B.n <= 0 || (B.n & 15) || S.count == 0 || !B.rows) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_train, dim3(static_cast<unsigned>(batch_rows(B.n))), dim3(kThreads), 0, s, M,
+                     B, S, step);
   return hipGetLastError();
 }
 
-hipError_t launch_adam(const Model& M, uint32_t step, float lr, float beta1, float beta2,
-                       float eps, hipStream_t s) {
+namespace {
+constexpr unsigned kSumBlocks = (kParams + 1 + kSumSlots - 1) / kSumSlots;
+}
+
+hipError_t launch_adam(const Model& M, const Batch& B, uint32_t step, float lr, float beta1,
+                       float beta2, float eps, hipStream_t s) {
   const double c1 = 1.0 - __builtin_pow(static_cast<double>(beta1), static_cast<double>(step));
   const double c2 = 1.0 - __builtin_pow(static_cast<double>(beta2), static_cast<double>(step));
-  hipLaunchKernelGGL(k_adam, dim3(blocks_for(kParams)), dim3(kThreads), 0, s, M, lr, beta1, beta2,
-                     eps, static_cast<float>(c1), static_cast<float>(c2));
+  hipLaunchKernelGGL(k_adam<true>, dim3(kSumBlocks), dim3(kThreads), 0, s, M, B.rows,
+                     batch_rows(B.n), lr, beta1, beta2, eps, static_cast<float>(c1),
+                     static_cast<float>(c2));
   return hipGetLastError();
 }
 
-hipError_t launch_zero_grad(const Model& M, hipStream_t s) {
-  hipLaunchKernelGGL(k_zero_grad, dim3(blocks_for(kParams)), dim3(kThreads), 0, s, M);
+hipError_t launch_gradient(const Model& M, const Batch& B, hipStream_t s) {
+  hipLaunchKernelGGL(k_adam<false>, dim3(kSumBlocks), dim3(kThreads), 0, s, M, B.rows,
+                     batch_rows(B.n), 0.0f, 0.0f, 0.0f, 0.0f, 1.0f, 1.0f);
   return hipGetLastError();
 }
 
