@@ -52,6 +52,9 @@ struct MeshGraphKey {
   iso::McBuffers B;
 };
 
+constexpr int kStageWords = 64;
+static_assert(iso::kLhmcCtlWords <= kStageWords, "read in one copy");
+
 struct iso_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -86,10 +89,10 @@ struct iso_ctx {
   unsigned long long* h_dc = nullptr;  // pinned
   // octree marching cubes: nodes, dense primal lattice (or the sorted path's
   // pairs and sort scratch), cubes, edge table, scan state
-  DevBuf oc_keys, oc_values, oc_leaf, oc_dense, oc_primal, oc_plevel, oc_corner, oc_case,
-      oc_base, oc_tkeys, oc_towner, oc_tid, sc_slot, sc_ctl, oc_pkeys, oc_plevels, oc_skeys,
+  DevBuf oc_keys, oc_values, oc_child, oc_dense, oc_primal, oc_plevel, oc_corner, oc_case,
+      oc_eslot, oc_tfirst, oc_split, oc_ctl, oc_tkeys, oc_towner, oc_tid, sc_slot, sc_ctl, oc_pkeys, oc_plevels, oc_skeys,
       oc_slevels, oc_sort;
-  unsigned long long* h_stage = nullptr;  // pinned, 8 words
+  unsigned long long* h_stage = nullptr;  // pinned, kStageWords
 
   // batched chunks: lowered programs, chunk table, sign words, offsets
   DevBuf b_ops, b_chunks, b_segstart, b_wordstart, b_tilestart, b_signs, b_voff, b_ioff, b_values;
@@ -332,7 +335,7 @@ int iso_ctx_create(int device, void* stream, iso_ctx** out) {
                     hipHostMallocDefault) != hipSuccess ||
       hipHostMalloc(reinterpret_cast<void**>(&c->h_dc), iso::kDcSlots * sizeof(unsigned long long),
                     hipHostMallocDefault) != hipSuccess ||
-      hipHostMalloc(reinterpret_cast<void**>(&c->h_stage), 8 * sizeof(unsigned long long),
+      hipHostMalloc(reinterpret_cast<void**>(&c->h_stage), kStageWords * sizeof(unsigned long long),
                     hipHostMallocDefault) != hipSuccess) {
     if (c->h_totals) (void)hipHostFree(c->h_totals);
     if (c->h_dc) (void)hipHostFree(c->h_dc);
@@ -364,8 +367,9 @@ int iso_ctx_destroy(iso_ctx* c) {
                     &c->agg,        &c->incl,       &c->active,    &c->totals,
                     &c->vout,       &c->iout,       &c->pts,       &c->vals,     &c->dc_normals, &c->dc_plist, &c->dc_pindex, &c->dc_samples,
                     &c->dc_values,  &c->dc_points,  &c->dc_mixed,  &c->dc_flags,  &c->dc_counters,
-                    &c->oc_keys,    &c->oc_values,  &c->oc_leaf,   &c->oc_dense, &c->oc_primal,
-                    &c->oc_plevel,  &c->oc_corner,  &c->oc_case,   &c->oc_base,  &c->oc_tkeys,
+                    &c->oc_keys,    &c->oc_values,  &c->oc_child,  &c->oc_dense, &c->oc_primal,
+                    &c->oc_plevel,  &c->oc_corner,  &c->oc_case,   &c->oc_eslot,
+                    &c->oc_tfirst,  &c->oc_split,   &c->oc_ctl,    &c->oc_tkeys,
                     &c->oc_towner,  &c->oc_tid,     &c->sc_slot,   &c->sc_ctl,
                     &c->oc_pkeys,   &c->oc_plevels, &c->oc_skeys,  &c->oc_slevels, &c->oc_sort,
                     &c->b_ops,      &c->b_chunks,   &c->b_segstart, &c->b_wordstart, &c->b_tilestart,
@@ -1410,27 +1414,6 @@ int iso_extract_dc(iso_ctx* c, const iso_grid_desc* desc, float epsilon, iso_mes
 
 namespace {
 
-// Grows a device buffer to `bytes`, keeping its first `keep` bytes.
-int grow_keep(iso_ctx* c, DevBuf* b, size_t bytes, size_t keep) {
-  if (b->bytes >= bytes && b->ptr) return ISO_OK;
-  size_t want = b->bytes ? b->bytes : 256;
-  while (want < bytes) want *= 2;
-  void* p = nullptr;
-  ISO_HIP(c, hipMalloc(&p, want));
-  if (keep && b->ptr) {
-    hipError_t e = hipMemcpyAsync(p, b->ptr, keep, hipMemcpyDeviceToDevice, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    if (e != hipSuccess) {
-      (void)hipFree(p);
-      return fail(c, ISO_ERR_DEVICE, std::string("grow copy: ") + hipGetErrorString(e));
-    }
-  }
-  release(b);
-  b->ptr = p;
-  b->bytes = want;
-  return ISO_OK;
-}
-
 // Scan state for scans of up to n items at one item per thread; err points
 // at the status word.
 int prepare_scan(iso_ctx* c, uint64_t n, iso::scan::State* st) {
@@ -1443,20 +1426,17 @@ int prepare_scan(iso_ctx* c, uint64_t n, iso::scan::State* st) {
   return ISO_OK;
 }
 
-// Reads ctl[0..4) of the scan state (total in [1], status bits in [2]);
-// `stage` names the failing pass in the error message.
-int read_ctl(iso_ctx* c, const iso::scan::State& st, const char* stage = "octree extraction") {
-  ISO_HIP(c, hipMemcpyAsync(c->h_stage, st.ctl, 4 * sizeof(unsigned long long),
+// Reads the octree extraction's control words.
+int read_lhmc(iso_ctx* c) {
+  ISO_HIP(c, hipMemcpyAsync(c->h_stage, c->oc_ctl.ptr,
+                            iso::kLhmcCtlWords * sizeof(unsigned long long),
                             hipMemcpyDeviceToHost, c->stream));
   ISO_HIP(c, hipStreamSynchronize(c->stream));
   collect_timing(c);
-  if (c->h_stage[2]) {
-    const unsigned long long e = c->h_stage[2];
+  if (const unsigned long long e = c->h_stage[iso::kLhmcErr])
     return fail(c, ISO_ERR_DEVICE,
-                std::string(stage) + " failed:" + ((e & iso::kLhmcErrScan) ? " scan" : "") +
-                    ((e & iso::kLhmcErrWalk) ? " dual-corner walk" : "") +
+                std::string("octree extraction failed:") + ((e & iso::kLhmcErrScan) ? " scan" : "") +
                     ((e & iso::kLhmcErrTable) ? " edge table" : ""));
-  }
   return ISO_OK;
 }
 
@@ -1474,159 +1454,206 @@ int iso_extract_lhmc(iso_ctx* c, int32_t max_depth, iso_mesh_out* out) {
   c->kept = false;
   ISO_HIP(c, hipSetDevice(c->device));
   int st = ISO_OK;
-  const iso::DevOp* ops = static_cast<const iso::DevOp*>(c->prog.ptr);
   const int d1 = (max_depth > 2 ? max_depth : 2) + 1;  // deepest possible node
-  const bool dense_primal = d1 <= iso::kLhmcDenseDepth;
-  const uint64_t n_dense = dense_primal ? 1ull << (3 * d1) : 0;
+  const bool bit_primal = d1 <= iso::kLhmcDenseDepth;
   // Morton::level's split points, found once with the host's libm log
   static uint64_t splits[iso::kLhmcMaxLevels];
   static std::once_flag splits_once;
   std::call_once(splits_once, [] { iso::lhmc_level_splits(splits); });
-  ISO_HIP(c, iso::launch_lhmc_levels(splits, c->stream));
-  iso::scan::State S{};
-  if ((st = prepare_scan(c, 1u << 16, &S)) != ISO_OK) return st;
-  // status word: cleared once, accumulated by every kernel below
-  ISO_HIP(c, iso::launch_fill_u32(reinterpret_cast<uint32_t*>(S.err), 2, 0u, c->stream));
-
-  // 1. octree, breadth first
-  iso::LhmcNodes N{};
-  N.n_levels = d1 + 1;
-  int64_t off[iso::kLhmcMaxLevels + 2] = {0};
-  off[0] = 0;
-  off[1] = 1;
-  {
-    const size_t cap = 4096;
-    if ((st = grow_keep(c, &c->oc_keys, cap * 8, 0)) != ISO_OK) return st;
-    c->h_stage[4] = 1ull;  // the root key
-    ISO_HIP(c, hipMemcpyAsync(c->oc_keys.ptr, &c->h_stage[4], sizeof(uint64_t),
-                              hipMemcpyHostToDevice, c->stream));
-    ISO_HIP(c, hipStreamSynchronize(c->stream));
+  if (!c->oc_split.ptr) {
+    ISO_HIP(c, ensure(&c->oc_split, sizeof splits));
+    hipError_t e = hipMemcpyAsync(c->oc_split.ptr, splits, sizeof splits, hipMemcpyHostToDevice,
+                                  c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    if (e != hipSuccess) release(&c->oc_split);
+    ISO_HIP(c, e);
   }
-  for (int d = 0; d <= d1; ++d) {
-    const int64_t n = off[d + 1] - off[d];
-    const int64_t next_cap = d < d1 ? 8 * n : 0;
-    const size_t need = static_cast<size_t>(off[d + 1] + next_cap);
-    if ((st = grow_keep(c, &c->oc_keys, need * 8, static_cast<size_t>(off[d + 1]) * 8)) != ISO_OK ||
-        (st = grow_keep(c, &c->oc_values, need * 4, static_cast<size_t>(off[d]) * 4)) != ISO_OK ||
-        (st = grow_keep(c, &c->oc_leaf, need, static_cast<size_t>(off[d]))) != ISO_OK)
-      return st;
-    if ((st = prepare_scan(c, static_cast<uint64_t>(n), &S)) != ISO_OK) return st;
-    ISO_HIP(c, timed(c, "lhmc_level", [&] {
-              return iso::launch_lhmc_level(
-                  ops, c->n_prog, max_depth, static_cast<uint64_t*>(c->oc_keys.ptr),
-                  static_cast<float*>(c->oc_values.ptr), static_cast<uint8_t*>(c->oc_leaf.ptr),
-                  off[d], n, next_cap, S, c->stream);
-            }));
-    if ((st = read_ctl(c, S)) != ISO_OK) return st;
-    const int64_t children = 8 * static_cast<int64_t>(c->h_stage[1]);
-    if (children > next_cap)
-      return fail(c, ISO_ERR_DEVICE, "octree refined past its deepest possible depth");
-    off[d + 2] = off[d + 1] + children;
-  }
-  N.keys = static_cast<uint64_t*>(c->oc_keys.ptr);
-  N.values = static_cast<float*>(c->oc_values.ptr);
-  N.leaf = static_cast<uint8_t*>(c->oc_leaf.ptr);
-  for (int d = 0; d <= N.n_levels; ++d) N.level_off[d] = off[d];
-  const int64_t n_nodes = off[N.n_levels];
-  if (n_nodes >= 0xffffffffll)
-    return fail(c, ISO_ERR_OVERFLOW, "octree has 2^32 or more nodes");
+  ISO_HIP(c, ensure(&c->oc_ctl, iso::kLhmcCtlWords * sizeof(unsigned long long)));
 
-  // 2. primal vertices in ascending Morton order
-  iso::LhmcCubes C{};
-  const uint64_t n_pairs = 8 * static_cast<uint64_t>(n_nodes);
-  uint64_t pv_cap = n_pairs;
-  if (dense_primal && pv_cap > n_dense) pv_cap = n_dense;
-  ISO_HIP(c, ensure(&c->oc_primal, pv_cap * sizeof(uint64_t)));
-  ISO_HIP(c, ensure(&c->oc_plevel, pv_cap));
-  C.primal = static_cast<uint64_t*>(c->oc_primal.ptr);
-  C.primal_level = static_cast<uint8_t*>(c->oc_plevel.ptr);
-  if ((st = prepare_scan(c, dense_primal ? n_dense : n_pairs, &S)) != ISO_OK) return st;
-  if (dense_primal) {
-    ISO_HIP(c, ensure(&c->oc_dense, n_dense * sizeof(uint32_t)));
-    ISO_HIP(c, timed(c, "lhmc_primal", [&] {
-              return iso::launch_lhmc_primal(N, d1, static_cast<uint32_t*>(c->oc_dense.ptr),
-                                             n_dense, C, pv_cap, S, c->stream);
-            }));
-  } else {
-    const size_t temp = iso::lhmc_sort_temp_bytes(n_pairs);
-    if (temp == 0) return fail(c, ISO_ERR_DEVICE, "radix sort size query failed");
-    ISO_HIP(c, ensure(&c->oc_pkeys, n_pairs * sizeof(uint64_t)));
-    ISO_HIP(c, ensure(&c->oc_skeys, n_pairs * sizeof(uint64_t)));
-    ISO_HIP(c, ensure(&c->oc_plevels, n_pairs));
-    ISO_HIP(c, ensure(&c->oc_slevels, n_pairs));
-    ISO_HIP(c, ensure(&c->oc_sort, temp));
-    ISO_HIP(c, timed(c, "lhmc_primal", [&] {
-              return iso::launch_lhmc_primal_sorted(
-                  N, static_cast<uint64_t*>(c->oc_pkeys.ptr),
-                  static_cast<uint8_t*>(c->oc_plevels.ptr),
-                  static_cast<uint64_t*>(c->oc_skeys.ptr),
-                  static_cast<uint8_t*>(c->oc_slevels.ptr), c->oc_sort.ptr, temp, C, pv_cap, S,
-                  c->stream);
-            }));
-  }
-  if ((st = read_ctl(c, S)) != ISO_OK) return st;
-  const uint64_t n_pv = c->h_stage[1];
-  if (n_pv > pv_cap) return fail(c, ISO_ERR_DEVICE, "primal vertex list overflow");
-  if (n_pv > 0x0fffffffull) return fail(c, ISO_ERR_OVERFLOW, "too many dual cubes");
-  C.n = static_cast<uint32_t>(n_pv);
-
-  // 3. dual cubes
-  ISO_HIP(c, ensure(&c->oc_corner, (n_pv ? n_pv : 1) * 8 * sizeof(uint32_t)));
-  ISO_HIP(c, ensure(&c->oc_case, n_pv ? n_pv : 1));
-  ISO_HIP(c, ensure(&c->oc_base, (n_pv ? n_pv : 1) * sizeof(unsigned long long)));
-  C.corner = static_cast<uint32_t*>(c->oc_corner.ptr);
-  C.cube_case = static_cast<uint8_t*>(c->oc_case.ptr);
-  C.base = static_cast<unsigned long long*>(c->oc_base.ptr);
-  ISO_HIP(c, timed(c, "lhmc_cubes", [&] { return iso::launch_lhmc_cubes(N, d1, C, S, c->stream); }));
-  if ((st = read_ctl(c, S)) != ISO_OK) return st;
-  const uint64_t n_tri = c->h_stage[1];
-
-  // 4. edge ownership and first ids
-  iso::LhmcEdgeTable T{};
-  uint64_t tcap = 1024;
-  while (tcap < 6 * n_tri) tcap *= 2;
-  ISO_HIP(c, ensure(&c->oc_tkeys, tcap * sizeof(unsigned long long)));
-  ISO_HIP(c, ensure(&c->oc_towner, tcap * sizeof(uint32_t)));
-  ISO_HIP(c, ensure(&c->oc_tid, tcap * sizeof(uint32_t)));
-  T.keys = static_cast<unsigned long long*>(c->oc_tkeys.ptr);
-  T.owner = static_cast<uint32_t*>(c->oc_towner.ptr);
-  T.id = static_cast<uint32_t*>(c->oc_tid.ptr);
-  T.mask = tcap - 1;
-  ISO_HIP(c, timed(c, "lhmc_own", [&] {
-            hipError_t e = iso::launch_lhmc_table_clear(T, c->stream);
-            if (e != hipSuccess) return e;
-            return iso::launch_lhmc_own(N, C, T, S.err, S, c->stream);
-          }));
-  if ((st = read_ctl(c, S)) != ISO_OK) return st;
-  const uint64_t nv = c->h_stage[1] & 0xffffffffull;
-  const uint64_t ni = 3 * (c->h_stage[1] >> 32);
-  if ((c->h_stage[1] >> 32) != n_tri) return fail(c, ISO_ERR_DEVICE, "triangle count mismatch");
-  if (ni > 0xffffffffull) return fail(c, ISO_ERR_OVERFLOW, "mesh exceeds u32 indices");
-  out->vertex_count = nv;
-  out->index_count = ni;
-
-  // 5. emit
+  // The buffers are as large as earlier calls left them, and the passes start
+  // over when one proves too small.
+  iso::LhmcTree N{};
+  N.ops = static_cast<const iso::DevOp*>(c->prog.ptr);
+  N.n_ops = c->n_prog;
+  N.max_depth = max_depth;
+  N.d1 = d1;
+  N.split = static_cast<const uint64_t*>(c->oc_split.ptr);
+  N.ctl = static_cast<unsigned long long*>(c->oc_ctl.ptr);
+  const bool on_device = out->memory == ISO_MEMORY_DEVICE;
+  uint64_t want_nodes = 1u << 16, want_primal = 1u << 16, want_cubes = 1u << 14,
+           want_table = 1u << 17, want_v = 1u << 15, want_i = 1u << 17;
+  uint64_t nv = 0, ni = 0, vcap = 0, icap = 0;
   float* vdst = nullptr;
   uint32_t* idst = nullptr;
-  uint64_t vcap = 0, icap = 0;
-  if (out->memory == ISO_MEMORY_DEVICE) {
-    vdst = out->vertices;
-    idst = out->indices;
-    vcap = out->vertices ? out->vertex_capacity : 0;
-    icap = out->indices ? out->index_capacity : 0;
-  } else {
-    ISO_HIP(c, ensure(&c->vout, (nv ? nv : 1) * 3 * sizeof(float)));
-    ISO_HIP(c, ensure(&c->iout, (ni ? ni : 1) * sizeof(uint32_t)));
-    vdst = static_cast<float*>(c->vout.ptr);
-    idst = static_cast<uint32_t*>(c->iout.ptr);
-    vcap = nv;
-    icap = ni;
+  while (true) {
+    ISO_HIP(c, ensure(&c->oc_keys, want_nodes * sizeof(uint64_t)));
+    ISO_HIP(c, ensure(&c->oc_values, want_nodes * sizeof(float)));
+    ISO_HIP(c, ensure(&c->oc_child, want_nodes * sizeof(uint32_t)));
+    N.keys = static_cast<uint64_t*>(c->oc_keys.ptr);
+    N.values = static_cast<float*>(c->oc_values.ptr);
+    N.child = static_cast<uint32_t*>(c->oc_child.ptr);
+    N.cap = std::min({c->oc_keys.bytes / sizeof(uint64_t), c->oc_values.bytes / sizeof(float),
+                      c->oc_child.bytes / sizeof(uint32_t)});
+    iso::LhmcCubes C{};
+    iso::LhmcEdgeTable T{};
+    auto edge_buffers = [&]() -> int {
+      ISO_HIP(c, ensure(&c->oc_tkeys, want_table * sizeof(unsigned long long)));
+      ISO_HIP(c, ensure(&c->oc_towner, want_table * sizeof(uint32_t)));
+      ISO_HIP(c, ensure(&c->oc_tid, want_table * sizeof(uint32_t)));
+      T.keys = static_cast<unsigned long long*>(c->oc_tkeys.ptr);
+      T.owner = static_cast<uint32_t*>(c->oc_towner.ptr);
+      T.id = static_cast<uint32_t*>(c->oc_tid.ptr);
+      C.table_capacity =
+          std::min({c->oc_tkeys.bytes / sizeof(unsigned long long),
+                    c->oc_towner.bytes / sizeof(uint32_t), c->oc_tid.bytes / sizeof(uint32_t)});
+      if (on_device) {
+        vdst = out->vertices;
+        idst = out->indices;
+        vcap = out->vertices ? out->vertex_capacity : 0;
+        icap = out->indices ? out->index_capacity : 0;
+      } else {
+        ISO_HIP(c, ensure(&c->vout, want_v * 3 * sizeof(float)));
+        ISO_HIP(c, ensure(&c->iout, want_i * sizeof(uint32_t)));
+        vdst = static_cast<float*>(c->vout.ptr);
+        idst = static_cast<uint32_t*>(c->iout.ptr);
+        vcap = c->vout.bytes / (3 * sizeof(float));
+        icap = c->iout.bytes / sizeof(uint32_t);
+      }
+      return ISO_OK;
+    };
+    auto cube_buffers = [&]() -> int {
+      ISO_HIP(c, ensure(&c->oc_corner, want_cubes * 8 * sizeof(uint32_t)));
+      ISO_HIP(c, ensure(&c->oc_eslot, want_cubes * 12 * sizeof(uint32_t)));
+      ISO_HIP(c, ensure(&c->oc_tfirst, want_cubes * sizeof(uint32_t)));
+      ISO_HIP(c, ensure(&c->oc_case, want_cubes));
+      C.primal = static_cast<uint64_t*>(c->oc_primal.ptr);
+      C.primal_capacity = c->oc_primal.bytes / sizeof(uint64_t);
+      C.corner = static_cast<uint32_t*>(c->oc_corner.ptr);
+      C.edge_slot = static_cast<uint32_t*>(c->oc_eslot.ptr);
+      C.tri_first = static_cast<uint32_t*>(c->oc_tfirst.ptr);
+      C.cube_case = static_cast<uint8_t*>(c->oc_case.ptr);
+      C.capacity = std::min({c->oc_corner.bytes / 32, c->oc_eslot.bytes / 48,
+                             c->oc_tfirst.bytes / sizeof(uint32_t), c->oc_case.bytes,
+                             size_t{0x0fffffff}});
+      return edge_buffers();
+    };
+    // 4. edge ownership, first ids and vertices; 5. indices
+    auto mesh = [&]() -> int {
+      ISO_HIP(c, timed(c, "lhmc_own", [&] {
+                return iso::launch_lhmc_own(N, C, T, vdst, vcap, c->stream);
+              }));
+      ISO_HIP(c, timed(c, "lhmc_emit", [&] {
+                return iso::launch_lhmc_emit(N, C, T, idst, icap, c->stream);
+              }));
+      return read_lhmc(c);
+    };
+
+    // 1. octree, breadth first; 2. primal vertices in ascending Morton order;
+    // 3. dual cubes
+    const uint64_t primal_slots = bit_primal ? iso::lhmc_primal_slots(d1) : 0;
+    uint64_t n_slots = primal_slots;
+    if (bit_primal) {
+      ISO_HIP(c, ensure(&c->oc_dense, (1ull << (3 * d1)) / 8));
+      N.bits = static_cast<uint32_t*>(c->oc_dense.ptr);
+      ISO_HIP(c, ensure(&c->oc_primal, want_primal * sizeof(uint64_t)));
+      if ((st = cube_buffers()) != ISO_OK) return st;
+      n_slots += C.primal_capacity / 1024 + 1;
+    }
+    ISO_HIP(c, ensure(&c->sc_slot,
+                      (n_slots + C.capacity / 256 + 1) * sizeof(unsigned long long)));
+    auto* slot = static_cast<unsigned long long*>(c->sc_slot.ptr);
+    C.slot = slot + primal_slots;
+    C.own_slot = slot + n_slots;
+    ISO_HIP(c, iso::launch_lhmc_clear(N, slot, n_slots, c->stream));
+    ISO_HIP(c, timed(c, "lhmc_level",
+                     [&] { return iso::launch_lhmc_levels(N, c->prog_kind, c->stream); }));
+    if (bit_primal) {
+      ISO_HIP(c, timed(c, "lhmc_primal", [&] {
+                return iso::launch_lhmc_primal(N, C, slot, c->stream);
+              }));
+      ISO_HIP(c, timed(c, "lhmc_cubes", [&] { return iso::launch_lhmc_cubes(N, C, c->stream); }));
+      if ((st = mesh()) != ISO_OK) return st;
+    } else if ((st = read_lhmc(c)) != ISO_OK) {
+      return st;
+    }
+    const unsigned long long* count = c->h_stage + iso::kLhmcCount;
+    uint64_t n_nodes = 0;
+    int d = 0;
+    for (; d <= d1 && n_nodes + count[d] <= N.cap; ++d) n_nodes += count[d];
+    if (d <= d1) {
+      // Depth d does not fit; the depths below it hold about four times as
+      // many nodes (they follow a surface).
+      n_nodes += count[d];
+      if (n_nodes >= 0xffffffffull)
+        return fail(c, ISO_ERR_OVERFLOW, "octree has 2^32 or more nodes");
+      want_nodes = d < d1 ? 4 * n_nodes : n_nodes;
+      continue;
+    }
+    if (count[d1 + 1])
+      return fail(c, ISO_ERR_DEVICE, "octree refined past its deepest possible depth");
+    if (n_nodes >= 0xffffffffull)
+      return fail(c, ISO_ERR_OVERFLOW, "octree has 2^32 or more nodes");
+    if (!bit_primal) {
+      const uint64_t n_pairs = 8 * n_nodes;
+      const size_t temp = iso::lhmc_sort_temp_bytes(n_pairs);
+      if (temp == 0) return fail(c, ISO_ERR_DEVICE, "radix sort size query failed");
+      // No more vertices than pairs: the list fits.
+      ISO_HIP(c, ensure(&c->oc_primal, n_pairs * sizeof(uint64_t)));
+      ISO_HIP(c, ensure(&c->oc_plevel, n_pairs));
+      ISO_HIP(c, ensure(&c->oc_pkeys, n_pairs * sizeof(uint64_t)));
+      ISO_HIP(c, ensure(&c->oc_skeys, n_pairs * sizeof(uint64_t)));
+      ISO_HIP(c, ensure(&c->oc_plevels, n_pairs));
+      ISO_HIP(c, ensure(&c->oc_slevels, n_pairs));
+      ISO_HIP(c, ensure(&c->oc_sort, temp));
+      if ((st = cube_buffers()) != ISO_OK) return st;
+      C.primal_level = static_cast<uint8_t*>(c->oc_plevel.ptr);
+      C.primal_capacity = n_pairs;
+      n_slots = n_pairs / 1024 + 1;
+      ISO_HIP(c, ensure(&c->sc_slot,
+                        (n_slots + C.capacity / 256 + 1) * sizeof(unsigned long long)));
+      C.slot = static_cast<unsigned long long*>(c->sc_slot.ptr);
+      C.own_slot = C.slot + n_slots;
+      ISO_HIP(c, timed(c, "lhmc_primal", [&] {
+                return iso::launch_lhmc_primal_sorted(
+                    N, static_cast<int64_t>(n_nodes), static_cast<uint64_t*>(c->oc_pkeys.ptr),
+                    static_cast<uint8_t*>(c->oc_plevels.ptr),
+                    static_cast<uint64_t*>(c->oc_skeys.ptr),
+                    static_cast<uint8_t*>(c->oc_slevels.ptr), c->oc_sort.ptr, temp, C, C.slot,
+                    c->stream);
+              }));
+      ISO_HIP(c, iso::launch_lhmc_cubes_reset(N, C, c->stream));
+      ISO_HIP(c, timed(c, "lhmc_cubes", [&] { return iso::launch_lhmc_cubes(N, C, c->stream); }));
+      if ((st = mesh()) != ISO_OK) return st;
+    }
+    const uint64_t n_pv = c->h_stage[iso::kLhmcPrimal + 1];
+    if (n_pv > 0x0fffffffull) return fail(c, ISO_ERR_OVERFLOW, "too many dual cubes");
+    if (n_pv > C.primal_capacity) {
+      want_primal = n_pv;
+      continue;
+    }
+    const unsigned long long cubes = c->h_stage[iso::kLhmcCubes + 1];
+    ni = 3 * (cubes & 0xffffffffull);
+    if (ni > 0xffffffffull) return fail(c, ISO_ERR_OVERFLOW, "mesh exceeds u32 indices");
+    want_table = iso::lhmc_table_size(cubes);
+    if ((cubes >> 32) > C.capacity) {
+      want_cubes = cubes >> 32;
+      continue;
+    }
+    // What remains can be run again by itself.
+    if (want_table > C.table_capacity || (!on_device && ni > icap)) {
+      want_i = ni;
+      if ((st = edge_buffers()) != ISO_OK || (st = mesh()) != ISO_OK) return st;
+    }
+    nv = c->h_stage[iso::kLhmcOwn + 1];
+    if (!on_device && nv > vcap) {
+      want_v = nv;
+      if ((st = edge_buffers()) != ISO_OK || (st = mesh()) != ISO_OK) return st;
+    }
+    break;
   }
-  ISO_HIP(c, timed(c, "lhmc_emit", [&] {
-            return iso::launch_lhmc_emit(N, C, T, vdst, vcap, idst, icap, S.err, c->stream);
-          }));
-  if ((st = read_ctl(c, S)) != ISO_OK) return st;
-  if (out->memory == ISO_MEMORY_DEVICE) {
+  out->vertex_count = nv;
+  out->index_count = ni;
+  if (on_device) {
     if (nv > vcap || ni > icap) return fail(c, ISO_ERR_CAPACITY, "output buffers too small");
     return ISO_OK;
   }

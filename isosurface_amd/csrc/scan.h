@@ -60,6 +60,48 @@ __global__ void k_reset(State st, int64_t n_blocks) {
   if (blockIdx.x == 0 && threadIdx.x < 2) st.ctl[threadIdx.x] = 0ull;
 }
 
+// What the workgroups before `blk` sum to: publishes blk's `total` and looks
+// back, 64 predecessors per step.  Called by one whole wavefront; workgroups
+// must have taken `blk` in order, so that every predecessor is running.
+__device__ __forceinline__ unsigned long long look_back(uint64_t blk, unsigned long long total,
+                                                        unsigned long long* slot,
+                                                        unsigned long long* err) {
+  const int lane = __lane_id();
+  unsigned long long prefix = 0ull;
+  if (blk == 0) {
+    if (lane == 0) slot_store(&slot[0], kInclusive | total);
+    return prefix;
+  }
+  if (lane == 0) slot_store(&slot[blk], kAggregate | total);
+  int64_t j = static_cast<int64_t>(blk) - 1;
+  uint32_t spins = 0;
+  while (true) {
+    const int64_t idx = j - lane;
+    // Blocks before the first one act as an inclusive zero.
+    const unsigned long long w = idx >= 0 ? slot_load(&slot[idx]) : kInclusive;
+    const uint64_t incl = __ballot((w >> 62) == 2ull);
+    const uint64_t zero = __ballot((w >> 62) == 0ull);
+    const int stop = incl ? __builtin_ctzll(incl) : 64;
+    const uint64_t upto = stop < 64 ? (2ull << stop) - 1ull : ~0ull;
+    if (zero & upto) {
+      if (++spins > kSpinLimit) {
+        if (lane == 0) atomicOr(err, 2ull);
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+      continue;
+    }
+    unsigned long long x = lane <= stop ? (w & kValueMask) : 0ull;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) x += __shfl_xor(x, d, 64);
+    prefix += x;
+    if (stop < 64) break;
+    j -= 64;
+  }
+  if (lane == 0) slot_store(&slot[blk], kInclusive | (prefix + total));
+  return prefix;
+}
+
 template <int I, class Load, class Sink>
 __global__ __launch_bounds__(kThreads) void k_scan(uint64_t n, Load load, Sink sink, State st) {
   constexpr uint64_t kTile = static_cast<uint64_t>(kThreads) * I;
@@ -92,42 +134,10 @@ __global__ __launch_bounds__(kThreads) void k_scan(uint64_t n, Load load, Sink s
   unsigned long long off = inc - sum;
   for (int i = 0; i < wv; ++i) off += s_wave[i];
 
-  // Look-back by the first wave: 64 predecessors per step.
   if (threadIdx.x < 64) {
     unsigned long long total = 0ull;
     for (int i = 0; i < kThreads / 64; ++i) total += s_wave[i];
-    unsigned long long prefix = 0ull;
-    if (blk == 0) {
-      if (lane == 0) slot_store(&st.slot[0], kInclusive | total);
-    } else {
-      if (lane == 0) slot_store(&st.slot[blk], kAggregate | total);
-      int64_t j = static_cast<int64_t>(blk) - 1;
-      uint32_t spins = 0;
-      while (true) {
-        const int64_t idx = j - lane;
-        // Blocks before the first one act as an inclusive zero.
-        const unsigned long long w = idx >= 0 ? slot_load(&st.slot[idx]) : kInclusive;
-        const uint64_t incl = __ballot((w >> 62) == 2ull);
-        const uint64_t zero = __ballot((w >> 62) == 0ull);
-        const int stop = incl ? __builtin_ctzll(incl) : 64;
-        const uint64_t upto = stop < 64 ? (2ull << stop) - 1ull : ~0ull;
-        if (zero & upto) {
-          if (++spins > kSpinLimit) {
-            if (lane == 0) atomicOr(st.err, 2ull);
-            break;
-          }
-          __builtin_amdgcn_s_sleep(1);
-          continue;
-        }
-        unsigned long long x = lane <= stop ? (w & kValueMask) : 0ull;
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) x += __shfl_xor(x, d, 64);
-        prefix += x;
-        if (stop < 64) break;
-        j -= 64;
-      }
-      if (lane == 0) slot_store(&st.slot[blk], kInclusive | (prefix + total));
-    }
+    const unsigned long long prefix = look_back(blk, total, st.slot, st.err);
     if (lane == 0) {
       s_prefix = prefix;
       if (blk == (n ? (n - 1) / kTile : 0)) st.ctl[1] = prefix + total;

@@ -30,7 +30,7 @@ namespace iso {
 // index is then a scalar load into scalar registers, whatever else the kernel
 // stores to (through an ordinary pointer that came from memory or a struct the
 // compiler must assume that a store may change it, and loads it per lane: 185
-// us instead of SPARSE_US for the 257^3 signs of 64 spheres minus a torus).
+// us instead of 135 for the 257^3 signs of 64 spheres minus a torus).
 using OpsPtr = const DevOp __attribute__((address_space(4)))*;
 __device__ __forceinline__ OpsPtr as_constant(const DevOp* ops) {
   return (OpsPtr)(reinterpret_cast<uintptr_t>(ops));
@@ -544,6 +544,127 @@ __device__ __forceinline__ void sdf_eval_list(OpsPtr ops, int first, const uint1
       }
     }
   }
+}
+
+// An operation held by lane `from` of the wavefront.
+__device__ __forceinline__ DevOp lane_op(const DevOp& mine, int from) {
+  auto f = [&](float x) {
+    return __builtin_bit_cast(float,
+                              __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), from));
+  };
+  DevOp o;
+  o.code = __builtin_amdgcn_readlane(mine.code, from);
+  o.combine = __builtin_amdgcn_readlane(mine.combine, from);
+  o.translated = 0;
+  o.k = f(mine.k);
+#pragma unroll
+  for (int a = 0; a < 4; ++a) o.prm[a] = f(mine.prm[a]);
+#pragma unroll
+  for (int a = 0; a < 3; ++a) o.off[a] = f(mine.off[a]);
+  o.off[3] = 0.0f;
+  return o;
+}
+
+// sdf_eval of a bounded program at one point a lane, for a wavefront whose
+// points lie close together and whose latency counts: it reads 64 operations
+// at once, one a lane, bounds the runs of min and smooth-min operands over the
+// box of its points, and evaluates out of those registers what can change a
+// value.  `head`: the first 64 operations (lane_ops), which the caller reads
+// when it has something to wait for.  Every lane takes part.
+__device__ __forceinline__ DevOp lane_ops(OpsPtr ops, int base, int n) {
+  const int j = base + static_cast<int>(__lane_id());
+  return load_op(ops, j < n ? j : n - 1);
+}
+
+template <bool kStack>
+__device__ __forceinline__ float sdf_eval_near(OpsPtr ops, int n, const DevOp& head, float px,
+                                               float py, float pz) {
+  const int lane = __lane_id();
+  const float base_p[3] = {px, py, pz};
+  float c[3] = {px, py, pz}, cl[3], ch[3];
+  auto box = [&] {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      cl[a] = wave_min(c[a]);
+      ch[a] = -wave_min(-c[a]);
+    }
+  };
+  box();
+  ShiftStack st;
+#pragma unroll
+  for (int i = 0; i < kMaxValueStack; ++i) st.v[i] = 0.0f;
+  ScopeStack scopes;
+  float top = kNoBound;
+  bool have_top = false;
+  for (int base = 0; base < n; base += 64) {
+    const DevOp mine = base == 0 ? head : lane_ops(ops, base, n);
+    const int e = n - base < 64 ? n - base : 64;
+    const uint64_t run = __ballot(base + lane < n && mine.code <= kCylinder &&
+                                  (mine.combine == kMin || mine.combine == kSmooth));
+    int p = 0;
+    while (p < e) {
+      const uint64_t from = run >> p;
+      uint64_t todo = 1ull << p;
+      int m = 1;
+      if (from & 1ull) {
+        m = ~from ? static_cast<int>(__builtin_ctzll(~from)) : 64;
+        const bool in = lane >= p && lane < p + m;
+        float vlo = kNoBound, vhi = kNoBound;
+        if (in) op_interval(mine, cl, ch, &vlo, &vhi);
+        // as bound_box, from the greatest running value itself
+        const float T = fminf(-wave_min(-top), wave_min_before(vhi));
+        todo = __ballot(in && !(mine.combine == kSmooth ? smooth_inactive(vlo - T, mine.k)
+                                                        : vlo > T));
+      }
+      p += m;
+      for (; todo; todo &= todo - 1) {
+        const int j = static_cast<int>(__builtin_ctzll(todo));
+        const DevOp op = lane_op(mine, j);
+        if (op.code <= kCylinder) {
+          float q[1][3], v[1];
+#pragma unroll
+          for (int a = 0; a < 3; ++a) q[0][a] = c[a] - op.off[a];  // (x - 0 is x)
+          prim_values(op.code, op.prm, q, v);
+          if (op.combine == kPush) {
+            if (kStack && have_top) st.push(top);
+            have_top = true;
+            top = v[0];
+          } else if (op.combine == kMin) {
+            top = fminf(top, v[0]);
+          } else if (op.combine == kSmooth) {
+            top = smooth_min(top, v[0], op.k);
+          } else {
+            // max(top, v), max(v, -top) or max(top, -v)
+            top = fmaxf(op.combine == kDiff ? -top : top, op.combine == kDiffRev ? -v[0] : v[0]);
+          }
+        } else if (op.code == kPushTranslate) {
+          scopes.push(base + j);
+#pragma unroll
+          for (int a = 0; a < 3; ++a) c[a] = c[a] - op.off[a];
+          box();
+        } else if (op.code == kPopTranslate) {
+          scopes.pop();
+#pragma unroll
+          for (int a = 0; a < 3; ++a) c[a] = base_p[a];
+          for (int s = 0; s < scopes.depth; ++s) {
+            const int o = scopes.at(s);
+#pragma unroll
+            for (int a = 0; a < 3; ++a) c[a] = c[a] - ops[o].off[a];
+          }
+          box();
+        } else if (kStack) {
+          const float w = st.pop();
+          if (op.code == kUnion)
+            top = fminf(w, top);
+          else if (op.code == kSmoothUnion)
+            top = smooth_min(w, top, op.k);
+          else  // max(w, t), max(t, -w) or max(w, -t)
+            top = fmaxf(op.code == kDifference ? -w : w, op.code == kDifferenceRev ? -top : top);
+        }
+      }
+    }
+  }
+  return top;
 }
 
 // A barrier for what the tile's wavefronts exchange in LDS: __syncthreads
