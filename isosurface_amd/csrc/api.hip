@@ -85,7 +85,7 @@ struct iso_ctx {
   // extended marching cubes: per active cell state, first ids, flip records
   DevBuf emc_cells, emc_first, emc_flips, emc_ctr, emc_cross;
   // dual contouring: primal samples, dual values and points, mixed list, counters
-  DevBuf dc_normals, dc_plist, dc_pindex, dc_samples, dc_values, dc_points, dc_mixed, dc_flags, dc_counters;
+  DevBuf dc_normals, dc_marks, dc_samples, dc_values, dc_points, dc_mixed, dc_counters;
   unsigned long long* h_dc = nullptr;  // pinned
   // octree marching cubes: nodes, dense primal lattice (or the sorted path's
   // pairs and sort scratch), cubes, edge table, scan state
@@ -333,7 +333,7 @@ int iso_ctx_create(int device, void* stream, iso_ctx** out) {
   }
   if (hipHostMalloc(reinterpret_cast<void**>(&c->h_totals), iso::kTotSlots * sizeof(unsigned long long),
                     hipHostMallocDefault) != hipSuccess ||
-      hipHostMalloc(reinterpret_cast<void**>(&c->h_dc), iso::kDcSlots * sizeof(unsigned long long),
+      hipHostMalloc(reinterpret_cast<void**>(&c->h_dc), sizeof(unsigned long long),
                     hipHostMallocDefault) != hipSuccess ||
       hipHostMalloc(reinterpret_cast<void**>(&c->h_stage), kStageWords * sizeof(unsigned long long),
                     hipHostMallocDefault) != hipSuccess) {
@@ -365,8 +365,8 @@ int iso_ctx_destroy(iso_ctx* c) {
   for (hipEvent_t e : c->event_pool) (void)hipEventDestroy(e);
   DevBuf* bufs[] = {&c->prog,       &c->grid_owned, &c->signs,     &c->seg,      &c->tplanes, &c->vplanes,
                     &c->agg,        &c->incl,       &c->active,    &c->totals,
-                    &c->vout,       &c->iout,       &c->pts,       &c->vals,     &c->dc_normals, &c->dc_plist, &c->dc_pindex, &c->dc_samples,
-                    &c->dc_values,  &c->dc_points,  &c->dc_mixed,  &c->dc_flags,  &c->dc_counters,
+                    &c->vout,       &c->iout,       &c->pts,       &c->vals,     &c->dc_normals, &c->dc_marks, &c->dc_samples,
+                    &c->dc_values,  &c->dc_points,  &c->dc_mixed,  &c->dc_counters,
                     &c->oc_keys,    &c->oc_values,  &c->oc_child,  &c->oc_dense, &c->oc_primal,
                     &c->oc_plevel,  &c->oc_corner,  &c->oc_case,   &c->oc_eslot,
                     &c->oc_tfirst,  &c->oc_split,   &c->oc_ctl,    &c->oc_tkeys,
@@ -1348,64 +1348,37 @@ int iso_extract_dc(iso_ctx* c, const iso_grid_desc* desc, float epsilon, iso_mes
   ISO_HIP(c, ensure(&c->dc_samples, n_points * sizeof(float)));
   ISO_HIP(c, ensure(&c->dc_values, n_cells * sizeof(float)));
   ISO_HIP(c, ensure(&c->dc_points, 3 * n_cells * sizeof(float)));
-  ISO_HIP(c, ensure(&c->dc_mixed, n_cells * sizeof(uint32_t)));
-  ISO_HIP(c, ensure(&c->dc_flags, n_cells));
+  ISO_HIP(c, ensure(&c->dc_mixed,
+                    iso::kDcSegments * iso::dc_segment_room(n_cells) * sizeof(uint32_t)));
+  ISO_HIP(c, ensure(&c->dc_marks, 64 * iso::dc_bricks(L).count()));
   ISO_HIP(c, ensure(&c->dc_counters, iso::kDcSlots * sizeof(unsigned long long)));
+  ISO_HIP(c, ensure(&c->dc_normals, 3 * n_points * sizeof(float)));
   iso::DcBuffers B;
   B.samples = static_cast<float*>(c->dc_samples.ptr);
   B.dual_values = static_cast<float*>(c->dc_values.ptr);
   B.dual_points = static_cast<float*>(c->dc_points.ptr);
   B.mixed = static_cast<uint32_t*>(c->dc_mixed.ptr);
-  B.mixed_flag = static_cast<uint8_t*>(c->dc_flags.ptr);
+  B.marks = static_cast<uint8_t*>(c->dc_marks.ptr);
   B.counters = static_cast<unsigned long long*>(c->dc_counters.ptr);
+  float* normals = static_cast<float*>(c->dc_normals.ptr);
   const iso::DevOp* ops = static_cast<const iso::DevOp*>(c->prog.ptr);
-  ISO_HIP(c, timed(c, "dc_sample",
-                   [&] { return iso::launch_dc_sample(ops, c->n_prog, L, B, c->stream); }));
-  iso::scan::State S{};
-  if ((st = prepare_scan(c, n_cells, &S)) != ISO_OK) return st;
-  ISO_HIP(c, timed(c, "dc_dual", [&] { return iso::launch_dc_dual(L, B, S, c->stream); }));
-  // Central differences evaluate the program six times per normal: the
-  // mixed cells' corners are listed once each and their normals shared.
-  // Analytic normals cost one evaluation: each cell corner takes its own.
-  const bool shared = epsilon > 0.0f;
-  uint32_t* plist = nullptr;
-  uint32_t* pindex = nullptr;
-  if (shared) {
-    ISO_HIP(c, ensure(&c->dc_plist, n_points * sizeof(uint32_t)));
-    ISO_HIP(c, ensure(&c->dc_pindex, n_points * sizeof(uint32_t)));
-    plist = static_cast<uint32_t*>(c->dc_plist.ptr);
-    pindex = static_cast<uint32_t*>(c->dc_pindex.ptr);
-    if ((st = prepare_scan(c, n_points, &S)) != ISO_OK) return st;
-    ISO_HIP(c, timed(c, "dc_points", [&] {
-              return iso::launch_dc_corner_points(L, B, plist, pindex, S, c->stream);
-            }));
-  }
-  // The counts size the normals and feature passes.
-  ISO_HIP(c, hipMemcpyAsync(c->h_dc, B.counters, iso::kDcSlots * sizeof(unsigned long long),
-                            hipMemcpyDeviceToHost, c->stream));
-  ISO_HIP(c, hipStreamSynchronize(c->stream));
-  if (c->h_dc[iso::kDcScanErr])
-    return fail(c, ISO_ERR_DEVICE, "a dual-contouring scan did not complete");
-  const uint64_t n_mixed = c->h_dc[iso::kDcMixed];
-  const uint64_t n_normals = shared ? c->h_dc[iso::kDcPoints] : 8 * n_mixed;
-  ISO_HIP(c, ensure(&c->dc_normals, (n_normals ? n_normals : 1) * 3 * sizeof(float)));
-  float* pnormals = static_cast<float*>(c->dc_normals.ptr);
+  ISO_HIP(c, timed(c, "dc_sample", [&] {
+            return iso::launch_dc_sample(ops, c->n_prog, c->prog_kind, L, B, c->stream);
+          }));
+  ISO_HIP(c, timed(c, "dc_dual", [&] { return iso::launch_dc_dual(L, B, c->stream); }));
   ISO_HIP(c, timed(c, "dc_normals", [&] {
-            return shared ? iso::launch_dc_normals(ops, c->n_prog, L, epsilon, plist, n_normals,
-                                                   pnormals, c->stream)
-                          : iso::launch_dc_cell_normals(ops, c->n_prog, L, epsilon, B, n_mixed,
-                                                        pnormals, c->stream);
+            return iso::launch_dc_normals(ops, c->n_prog, c->prog_kind, L, epsilon, B, normals,
+                                          c->stream);
           }));
-  ISO_HIP(c, timed(c, "dc_feature", [&] {
-            return iso::launch_dc_feature(L, B, n_mixed, pindex, pnormals, c->stream);
-          }));
-  st = extract_lattice(c, Ld, B.dual_values, B.dual_points, out);
-  // The stall flag is final once the stream has passed the feature kernel,
-  // which every extract_lattice path has synchronised past.
-  ISO_HIP(c, hipMemcpyAsync(c->h_dc, B.counters, iso::kDcSlots * sizeof(unsigned long long),
+  ISO_HIP(c, timed(c, "dc_feature",
+                   [&] { return iso::launch_dc_feature(L, B, normals, c->stream); }));
+  // The stall flag is final here; it is read after the mesh, whose round trip
+  // it shares.
+  ISO_HIP(c, hipMemcpyAsync(c->h_dc, B.counters + iso::kDcStalled, sizeof(unsigned long long),
                             hipMemcpyDeviceToHost, c->stream));
+  st = extract_lattice(c, Ld, B.dual_values, B.dual_points, out);
   ISO_HIP(c, hipStreamSynchronize(c->stream));
-  if (c->h_dc[iso::kDcStalled])
+  if (c->h_dc[0])
     return fail(c, ISO_ERR_DEVICE, "a feature point's SVD did not converge");
   return st;
 }

@@ -188,10 +188,14 @@ __device__ __forceinline__ DevOp node_ops(const LhmcTree& T) {
 }
 template <int kKind>
 __device__ __forceinline__ float node_value(const LhmcTree& T, const DevOp& head, const F3& c) {
-  if constexpr (kKind == 0)
+  if constexpr (kKind == 0) {
     return sdf_eval(T.ops, T.n_ops, c.x, c.y, c.z);
-  else
-    return sdf_eval_near<kKind == 2>(as_constant(T.ops), T.n_ops, head, c.x, c.y, c.z);
+  } else {
+    const float p[1][3] = {{c.x, c.y, c.z}};
+    float v[1];
+    sdf_eval_near<1, kKind == 2>(as_constant(T.ops), T.n_ops, head, p, v);
+    return v[0];
+  }
 }
 
 // Signed::within_extent (distance.rs:60-62)

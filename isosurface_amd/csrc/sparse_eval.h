@@ -565,8 +565,8 @@ __device__ __forceinline__ DevOp lane_op(const DevOp& mine, int from) {
   return o;
 }
 
-// sdf_eval of a bounded program at one point a lane, for a wavefront whose
-// points lie close together and whose latency counts: it reads 64 operations
+// sdf_eval of a bounded program at K points a lane, for a wavefront whose
+// points lie close together: it reads 64 operations
 // at once, one a lane, bounds the runs of min and smooth-min operands over the
 // box of its points, and evaluates out of those registers what can change a
 // value.  `head`: the first 64 operations (lane_ops), which the caller reads
@@ -576,25 +576,35 @@ __device__ __forceinline__ DevOp lane_ops(OpsPtr ops, int base, int n) {
   return load_op(ops, j < n ? j : n - 1);
 }
 
-template <bool kStack>
-__device__ __forceinline__ float sdf_eval_near(OpsPtr ops, int n, const DevOp& head, float px,
-                                               float py, float pz) {
+template <int K, bool kStack>
+__device__ __forceinline__ void sdf_eval_near(OpsPtr ops, int n, const DevOp& head,
+                                              const float (&base_p)[K][3], float (&top)[K]) {
   const int lane = __lane_id();
-  const float base_p[3] = {px, py, pz};
-  float c[3] = {px, py, pz}, cl[3], ch[3];
+  float c[K][3], cl[3], ch[3];
   auto box = [&] {
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      cl[a] = wave_min(c[a]);
-      ch[a] = -wave_min(-c[a]);
+      float lo = c[0][a], hi = c[0][a];
+#pragma unroll
+      for (int k = 1; k < K; ++k) {
+        lo = fminf(lo, c[k][a]);
+        hi = fmaxf(hi, c[k][a]);
+      }
+      cl[a] = wave_min(lo);
+      ch[a] = -wave_min(-hi);
     }
   };
-  box();
-  ShiftStack st;
+  ShiftStack st[K];
 #pragma unroll
-  for (int i = 0; i < kMaxValueStack; ++i) st.v[i] = 0.0f;
+  for (int k = 0; k < K; ++k) {
+    top[k] = kNoBound;
+#pragma unroll
+    for (int i = 0; i < kMaxValueStack; ++i) st[k].v[i] = 0.0f;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) c[k][a] = base_p[k][a];
+  }
+  box();
   ScopeStack scopes;
-  float top = kNoBound;
   bool have_top = false;
   for (int base = 0; base < n; base += 64) {
     const DevOp mine = base == 0 ? head : lane_ops(ops, base, n);
@@ -612,7 +622,10 @@ __device__ __forceinline__ float sdf_eval_near(OpsPtr ops, int n, const DevOp& h
         float vlo = kNoBound, vhi = kNoBound;
         if (in) op_interval(mine, cl, ch, &vlo, &vhi);
         // as bound_box, from the greatest running value itself
-        const float T = fminf(-wave_min(-top), wave_min_before(vhi));
+        float most = top[0];
+#pragma unroll
+        for (int k = 1; k < K; ++k) most = fmaxf(most, top[k]);
+        const float T = fminf(-wave_min(-most), wave_min_before(vhi));
         todo = __ballot(in && !(mine.combine == kSmooth ? smooth_inactive(vlo - T, mine.k)
                                                         : vlo > T));
       }
@@ -621,50 +634,63 @@ __device__ __forceinline__ float sdf_eval_near(OpsPtr ops, int n, const DevOp& h
         const int j = static_cast<int>(__builtin_ctzll(todo));
         const DevOp op = lane_op(mine, j);
         if (op.code <= kCylinder) {
-          float q[1][3], v[1];
+          float q[K][3], v[K];
 #pragma unroll
-          for (int a = 0; a < 3; ++a) q[0][a] = c[a] - op.off[a];  // (x - 0 is x)
+          for (int k = 0; k < K; ++k)
+#pragma unroll
+            for (int a = 0; a < 3; ++a) q[k][a] = c[k][a] - op.off[a];  // (x - 0 is x)
           prim_values(op.code, op.prm, q, v);
-          if (op.combine == kPush) {
-            if (kStack && have_top) st.push(top);
-            have_top = true;
-            top = v[0];
-          } else if (op.combine == kMin) {
-            top = fminf(top, v[0]);
-          } else if (op.combine == kSmooth) {
-            top = smooth_min(top, v[0], op.k);
-          } else {
-            // max(top, v), max(v, -top) or max(top, -v)
-            top = fmaxf(op.combine == kDiff ? -top : top, op.combine == kDiffRev ? -v[0] : v[0]);
+          const uint32_t mode = op.combine;
+          if (kStack && mode == kPush && have_top) {
+#pragma unroll
+            for (int k = 0; k < K; ++k) st[k].push(top[k]);
           }
+          if (mode == kPush) have_top = true;
+          // max(top, v), max(v, -top) or max(top, -v)
+          const uint32_t nt = mode == kDiff ? 0x80000000u : 0u;
+          const uint32_t nv = mode == kDiffRev ? 0x80000000u : 0u;
+#pragma unroll
+          for (int k = 0; k < K; ++k)
+            top[k] = mode == kPush     ? v[k]
+                     : mode == kMin    ? fminf(top[k], v[k])
+                     : mode == kSmooth ? smooth_min(top[k], v[k], op.k)
+                                       : fmaxf(flip_sign(top[k], nt), flip_sign(v[k], nv));
         } else if (op.code == kPushTranslate) {
           scopes.push(base + j);
 #pragma unroll
-          for (int a = 0; a < 3; ++a) c[a] = c[a] - op.off[a];
+          for (int k = 0; k < K; ++k)
+#pragma unroll
+            for (int a = 0; a < 3; ++a) c[k][a] = c[k][a] - op.off[a];
           box();
         } else if (op.code == kPopTranslate) {
           scopes.pop();
 #pragma unroll
-          for (int a = 0; a < 3; ++a) c[a] = base_p[a];
+          for (int k = 0; k < K; ++k)
+#pragma unroll
+            for (int a = 0; a < 3; ++a) c[k][a] = base_p[k][a];
           for (int s = 0; s < scopes.depth; ++s) {
             const int o = scopes.at(s);
 #pragma unroll
-            for (int a = 0; a < 3; ++a) c[a] = c[a] - ops[o].off[a];
+            for (int k = 0; k < K; ++k)
+#pragma unroll
+              for (int a = 0; a < 3; ++a) c[k][a] = c[k][a] - ops[o].off[a];
           }
           box();
         } else if (kStack) {
-          const float w = st.pop();
-          if (op.code == kUnion)
-            top = fminf(w, top);
-          else if (op.code == kSmoothUnion)
-            top = smooth_min(w, top, op.k);
-          else  // max(w, t), max(t, -w) or max(w, -t)
-            top = fmaxf(op.code == kDifference ? -w : w, op.code == kDifferenceRev ? -top : top);
+          const uint32_t nw = op.code == kDifference ? 0x80000000u : 0u;
+          const uint32_t nt = op.code == kDifferenceRev ? 0x80000000u : 0u;
+#pragma unroll
+          for (int k = 0; k < K; ++k) {
+            const float w = st[k].pop();
+            top[k] = op.code == kUnion         ? fminf(w, top[k])
+                     : op.code == kSmoothUnion ? smooth_min(w, top[k], op.k)
+                                               // max(w, t), max(t, -w) or max(w, -t)
+                                               : fmaxf(flip_sign(w, nw), flip_sign(top[k], nt));
+          }
         }
       }
     }
   }
-  return top;
 }
 
 // A barrier for what the tile's wavefronts exchange in LDS: __syncthreads

@@ -52,6 +52,12 @@ int64_t tile_count(int64_t nx, int64_t ny, int64_t nz);
 hipError_t launch_signs_sparse(const DevOp* ops, int n_ops, bool stack, const Lattice& L,
                                const McDims& D, const McBuffers& B, float* values, hipStream_t s);
 
+// Samples of a lattice for dual contouring: the program's value near the
+// surface, and 1 or -1 at samples whose own and whose neighbours' dual values
+// are only read for their sign.
+hipError_t launch_samples_sparse(const DevOp* ops, int n_ops, bool stack, const Lattice& L,
+                                 float* samples, hipStream_t s);
+
 // The same for every chunk of a batch (P.sparse), and the extraction's state
 // reset for n_blocks look-back words.
 hipError_t launch_batch_signs_sparse(const BatchPlan& P, const McBuffers& B, int64_t n_blocks,

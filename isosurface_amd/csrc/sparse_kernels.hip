@@ -38,7 +38,6 @@ namespace {
 using namespace mcd;
 
 constexpr int kBricks = 64;      // bricks of a tile: 4 x 4 x 4
-constexpr int kTileCoords = kTileSide + 2;  // coordinates along an axis, neighbours included
 constexpr int kListCap = 512;    // operations of a tile's list; a longer one is not kept
 constexpr uint32_t kSparseXcds = 8;
 
@@ -75,16 +74,26 @@ struct BatchTiles {
 // W wavefronts per tile: one where tiles alone fill the chip, four where a
 // small lattice leaves it idle (the bricks of a tile are then spread over
 // four SIMDs; the bounds are one wavefront's work either way).
-template <class Tiles, int W, bool kStack>
+//
+// kSamples: for dual contouring, which takes no sign words but reads all
+// samples, a dual value being half the sum of two opposite corners of a cell.
+// A sample of a proven brick is 1 or -1 there.  A dual value is read for more
+// than its sign only where its dual neighbour's differs, and the samples of
+// both lie within two of any of them: the bounds are taken two samples wider,
+// and from 1e-30 on where half a sample could round to zero.
+template <class Tiles, int W, bool kStack, bool kSamples>
 __global__ __launch_bounds__(64 * W) void k_signs_sparse(Tiles tiles, uint32_t n_tiles,
                                                          uint32_t group, ResetArgs R) {
+  constexpr int kMargin = kSamples ? 2 : 1;  // neighbours in a brick's box
+  constexpr int kTileCoords = kTileSide + 2 * kMargin;  // coordinates along an axis
+  constexpr float kOutside = kSamples ? 1.0e-30f : 0.0f;
   __shared__ uint64_t s_sign[kBricks];  // sign bits of a brick's samples, x fastest
   __shared__ uint16_t s_list[kListCap];  // operations that matter in the tile
   __shared__ uint64_t s_mask[kListCap];  // and the bricks each of them matters in
   __shared__ float s_coord[3 * kTileCoords];
   __shared__ int s_len;
   __shared__ uint64_t s_todo;
-  reset_state(R);
+  if (!kSamples) reset_state(R);
   // Groups of consecutive tiles (a row's neighbours share lines of sign words
   // and values) go to one XCD, the groups round robin.
   const uint32_t q = blockIdx.x / kSparseXcds;
@@ -117,7 +126,7 @@ __global__ __launch_bounds__(64 * W) void k_signs_sparse(Tiles tiles, uint32_t n
     if (lane < 3 * kTileCoords) {
       const int a = lane / kTileCoords;
       const int32_t na = a == 0 ? nx : a == 1 ? ny : nz;
-      int32_t i = (a == 0 ? s0[0] : a == 1 ? s0[1] : s0[2]) + lane - kTileCoords * a - 1;
+      int32_t i = (a == 0 ? s0[0] : a == 1 ? s0[1] : s0[2]) + lane - kTileCoords * a - kMargin;
       i = i < 0 ? 0 : i < na ? i : na - 1;
       const float o = a == 0 ? C.origin[0] : a == 1 ? C.origin[1] : C.origin[2];
       const float d = a == 0 ? C.spacing[0] : a == 1 ? C.spacing[1] : C.spacing[2];
@@ -137,7 +146,7 @@ __global__ __launch_bounds__(64 * W) void k_signs_sparse(Tiles tiles, uint32_t n
     }
     float lo, hi;
     int len = bound_box<kStack>(ops, first, n_ops, blo, bhi, s_list, kListCap, &lo, &hi);
-    bool outside = lo > 0.0f, inside = hi <= 0.0f;
+    bool outside = lo > kOutside, inside = hi <= 0.0f;
     bool active = true;
     if (!outside && !inside) {
       // Then its bricks', each with its samples' neighbours.
@@ -146,7 +155,7 @@ __global__ __launch_bounds__(64 * W) void k_signs_sparse(Tiles tiles, uint32_t n
       for (int a = 0; a < 3; ++a) {
         active = active && s0[a] + 4 * b[a] < n[a];
         const float c0 = s_coord[kTileCoords * a + 4 * b[a]];
-        const float c1 = s_coord[kTileCoords * a + 4 * b[a] + 5];
+        const float c1 = s_coord[kTileCoords * a + 4 * b[a] + 3 + 2 * kMargin];
         blo[a] = fminf(c0, c1);
         bhi[a] = fmaxf(c0, c1);
       }
@@ -155,7 +164,7 @@ __global__ __launch_bounds__(64 * W) void k_signs_sparse(Tiles tiles, uint32_t n
       const int left = bound_lanes<kStack>(ops, first, fits ? len : n_ops - first, blo, bhi,
                                            active, fits ? s_list : nullptr, s_mask, &lo, &hi);
       if (fits) len = left;
-      outside = lo > 0.0f;
+      outside = lo > kOutside;
       inside = hi <= 0.0f;
     }
     s_sign[lane] = inside ? ~0ull : 0ull;
@@ -175,6 +184,17 @@ __global__ __launch_bounds__(64 * W) void k_signs_sparse(Tiles tiles, uint32_t n
            (static_cast<uint64_t>(static_cast<uint32_t>(
                 __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(t >> 32))))
             << 32);
+  }
+  if (kSamples && ~todo) {
+    // rows of sixteen samples, four a wavefront's store
+    float* grid = const_cast<float*>(C.grid);
+    for (int i = threadIdx.x; i < kTileSide * kTileSide * kTileSide; i += 64 * W) {
+      const int x = i & 15, y = (i >> 4) & 15, z = i >> 8;
+      const int b = (z >> 2) * 16 + (y & 12) + (x >> 2);
+      if ((todo >> b & 1) || s0[0] + x >= nx || s0[1] + y >= ny || s0[2] + z >= nz) continue;
+      grid[(static_cast<int64_t>(s0[2] + z) * ny + s0[1] + y) * nx + s0[0] + x] =
+          s_sign[b] ? -1.0f : 1.0f;
+    }
   }
   const uint16_t* list = len <= kListCap ? s_list : nullptr;
   const int m = len <= kListCap ? len : n_ops - first;
@@ -205,9 +225,9 @@ __global__ __launch_bounds__(64 * W) void k_signs_sparse(Tiles tiles, uint32_t n
 #pragma unroll
     for (int j = 0; j < kPoints; ++j) {
       const int b = brick[j];
-      p[j][0] = s_coord[1 + 4 * (b & 3) + lx];
-      p[j][1] = s_coord[kTileCoords + 1 + (b & 12) + ly];
-      p[j][2] = s_coord[2 * kTileCoords + 1 + 4 * (b >> 4) + lz];
+      p[j][0] = s_coord[kMargin + 4 * (b & 3) + lx];
+      p[j][1] = s_coord[kTileCoords + kMargin + (b & 12) + ly];
+      p[j][2] = s_coord[2 * kTileCoords + kMargin + 4 * (b >> 4) + lz];
     }
     sdf_eval_list<kPoints, kStack>(ops, first, list, s_mask, bricks, m, p, v);
     uint64_t mine = 0;
@@ -224,12 +244,14 @@ __global__ __launch_bounds__(64 * W) void k_signs_sparse(Tiles tiles, uint32_t n
       const uint64_t in = __ballot(valid && !(v[j] > 0.0f));
       if (lane == j) mine = in;
     }
+    if (kSamples) continue;
     // (a spare point repeats the first brick)
     int slot = brick[0];
 #pragma unroll
     for (int j = 1; j < kPoints; ++j) slot = lane == j ? brick[j] : slot;
     if (lane < kPoints) s_sign[slot] = mine;
   }
+  if (kSamples) return;
   lds_barrier<W>();
   store_tile_signs(C, s_sign, s0, tx, threadIdx.x, 64 * W);
 }
@@ -327,10 +349,25 @@ hipError_t launch_signs_sparse(const DevOp* ops, int n_ops, bool stack, const La
   const int64_t n = tile_count(L.nx, L.ny, L.nz);
   const int64_t group = (L.nx + kTileSide - 1) >> kTileShift;
   if (n >= kManyTiles)
-    return stack ? launch_tiles(k_signs_sparse<SingleTiles, 1, true>, 64, t, n, group, R, s)
-                 : launch_tiles(k_signs_sparse<SingleTiles, 1, false>, 64, t, n, group, R, s);
-  return stack ? launch_tiles(k_signs_sparse<SingleTiles, 4, true>, 256, t, n, group, R, s)
-               : launch_tiles(k_signs_sparse<SingleTiles, 4, false>, 256, t, n, group, R, s);
+    return stack ? launch_tiles(k_signs_sparse<SingleTiles, 1, true, false>, 64, t, n, group, R, s)
+                 : launch_tiles(k_signs_sparse<SingleTiles, 1, false, false>, 64, t, n, group, R, s);
+  return stack ? launch_tiles(k_signs_sparse<SingleTiles, 4, true, false>, 256, t, n, group, R, s)
+               : launch_tiles(k_signs_sparse<SingleTiles, 4, false, false>, 256, t, n, group, R, s);
+}
+
+hipError_t launch_samples_sparse(const DevOp* ops, int n_ops, bool stack, const Lattice& L,
+                                 float* samples, hipStream_t s) {
+  if (!ops || !samples) return hipErrorInvalidValue;
+  const SingleTiles t{
+      single_cell_space(L, mc_dims_pitched(L), nullptr, ops, n_ops, samples, nullptr)};
+  const int64_t n = tile_count(L.nx, L.ny, L.nz);
+  const int64_t group = (L.nx + kTileSide - 1) >> kTileShift;
+  const ResetArgs R{};
+  if (n >= kManyTiles)
+    return stack ? launch_tiles(k_signs_sparse<SingleTiles, 1, true, true>, 64, t, n, group, R, s)
+                 : launch_tiles(k_signs_sparse<SingleTiles, 1, false, true>, 64, t, n, group, R, s);
+  return stack ? launch_tiles(k_signs_sparse<SingleTiles, 4, true, true>, 256, t, n, group, R, s)
+               : launch_tiles(k_signs_sparse<SingleTiles, 4, false, true>, 256, t, n, group, R, s);
 }
 
 hipError_t launch_batch_signs_sparse(const BatchPlan& P, const McBuffers& B, int64_t n_blocks,
@@ -346,10 +383,10 @@ hipError_t launch_batch_signs_sparse(const BatchPlan& P, const McBuffers& B, int
   R.totals = B.totals;
   constexpr int64_t kGroup = 4;  // about a row of a chunk's tiles
   if (P.n_tiles >= kManyTiles)
-    return P.stack ? launch_tiles(k_signs_sparse<BatchTiles, 1, true>, 64, t, P.n_tiles, kGroup, R, s)
-                   : launch_tiles(k_signs_sparse<BatchTiles, 1, false>, 64, t, P.n_tiles, kGroup, R, s);
-  return P.stack ? launch_tiles(k_signs_sparse<BatchTiles, 4, true>, 256, t, P.n_tiles, kGroup, R, s)
-                 : launch_tiles(k_signs_sparse<BatchTiles, 4, false>, 256, t, P.n_tiles, kGroup, R, s);
+    return P.stack ? launch_tiles(k_signs_sparse<BatchTiles, 1, true, false>, 64, t, P.n_tiles, kGroup, R, s)
+                   : launch_tiles(k_signs_sparse<BatchTiles, 1, false, false>, 64, t, P.n_tiles, kGroup, R, s);
+  return P.stack ? launch_tiles(k_signs_sparse<BatchTiles, 4, true, false>, 256, t, P.n_tiles, kGroup, R, s)
+                 : launch_tiles(k_signs_sparse<BatchTiles, 4, false, false>, 256, t, P.n_tiles, kGroup, R, s);
 }
 
 }  // namespace iso
