@@ -1120,7 +1120,8 @@ int iso_extract_emc(iso_ctx* c, const iso_grid_desc* desc, float epsilon, iso_me
   c->kept = false;
   c->band_valid = false;
   ISO_HIP(c, hipSetDevice(c->device));
-  const iso::McDims D = iso::mc_dims(L);
+  const bool sparse = iso::sparse_lattice(L, c->prog_kind.bounded);
+  const iso::McDims D = sparse ? iso::mc_dims_pitched(L) : iso::mc_dims(L);
   if (D.n_segs >= (int64_t(1) << 26))
     return fail(c, ISO_ERR_INVALID_ARGUMENT, "lattice has 2^26 or more 64-cell segments");
   iso::McBuffers B{};
@@ -1132,7 +1133,9 @@ int iso_extract_emc(iso_ctx* c, const iso_grid_desc* desc, float epsilon, iso_me
   uint64_t n_act = 0;
   for (int attempt = 0; attempt < 2; ++attempt) {
     ISO_HIP(c, timed(c, "mc_signs_directed", [&] {
-              return iso::launch_signs_directed(ops, c->n_prog, L, D, B, vals, c->stream);
+              return sparse ? iso::launch_directed_sparse(ops, c->n_prog, c->prog_kind.stack, L, D,
+                                                          B, vals, c->stream)
+                            : iso::launch_signs_directed(ops, c->n_prog, L, D, B, vals, c->stream);
             }));
     ISO_HIP(c, timed(c, "mc_count", [&] { return iso::launch_count(L, D, B, c->stream); }));
     if ((st = read_totals(c, B)) != ISO_OK) return st;
@@ -1167,7 +1170,9 @@ int iso_extract_emc(iso_ctx* c, const iso_grid_desc* desc, float epsilon, iso_me
   A.counters = static_cast<unsigned long long*>(c->emc_ctr.ptr);
   ISO_HIP(c, ensure(&c->emc_cross, na * 72 * sizeof(float)));
   A.crossings = static_cast<float*>(c->emc_cross.ptr);
-  ISO_HIP(c, timed(c, "emc_crossings", [&] { return iso::launch_emc_crossings(A, c->stream); }));
+  ISO_HIP(c, timed(c, "emc_crossings", [&] {
+            return iso::launch_emc_crossings(A, c->prog_kind, c->stream);
+          }));
   ISO_HIP(c, timed(c, "emc_cells", [&] { return iso::launch_emc_cells(A, S, c->stream); }));
   ISO_HIP(c, hipMemcpyAsync(c->h_stage, S.ctl, 4 * sizeof(unsigned long long),
                             hipMemcpyDeviceToHost, c->stream));

@@ -182,7 +182,7 @@ __global__ __launch_bounds__(256) void k_sample_normals(const DevOp* __restrict_
 // stack, 2 bounded with one: then the operations are bounded over the brick's
 // marked points and only those that can change a value there are evaluated, at
 // the six points of a central difference at once.  (The normals of a 128^3
-// lattice over 32 boxes: 41 us; listing the points by a scan and evaluating
+// lattice over 32 boxes: 43 us; listing the points by a scan and evaluating
 // all 32 at each took 35 and 87.)
 template <int kKind>
 __global__ __launch_bounds__(256) void k_dc_normals(const DevOp* __restrict__ ops, int n_ops,

@@ -22,6 +22,7 @@
 
 #include "mc_kernels.h"
 #include "scan.h"
+#include "sparse_kernels.h"
 
 namespace iso {
 
@@ -59,7 +60,7 @@ struct EmcArgs {
 
 // Stage 0: the crossing points and normals of every active cell's crossed
 // edges, one thread per (cell, edge).
-hipError_t launch_emc_crossings(const EmcArgs& A, hipStream_t s);
+hipError_t launch_emc_crossings(const EmcArgs& A, const ProgramKind& kind, hipStream_t s);
 // Stage 1: cells + scan (state for n_act items at one item per thread).
 // The totals land in scan state ctl[1]: triangles << 32 | vertices.
 hipError_t launch_emc_cells(const EmcArgs& A, const scan::State& st, hipStream_t s);

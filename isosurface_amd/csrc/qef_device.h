@@ -12,6 +12,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 namespace iso {
 namespace qef {
 
@@ -39,6 +41,14 @@ __device__ __forceinline__ Vec3f normalised_or_zero(Vec3f v) {
 
 // The SVD of a rows x 3 matrix (rows <= R): every loop over rows runs to
 // `rows`, so the arithmetic is that of the reference's rows-row matrix.
+//
+// One thread's solve is a serial chain of f64 operations, and latency bounds
+// it: a launch has about one wavefront for each SIMD.  So indices are constants
+// once the loops are unrolled (the column window is a template argument, a
+// run-time column becomes a choice between constants), and cases that differ
+// in their operands choose those first and share one chain: the feature pass
+// of 128^3 dual contouring over 32 boxes takes 37 us, with run-time columns and
+// a division in every branch 48.
 template <int R>
 struct SvdT {
   double u[R][3];
@@ -47,8 +57,9 @@ struct SvdT {
   int rows;
 };
 
-// Householder reflection of the n entries x[0], x[stride], ... (svd.rs:251-293).
-__device__ __forceinline__ double householder(double* x, int n, int stride) {
+// Householder reflection of the n <= N entries x[0], x[stride], ... (svd.rs:251-293).
+template <int N, int stride>
+__device__ __forceinline__ double householder(double* x, int n) {
   double tau = 0.0;
   if (n > 1) {
     double xnorm;
@@ -56,15 +67,15 @@ __device__ __forceinline__ double householder(double* x, int n, int stride) {
       xnorm = __builtin_fabs(x[stride]);
     } else {
       double scl = 0.0, ssq = 1.0;
-      for (int i = 1; i < n; ++i) {
+#pragma unroll
+      for (int i = 1; i < N; ++i) {
+        if (i >= n) continue;
         const double a = __builtin_fabs(x[i * stride]);
-        if (a != 0.0) {
-          if (scl < a) {
-            ssq = 1.0 + ssq * (scl / a) * (scl / a);
-            scl = a;
-          } else {
-            ssq += a / scl * (a / scl);
-          }
+        if (a != 0.0) {  // (one division for both cases)
+          const bool up = scl < a;
+          const double r = (up ? scl : a) / (up ? a : scl);
+          ssq = up ? 1.0 + ssq * r * r : ssq + r * r;
+          scl = up ? a : scl;
         }
       }
       xnorm = scl * __builtin_sqrt(ssq);
@@ -76,63 +87,85 @@ __device__ __forceinline__ double householder(double* x, int n, int stride) {
       tau = (beta - alpha) / beta;
       const double scl = 1.0 / (alpha - beta);
       x[0] = beta;
-      for (int i = 1; i < n; ++i) x[i * stride] *= scl;
+#pragma unroll
+      for (int i = 1; i < N; ++i)
+        if (i < n) x[i * stride] *= scl;
     }
   }
   return tau;
 }
 
-// Bidiagonal factorisation (svd.rs:149-249).
-template <int R>
-__device__ __forceinline__ void bidiagonalise(double m[R][3], double tau_u[3], double tau_v[2],
-                                              int rows) {
-  for (int i = 0; i < 3; ++i) {
-    double tau = householder(&m[i][i], rows - i, 3);
-    tau_u[i] = tau;
-    if (i + 1 < 3) {
-      if (tau != 0.0) {
-        for (int x = i + 1; x < 3; ++x) {
-          double wx = m[i][x];
-          for (int y = i + 1; y < rows; ++y) wx += m[y][x] * m[y][i];
-          const double tw = tau * wx;
-          m[i][x] -= tw;
-          for (int y = i + 1; y < rows; ++y) m[y][x] -= tw * m[y][i];
-        }
+// Step i of the bidiagonal factorisation (svd.rs:149-249).
+template <int R, int i>
+__device__ __forceinline__ void bidiagonalise_step(double m[R][3], double tau_u[3], double tau_v[2],
+                                                   int rows) {
+  double tau = householder<R - i, 3>(&m[i][i], rows - i);
+  tau_u[i] = tau;
+  if constexpr (i + 1 < 3) {
+    if (tau != 0.0) {
+#pragma unroll
+      for (int x = i + 1; x < 3; ++x) {
+        double wx = m[i][x];
+#pragma unroll
+        for (int y = i + 1; y < R; ++y)
+          if (y < rows) wx += m[y][x] * m[y][i];
+        const double tw = tau * wx;
+        m[i][x] -= tw;
+#pragma unroll
+        for (int y = i + 1; y < R; ++y)
+          if (y < rows) m[y][x] -= tw * m[y][i];
       }
-      tau = householder(&m[i][i + 1], i == 0 ? 2 : 1, 1);
-      tau_v[i] = tau;
-      if (tau != 0.0) {
-        for (int y = i + 1; y < rows; ++y) {
-          double wy = m[y][i + 1];
-          if (i == 0) wy += m[y][i + 2] * m[i][i + 2];
-          const double tw = tau * wy;
-          m[y][i + 1] -= tw;
-          if (i == 0) m[y][i + 2] -= tw * m[i][i + 2];
-        }
+    }
+    tau = householder<2 - i, 1>(&m[i][i + 1], 2 - i);
+    tau_v[i] = tau;
+    if (tau != 0.0) {
+#pragma unroll
+      for (int y = i + 1; y < R; ++y) {
+        if (y >= rows) continue;
+        double wy = m[y][i + 1];
+        if constexpr (i == 0) wy += m[y][i + 2] * m[i][i + 2];
+        const double tw = tau * wy;
+        m[y][i + 1] -= tw;
+        if constexpr (i == 0) m[y][i + 2] -= tw * m[i][i + 2];
       }
     }
   }
+}
+template <int R>
+__device__ __forceinline__ void bidiagonalise(double m[R][3], double tau_u[3], double tau_v[2],
+                                              int rows) {
+  bidiagonalise_step<R, 0>(m, tau_u, tau_v, rows);
+  bidiagonalise_step<R, 1>(m, tau_u, tau_v, rows);
+  bidiagonalise_step<R, 2>(m, tau_u, tau_v, rows);
 }
 
 // Accumulates the reflections into U and V (svd.rs:295-410).
 template <int R>
 __device__ __forceinline__ void unpack(double u[R][3], double v[3][3], double tau_u[3],
                                        double tau_v[2], int rows) {
+#pragma unroll
   for (int i = 0; i < 3; ++i)
+#pragma unroll
     for (int j = 0; j < 3; ++j) v[i][j] = i == j ? 1.0 : 0.0;
+#pragma unroll
   for (int i = 1; i >= 0; --i) {
     const double tau = tau_v[i];
     if (tau != 0.0) {
+#pragma unroll
       for (int x = i + 1; x < 3; ++x) {
         double wx = v[i + 1][x];
+#pragma unroll
         for (int y = i + 2; y < 3; ++y) wx += v[y][x] * u[i][y];
         const double tw = tau * wx;
         v[i + 1][x] -= tw;
+#pragma unroll
         for (int y = i + 2; y < 3; ++y) v[y][x] -= tw * u[i][y];
       }
     }
   }
+#pragma unroll
   for (int i = 0; i < 2; ++i) tau_v[i] = u[i][i + 1];
+#pragma unroll
   for (int i = 2; i >= 0; --i) {
     const double tau = tau_u[i];
     tau_u[i] = u[i][i];
@@ -142,36 +175,39 @@ __device__ __forceinline__ void unpack(double u[R][3], double v[3][3], double ta
         u[i][2] = 0.0;
         if (i < 1) u[i][1] = 0.0;
       }
-      for (int y = i + 1; y < rows; ++y) u[y][i] = 0.0;
+#pragma unroll
+      for (int y = i + 1; y < R; ++y)
+        if (y < rows) u[y][i] = 0.0;
     } else {
+#pragma unroll
       for (int x = i + 1; x < 3; ++x) {
         double wx = 0.0;
-        for (int y = i + 1; y < rows; ++y) wx += u[y][x] * u[y][i];
+#pragma unroll
+        for (int y = i + 1; y < R; ++y)
+          if (y < rows) wx += u[y][x] * u[y][i];
         const double tw = tau * wx;
         u[i][x] = -tw;
-        for (int y = i + 1; y < rows; ++y) u[y][x] -= tw * u[y][i];
+#pragma unroll
+        for (int y = i + 1; y < R; ++y)
+          if (y < rows) u[y][x] -= tw * u[y][i];
       }
-      for (int y = i + 1; y < rows; ++y) u[y][i] = u[y][i] * -tau;
+#pragma unroll
+      for (int y = i + 1; y < R; ++y)
+        if (y < rows) u[y][i] = u[y][i] * -tau;
       u[i][i] = 1.0 - tau;
     }
   }
 }
 
+// The cases of the next three differ in their operands: chosen first, each is
+// one chain of divisions and square roots for the whole wavefront.
 __device__ __forceinline__ void givens(double a, double b, double* c, double* s) {  // svd.rs:825-842
-  if (b == 0.0) {
-    *c = 1.0;
-    *s = 0.0;
-  } else if (__builtin_fabs(b) > __builtin_fabs(a)) {
-    const double t = -a / b;
-    const double s1 = 1.0 / __builtin_sqrt(1.0 + t * t);
-    *s = s1;
-    *c = s1 * t;
-  } else {
-    const double t = -b / a;
-    const double c1 = 1.0 / __builtin_sqrt(1.0 + t * t);
-    *c = c1;
-    *s = c1 * t;
-  }
+  const bool steep = __builtin_fabs(b) > __builtin_fabs(a);
+  const double t = -(steep ? a : b) / (steep ? b : a);
+  const double r = 1.0 / __builtin_sqrt(1.0 + t * t);
+  const double rt = r * t;
+  *c = b == 0.0 ? 1.0 : steep ? rt : r;
+  *s = b == 0.0 ? 0.0 : steep ? r : rt;
 }
 
 __device__ __forceinline__ void schur(double a1, double a2, double a3, double* c, double* s) {  // svd.rs:844-865
@@ -181,65 +217,69 @@ __device__ __forceinline__ void schur(double a1, double a2, double a3, double* c
     *s = 0.0;
   } else {
     const double tau = (a2 * a2 + (a3 + a1) * (a3 - a1)) / apq;
-    const double t = tau >= 0.0 ? 1.0 / (tau + __builtin_sqrt(1.0 + tau * tau))
-                                : -1.0 / (__builtin_sqrt(1.0 + tau * tau) - tau);
+    const double q = __builtin_sqrt(1.0 + tau * tau);
+    const double r = 1.0 / (tau >= 0.0 ? tau + q : q - tau);
+    const double t = tau >= 0.0 ? r : -r;
     *c = 1.0 / __builtin_sqrt(1.0 + t * t);
     *s = t * *c;
   }
 }
 
-__device__ __forceinline__ void chop(double* a, double* b, int n) {  // svd.rs:481-493
-  double ai = a[0];
-  for (int i = 0; i < n - 1; ++i) {
-    const double bi = b[i];
-    const double ai1 = a[i + 1];
-    if (__builtin_fabs(bi) < 1e-5 * (__builtin_fabs(ai) + __builtin_fabs(ai1))) b[i] = 0.0;
-    ai = ai1;
-  }
+// On the n columns from a on (svd.rs:481-493).
+template <int a, int n>
+__device__ __forceinline__ void chop(double tu[3], double tv[2]) {
+#pragma unroll
+  for (int i = a; i < a + n - 1; ++i)
+    if (__builtin_fabs(tv[i]) < 1e-5 * (__builtin_fabs(tu[i]) + __builtin_fabs(tu[i + 1])))
+      tv[i] = 0.0;
 }
 
-// Rotates columns p and q (absolute) of the first `rows` rows by (c, s).
-template <int R>
-__device__ __forceinline__ void rotate(double m[R][3], int rows, int p, int q, double c,
-                                       double s) {
-  for (int i = 0; i < rows; ++i) {
+// Rotates columns p and q of the first `rows` rows by (c, s).
+template <int R, int p, int q>
+__device__ __forceinline__ void rotate(double m[R][3], int rows, double c, double s) {
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    if (i >= rows) continue;
     const double mp = m[i][p], mq = m[i][q];
     m[i][p] = mp * c - mq * s;
     m[i][q] = mp * s + mq * c;
   }
 }
 
-__device__ __forceinline__ void swap_cols01(double v[3][3], int a) {
-  for (int i = 0; i < 3; ++i) {
-    const double t = v[i][a];
-    v[i][a] = v[i][a + 1];
-    v[i][a + 1] = t;
+template <int a, int b, int R>
+__device__ __forceinline__ void swap_cols(double m[R][3], int rows) {
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    if (i >= rows) continue;
+    const double t = m[i][a];
+    m[i][a] = m[i][b];
+    m[i][b] = t;
   }
 }
 
 // QR step on the 2-column window [a, a+1] (svd.rs:689-823).
-template <int R>
-__device__ __forceinline__ void qr_cols2(SvdT<R>& S, double* tu, double* tv, int a) {
+template <int a, int R>
+__device__ __forceinline__ void qr_cols2(SvdT<R>& S, double tu[3], double tv[2]) {
   double c, s;
-  if (tu[0] == 0.0) {
-    givens(tv[0], tu[1], &c, &s);
-    tu[0] = tv[0] * c - tu[1] * s;
-    tv[0] = tv[0] * s + tu[1] * c;
-    tu[1] = 0.0;
-    rotate<R>(S.u, S.rows, a, a + 1, c, s);
-    swap_cols01(S.v, a);
-  } else if (tu[1] == 0.0) {
-    givens(tu[0], tv[0], &c, &s);
-    tu[0] = tu[0] * c - tv[0] * s;
-    tv[0] = 0.0;
-    rotate<3>(S.v, 3, a, a + 1, c, s);
+  if (tu[a] == 0.0) {
+    givens(tv[a], tu[a + 1], &c, &s);
+    tu[a] = tv[a] * c - tu[a + 1] * s;
+    tv[a] = tv[a] * s + tu[a + 1] * c;
+    tu[a + 1] = 0.0;
+    rotate<R, a, a + 1>(S.u, S.rows, c, s);
+    swap_cols<a, a + 1, 3>(S.v, 3);
+  } else if (tu[a + 1] == 0.0) {
+    givens(tu[a], tv[a], &c, &s);
+    tu[a] = tu[a] * c - tv[a] * s;
+    tv[a] = 0.0;
+    rotate<3, a, a + 1>(S.v, 3, c, s);
   } else {
-    schur(tu[0], tv[0], tu[1], &c, &s);
-    double a11 = tu[0] * c - tv[0] * s;
-    double a21 = -tu[1] * s;
-    double a12 = tu[0] * s + tv[0] * c;
-    double a22 = tu[1] * c;
-    rotate<3>(S.v, 3, a, a + 1, c, s);
+    schur(tu[a], tv[a], tu[a + 1], &c, &s);
+    double a11 = tu[a] * c - tv[a] * s;
+    double a21 = -tu[a + 1] * s;
+    double a12 = tu[a] * s + tv[a] * c;
+    double a22 = tu[a + 1] * c;
+    rotate<3, a, a + 1>(S.v, 3, c, s);
     if (a11 * a11 + a21 * a21 < a12 * a12 + a22 * a22) {
       double t = a11;
       a11 = a12;
@@ -247,32 +287,34 @@ __device__ __forceinline__ void qr_cols2(SvdT<R>& S, double* tu, double* tv, int
       t = a21;
       a21 = a22;
       a22 = t;
-      swap_cols01(S.v, a);
+      swap_cols<a, a + 1, 3>(S.v, 3);
     }
     givens(a11, a21, &c, &s);
-    tu[0] = a11 * c - a21 * s;
-    tv[0] = a12 * c - a22 * s;
-    tu[1] = a12 * s + a22 * c;
-    rotate<R>(S.u, S.rows, a, a + 1, c, s);
+    tu[a] = a11 * c - a21 * s;
+    tv[a] = a12 * c - a22 * s;
+    tu[a + 1] = a12 * s + a22 * c;
+    rotate<R, a, a + 1>(S.u, S.rows, c, s);
   }
 }
 
-// A zero on the diagonal inside the 3-column window (svd.rs:604-641).
-template <int R>
-__device__ __forceinline__ void qr_middle(SvdT<R>& S, double* tu, double* tv, int cols,
-                                          int col) {
+// A zero on the diagonal at `col` inside the 3-column window (svd.rs:604-641).
+template <int col, int R>
+__device__ __forceinline__ void qr_middle(SvdT<R>& S, double tu[3], double tv[2]) {
   double x = tv[col], y = tu[col + 1];
-  for (int j = col; j < cols - 1; ++j) {
+#pragma unroll
+  for (int j = col; j < 2; ++j) {
     double c, s;
     givens(y, -x, &c, &s);
-    for (int i = 0; i < S.rows; ++i) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      if (i >= S.rows) continue;
       const double up = S.u[i][col], uq = S.u[i][j + 1];
       S.u[i][col] = up * c - uq * s;
       S.u[i][j + 1] = up * s + uq * c;
     }
     tu[j + 1] = x * s + y * c;
     if (j == col) tv[j] = x * c - y * s;
-    if (j < cols - 2) {
+    if (j < 1) {
       const double z = tv[j + 1];
       tv[j + 1] *= c;
       x = z * -s;
@@ -283,11 +325,13 @@ __device__ __forceinline__ void qr_middle(SvdT<R>& S, double* tu, double* tv, in
 
 // A zero at the end of the diagonal (svd.rs:643-671).
 template <int R>
-__device__ __forceinline__ void qr_end(SvdT<R>& S, double* tu, double* tv) {
+__device__ __forceinline__ void qr_end(SvdT<R>& S, double tu[3], double tv[2]) {
   double x = tu[1], y = tv[1];
+#pragma unroll
   for (int k = 1; k >= 0; --k) {
     double c, s;
     givens(x, y, &c, &s);
+#pragma unroll
     for (int i = 0; i < 3; ++i) {
       const double vp = S.v[i][k], vq = S.v[i][2];
       S.v[i][k] = vp * c - vq * s;
@@ -309,25 +353,64 @@ __device__ __forceinline__ double qr_shift(const double* tu, const double* tv) {
   const double tb = tu[2] * tu[2] + tv[1] * tv[1];
   const double tab = tu[1] * tv[1];
   const double dt = (ta - tb) / 2.0;
-  if (dt >= 0.0) return tb - tab * tab / (dt + __builtin_sqrt(dt * dt + tab * tab));
-  return tb + tab * tab / (__builtin_sqrt(dt * dt + tab * tab) - dt);
+  const double q = __builtin_sqrt(dt * dt + tab * tab);
+  const double r = tab * tab / (dt >= 0.0 ? dt + q : q - dt);
+  return dt >= 0.0 ? tb - r : tb + r;
 }
 
-// One implicit-shift QR sweep on the window [a, a+cols) (svd.rs:495-602).
+// Column k of a sweep over the whole matrix.
+template <int k, int R>
+__device__ __forceinline__ void qr_column(SvdT<R>& S, double tu[3], double tv[2], double& y,
+                                          double& z, double& ak, double& bk, double& zk, double& ap,
+                                          double& bp, double& aq) {
+  double c, s;
+  givens(y, z, &c, &s);
+  rotate<3, k, k + 1>(S.v, 3, c, s);
+  double bk1 = bk * c - z * s;
+  double ap1 = ap * c - bp * s;
+  double bp1 = ap * s + bp * c;
+  const double zp1 = aq * -s;
+  const double aq1 = aq * c;
+  if constexpr (k > 0) tv[k - 1] = bk1;
+  ak = ap1;
+  bk = bp1;
+  zk = zp1;
+  ap = aq1;
+  bp = 0.0;
+  if constexpr (k < 1) bp = tv[k + 1];
+  y = ak;
+  z = zk;
+  givens(y, z, &c, &s);
+  rotate<R, k, k + 1>(S.u, S.rows, c, s);
+  const double ak1 = ak * c - zk * s;
+  bk1 = bk * c - ap * s;
+  const double zk1 = bp * -s;
+  ap1 = bk * s + ap * c;
+  bp1 = bp * c;
+  tu[k] = ak1;
+  ak = ak1;
+  bk = bk1;
+  zk = zk1;
+  ap = ap1;
+  bp = bp1;
+  aq = 0.0;
+  if constexpr (k < 1) aq = tu[k + 2];
+  y = bk;
+  z = zk;
+}
+
+// One implicit-shift QR sweep over all three columns (svd.rs:495-602).
 template <int R>
-__device__ __forceinline__ void qr_step(SvdT<R>& S, double* tu, double* tv, int a, int cols) {
-  if (cols == 2) {
-    qr_cols2(S, tu, tv, a);
+__device__ __forceinline__ void qr_cols3(SvdT<R>& S, double tu[3], double tv[2]) {
+  if (tu[0] == 0.0) {
+    qr_middle<0>(S, tu, tv);
     return;
   }
-  // cols == 3 here, so the window is the whole matrix (a == 0).
-  for (int i = 0; i < cols - 1; ++i) {
-    if (tu[i] == 0.0) {
-      qr_middle(S, tu, tv, cols, i);
-      return;
-    }
+  if (tu[1] == 0.0) {
+    qr_middle<1>(S, tu, tv);
+    return;
   }
-  if (tu[cols - 1] == 0.0) {
+  if (tu[2] == 0.0) {
     qr_end(S, tu, tv);
     return;
   }
@@ -336,121 +419,103 @@ __device__ __forceinline__ void qr_step(SvdT<R>& S, double* tu, double* tv, int 
   double z = tu[0] * tv[0];
   double ak = 0.0, bk = 0.0, zk = 0.0;
   double ap = tu[0], bp = tv[0], aq = tu[1];
-  for (int k = 0; k < cols - 1; ++k) {
-    double c, s;
-    givens(y, z, &c, &s);
-    rotate<3>(S.v, 3, k, k + 1, c, s);
-    double bk1 = bk * c - z * s;
-    double ap1 = ap * c - bp * s;
-    double bp1 = ap * s + bp * c;
-    double zp1 = aq * -s;
-    double aq1 = aq * c;
-    if (k > 0) tv[k - 1] = bk1;
-    ak = ap1;
-    bk = bp1;
-    zk = zp1;
-    ap = aq1;
-    bp = k < cols - 2 ? tv[k + 1] : 0.0;
-    y = ak;
-    z = zk;
-    givens(y, z, &c, &s);
-    rotate<R>(S.u, S.rows, k, k + 1, c, s);
-    const double ak1 = ak * c - zk * s;
-    bk1 = bk * c - ap * s;
-    const double zk1 = bp * -s;
-    ap1 = bk * s + ap * c;
-    bp1 = bp * c;
-    tu[k] = ak1;
-    ak = ak1;
-    bk = bk1;
-    zk = zk1;
-    ap = ap1;
-    bp = bp1;
-    aq = k < cols - 2 ? tu[k + 2] : 0.0;
-    y = bk;
-    z = zk;
-  }
-  tv[cols - 2] = bk;
-  tu[cols - 1] = ap;
+  qr_column<0>(S, tu, tv, y, z, ak, bk, zk, ap, bp, aq);
+  qr_column<1>(S, tu, tv, y, z, ak, bk, zk, ap, bp, aq);
+  tv[1] = bk;
+  tu[2] = ap;
 }
 
 // Diagonalisation (svd.rs:413-479).  The reference has no iteration cap;
 // `max_sweeps` bounds the loop on the device so that every thread finishes
-// (a cell that hits it is reported through *stalled).
+// (a cell that hits it is reported through *stalled).  The window is the last
+// run of nonzero off-diagonal entries; one that has become zero at the end
+// stays so.
 template <int R>
 __device__ __forceinline__ void diagonalise(SvdT<R>& S, double tu[3], double tv[2], int max_sweeps,
                                             bool* stalled) {
-  chop(tu, tv, 3);
-  int b = 2;
-  int sweeps = 0;
-  while (b > 0) {
-    if (tv[b - 1] == 0.0) {
-      --b;
-      continue;
-    }
-    if (++sweeps > max_sweeps) {
+  chop<0, 3>(tu, tv);
+  for (int sweeps = 0; tv[0] != 0.0 || tv[1] != 0.0; ++sweeps) {
+    if (sweeps >= max_sweeps) {
       *stalled = true;
       return;
     }
-    int a = b - 1;
-    while (a > 0 && tv[a - 1] != 0.0) --a;
-    const int n = b - a + 1;
-    qr_step(S, &tu[a], &tv[a], a, n);
-    chop(&tu[a], &tv[a], n);
+    if (tv[1] == 0.0) {
+      qr_cols2<0>(S, tu, tv);
+      chop<0, 2>(tu, tv);
+    } else if (tv[0] == 0.0) {
+      qr_cols2<1>(S, tu, tv);
+      chop<1, 2>(tu, tv);
+    } else {
+      qr_cols3(S, tu, tv);
+      chop<0, 3>(tu, tv);
+    }
   }
 }
 
+// Puts the greatest of the singular values from i on first (svd.rs:867-926).
+template <int i, int R>
+__device__ __forceinline__ void sort_column(SvdT<R>& S) {
+  double dmax = S.d[i];
+  int imax = i;
+#pragma unroll
+  for (int j = i + 1; j < 3; ++j) {
+    if (S.d[j] > dmax) {
+      dmax = S.d[j];
+      imax = j;
+    }
+  }
+  auto exchange = [&](auto to) {
+    constexpr int j = decltype(to)::value;
+    const double t = S.d[i];
+    S.d[i] = S.d[j];
+    S.d[j] = t;
+    swap_cols<i, j, R>(S.u, S.rows);
+    swap_cols<i, j, 3>(S.v, 3);
+  };
+  if constexpr (i == 0) {
+    if (imax == 1) exchange(std::integral_constant<int, 1>{});
+  }
+  if (imax == 2) exchange(std::integral_constant<int, 2>{});
+}
+
 template <int R>
-__device__ __forceinline__ void sort_singular(SvdT<R>& S) {  // svd.rs:867-926
+__device__ __forceinline__ void sort_singular(SvdT<R>& S) {
+#pragma unroll
   for (int j = 0; j < 3; ++j) {
     if (S.d[j] < 0.0) {
+#pragma unroll
       for (int i = 0; i < 3; ++i) S.v[i][j] = -S.v[i][j];
       S.d[j] = -S.d[j];
     }
   }
-  for (int i = 0; i < 3; ++i) {
-    double dmax = S.d[i];
-    int imax = i;
-    for (int j = i + 1; j < 3; ++j) {
-      if (S.d[j] > dmax) {
-        dmax = S.d[j];
-        imax = j;
-      }
-    }
-    if (imax != i) {
-      double t = S.d[i];
-      S.d[i] = S.d[imax];
-      S.d[imax] = t;
-      for (int y = 0; y < S.rows; ++y) {
-        t = S.u[y][i];
-        S.u[y][i] = S.u[y][imax];
-        S.u[y][imax] = t;
-      }
-      for (int y = 0; y < 3; ++y) {
-        t = S.v[y][i];
-        S.v[y][i] = S.v[y][imax];
-        S.v[y][imax] = t;
-      }
-    }
-  }
+  sort_column<0>(S);
+  sort_column<1>(S);
 }
 
 // TangentPlanes::new (feature/mod.rs:91-148) over n <= R points and normals
 // + MinimiseQEF::place_feature_with_tangents (qef.rs:36-68); *feature
 // receives whether the planes were classified Edge or Corner.
-template <int R>
+// kFull: n is R (the loops over the points are then unrolled, too).
+template <int R, bool kFull>
 __device__ __forceinline__ Vec3f place_feature_n(const Vec3f* corners, const Vec3f* normals,
                                                  int n, bool* stalled, bool* feature) {
   const float kFeatureAngle = 0.866025388f;  // f32(0.8660254037844387), mod.rs:22
-  Vec3f com{0.0f, 0.0f, 0.0f}, axis{0.0f, 0.0f, 0.0f};
+  constexpr int kUnroll = kFull ? R : 1;
+  if (kFull) n = R;
+  Vec3f com{0.0f, 0.0f, 0.0f};
+  int first = 0, second = 0;
   float min_angle = 3.40282347e+38f;
   float count = 0.0f;
   *feature = false;
+#pragma unroll kUnroll
   for (int i = 0; i < n; ++i) {
-    for (int j = 0; j < n; ++j) {
+    // (j < i repeats the angle of an earlier pair, which is not below itself)
+#pragma unroll kUnroll
+    for (int j = i; j < n; ++j) {
       const float angle = dot3(normals[i], normals[j]);
       if (angle < min_angle) {
-        axis = cross3(normals[i], normals[j]);
+        first = i;
+        second = j;
         min_angle = angle;
       }
     }
@@ -464,8 +529,20 @@ __device__ __forceinline__ Vec3f place_feature_n(const Vec3f* corners, const Vec
   com.z /= count;
   if (min_angle > kFeatureAngle) return com;  // planar
   *feature = true;
-  axis = normalised_or_zero(axis);
+  Vec3f na{0.0f, 0.0f, 0.0f}, nb{0.0f, 0.0f, 0.0f};
+  if (kFull) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      if (i == first) na = normals[i];
+      if (i == second) nb = normals[i];
+    }
+  } else {
+    na = normals[first];
+    nb = normals[second];
+  }
+  const Vec3f axis = normalised_or_zero(cross3(na, nb));
   float min_c = 1.0f, max_c = -1.0f;
+#pragma unroll kUnroll
   for (int i = 0; i < n; ++i) {
     const float c = dot3(axis, normals[i]);
     min_c = fminf(min_c, c);
@@ -478,7 +555,10 @@ __device__ __forceinline__ Vec3f place_feature_n(const Vec3f* corners, const Vec
   SvdT<R> S;
   S.rows = n;
   double b[R];
-  for (int i = 0; i < n; ++i) {
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    S.u[i][0] = S.u[i][1] = S.u[i][2] = b[i] = 0.0;
+    if (i >= n) continue;
     S.u[i][0] = normals[i].x;
     S.u[i][1] = normals[i].y;
     S.u[i][2] = normals[i].z;
@@ -493,27 +573,35 @@ __device__ __forceinline__ Vec3f place_feature_n(const Vec3f* corners, const Vec
   if (edge) {  // qef.rs:51-63: drop the smallest singular value
     double smin = 1.7976931348623157e308;
     int id = 0;
+#pragma unroll
     for (int i = 0; i < 3; ++i) {
       if (S.d[i] < smin) {
         smin = S.d[i];
         id = i;
       }
     }
-    S.d[id] = 0.0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      if (i == id) S.d[i] = 0.0;
   }
   // SVD::solve (svd.rs:55-84) + solveSVD (svd.rs:928-972)
   if (S.d[2] < 0.1) S.d[2] = 0.0;
   if (S.d[1] < 0.1) S.d[1] = 0.0;
   if (S.d[0] < 0.1) S.d[0] = 0.0;
   double w[3] = {0.0, 0.0, 0.0};
-  for (int i = 0; i < n; ++i)
-    if (b[i] != 0.0)
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+    if (i < n && b[i] != 0.0)
+#pragma unroll
       for (int j = 0; j < 3; ++j) w[j] += b[i] * S.u[i][j];
+#pragma unroll
   for (int i = 0; i < 3; ++i)
     if (S.d[i] != 0.0) w[i] /= S.d[i];
   float x[3];
+#pragma unroll
   for (int i = 0; i < 3; ++i) {
     double t = 0.0;
+#pragma unroll
     for (int j = 0; j < 3; ++j) t += w[j] * S.v[i][j];
     x[i] = static_cast<float>(t);
   }
@@ -524,7 +612,7 @@ __device__ __forceinline__ Vec3f place_feature_n(const Vec3f* corners, const Vec
 __device__ __forceinline__ Vec3f place_feature(const Vec3f corners[8], const Vec3f normals[8],
                                                bool* stalled) {
   bool feature;
-  return place_feature_n<kRows>(corners, normals, kRows, stalled, &feature);
+  return place_feature_n<kRows, true>(corners, normals, kRows, stalled, &feature);
 }
 
 }  // namespace qef

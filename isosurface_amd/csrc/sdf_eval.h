@@ -20,6 +20,67 @@ __device__ __forceinline__ float f_len3(float x, float y, float z) {
   return __builtin_sqrtf((x * x + y * y) + z * z);
 }
 
+// A program in the constant address space: an operation read at a uniform
+// index is then a scalar load into scalar registers, whatever else the kernel
+// stores to (through an ordinary pointer that came from memory or a struct the
+// compiler must assume that a store may change it, and loads it per lane: 185
+// us instead of 135 for the 257^3 signs of 64 spheres minus a torus).
+using OpsPtr = const DevOp __attribute__((address_space(4)))*;
+__device__ __forceinline__ OpsPtr as_constant(const DevOp* ops) {
+  return (OpsPtr)(reinterpret_cast<uintptr_t>(ops));
+}
+__device__ __forceinline__ DevOp load_op(OpsPtr ops, int i) {
+  DevOp o;
+  o.code = ops[i].code;
+  o.combine = ops[i].combine;
+  o.translated = ops[i].translated;
+  o.k = ops[i].k;
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    o.prm[a] = ops[i].prm[a];
+    o.off[a] = ops[i].off[a];
+  }
+  return o;
+}
+
+// A value stack of registers: pushes and pops move the entries, so no entry
+// is addressed by a run-time index (a program seldom pushes).
+struct ShiftStack {
+  float v[kMaxValueStack];
+  __device__ __forceinline__ void push(float x) {
+#pragma unroll
+    for (int i = kMaxValueStack - 1; i > 0; --i) v[i] = v[i - 1];
+    v[0] = x;
+  }
+  __device__ __forceinline__ float pop() {
+    const float x = v[0];
+#pragma unroll
+    for (int i = 0; i + 1 < kMaxValueStack; ++i) v[i] = v[i + 1];
+    return x;
+  }
+};
+
+// The open translation scopes, innermost in the low bits: op indices of
+// their kPushTranslate, 16 bits each (a program has at most 8192 ops and
+// kMaxPointStack nested scopes).  Leaving a scope re-applies the remaining
+// ones to the base point, outermost first.
+struct ScopeStack {
+  uint64_t ops = 0;
+  int depth = 0;
+  __device__ __forceinline__ void push(int op) {
+    ops = (ops << 16) | static_cast<uint64_t>(op);
+    ++depth;
+  }
+  __device__ __forceinline__ void pop() {
+    ops >>= 16;
+    --depth;
+  }
+  __device__ __forceinline__ int at(int level) const {  // level 0: outermost
+    return static_cast<int>((ops >> (16 * (depth - 1 - level))) & 0xFFFFull);
+  }
+};
+static_assert(kMaxPointStack <= 4 && kMaxProgramOps <= 65536, "ScopeStack packs four op indices");
+
 // Correctly rounded square roots of K nonnegative values, bit for bit
 // __builtin_sqrtf's: the hardware's reciprocal square root and one Markstein
 // correction (six instructions; the compiler's sequence for any operand takes
@@ -725,60 +786,49 @@ __device__ __forceinline__ void prim_normal(uint32_t code, const float* prm, flo
   }
 }
 
-__device__ __forceinline__ void sdf_eval_hermite(const DevOp* __restrict__ ops, int n, float px,
-                                                 float py, float pz, float* out) {
+__device__ __forceinline__ void sdf_eval_hermite(const DevOp* ops_at, int n, float px, float py,
+                                                 float pz, float* out) {
+  const OpsPtr ops = as_constant(ops_at);
   float top[3] = {0.0f, 0.0f, 0.0f};
-  float st[kMaxValueStack][3];
-  int sp = 0;
-  float cx = px, cy = py, cz = pz;
-  float sx[kMaxPointStack], sy[kMaxPointStack], sz[kMaxPointStack];
-  int psp = 0;
+  ShiftStack st[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+#pragma unroll
+    for (int i = 0; i < kMaxValueStack; ++i) st[a].v[i] = 0.0f;
+  float c[3] = {px, py, pz};
+  ScopeStack scopes;
   bool have_top = false;
   for (int i = 0; i < n; ++i) {
-    const uint32_t code = ops[i].code;
-    if (code <= kCylinder) {
-      float qx = cx, qy = cy, qz = cz;
-      if (ops[i].translated) {
-        qx = cx - ops[i].off[0];
-        qy = cy - ops[i].off[1];
-        qz = cz - ops[i].off[2];
-      }
+    const DevOp op = load_op(ops, i);
+    if (op.code <= kCylinder) {
       float v[3];
-      prim_normal(code, ops[i].prm, qx, qy, qz, v);
-      if (ops[i].combine == kPush) {
-        if (have_top) {
-          st[sp][0] = top[0];
-          st[sp][1] = top[1];
-          st[sp][2] = top[2];
-          ++sp;
-        }
-        top[0] = v[0];
-        top[1] = v[1];
-        top[2] = v[2];
-        have_top = true;
-      } else {  // kMin: Union(top, v)
-        top[0] = fminf(top[0], v[0]);
-        top[1] = fminf(top[1], v[1]);
-        top[2] = fminf(top[2], v[2]);
+      // (an untranslated primitive's offset is 0, and x - 0 is x)
+      prim_normal(op.code, op.prm, c[0] - op.off[0], c[1] - op.off[1], c[2] - op.off[2], v);
+      const bool push = op.combine == kPush;
+      if (push && have_top) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) st[a].push(top[a]);
       }
-    } else if (code == kPushTranslate) {
-      sx[psp] = cx;
-      sy[psp] = cy;
-      sz[psp] = cz;
-      ++psp;
-      cx = cx - ops[i].off[0];
-      cy = cy - ops[i].off[1];
-      cz = cz - ops[i].off[2];
-    } else if (code == kPopTranslate) {
-      --psp;
-      cx = sx[psp];
-      cy = sy[psp];
-      cz = sz[psp];
+      have_top = true;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) top[a] = push ? v[a] : fminf(top[a], v[a]);  // kMin: Union(top, v)
+    } else if (op.code == kPushTranslate) {
+      scopes.push(i);
+#pragma unroll
+      for (int a = 0; a < 3; ++a) c[a] = c[a] - op.off[a];
+    } else if (op.code == kPopTranslate) {
+      scopes.pop();
+      c[0] = px;
+      c[1] = py;
+      c[2] = pz;
+      for (int s = 0; s < scopes.depth; ++s) {
+        const int o = scopes.at(s);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) c[a] = c[a] - ops[o].off[a];
+      }
     } else {  // kUnion of (below, top)
-      --sp;
-      top[0] = fminf(st[sp][0], top[0]);
-      top[1] = fminf(st[sp][1], top[1]);
-      top[2] = fminf(st[sp][2], top[2]);
+#pragma unroll
+      for (int a = 0; a < 3; ++a) top[a] = fminf(st[a].pop(), top[a]);
     }
   }
   out[0] = top[0];

@@ -26,67 +26,6 @@
 
 namespace iso {
 
-// A program in the constant address space: an operation read at a uniform
-// index is then a scalar load into scalar registers, whatever else the kernel
-// stores to (through an ordinary pointer that came from memory or a struct the
-// compiler must assume that a store may change it, and loads it per lane: 185
-// us instead of 135 for the 257^3 signs of 64 spheres minus a torus).
-using OpsPtr = const DevOp __attribute__((address_space(4)))*;
-__device__ __forceinline__ OpsPtr as_constant(const DevOp* ops) {
-  return (OpsPtr)(reinterpret_cast<uintptr_t>(ops));
-}
-__device__ __forceinline__ DevOp load_op(OpsPtr ops, int i) {
-  DevOp o;
-  o.code = ops[i].code;
-  o.combine = ops[i].combine;
-  o.translated = ops[i].translated;
-  o.k = ops[i].k;
-#pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    o.prm[a] = ops[i].prm[a];
-    o.off[a] = ops[i].off[a];
-  }
-  return o;
-}
-
-// A value stack of registers: pushes and pops move the entries, so no entry
-// is addressed by a run-time index (a program seldom pushes).
-struct ShiftStack {
-  float v[kMaxValueStack];
-  __device__ __forceinline__ void push(float x) {
-#pragma unroll
-    for (int i = kMaxValueStack - 1; i > 0; --i) v[i] = v[i - 1];
-    v[0] = x;
-  }
-  __device__ __forceinline__ float pop() {
-    const float x = v[0];
-#pragma unroll
-    for (int i = 0; i + 1 < kMaxValueStack; ++i) v[i] = v[i + 1];
-    return x;
-  }
-};
-
-// The open translation scopes, innermost in the low bits: op indices of
-// their kPushTranslate, 16 bits each (a program has at most 8192 ops and
-// kMaxPointStack nested scopes).  Leaving a scope re-applies the remaining
-// ones to the base point, outermost first.
-struct ScopeStack {
-  uint64_t ops = 0;
-  int depth = 0;
-  __device__ __forceinline__ void push(int op) {
-    ops = (ops << 16) | static_cast<uint64_t>(op);
-    ++depth;
-  }
-  __device__ __forceinline__ void pop() {
-    ops >>= 16;
-    --depth;
-  }
-  __device__ __forceinline__ int at(int level) const {  // level 0: outermost
-    return static_cast<int>((ops >> (16 * (depth - 1 - level))) & 0xFFFFull);
-  }
-};
-static_assert(kMaxPointStack <= 4 && kMaxProgramOps <= 65536, "ScopeStack packs four op indices");
-
 // Bounds of the correctly rounded square root by the hardware's, which is
 // within one ulp of it (two for certain: four are allowed), and within 2^-62
 // of it where its operand is too small to be normal.
@@ -297,6 +236,74 @@ __device__ __forceinline__ void op_interval(const DevOp& op, const float* cl, co
   prim_interval(op.code, op.prm, ql, qh, vlo, vhi);
 }
 
+// The same for a primitive's Directed value, three components of which each is
+// the signed distance along its axis, or kDirectedMiss where the axis' line
+// misses the shape.  They are ordered by what is known of all three:
+//   4         all kDirectedMiss at every point of the box: no component of any
+//             other value is greater;
+//   1 to 3    all positive; -1 to -3: all negative; -3 to 3: not known.
+// (The negatives' bounds mirror these.)  Minima and maxima of values follow
+// those of the bounds, so Bounds combines them, and what it finds idle leaves
+// every component as it is.  A torus is not bounded.
+__device__ __forceinline__ void directed_interval(const DevOp& op, const float* cl,
+                                                  const float* ch, float* vlo, float* vhi) {
+  float an[3], af[3];  // least and greatest |q_c|
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const float lo = cl[a] - op.off[a], hi = ch[a] - op.off[a];
+    an[a] = fmaxf(fmaxf(lo, -hi), 0.0f);
+    af[a] = fmaxf(-lo, hi);
+  }
+  bool out[3];        // outside along the axis
+  bool in = true;     // all negative
+  if (op.code == kBox) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      out[a] = an[a] > op.prm[a];
+      in = in && af[a] < op.prm[a];
+    }
+    // outside along two axes: every axis' line misses
+    const int n = out[0] + out[1] + out[2];
+    *vlo = n >= 2 ? 4.0f : n ? 1.0f : -3.0f;
+    *vhi = n >= 2 ? 4.0f : in ? -1.0f : 3.0f;
+    return;
+  }
+  *vlo = -3.0f;
+  *vhi = 3.0f;
+  if (op.code == kTorus) return;
+  // Squares: far enough from the surface that no rounding of the squares, their
+  // sums and the root (a few 2^-24 of r^2) changes a comparison.
+  const float rr = op.prm[0] * op.prm[0];
+  const float far = rr * 1.00002f + 1.0e-30f, near = rr * 0.99998f - 1.0e-30f;
+  const float xy = an[0] * an[0] + an[1] * an[1];
+  if (op.code == kSphere) {
+    const float xz = an[0] * an[0] + an[2] * an[2], yz = an[1] * an[1] + an[2] * an[2];
+    if (xy > far && xz > far && yz > far)
+      *vlo = *vhi = 4.0f;
+    else if (xy + an[2] * an[2] > far)
+      *vlo = 1.0f;
+    else if ((af[0] * af[0] + af[1] * af[1]) + af[2] * af[2] < near)
+      *vhi = -1.0f;
+  } else {  // kCylinder
+    const bool above = an[2] > op.prm[1], beside = xy > far;
+    if (above && beside)
+      *vlo = *vhi = 4.0f;
+    else if (above || beside)
+      *vlo = 1.0f;
+    else if (op.prm[0] > 0.0f && af[2] < op.prm[1] && af[0] * af[0] + af[1] * af[1] < near)
+      *vhi = -1.0f;
+  }
+}
+
+template <bool kDirected>
+__device__ __forceinline__ void value_interval(const DevOp& op, const float* cl, const float* ch,
+                                               float* vlo, float* vhi) {
+  if constexpr (kDirected)
+    directed_interval(op, cl, ch, vlo, vhi);
+  else
+    op_interval(op, cl, ch, vlo, vhi);
+}
+
 // Scopes that hold the whole program (a recentring wrapper): as many as open
 // it and close it together.  The callers give boxes and points inside them,
 // and walk the operations after their openings, with them already open.
@@ -312,7 +319,7 @@ __device__ __forceinline__ int leading_scopes(OpsPtr ops, int n) {
 // `cap`: they do not fit, and the list is not usable).  Runs of min and
 // smooth-min operands are bounded 64 at a time, one a lane, each against the
 // running upper bound before it.
-template <bool kStack>
+template <bool kStack, bool kDirected = false>
 __device__ __forceinline__ int bound_box(OpsPtr ops, int first, int n, const float* tlo,
                                          const float* thi, uint16_t* list, int cap, float* out_lo,
                                          float* out_hi) {
@@ -335,7 +342,7 @@ __device__ __forceinline__ int bound_box(OpsPtr ops, int first, int n, const flo
         const int m = ~from ? static_cast<int>(__builtin_ctzll(~from)) : 64;
         const bool in = lane >= p && lane < p + m;
         float vlo = kNoBound, vhi = kNoBound;
-        if (in) op_interval(mine, cl, ch, &vlo, &vhi);
+        if (in) value_interval<kDirected>(mine, cl, ch, &vlo, &vhi);
         const bool smooth = mine.combine == kSmooth;
         const float T = fminf(B.hi, wave_min_before(vhi));
         const bool kept = in && !(smooth ? smooth_inactive(vlo - T, mine.k) : vlo > T);
@@ -363,7 +370,7 @@ __device__ __forceinline__ int bound_box(OpsPtr ops, int first, int n, const flo
       if (op.code <= kCylinder) {
         float vlo, vhi;
         uint64_t matters;
-        op_interval(op, cl, ch, &vlo, &vhi);
+        value_interval<kDirected>(op, cl, ch, &vlo, &vhi);
         if (!B.join(op.combine, op.k, vlo, vhi, true, &matters)) continue;
       } else if (op.code == kPushTranslate) {
         scopes.push(i);
@@ -389,7 +396,7 @@ __device__ __forceinline__ int bound_box(OpsPtr ops, int first, int n, const flo
 // [first, first + m)).  With a list, the operations that matter to no lane are
 // taken out of it, and mask[j] names the lanes that the j-th remaining one
 // matters to.  Returns the number of operations left.
-template <bool kStack>
+template <bool kStack, bool kDirected = false>
 __device__ __forceinline__ int bound_lanes(OpsPtr ops, int first, int m, const float* blo,
                                            const float* bhi, bool active, uint16_t* list,
                                            uint64_t* mask, float* out_lo, float* out_hi) {
@@ -408,7 +415,7 @@ __device__ __forceinline__ int bound_lanes(OpsPtr ops, int first, int m, const f
     uint64_t matters = ~0ull;
     if (op.code <= kCylinder) {
       float vlo, vhi;
-      op_interval(op, cl, ch, &vlo, &vhi);
+      value_interval<kDirected>(op, cl, ch, &vlo, &vhi);
       if (!B.join(op.combine, op.k, vlo, vhi, active, &matters)) continue;
     } else if (op.code == kPushTranslate) {
       scopes.push(i);
@@ -541,6 +548,103 @@ __device__ __forceinline__ void sdf_eval_list(OpsPtr ops, int first, const uint1
           else  // max(w, t), max(t, -w) or max(w, -t)
             top[k] = fmaxf(flip_sign(w, nw), flip_sign(top[k], nt));
         }
+      }
+    }
+  }
+}
+
+// sdf_eval_vector (Directed values) over a list of operations, as sdf_eval_list.
+template <int K, bool kStack>
+__device__ __forceinline__ void sdf_eval_vector_list(OpsPtr ops, int first, const uint16_t* list,
+                                                     const uint64_t* mask, uint64_t bricks, int m,
+                                                     const float (&p)[K][3], float (&top)[K][3]) {
+  const int lane = __lane_id();
+  ShiftStack st[K][3];
+  float c[K][3];
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      top[k][a] = __builtin_inff();  // min(inf, v) is v: the first push is read as a min
+      c[k][a] = p[k][a];
+#pragma unroll
+      for (int i = 0; i < kMaxValueStack; ++i) st[k][a].v[i] = 0.0f;
+    }
+  ScopeStack scopes;
+  bool have_top = false;
+  for (int base = 0; base < m; base += 64) {
+    int mine = first + base + lane;
+    bool use = base + lane < m;
+    if (list && use) {
+      mine = list[base + lane];
+      use = (mask[base + lane] & bricks) != 0ull;
+    }
+    uint64_t todo = __ballot(use);
+    while (todo) {
+      const int i = __builtin_amdgcn_readlane(mine, static_cast<int>(__builtin_ctzll(todo)));
+      todo &= todo - 1;
+      const DevOp op = load_op(ops, i);
+      const uint32_t code = op.code;
+      if (code <= kCylinder) {
+        const uint32_t mode = op.combine;
+        const bool least = mode == kMin || (!kStack && mode == kPush);
+        const uint32_t nt = mode == kDiff ? 0x80000000u : 0u;
+        const uint32_t nv = mode == kDiffRev ? 0x80000000u : 0u;
+        if (kStack && mode == kPush && have_top) {
+#pragma unroll
+          for (int k = 0; k < K; ++k)
+#pragma unroll
+            for (int a = 0; a < 3; ++a) st[k][a].push(top[k][a]);
+        }
+        if (mode == kPush) have_top = true;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          float v[3];
+          prim_vector(code, op.prm, c[k][0] - op.off[0], c[k][1] - op.off[1],
+                      c[k][2] - op.off[2], v);  // (x - 0 is x)
+#pragma unroll
+          for (int a = 0; a < 3; ++a) {
+            // min, or max(top, v), max(v, -top), max(top, -v)
+            if (kStack && mode == kPush)
+              top[k][a] = v[a];
+            else if (least)
+              top[k][a] = fminf(top[k][a], v[a]);
+            else
+              top[k][a] = fmaxf(flip_sign(top[k][a], nt), flip_sign(v[a], nv));
+          }
+        }
+      } else if (code == kPushTranslate) {
+        scopes.push(i);
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+#pragma unroll
+          for (int a = 0; a < 3; ++a) c[k][a] = c[k][a] - op.off[a];
+      } else if (code == kPopTranslate) {
+        if (scopes.depth == 0) continue;
+        scopes.pop();
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+#pragma unroll
+          for (int a = 0; a < 3; ++a) c[k][a] = p[k][a];
+        for (int s = 0; s < scopes.depth; ++s) {
+          const int o = scopes.at(s);
+#pragma unroll
+          for (int k = 0; k < K; ++k)
+#pragma unroll
+            for (int a = 0; a < 3; ++a) c[k][a] = c[k][a] - ops[o].off[a];
+        }
+      } else if (kStack) {
+        const uint32_t nw = code == kDifference ? 0x80000000u : 0u;
+        const uint32_t nt = code == kDifferenceRev ? 0x80000000u : 0u;
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+#pragma unroll
+          for (int a = 0; a < 3; ++a) {
+            const float w = st[k][a].pop();
+            // min, or max(w, t), max(t, -w), max(w, -t)
+            top[k][a] = code == kUnion ? fminf(w, top[k][a])
+                                       : fmaxf(flip_sign(w, nw), flip_sign(top[k][a], nt));
+          }
       }
     }
   }

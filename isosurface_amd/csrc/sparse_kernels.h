@@ -52,6 +52,12 @@ int64_t tile_count(int64_t nx, int64_t ny, int64_t nz);
 hipError_t launch_signs_sparse(const DevOp* ops, int n_ops, bool stack, const Lattice& L,
                                const McDims& D, const McBuffers& B, float* values, hipStream_t s);
 
+// Directed signs and values like launch_signs_directed (3 floats a sample,
+// those of the unproven bricks), from dims of mc_dims_pitched.
+hipError_t launch_directed_sparse(const DevOp* ops, int n_ops, bool stack, const Lattice& L,
+                                  const McDims& D, const McBuffers& B, float* values,
+                                  hipStream_t s);
+
 // Samples of a lattice for dual contouring: the program's value near the
 // surface, and 1 or -1 at samples whose own and whose neighbours' dual values
 // are only read for their sign.

@@ -71,9 +71,9 @@ struct BatchTiles {
   }
 };
 
-// W wavefronts per tile: one where tiles alone fill the chip, four where a
-// small lattice leaves it idle (the bricks of a tile are then spread over
-// four SIMDs; the bounds are one wavefront's work either way).
+// W wavefronts per tile: one where tiles alone fill the chip, four or eight
+// where a small lattice leaves it idle (the bricks of a tile are then spread
+// over the SIMDs; the bounds are one wavefront's work either way).
 //
 // kSamples: for dual contouring, which takes no sign words but reads all
 // samples, a dual value being half the sum of two opposite corners of a cell.
@@ -81,19 +81,26 @@ struct BatchTiles {
 // than its sign only where its dual neighbour's differs, and the samples of
 // both lie within two of any of them: the bounds are taken two samples wider,
 // and from 1e-30 on where half a sample could round to zero.
-template <class Tiles, int W, bool kStack, bool kSamples>
+//
+// kDirected: Directed values (three floats a sample) and their signs.  A brick
+// is proven where all components of all its samples, and its neighbours',
+// have one sign (directed_interval), and the evaluated bricks again hold every
+// value that is read, those of all corners of a mixed cell.
+enum SparseMode : int { kSigns, kSamples, kDirected };
+
+template <class Tiles, int W, bool kStack, int kMode>
 __global__ __launch_bounds__(64 * W) void k_signs_sparse(Tiles tiles, uint32_t n_tiles,
                                                          uint32_t group, ResetArgs R) {
-  constexpr int kMargin = kSamples ? 2 : 1;  // neighbours in a brick's box
+  constexpr int kMargin = kMode == kSamples ? 2 : 1;  // neighbours in a brick's box
   constexpr int kTileCoords = kTileSide + 2 * kMargin;  // coordinates along an axis
-  constexpr float kOutside = kSamples ? 1.0e-30f : 0.0f;
+  constexpr float kOutside = kMode == kSamples ? 1.0e-30f : 0.0f;
   __shared__ uint64_t s_sign[kBricks];  // sign bits of a brick's samples, x fastest
   __shared__ uint16_t s_list[kListCap];  // operations that matter in the tile
   __shared__ uint64_t s_mask[kListCap];  // and the bricks each of them matters in
   __shared__ float s_coord[3 * kTileCoords];
   __shared__ int s_len;
   __shared__ uint64_t s_todo;
-  if (!kSamples) reset_state(R);
+  if (kMode != kSamples) reset_state(R);
   // Groups of consecutive tiles (a row's neighbours share lines of sign words
   // and values) go to one XCD, the groups round robin.
   const uint32_t q = blockIdx.x / kSparseXcds;
@@ -145,7 +152,7 @@ __global__ __launch_bounds__(64 * W) void k_signs_sparse(Tiles tiles, uint32_t n
       bhi[a] = fmaxf(c0, c1);
     }
     float lo, hi;
-    int len = bound_box<kStack>(ops, first, n_ops, blo, bhi, s_list, kListCap, &lo, &hi);
+    int len = bound_box<kStack, kMode == kDirected>(ops, first, n_ops, blo, bhi, s_list, kListCap, &lo, &hi);
     bool outside = lo > kOutside, inside = hi <= 0.0f;
     bool active = true;
     if (!outside && !inside) {
@@ -161,8 +168,9 @@ __global__ __launch_bounds__(64 * W) void k_signs_sparse(Tiles tiles, uint32_t n
       }
       lds_barrier<1>();
       const bool fits = len <= kListCap;
-      const int left = bound_lanes<kStack>(ops, first, fits ? len : n_ops - first, blo, bhi,
-                                           active, fits ? s_list : nullptr, s_mask, &lo, &hi);
+      const int left = bound_lanes<kStack, kMode == kDirected>(
+          ops, first, fits ? len : n_ops - first, blo, bhi, active, fits ? s_list : nullptr, s_mask,
+          &lo, &hi);
       if (fits) len = left;
       outside = lo > kOutside;
       inside = hi <= 0.0f;
@@ -185,7 +193,7 @@ __global__ __launch_bounds__(64 * W) void k_signs_sparse(Tiles tiles, uint32_t n
                 __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(t >> 32))))
             << 32);
   }
-  if (kSamples && ~todo) {
+  if (kMode == kSamples && ~todo) {
     // rows of sixteen samples, four a wavefront's store
     float* grid = const_cast<float*>(C.grid);
     for (int i = threadIdx.x; i < kTileSide * kTileSide * kTileSide; i += 64 * W) {
@@ -229,7 +237,15 @@ __global__ __launch_bounds__(64 * W) void k_signs_sparse(Tiles tiles, uint32_t n
       p[j][1] = s_coord[kTileCoords + kMargin + (b & 12) + ly];
       p[j][2] = s_coord[2 * kTileCoords + kMargin + 4 * (b >> 4) + lz];
     }
-    sdf_eval_list<kPoints, kStack>(ops, first, list, s_mask, bricks, m, p, v);
+    float d[kPoints][3];
+    if constexpr (kMode == kDirected) {
+      sdf_eval_vector_list<kPoints, kStack>(ops, first, list, s_mask, bricks, m, p, d);
+#pragma unroll
+      for (int j = 0; j < kPoints; ++j)  // Directed::is_positive, distance.rs:76-79
+        v[j] = d[j][0] > 0.0f || d[j][1] > 0.0f || d[j][2] > 0.0f ? 1.0f : -1.0f;
+    } else {
+      sdf_eval_list<kPoints, kStack>(ops, first, list, s_mask, bricks, m, p, v);
+    }
     uint64_t mine = 0;
 #pragma unroll
     for (int j = 0; j < kPoints; ++j) {
@@ -237,21 +253,28 @@ __global__ __launch_bounds__(64 * W) void k_signs_sparse(Tiles tiles, uint32_t n
       const int32_t x0 = s0[0] + 4 * (b & 3), y0 = s0[1] + (b & 12), z0 = s0[2] + 4 * (b >> 4);
       const bool valid = full || (x0 + lx < nx && y0 + ly < ny && z0 + lz < nz);
       if (C.grid && valid && ((have >> j) & 1u)) {
-        float* at = const_cast<float*>(C.grid) + (static_cast<int64_t>(z0) * ny + y0) * nx + x0;
-        at[within] = v[j];
+        const int64_t s = (static_cast<int64_t>(z0) * ny + y0) * nx + x0 + within;
+        float* at = const_cast<float*>(C.grid);
+        if constexpr (kMode == kDirected) {
+          at[3 * s + 0] = d[j][0];
+          at[3 * s + 1] = d[j][1];
+          at[3 * s + 2] = d[j][2];
+        } else {
+          at[s] = v[j];
+        }
       }
       // classify_corners, distance.rs:52-54
       const uint64_t in = __ballot(valid && !(v[j] > 0.0f));
       if (lane == j) mine = in;
     }
-    if (kSamples) continue;
+    if (kMode == kSamples) continue;
     // (a spare point repeats the first brick)
     int slot = brick[0];
 #pragma unroll
     for (int j = 1; j < kPoints; ++j) slot = lane == j ? brick[j] : slot;
     if (lane < kPoints) s_sign[slot] = mine;
   }
-  if (kSamples) return;
+  if (kMode == kSamples) return;
   lds_barrier<W>();
   store_tile_signs(C, s_sign, s0, tx, threadIdx.x, 64 * W);
 }
@@ -279,10 +302,15 @@ hipError_t launch_tiles(Kernel kernel, int threads, const Tiles& tiles, int64_t 
   return hipGetLastError();
 }
 
-// Tiles from which one wavefront each is the better split.  Kernel times with
-// one / four wavefronts a tile, 64 spheres minus a torus: 75 / 44 us at 257^3
-// (4913 tiles), 87 / 83 at 385^3 (15625), 119 / 151 at 513^3 (35937).
+// Tiles from which one wavefront each is the better split, and up to which
+// eight are: a chain's latency counts there.  Kernel times with one / four
+// wavefronts a tile, 64 spheres minus a torus: 75 / 44 us at 257^3 (4913
+// tiles), 87 / 83 at 385^3 (15625), 119 / 151 at 513^3 (35937).  Whole
+// extractions with four / eight: 74 / 65 us at 129^3 (729 tiles), 76 / 78 at
+// 193^3 (2197), 94 / 110 at 257^3; directed values of 32 boxes at 128^3 (512
+// tiles) 94 / 72, dual contouring's samples there 40 / 35.
 constexpr int64_t kManyTiles = 16384;
+constexpr int64_t kFewTiles = 2048;
 
 // Parameters and coordinates below this: no square or sum of squares of a
 // primitive's operands overflows.
@@ -335,10 +363,24 @@ ProgramKind program_kind(const DevOp* ops, int n_ops) {
   return K;
 }
 
-hipError_t launch_signs_sparse(const DevOp* ops, int n_ops, bool stack, const Lattice& L,
-                               const McDims& D, const McBuffers& B, float* values, hipStream_t s) {
-  if (!ops || !B.signs || (D.sign_pitch & 63)) return hipErrorInvalidValue;
-  const SingleTiles t{single_cell_space(L, D, B.signs, ops, n_ops, values, nullptr)};
+namespace {
+
+template <int kMode>
+hipError_t launch_single(const SingleTiles& t, bool stack, const Lattice& L, const ResetArgs& R,
+                         hipStream_t s) {
+  const int64_t n = tile_count(L.nx, L.ny, L.nz);
+  const int64_t group = (L.nx + kTileSide - 1) >> kTileShift;
+  if (n >= kManyTiles)
+    return stack ? launch_tiles(k_signs_sparse<SingleTiles, 1, true, kMode>, 64, t, n, group, R, s)
+                 : launch_tiles(k_signs_sparse<SingleTiles, 1, false, kMode>, 64, t, n, group, R, s);
+  if (n <= kFewTiles)
+    return stack ? launch_tiles(k_signs_sparse<SingleTiles, 8, true, kMode>, 512, t, n, group, R, s)
+                 : launch_tiles(k_signs_sparse<SingleTiles, 8, false, kMode>, 512, t, n, group, R, s);
+  return stack ? launch_tiles(k_signs_sparse<SingleTiles, 4, true, kMode>, 256, t, n, group, R, s)
+               : launch_tiles(k_signs_sparse<SingleTiles, 4, false, kMode>, 256, t, n, group, R, s);
+}
+
+ResetArgs reset_args(const McDims& D, const McBuffers& B) {
   ResetArgs R;
   R.signs = B.signs;
   R.n_words = D.n_sign_words;
@@ -346,13 +388,24 @@ hipError_t launch_signs_sparse(const DevOp* ops, int n_ops, bool stack, const La
   R.incl = B.incl;
   R.n_blocks = D.n_blocks;
   R.totals = B.totals;
-  const int64_t n = tile_count(L.nx, L.ny, L.nz);
-  const int64_t group = (L.nx + kTileSide - 1) >> kTileShift;
-  if (n >= kManyTiles)
-    return stack ? launch_tiles(k_signs_sparse<SingleTiles, 1, true, false>, 64, t, n, group, R, s)
-                 : launch_tiles(k_signs_sparse<SingleTiles, 1, false, false>, 64, t, n, group, R, s);
-  return stack ? launch_tiles(k_signs_sparse<SingleTiles, 4, true, false>, 256, t, n, group, R, s)
-               : launch_tiles(k_signs_sparse<SingleTiles, 4, false, false>, 256, t, n, group, R, s);
+  return R;
+}
+
+}  // namespace
+
+hipError_t launch_signs_sparse(const DevOp* ops, int n_ops, bool stack, const Lattice& L,
+                               const McDims& D, const McBuffers& B, float* values, hipStream_t s) {
+  if (!ops || !B.signs || (D.sign_pitch & 63)) return hipErrorInvalidValue;
+  const SingleTiles t{single_cell_space(L, D, B.signs, ops, n_ops, values, nullptr)};
+  return launch_single<kSigns>(t, stack, L, reset_args(D, B), s);
+}
+
+hipError_t launch_directed_sparse(const DevOp* ops, int n_ops, bool stack, const Lattice& L,
+                                  const McDims& D, const McBuffers& B, float* values,
+                                  hipStream_t s) {
+  if (!ops || !B.signs || !values || (D.sign_pitch & 63)) return hipErrorInvalidValue;
+  const SingleTiles t{single_cell_space(L, D, B.signs, ops, n_ops, values, nullptr)};
+  return launch_single<kDirected>(t, stack, L, reset_args(D, B), s);
 }
 
 hipError_t launch_samples_sparse(const DevOp* ops, int n_ops, bool stack, const Lattice& L,
@@ -360,14 +413,7 @@ hipError_t launch_samples_sparse(const DevOp* ops, int n_ops, bool stack, const 
   if (!ops || !samples) return hipErrorInvalidValue;
   const SingleTiles t{
       single_cell_space(L, mc_dims_pitched(L), nullptr, ops, n_ops, samples, nullptr)};
-  const int64_t n = tile_count(L.nx, L.ny, L.nz);
-  const int64_t group = (L.nx + kTileSide - 1) >> kTileShift;
-  const ResetArgs R{};
-  if (n >= kManyTiles)
-    return stack ? launch_tiles(k_signs_sparse<SingleTiles, 1, true, true>, 64, t, n, group, R, s)
-                 : launch_tiles(k_signs_sparse<SingleTiles, 1, false, true>, 64, t, n, group, R, s);
-  return stack ? launch_tiles(k_signs_sparse<SingleTiles, 4, true, true>, 256, t, n, group, R, s)
-               : launch_tiles(k_signs_sparse<SingleTiles, 4, false, true>, 256, t, n, group, R, s);
+  return launch_single<kSamples>(t, stack, L, ResetArgs{}, s);
 }
 
 hipError_t launch_batch_signs_sparse(const BatchPlan& P, const McBuffers& B, int64_t n_blocks,
@@ -383,10 +429,10 @@ hipError_t launch_batch_signs_sparse(const BatchPlan& P, const McBuffers& B, int
   R.totals = B.totals;
   constexpr int64_t kGroup = 4;  // about a row of a chunk's tiles
   if (P.n_tiles >= kManyTiles)
-    return P.stack ? launch_tiles(k_signs_sparse<BatchTiles, 1, true, false>, 64, t, P.n_tiles, kGroup, R, s)
-                   : launch_tiles(k_signs_sparse<BatchTiles, 1, false, false>, 64, t, P.n_tiles, kGroup, R, s);
-  return P.stack ? launch_tiles(k_signs_sparse<BatchTiles, 4, true, false>, 256, t, P.n_tiles, kGroup, R, s)
-                 : launch_tiles(k_signs_sparse<BatchTiles, 4, false, false>, 256, t, P.n_tiles, kGroup, R, s);
+    return P.stack ? launch_tiles(k_signs_sparse<BatchTiles, 1, true, kSigns>, 64, t, P.n_tiles, kGroup, R, s)
+                   : launch_tiles(k_signs_sparse<BatchTiles, 1, false, kSigns>, 64, t, P.n_tiles, kGroup, R, s);
+  return P.stack ? launch_tiles(k_signs_sparse<BatchTiles, 4, true, kSigns>, 256, t, P.n_tiles, kGroup, R, s)
+                 : launch_tiles(k_signs_sparse<BatchTiles, 4, false, kSigns>, 256, t, P.n_tiles, kGroup, R, s);
 }
 
 }  // namespace iso
