@@ -83,7 +83,7 @@ struct iso_ctx {
   DevBuf dgrid, dvals;
   int64_t dgnx = 0, dgny = 0, dgnz = 0;
   // extended marching cubes: per active cell state, first ids, flip records
-  DevBuf emc_cells, emc_first, emc_flips, emc_ctr, emc_cross;
+  DevBuf emc_cells, emc_index, emc_first, emc_flips, emc_ctr, emc_cross;
   // dual contouring: primal samples, dual values and points, mixed list, counters
   DevBuf dc_normals, dc_marks, dc_samples, dc_values, dc_points, dc_mixed, dc_counters;
   unsigned long long* h_dc = nullptr;  // pinned
@@ -379,7 +379,7 @@ int iso_ctx_destroy(iso_ctx* c) {
                     &c->nn_pts,   &c->nn_t,
                     &c->nn_w,       &c->nn_out,     &c->br_centres, &c->br_hd,   &c->br_pred,
                     &c->br_flags,   &c->br_count,  &c->pvals,  &c->dense_check,  &c->nrm,
-                    &c->dgrid,      &c->dvals,      &c->emc_cells, &c->emc_first, &c->emc_cross,
+                    &c->dgrid,      &c->dvals,      &c->emc_cells, &c->emc_index, &c->emc_first, &c->emc_cross,
                     &c->emc_flips,  &c->emc_ctr,    &c->br_coarse, &c->br_proof,
                     &c->f_signs,    &c->f_flags,    &c->f_slots,   &c->f_rowbase, &c->f_ctl};
   if (c->b_graph) (void)hipGraphExecDestroy(c->b_graph);
@@ -1129,6 +1129,14 @@ int iso_extract_emc(iso_ctx* c, const iso_grid_desc* desc, float epsilon, iso_me
   ISO_HIP(c, ensure(&c->dvals, static_cast<size_t>(D.n_points) * 3 * sizeof(float)));
   float* vals = static_cast<float*>(c->dvals.ptr);
   const iso::DevOp* ops = static_cast<const iso::DevOp*>(c->prog.ptr);
+  // Status words, before anything waits.
+  ISO_HIP(c, ensure(&c->emc_ctr, iso::kEmcSlots * sizeof(unsigned long long)));
+  ISO_HIP(c, iso::launch_fill_u32(static_cast<uint32_t*>(c->emc_ctr.ptr), 2 * iso::kEmcSlots, 0u,
+                                  c->stream));
+  iso::scan::State S;
+  if ((st = prepare_scan(c, 1, &S)) != ISO_OK) return st;
+  ISO_HIP(c, iso::launch_fill_u32(reinterpret_cast<uint32_t*>(S.err), 2, 0u, c->stream));
+  ISO_HIP(c, ensure(&c->emc_index, static_cast<size_t>(D.n_cells) * sizeof(uint32_t)));
   // Directed signs and the active (mixed) cells.
   uint64_t n_act = 0;
   for (int attempt = 0; attempt < 2; ++attempt) {
@@ -1149,12 +1157,7 @@ int iso_extract_emc(iso_ctx* c, const iso_grid_desc* desc, float epsilon, iso_me
   const uint64_t na = n_act ? n_act : 1;
   ISO_HIP(c, ensure(&c->emc_cells, na * sizeof(iso::EmcCell)));
   ISO_HIP(c, ensure(&c->emc_first, 2 * na * sizeof(uint32_t)));
-  ISO_HIP(c, ensure(&c->emc_ctr, iso::kEmcSlots * sizeof(unsigned long long)));
-  ISO_HIP(c, hipMemsetAsync(c->emc_ctr.ptr, 0, iso::kEmcSlots * sizeof(unsigned long long),
-                            c->stream));
-  iso::scan::State S;
   if ((st = prepare_scan(c, n_act, &S)) != ISO_OK) return st;
-  ISO_HIP(c, iso::launch_fill_u32(reinterpret_cast<uint32_t*>(S.err), 2, 0u, c->stream));
   iso::EmcArgs A{};
   A.L = L;
   A.segs_per_row = static_cast<uint32_t>(D.segs_per_row);
@@ -1167,6 +1170,7 @@ int iso_extract_emc(iso_ctx* c, const iso_grid_desc* desc, float epsilon, iso_me
   A.cells = static_cast<iso::EmcCell*>(c->emc_cells.ptr);
   A.vfirst = static_cast<uint32_t*>(c->emc_first.ptr);
   A.tfirst = A.vfirst + na;
+  A.index_of = static_cast<uint32_t*>(c->emc_index.ptr);
   A.counters = static_cast<unsigned long long*>(c->emc_ctr.ptr);
   ISO_HIP(c, ensure(&c->emc_cross, na * 72 * sizeof(float)));
   A.crossings = static_cast<float*>(c->emc_cross.ptr);

@@ -11,7 +11,7 @@
 //      numbering (a feature vertex comes first in its cell, then the cell's
 //      edges in the order its fans or triangles first use them);
 //   2. emit: vertices and index triples, each edge's vertex resolved in the
-//      cell that owns it (found by binary search of the active list);
+//      cell that owns it (found through a map from cells to the list);
 //   3. the edge flips of flip_feature_edges: a fan edge whose two faces
 //      both have feature vertices opposite is rotated; every such edge lies
 //      in one cell or across one cube face, so each is found from one of its
@@ -48,6 +48,7 @@ struct EmcArgs {
   // 72 per active cell: per local edge e, the crossing point (floats 6e..6e+2)
   // and its normalised normal (6e+3..6e+5), written for crossed edges only
   float* crossings;
+  uint32_t* index_of;      // per lattice cell: an active cell's index (else undefined)
   EmcCell* cells;          // n_act
   uint32_t* vfirst;        // n_act: first vertex id of each cell
   uint32_t* tfirst;        // n_act: first triangle of each cell
@@ -59,7 +60,7 @@ struct EmcArgs {
 };
 
 // Stage 0: the crossing points and normals of every active cell's crossed
-// edges, one thread per (cell, edge).
+// edges, one thread per crossing, and index_of.
 hipError_t launch_emc_crossings(const EmcArgs& A, const ProgramKind& kind, hipStream_t s);
 // Stage 1: cells + scan (state for n_act items at one item per thread).
 // The totals land in scan state ctl[1]: triangles << 32 | vertices.
