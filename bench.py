@@ -149,9 +149,9 @@ def measured_traffic():
 
 
 # VALU issue peak: 256 CUs x 4 SIMDs at 2.4 GHz, one wave64 FP32 VALU
-# instruction per SIMD every 2 clocks (32 lanes a clock: the rate behind the
-# 157.3 TFLOP/s FP32 vector figure).
-VALU_PEAK_GINSTR = 256 * 4 * 2.4e9 / 2 / 1e9
+# instruction per SIMD every 4 clocks (16 lanes a clock; the 157.3 TFLOP/s FP32
+# vector figure counts packed instructions, which the kernels are built without).
+VALU_PEAK_GINSTR = 256 * 4 * 2.4e9 / 4 / 1e9
 FP32_PEAK_TFLOPS = 157.3
 
 
