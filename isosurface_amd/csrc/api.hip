@@ -1462,8 +1462,10 @@ int iso_extract_lhmc(iso_ctx* c, int32_t max_depth, iso_mesh_out* out) {
   N.split = static_cast<const uint64_t*>(c->oc_split.ptr);
   N.ctl = static_cast<unsigned long long*>(c->oc_ctl.ptr);
   const bool on_device = out->memory == ISO_MEMORY_DEVICE;
-  uint64_t want_nodes = 1u << 16, want_primal = 1u << 16, want_cubes = 1u << 14,
-           want_table = 1u << 17, want_v = 1u << 15, want_i = 1u << 17;
+  // (a first call's buffers, 35 MB, hold a surface at depth 7: starting over
+  // costs its allocations again)
+  uint64_t want_nodes = 1u << 19, want_primal = 1u << 19, want_cubes = 1u << 16,
+           want_table = 1u << 19, want_v = 1u << 17, want_i = 1u << 19;
   uint64_t nv = 0, ni = 0, vcap = 0, icap = 0;
   float* vdst = nullptr;
   uint32_t* idst = nullptr;
