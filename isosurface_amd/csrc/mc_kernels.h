@@ -71,7 +71,6 @@ struct CellSpace {
   float origin[3];
   float spacing[3];
   const uint64_t* signs;    // the lattice's sign bits, row (y, z) at bit (z ny + y) sign_pitch
-  int64_t sign_pitch;       // nx (flat), or a multiple of 64 (row-aligned)
   uint32_t segs_per_row;
   uint32_t seg_off;         // global index of the lattice's first segment
   const DevOp* ops;         // program source
@@ -79,6 +78,7 @@ struct CellSpace {
   int32_t reserved;
   const float* grid;        // dense samples (a batch's stored program samples), or null
   const float* positions;   // per-point vertex positions, or null
+  int64_t sign_pitch;       // nx (flat), or a multiple of 64 (row-aligned)
 };
 
 // Entry i (the same for every lane) of a chunk table, by scalar loads.

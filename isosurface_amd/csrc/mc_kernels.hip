@@ -235,8 +235,15 @@ __global__ __launch_bounds__(256) void k_batch_signs(const CellSpace* __restrict
 // 2. count + single-pass scan (decoupled look-back)
 // ---------------------------------------------------------------------------
 // The lattice of one extraction, passed by value: every field is uniform.
+// kPitched: the sign rows may be row-aligned.  Where they are flat, a cell's
+// sign bits sit at its samples' index, and emit reckons one address for both.
+// (count and the program's emit read the pitch at no cost: same instructions.)
+template <bool kPitched>
 struct SingleSpace {
   CellSpace C;
+  __device__ __forceinline__ static int64_t pitch(const CellSpace& c) {
+    return kPitched ? c.sign_pitch : c.nx;
+  }
   __device__ __forceinline__ const CellSpace& at(uint32_t g, uint32_t* local) const {
     *local = g;
     return C;
@@ -251,6 +258,7 @@ struct BatchSpace {
   const CellSpace* chunks;
   const uint32_t* seg_start;  // n_chunks + 1 ascending first segments
   uint32_t n_chunks;
+  __device__ __forceinline__ static int64_t pitch(const CellSpace& c) { return c.sign_pitch; }
   __device__ __forceinline__ CellSpace at(uint32_t g, uint32_t* local) const {
     using U32 = const uint32_t __attribute__((address_space(4)))*;
     const U32 first = (U32)(reinterpret_cast<uintptr_t>(seg_start));
@@ -302,7 +310,7 @@ __global__ __launch_bounds__(kCountBlock) void k_count(Space sp, int64_t n_segs,
       const CellSpace& C = sp.at(static_cast<uint32_t>(g), &gg);
       const uint64_t* __restrict__ S = C.signs;
       const int64_t nx = C.nx, ny = C.ny;
-      const int64_t pitch = C.sign_pitch;
+      const int64_t pitch = Space::pitch(C);
       const uint32_t spr = C.segs_per_row;
       const uint32_t cyn = static_cast<uint32_t>(ny - 1);
       const uint32_t row = gg / spr;
@@ -674,7 +682,7 @@ __global__ __launch_bounds__(kEmitThreads) void k_emit(EmitArgs A, Space sp) {
     // x-1, x, x+1, read straight from the flat sign array (the guard words
     // cover x-1 at the array's start; bits of rows or columns outside the
     // lattice are never used).
-    const int64_t pitch = C.sign_pitch;
+    const int64_t pitch = Space::pitch(C);
     const int64_t fs = (static_cast<int64_t>(cz) * ny + cy) * pitch + cx;
     uint32_t cube = 0;
 #pragma unroll
@@ -1073,12 +1081,6 @@ hipError_t launch_signs_program(const DevOp* ops, int n_ops, const Lattice& L, c
 
 namespace {
 
-SingleSpace single_space(const Lattice& L, const McDims& D, const uint64_t* signs,
-                         const DevOp* ops, int n_ops, const float* grid,
-                         const float* positions) {
-  return SingleSpace{single_cell_space(L, D, signs, ops, n_ops, grid, positions)};
-}
-
 EmitArgs emit_args(const McBuffers& B) {
   EmitArgs A;
   A.seg = B.seg;
@@ -1121,12 +1123,20 @@ unsigned emit_blocks(const McBuffers& B, int per_cu, K kernel, int64_t n_cells =
   return static_cast<unsigned>(blocks);
 }
 
+template <int kSrc, bool kPitched>
+void launch_emit_single(const EmitArgs& A, const CellSpace& C, const McDims& D, const McBuffers& B,
+                        hipStream_t s) {
+  auto k = k_emit<kSrc, SingleSpace<kPitched>>;
+  launch_k(k, dim3(emit_blocks(B, 0, k, D.n_cells)), dim3(kEmitThreads), s, A,
+           SingleSpace<kPitched>{C});
+}
+
 }  // namespace
 
 hipError_t launch_count(const Lattice& L, const McDims& D, const McBuffers& B, hipStream_t s) {
   if (D.n_blocks > 0x7fffffff) return hipErrorInvalidValue;
-  const SingleSpace sp = single_space(L, D, B.signs, nullptr, 0, nullptr, nullptr);
-  launch_k(k_count<SingleSpace, kCountRounds>, dim3(static_cast<unsigned>(D.n_blocks)),
+  const SingleSpace<true> sp{single_cell_space(L, D, B.signs, nullptr, 0, nullptr, nullptr)};
+  launch_k(k_count<SingleSpace<true>, kCountRounds>, dim3(static_cast<unsigned>(D.n_blocks)),
            dim3(kCountBlock), s, sp, D.n_segs, D.n_blocks, B);
   return hipGetLastError();
 }
@@ -1135,16 +1145,16 @@ hipError_t launch_emit(const float* grid, const DevOp* ops, int n_ops, const flo
                        const Lattice& L, const McDims& D, const McBuffers& B, hipStream_t s) {
   if ((positions && !grid) || (!grid && !ops)) return hipErrorInvalidValue;
   const EmitArgs A = emit_args(B);
-  const SingleSpace sp = single_space(L, D, B.signs, ops, n_ops, grid, positions);
+  const CellSpace C = single_cell_space(L, D, B.signs, ops, n_ops, grid, positions);
+  const bool flat = D.sign_pitch == L.nx;
   if (grid && positions) {
-    auto k = k_emit<kEmitPositions, SingleSpace>;
-    launch_k(k, dim3(emit_blocks(B, 0, k, D.n_cells)), dim3(kEmitThreads), s, A, sp);
+    if (!flat) return hipErrorInvalidValue;  // (a grid's signs)
+    launch_emit_single<kEmitPositions, false>(A, C, D, B, s);
   } else if (grid) {
-    auto k = k_emit<kEmitGrid, SingleSpace>;
-    launch_k(k, dim3(emit_blocks(B, 0, k, D.n_cells)), dim3(kEmitThreads), s, A, sp);
+    if (flat) launch_emit_single<kEmitGrid, false>(A, C, D, B, s);
+    else launch_emit_single<kEmitGrid, true>(A, C, D, B, s);
   } else {
-    auto k = k_emit<kEmitProgram, SingleSpace>;
-    launch_k(k, dim3(emit_blocks(B, 0, k, D.n_cells)), dim3(kEmitThreads), s, A, sp);
+    launch_emit_single<kEmitProgram, true>(A, C, D, B, s);
   }
   return hipGetLastError();
 }
@@ -1162,11 +1172,9 @@ hipError_t launch_signs_directed(const DevOp* ops, int n_ops, const Lattice& L, 
 
 hipError_t launch_emit_directed(const float* values, const Lattice& L, const McDims& D,
                                 const McBuffers& B, hipStream_t s) {
-  if (!values) return hipErrorInvalidValue;
-  const EmitArgs A = emit_args(B);
-  const SingleSpace sp = single_space(L, D, B.signs, nullptr, 0, values, nullptr);
-  auto k = k_emit<kEmitDirected, SingleSpace>;
-  launch_k(k, dim3(emit_blocks(B, 0, k, D.n_cells)), dim3(kEmitThreads), s, A, sp);
+  if (!values || D.sign_pitch != L.nx) return hipErrorInvalidValue;  // (k_signs_directed's signs)
+  launch_emit_single<kEmitDirected, false>(
+      emit_args(B), single_cell_space(L, D, B.signs, nullptr, 0, values, nullptr), D, B, s);
   return hipGetLastError();
 }
 
@@ -1193,9 +1201,8 @@ hipError_t launch_emit_band(const float* values, const uint8_t* brick_flags, int
   A.nbx = nbx;
   A.nby = nby;
   A.brick_shift = brick_shift;
-  const SingleSpace sp = single_space(L, D, B.signs, ops, n_ops, values, nullptr);
-  auto k = k_emit<kEmitBand, SingleSpace>;
-  launch_k(k, dim3(emit_blocks(B, 0, k, D.n_cells)), dim3(kEmitThreads), s, A, sp);
+  launch_emit_single<kEmitBand, true>(
+      A, single_cell_space(L, D, B.signs, ops, n_ops, values, nullptr), D, B, s);
   return hipGetLastError();
 }
 
