@@ -261,19 +261,22 @@ __global__ __launch_bounds__(256) void k_brick_flags(
 // them at a time however few each block has; with sound bounds they are
 // evaluated over the operations that matter in the tile and, of those, in the
 // blocks that the 256 come from.  Row-aligned sign words, one 16-bit store a
-// row.  Bound by instruction issue: 98.4 M samples of 1024 smoothly joined
-// spheres at 1025^3 take 4.8 ms, where the flat background pass and a
-// culled evaluation of the whole program took 19.2 ms.
+// row.  kKind: 0 any program, 1 bounded without a stack, 2 bounded with one;
+// without sound bounds each wavefront skips by sdf_eval_culled what cannot
+// change its own 64 samples.  Bound by instruction issue: 98.4 M samples of
+// 1024 smoothly joined spheres at 1025^3 take 4.8 ms, where the flat background
+// pass and a culled evaluation of the whole program took 19.2 ms.
 constexpr int kTileBlocks = 64;
 constexpr int kTileSamples = kTileSide * kTileSide * kTileSide;
 constexpr int kBandListCap = 512;
 constexpr int kBandCoords = kTileSide + 2;
 constexpr int kBandWaves = 4;
 
-template <bool kStack>
+template <int kKind>
 __global__ __launch_bounds__(64 * kBandWaves) void k_band_tiles(
-    CellSpace C, BrickGrid G, int bounded, const uint8_t* __restrict__ flags, uint32_t n_tiles,
+    CellSpace C, BrickGrid G, const uint8_t* __restrict__ flags, uint32_t n_tiles,
     unsigned long long* evaluated, ResetArgs R) {
+  constexpr bool kStack = kKind == 2;
   __shared__ uint64_t s_sign[kTileBlocks];
   __shared__ uint64_t s_mask[kBandListCap];
   __shared__ uint64_t s_from[kTileSamples / 64];  // blocks that each 64 queue entries come from
@@ -390,7 +393,7 @@ __global__ __launch_bounds__(64 * kBandWaves) void k_band_tiles(
   if (total) {
     const OpsPtr ops = as_constant(C.ops);
     const int n_ops = C.n_ops;
-    const int first = leading_scopes(ops, n_ops);
+    const int first = kKind ? leading_scopes(ops, n_ops) : 0;
     if (wv == 0) {
       if (lane < 3 * kBandCoords) {
         const int a = lane / kBandCoords;
@@ -406,7 +409,7 @@ __global__ __launch_bounds__(64 * kBandWaves) void k_band_tiles(
       }
       lds_barrier<1>();
       int len = kBandListCap + 1;
-      if (bounded) {
+      if constexpr (kKind != 0) {
         float blo[3], bhi[3], vlo, vhi;
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
@@ -436,7 +439,7 @@ __global__ __launch_bounds__(64 * kBandWaves) void k_band_tiles(
     const int len = __builtin_amdgcn_readfirstlane(s_len);
     const uint16_t* list = len <= kBandListCap ? s_list : nullptr;
     const int m = len <= kBandListCap ? len : n_ops - first;
-    constexpr int kPoints = kStack ? 2 : 4;
+    constexpr int kPoints = kKind == 0 ? 1 : kStack ? 2 : 4;
     const int64_t base = (static_cast<int64_t>(s0[2]) * n[1] + s0[1]) * n[0] + s0[0];
     for (uint32_t q0 = static_cast<uint32_t>(wv) * 64 * kPoints; q0 < total;
          q0 += 64 * kPoints * kBandWaves) {
@@ -455,7 +458,10 @@ __global__ __launch_bounds__(64 * kBandWaves) void k_band_tiles(
       }
       // (spare points repeat the queue's last entry)
       from |= s_from[(total - 1) >> 6];
-      sdf_eval_list<kPoints, kStack>(ops, first, list, s_mask, from, m, p, v);
+      if constexpr (kKind == 0)
+        v[0] = sdf_eval_culled(C.ops, n_ops, p[0][0], p[0][1], p[0][2]);
+      else
+        sdf_eval_list<kPoints, kStack>(ops, first, list, s_mask, from, m, p, v);
 #pragma unroll
       for (int j = 0; j < kPoints; ++j) {
         if (q0 + 64 * j + lane >= total) continue;
@@ -471,8 +477,8 @@ __global__ __launch_bounds__(64 * kBandWaves) void k_band_tiles(
       }
     }
     __syncthreads();
-    // One counter line for every 64 tiles: thousands of tiles adding to one
-    // word would wait for each other.
+    // Tiles add to kCounterLines lines in turn: thousands of them adding to
+    // one word would wait for each other.
     if (threadIdx.x == 0) atomicAdd(evaluated + kCounterStride * (tile % kCounterLines), total);
   }
   store_tile_signs(C, s_sign, s0, tx, threadIdx.x, 64 * kBandWaves);
@@ -626,16 +632,11 @@ hipError_t launch_band_tiles(const DevOp* ops, int n_ops, const ProgramKind& kin
   R.n_blocks = D.n_blocks;
   R.totals = B.totals;
   const CellSpace C = single_cell_space(L, D, B.signs, ops, n_ops, values, nullptr);
-  const int bounded = kind.bounded && lattice_bounded(L) ? 1 : 0;
-  const dim3 grid(static_cast<unsigned>(n_tiles)), block(64 * kBandWaves);
-  // (without sound bounds the first push must be kept as it is: no shortcut
-  // for it, as the interpreter without a stack takes)
-  if (kind.stack || !bounded)
-    hipLaunchKernelGGL(k_band_tiles<true>, grid, block, 0, s, C, G, bounded, flags,
-                       static_cast<uint32_t>(n_tiles), evaluated, R);
-  else
-    hipLaunchKernelGGL(k_band_tiles<false>, grid, block, 0, s, C, G, bounded, flags,
-                       static_cast<uint32_t>(n_tiles), evaluated, R);
+  const auto kernel = !kind.bounded || !lattice_bounded(L) ? k_band_tiles<0>
+                      : kind.stack                           ? k_band_tiles<2>
+                                                             : k_band_tiles<1>;
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(n_tiles)), dim3(64 * kBandWaves), 0, s, C, G,
+                     flags, static_cast<uint32_t>(n_tiles), evaluated, R);
   return hipGetLastError();
 }
 

@@ -31,11 +31,11 @@ def desc(n, origin=(0.0, 0.0, 0.0), spacing=None):
     return d
 
 
-def smooth(n):
+def smooth(n, more=()):
     r = W.SplitMix64(41)
     return DemoSource(smooth_union_all(
         [Translate(tuple(r.uniform(-0.4, 0.4) for _ in range(3)), Sphere(r.uniform(0.02, 0.06)))
-         for _ in range(n)], 0.02))
+         for _ in range(n)] + list(more), 0.02))
 
 
 def tree():
@@ -49,6 +49,7 @@ SOURCES = {
     "smooth700": lambda: smooth(700),
     "tree": tree,
     "unbounded": lambda: DemoSource(Union(Sphere(0.3), Translate((1e30, 0.0, 0.0), Sphere(0.1)))),
+    "unbounded100": lambda: smooth(100, [Translate((1e30, 0.0, 0.0), Sphere(0.1))]),
 }
 
 
