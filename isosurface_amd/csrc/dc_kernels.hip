@@ -178,12 +178,15 @@ __global__ __launch_bounds__(256) void k_sample_normals(const DevOp* __restrict_
 }
 
 // The normal at each marked lattice point of a brick of 4^3, 12 bytes at the
-// point's place in the lattice.  kKind: 0 any program, 1 bounded without a
-// stack, 2 bounded with one: then the operations are bounded over the brick's
-// marked points and only those that can change a value there are evaluated, at
-// the six points of a central difference at once.  (The normals of a 128^3
-// lattice over 32 boxes: 43 us; listing the points by a scan and evaluating
-// all 32 at each took 35 and 87.)
+// point's place in the lattice.  kKind: 1 a bounded program without a stack, 2
+// one with a stack: then the operations are bounded over the brick's marked
+// points and only those that can change a value there are evaluated, at the six
+// points of a central difference at once.  (The normals of a 128^3 lattice over
+// 32 boxes: 43 us; listing the points by a scan and evaluating all 32 at each
+// took 35 and 87.)  0: without sound bounds on the program, its culled
+// evaluation one point after the other; kEach: nor on the points, each lane by
+// itself (a brick has few marked points, and the lanes of the others idle).
+constexpr int kEach = 3;
 template <int kKind>
 __global__ __launch_bounds__(256) void k_dc_normals(const DevOp* __restrict__ ops, int n_ops,
                                                     Lattice L, DcBricks K, float eps,
@@ -206,16 +209,21 @@ __global__ __launch_bounds__(256) void k_dc_normals(const DevOp* __restrict__ op
     const float px = lattice_coord(L, 0, x), py = lattice_coord(L, 1, y),
                 pz = lattice_coord(L, 2, z);
     qef::Vec3f nrm;
-    if (kKind == 0 || eps == 0.0f) {
+    if (kKind == kEach || eps == 0.0f) {
       nrm = central_normal(ops, n_ops, px, py, pz, eps);
     } else {
-      const OpsPtr list = as_constant(ops);
       // the points of central_normal
       const float p[6][3] = {{px + eps, py + 0.0f, pz + 0.0f}, {px - eps, py - 0.0f, pz - 0.0f},
                              {px + 0.0f, py + eps, pz + 0.0f}, {px - 0.0f, py - eps, pz - 0.0f},
                              {px + 0.0f, py + 0.0f, pz + eps}, {px - 0.0f, py - 0.0f, pz - eps}};
       float v[6];
-      sdf_eval_near<6, kKind == 2>(list, n_ops, lane_ops(list, 0, n_ops), p, v);
+      if constexpr (kKind == 0) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) v[k] = sdf_eval_culled(ops, n_ops, p[k][0], p[k][1], p[k][2]);
+      } else {
+        const OpsPtr list = as_constant(ops);
+        sdf_eval_near<6, kKind == 2>(list, n_ops, lane_ops(list, 0, n_ops), p, v);
+      }
       const float e2 = 2.0f * eps;
       nrm = qef::normalised_or_zero(
           qef::Vec3f{(v[0] - v[1]) / e2, (v[2] - v[3]) / e2, (v[4] - v[5]) / e2});
@@ -312,8 +320,11 @@ hipError_t launch_dc_normals(const DevOp* ops, int n_ops, const ProgramKind& kin
   uint64_t blocks = (K.count() + 3) / 4;
   if (blocks > 65536) blocks = 65536;
   // (epsilon widens the points' box: bounds need it small as well)
-  const bool bounded = kind.bounded && lattice_bounded(L) && epsilon < 1.0e15f;
-  const auto kernel = !bounded ? k_dc_normals<0> : kind.stack ? k_dc_normals<2> : k_dc_normals<1>;
+  const bool near = lattice_bounded(L) && epsilon < 1.0e15f;
+  const auto kernel = !near          ? k_dc_normals<kEach>
+                      : !kind.bounded ? k_dc_normals<0>
+                      : kind.stack    ? k_dc_normals<2>
+                                      : k_dc_normals<1>;
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, ops, n_ops, L, K,
                      epsilon, B.marks, normals);
   return hipGetLastError();

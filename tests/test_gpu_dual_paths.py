@@ -38,10 +38,10 @@ def check(ctx, src, d, eps=1e-6, want_mesh=True):
     assert not want_mesh or len(ref.indices) > 0
 
 
-def spheres(n, k):
+def spheres(n, k, more=()):
     r = W.SplitMix64(31)
     parts = [Translate(tuple(r.uniform(-0.4, 0.4) for _ in range(3)), Sphere(r.uniform(0.02, 0.1)))
-             for _ in range(n)]
+             for _ in range(n)] + list(more)
     return DemoSource(smooth_union_all(parts, k) if k else union_all(parts))
 
 
@@ -58,6 +58,7 @@ SOURCES = {
     "smooth130": lambda: spheres(130, 0.03),
     "tree": tree,
     "unbounded": lambda: DemoSource(Union(Sphere(0.3), Translate((1e30, 0.0, 0.0), Sphere(0.1)))),
+    "unbounded100": lambda: spheres(100, 0.03, [Translate((1e30, 0.0, 0.0), Sphere(0.1))]),
 }
 
 
@@ -71,6 +72,16 @@ def test_programs_on_ragged_lattices(ctx, name, n):
 @pytest.mark.parametrize("eps", [1e-3, 0.25])
 def test_small_lattices(ctx, n, eps):
     check(ctx, tree(), desc(n), eps, want_mesh=min(n) > 20)
+
+
+@pytest.mark.parametrize("eps", [1e11, 1e16])  # beyond what bounds of the points allow, too
+def test_lattice_without_sound_bounds(ctx, eps):
+    src = Union(Sphere(1.0e16), Translate((0.0, 0.0, 1.0e16), Sphere(5.0e15)))
+    check(ctx, src, desc((41, 42, 43), origin=(-2.0e16,) * 3, spacing=(1.0e15,) * 3), eps)
+
+
+def test_steps_without_sound_bounds(ctx):
+    check(ctx, tree(), desc((33, 34, 35)), 1e16)
 
 
 def test_analytic_normals(ctx):
