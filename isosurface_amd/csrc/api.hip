@@ -1,6 +1,7 @@
 // C ABI of isosurface_amd: contexts, sources, extraction, timing.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cmath>
 #include <cstring>
@@ -1462,10 +1463,15 @@ int iso_extract_lhmc(iso_ctx* c, int32_t max_depth, iso_mesh_out* out) {
   N.split = static_cast<const uint64_t*>(c->oc_split.ptr);
   N.ctl = static_cast<unsigned long long*>(c->oc_ctl.ptr);
   const bool on_device = out->memory == ISO_MEMORY_DEVICE;
-  // (a first call's buffers, 35 MB, hold a surface at depth 7: starting over
-  // costs its allocations again)
-  uint64_t want_nodes = 1u << 19, want_primal = 1u << 19, want_cubes = 1u << 16,
-           want_table = 1u << 19, want_v = 1u << 17, want_i = 1u << 19;
+  // A context's first call has room for the surface of some dozens of shapes at
+  // depth 6, and at lesser depths a quarter for each (a union of 32 boxes has
+  // 585, 3985, 20 k and 90 k nodes at depths 3 to 6, as many primal vertices and
+  // a quarter as many cubes).  More would cost the calls that do not need it
+  // more than starting over costs those that do: up to 2 MB a buffer, as here,
+  // the allocations take 0.1 ms in all, four times larger ones 1.3 to 1.7 ms.
+  uint64_t want_nodes = 1ull << (5 + 2 * std::clamp(max_depth, 3, 6));
+  uint64_t want_primal = want_nodes, want_cubes = want_nodes / 4, want_table = 2 * want_nodes,
+           want_v = want_nodes / 4, want_i = want_nodes;
   uint64_t nv = 0, ni = 0, vcap = 0, icap = 0;
   float* vdst = nullptr;
   uint32_t* idst = nullptr;
@@ -1565,12 +1571,21 @@ int iso_extract_lhmc(iso_ctx* c, int32_t max_depth, iso_mesh_out* out) {
     int d = 0;
     for (; d <= d1 && n_nodes + count[d] <= N.cap; ++d) n_nodes += count[d];
     if (d <= d1) {
-      // Depth d does not fit; the depths below it hold about four times as
-      // many nodes (they follow a surface).
+      // Depth d does not fit.  The depths below it hold four to five times as
+      // many nodes (they follow a surface), but for the last, which holds the
+      // children of few.
       n_nodes += count[d];
       if (n_nodes >= 0xffffffffull)
         return fail(c, ISO_ERR_OVERFLOW, "octree has 2^32 or more nodes");
-      want_nodes = d < d1 ? 4 * n_nodes : n_nodes;
+      want_nodes = d < d1 - 1 ? 5 * n_nodes : n_nodes + n_nodes / 16 + 64;
+      // The other buffers with it, so that they need no start of their own (of a
+      // large tree one by one, for memory).
+      if (want_nodes <= 1ull << 24) {
+        want_primal = want_nodes + want_nodes / 8;
+        want_cubes = want_v = want_nodes / 4;
+        want_i = want_nodes + want_nodes / 2;
+        want_table = iso::lhmc_table_size(want_i / 3);
+      }
       continue;
     }
     if (count[d1 + 1])

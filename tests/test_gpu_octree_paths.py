@@ -5,8 +5,8 @@ Nodes are evaluated over the operations that can change a value among a
 wavefront's 64 (runs longer than 64 operations, operands below on the value
 stack, nested translations, programs whose bounds are not sound), depths of
 fewer nodes than a wavefront and of many workgroups, primal vertices on a bit
-lattice or sorted, and every buffer starts too small in a fresh context, or
-larger than needed after a larger call."""
+lattice or sorted, and buffers that are too small in a fresh context, each in
+its turn, or larger than needed after a larger call."""
 import ctypes as C
 
 import numpy as np
@@ -70,6 +70,50 @@ def test_buffers_grow_and_are_reused(ctx):
             same(fresh, DemoSource(Sphere(0.3)), depth)
     finally:
         fresh.close()
+
+
+# From depth 6 on a fresh context has room for 131072 nodes and primal vertices,
+# 32768 cubes and vertices, 131072 indices and a table for 43690 triangles.
+# (radius, depth): nodes, primal vertices, mesh vertices (two less than cubes),
+# indices.
+OUTGROWN = {
+    "nothing": (0.2, 6),
+    "table_and_indices": (0.3, 7),     # 84113, 101269, 27768, 166596
+    "cubes_and_vertices": (0.33, 7),   # 104465, 124903, 33552, 201300
+    "primal_vertices": (0.35, 7),      # 116561, 139567, 37920, 227508
+    "nodes_of_last_depth": (0.3, 8),   # 339153 (84113 without it)
+    "nodes_before_it": (0.45, 8),      # 772689 (193169 without it)
+}
+
+
+@pytest.mark.parametrize("device", [False, True])
+@pytest.mark.parametrize("what", sorted(OUTGROWN))
+def test_each_buffer_outgrown_on_the_bit_lattice(what, device):
+    import torch
+    radius, depth = OUTGROWN[what]
+    src = DemoSource(Sphere(radius))
+    fresh = Context(0)
+    try:
+        if not device:
+            ref = same(fresh, src, depth)
+        else:
+            ref = O.extract_lhmc(src.program(), depth, 0)
+            nv, ni = len(ref.vertices), len(ref.indices)
+            v = torch.zeros((nv, 3), device="cuda")
+            i = torch.zeros(ni, dtype=torch.int32, device="cuda")
+            torch.cuda.synchronize()
+            fresh.upload_program(src.program())
+            out = A.IsoMeshOut(v.data_ptr(), i.data_ptr(), nv, ni, 0, 0, A.ISO_MEMORY_DEVICE, 0)
+            assert fresh.lib.iso_extract_lhmc(fresh.handle, depth, C.byref(out)) == 0
+            assert (out.vertex_count, out.index_count) == (nv, ni)
+            assert v.cpu().numpy().tobytes() == ref.vertices.tobytes()
+            assert np.array_equal(i.cpu().numpy().view(np.uint32), ref.indices)
+    finally:
+        fresh.close()
+    nodes = len(O.lhmc_octree(src.program(), depth)[0])
+    assert (nodes > 131072) == what.startswith("nodes")
+    assert (len(ref.vertices) > 32768) == (what not in ("nothing", "table_and_indices"))
+    assert (len(ref.indices) > 131072) == (what != "nothing")
 
 
 def test_device_buffers_too_small(ctx):
