@@ -455,9 +455,13 @@ hipError_t launch_emc_crossings(const EmcArgs& A, const ProgramKind& kind, hipSt
   if (!A.crossings) return hipErrorInvalidValue;
   const uint64_t blocks = (A.n_act + kGroup - 1) / kGroup;
   if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
-  // (crossings interpolate lattice points, epsilon moves off them)
-  const bool near =
-      A.epsilon > 0.0f && A.epsilon < 1.0e15f && kind.bounded && lattice_bounded(A.L);
+  // A crossing can lie off its edge: a corner is outside if any component is
+  // positive, so the edge's own can have one sign at both ends (inside a spindle
+  // torus).  -a / (b - a) is then at most 2^24, as the difference of two floats is
+  // no less than an ulp of either, and the point 2^25 times as far out as they
+  // are.  Epsilon moves off it.
+  const bool near = A.epsilon > 0.0f && A.epsilon < 1.0e15f && kind.bounded &&
+                    lattice_bounded(A.L, 33554432.0f);
   const auto kernel = !near        ? k_emc_crossings<false, false>
                       : kind.stack ? k_emc_crossings<true, true>
                                    : k_emc_crossings<true, false>;

@@ -14,8 +14,9 @@ constexpr int kTileSide = 1 << kTileShift;
 
 // Whether interval bounds of the program over this lattice are sound: every
 // parameter and coordinate is finite and far from overflowing a square.
+// `reach`: and so are points that many times as far out as the lattice's.
 bool program_bounded(const DevOp* ops, int n_ops);
-bool lattice_bounded(const Lattice& L);
+bool lattice_bounded(const Lattice& L, float reach = 1.0f);
 // Whether the program holds values below the running one.
 bool program_needs_stack(const DevOp* ops, int n_ops);
 

@@ -329,10 +329,11 @@ bool program_bounded(const DevOp* ops, int n_ops) {
   return true;
 }
 
-bool lattice_bounded(const Lattice& L) {
+bool lattice_bounded(const Lattice& L, float reach) {
   const int64_t n[3] = {L.nx, L.ny, L.nz};
   for (int a = 0; a < 3; ++a)
-    if (!small(L.origin[a]) || !small(L.spacing[a] * static_cast<float>(n[a]))) return false;
+    if (!small(reach * L.origin[a]) || !small(reach * (L.spacing[a] * static_cast<float>(n[a]))))
+      return false;
   return true;
 }
 

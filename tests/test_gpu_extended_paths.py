@@ -75,6 +75,27 @@ def test_unions(ctx, name, eps):
     check(ctx, src, desc((96, 97, 98)), eps)
 
 
+# With the coordinates of the last scale times 2^25, bounds of the crossings' box
+# are not sound any more.
+@pytest.mark.parametrize("scale", [1.0, 2.0**20, 2.0**40])
+def test_crossings_off_their_edges(ctx, scale):
+    """Inside a spindle torus a corner can be positive in one component only, and
+    the crossing of an edge along another lies far outside the edge."""
+    src = Union(Torus(0.05 * scale, 0.3 * scale),
+                union_all(Translate(tuple(scale * c for c in (0.1 * i - 0.4, 0.05 * i, -0.3)),
+                                    Sphere(0.1 * scale)) for i in range(8)))
+    d = desc((40, 41, 42), tuple(scale * c for c in (-0.437, -0.463, -0.4)),
+             tuple(0.9 * scale / k for k in (39, 40, 41)))
+    x, y = (float(np.float32(d.origin[a]) + np.float32(i) * np.float32(d.spacing[a]))
+            for a, i in ((0, 12), (1, 20)))
+    column = [O.sample_vector(src.program(), x, y,
+                              float(np.float32(d.origin[2]) + np.float32(i) * np.float32(d.spacing[2])))
+              for i in range(d.nz)]
+    ends = [(a[2], b[2]) for a, b in zip(column, column[1:]) if (a > 0).any() != (b > 0).any()]
+    assert any(a * b > 0 for a, b in ends)  # a crossing that no interpolation gives
+    check(ctx, src, d, 1e-4 * scale)
+
+
 def test_small_lattices(ctx):
     for n in ((2, 3, 2), (9, 8, 7), (33, 34, 35)):
         check(ctx, tree(3, 8), desc(n), 1e-5, want_mesh=min(n) > 20)
