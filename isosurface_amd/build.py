@@ -60,6 +60,7 @@ def build(verbose: bool = False) -> Path:
     subprocess.run(cmd, check=True, cwd=str(ROOT))
     os.replace(tmp, LIB)
     build_example(verbose)
+    build_sqrt_check(verbose)
     return LIB
 
 
@@ -74,6 +75,19 @@ def build_example(verbose: bool = False) -> Path:
         print(" ".join(cmd), flush=True)
     subprocess.run(cmd, check=True, cwd=str(ROOT))
     return EXAMPLE
+
+
+SQRT_CHECK = ROOT / "tests" / "native" / "libsqrt_check.so"
+
+
+def build_sqrt_check(verbose: bool = False) -> Path:
+    """Compiles the kernels that a GPU test compares the device square root with."""
+    cmd = [hipcc(), *HIP_FLAGS, "-shared", "-x", "hip",
+           str(SQRT_CHECK.with_name("sqrt_check.hip")), "-o", str(SQRT_CHECK)]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.run(cmd, check=True, cwd=str(ROOT))
+    return SQRT_CHECK
 
 
 if __name__ == "__main__":
