@@ -2,11 +2,11 @@
 dc_kernels.hip) against the oracle byte for byte.
 
 Lattices of at least 92^3 samples take the sparse samples: sides around the
-4^3 bricks and 16^3 tiles, one wavefront a tile and four, surfaces through
-lattice points and dual points, descending lattices.  Normals of every kind of
-program: long runs, operands below on the value stack, nested translations,
-programs whose bounds are not sound; by central differences of small and large
-steps, and the program's own."""
+4^3 bricks and 16^3 tiles, one wavefront a tile (the other splits:
+test_gpu_wavefronts.py), surfaces through lattice points and dual points,
+descending lattices.  Normals of every kind of program: long runs, operands below
+on the value stack, nested translations, programs whose bounds are not sound; by
+central differences of small and large steps, and the program's own."""
 import numpy as np
 import pytest
 

@@ -4,8 +4,9 @@
 Lattices of at least 92^3 samples take the sparse values: every primitive and
 operator (lines that miss, tori, which no bound proves, operands below on the
 value stack, nested translations, runs of more than 64), sides around bricks
-and tiles, surfaces on lattice points, one wavefront a tile, unbounded
-programs; analytic normals and central differences of small and large steps."""
+and tiles, surfaces on lattice points, one wavefront a tile (the other splits:
+test_gpu_wavefronts.py), crossings off their edges, unbounded programs; analytic
+normals and central differences of small and large steps."""
 import numpy as np
 import pytest
 

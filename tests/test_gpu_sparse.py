@@ -3,11 +3,12 @@
 Bounds prove the sign of whole 4^3 bricks and only the others are evaluated,
 over the operations that matter in their 16^3 tile.  The cases sit where that
 can go wrong: lattice sides around the brick and tile edges (all of at least
-92^3 samples, where the sparse pass takes over), one wavefront per tile and four, every primitive and operator (runs longer than 64 operands,
-tiles whose list does not fit, nested translations, operands below on the value
-stack), surfaces that pass exactly through lattice points, negative spacings,
-and programs or lattices whose bounds are not sound.  The mesh must equal the
-oracle's byte for byte."""
+92^3 samples, where the sparse pass takes over), every primitive and operator
+(runs longer than 64 operands, tiles whose list does not fit, nested
+translations, operands below on the value stack), surfaces that pass exactly
+through lattice points, negative spacings, and programs or lattices whose bounds
+are not sound.  The mesh must equal the oracle's byte for byte.  (The splits of a
+tile among wavefronts: test_gpu_wavefronts.py.)"""
 import numpy as np
 import pytest
 
