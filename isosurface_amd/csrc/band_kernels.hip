@@ -262,8 +262,8 @@ __global__ __launch_bounds__(256) void k_brick_flags(
 // evaluated over the operations that matter in the tile and, of those, in the
 // blocks that the 256 come from.  Row-aligned sign words, one 16-bit store a
 // row.  kKind: 0 any program, 1 bounded without a stack, 2 bounded with one;
-// without sound bounds each wavefront skips by sdf_eval_culled what cannot
-// change its own 64 samples.  Bound by instruction issue: 98.4 M samples of
+// of the first each wavefront skips by sdf_eval_culled what cannot change its own
+// 64 samples.  Bound by instruction issue: 98.4 M samples of
 // 1024 smoothly joined spheres at 1025^3 take 4.8 ms, where the flat background
 // pass and a culled evaluation of the whole program took 19.2 ms.
 constexpr int kTileBlocks = 64;
@@ -271,9 +271,16 @@ constexpr int kTileSamples = kTileSide * kTileSide * kTileSide;
 constexpr int kBandListCap = 512;
 constexpr int kBandCoords = kTileSide + 2;
 constexpr int kBandWaves = 4;
+// A program longer than a tile's list on a lattice of few tiles: a tile then
+// spans much of the domain and its list seldom fits, so wavefronts that cull for
+// themselves do better, and there are few of them: sixteen a tile.  1000
+// smoothly joined spheres, exact samples alone, listed by four wavefronts /
+// culled by four / culled by sixteen: XXX.
+constexpr int64_t kBandFewTiles = 128;
+constexpr int kBandManyWaves = 16;
 
-template <int kKind>
-__global__ __launch_bounds__(64 * kBandWaves) void k_band_tiles(
+template <int kKind, int W>
+__global__ __launch_bounds__(64 * W) void k_band_tiles(
     CellSpace C, BrickGrid G, const uint8_t* __restrict__ flags, uint32_t n_tiles,
     unsigned long long* evaluated, ResetArgs R) {
   constexpr bool kStack = kKind == 2;
@@ -353,7 +360,7 @@ __global__ __launch_bounds__(64 * kBandWaves) void k_band_tiles(
   if (!work) {
     if (wv == 0) s_sign[lane] = around & 256u ? ~0ull : 0ull;
     __syncthreads();
-    store_tile_signs(C, s_sign, s0, tx, threadIdx.x, 64 * kBandWaves);
+    store_tile_signs(C, s_sign, s0, tx, threadIdx.x, 64 * W);
     return;
   }
   // Each block, a wavefront at a time: signs of the samples that are not
@@ -365,7 +372,7 @@ __global__ __launch_bounds__(64 * kBandWaves) void k_band_tiles(
     held |= (!(k & 1) || l[0] == 0) && (!(k & 2) || l[1] == 0) && (!(k & 4) || l[2] == 0) ? 1u << k : 0u;
   const bool full =
       s0[0] + kTileSide <= n[0] && s0[1] + kTileSide <= n[1] && s0[2] + kTileSide <= n[2];
-  for (int blk = wv; blk < kTileBlocks; blk += kBandWaves) {
+  for (int blk = wv; blk < kTileBlocks; blk += W) {
     const uint32_t w = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(around), blk));
     const bool valid = full || (s0[0] + 4 * (blk & 3) + l[0] < n[0] &&
                                 s0[1] + (blk & 12) + l[1] < n[1] &&
@@ -442,7 +449,7 @@ __global__ __launch_bounds__(64 * kBandWaves) void k_band_tiles(
     constexpr int kPoints = kKind == 0 ? 1 : kStack ? 2 : 4;
     const int64_t base = (static_cast<int64_t>(s0[2]) * n[1] + s0[1]) * n[0] + s0[0];
     for (uint32_t q0 = static_cast<uint32_t>(wv) * 64 * kPoints; q0 < total;
-         q0 += 64 * kPoints * kBandWaves) {
+         q0 += 64 * kPoints * W) {
       float p[kPoints][3], v[kPoints];
       int id[kPoints];
       uint64_t from = 0;
@@ -481,7 +488,7 @@ __global__ __launch_bounds__(64 * kBandWaves) void k_band_tiles(
     // one word would wait for each other.
     if (threadIdx.x == 0) atomicAdd(evaluated + kCounterStride * (tile % kCounterLines), total);
   }
-  store_tile_signs(C, s_sign, s0, tx, threadIdx.x, 64 * kBandWaves);
+  store_tile_signs(C, s_sign, s0, tx, threadIdx.x, 64 * W);
 }
 
 // Cells whose marching-cubes case differs between two sign arrays of the
@@ -632,11 +639,15 @@ hipError_t launch_band_tiles(const DevOp* ops, int n_ops, const ProgramKind& kin
   R.n_blocks = D.n_blocks;
   R.totals = B.totals;
   const CellSpace C = single_cell_space(L, D, B.signs, ops, n_ops, values, nullptr);
-  const auto kernel = !kind.bounded || !lattice_bounded(L) ? k_band_tiles<0>
-                      : kind.stack                           ? k_band_tiles<2>
-                                                             : k_band_tiles<1>;
-  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(n_tiles)), dim3(64 * kBandWaves), 0, s, C, G,
-                     flags, static_cast<uint32_t>(n_tiles), evaluated, R);
+  const bool few = n_tiles <= kBandFewTiles;
+  const bool cull = !kind.bounded || !lattice_bounded(L) || (few && n_ops > kBandListCap);
+  const auto kernel = cull ? (few ? k_band_tiles<0, kBandManyWaves> : k_band_tiles<0, kBandWaves>)
+                      : kind.stack ? k_band_tiles<2, kBandWaves>
+                                   : k_band_tiles<1, kBandWaves>;
+  const int waves = cull && few ? kBandManyWaves : kBandWaves;
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(n_tiles)),
+                     dim3(static_cast<unsigned>(64 * waves)), 0, s, C, G, flags,
+                     static_cast<uint32_t>(n_tiles), evaluated, R);
   return hipGetLastError();
 }
 

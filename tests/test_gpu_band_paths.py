@@ -31,11 +31,11 @@ def desc(n, origin=(0.0, 0.0, 0.0), spacing=None):
     return d
 
 
-def smooth(n, more=()):
+def smooth(n, more=(), k=0.02):
     r = W.SplitMix64(41)
     return DemoSource(smooth_union_all(
         [Translate(tuple(r.uniform(-0.4, 0.4) for _ in range(3)), Sphere(r.uniform(0.02, 0.06)))
-         for _ in range(n)] + list(more), 0.02))
+         for _ in range(n)] + list(more), k))
 
 
 def tree():
@@ -50,13 +50,16 @@ SOURCES = {
     "tree": tree,
     "unbounded": lambda: DemoSource(Union(Sphere(0.3), Translate((1e30, 0.0, 0.0), Sphere(0.1)))),
     "unbounded100": lambda: smooth(100, [Translate((1e30, 0.0, 0.0), Sphere(0.1))]),
+    "blended600": lambda: smooth(600, k=0.3),
 }
 
 
 @pytest.mark.parametrize("name", sorted(SOURCES))
 @pytest.mark.parametrize("brick", [0, A.ISO_BAND_BRICK8])
-@pytest.mark.parametrize("n", [(17, 33, 18), (33, 32, 31), (67, 50, 40), (9, 8, 130)])
+@pytest.mark.parametrize("n", [(17, 33, 18), (33, 32, 31), (67, 50, 40), (9, 8, 130), (83, 81, 70)])
 def test_certified_band_is_the_oracles_mesh(ctx, name, brick, n):
+    # (the last has more than 128 tiles: lists however long the program, and
+    # programs without sound bounds by four wavefronts)
     src = SOURCES[name]()
     band = NarrowBand(ctx)
     ctx.upload_program(src.program())
