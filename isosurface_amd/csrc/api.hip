@@ -1687,7 +1687,7 @@ int iso_batch_upload(iso_ctx* c, const iso_node* nodes, uint64_t n_nodes,
   std::vector<iso::DevOp> ops;
   std::vector<uint32_t> op_off(n_chunks), seg_start(n_chunks + 1), tile_start(n_chunks + 1);
   std::vector<uint64_t> word_start(n_chunks + 1), sign_off(n_chunks), row_off(n_chunks);
-  uint64_t segs = 0, words = 0, sign_words = 0, row_words = 0, tiles = 0, cells = 0;
+  uint64_t segs = 0, words = 0, sign_words = 0, row_words = 0, tiles = 0, samples = 0, cells = 0;
   bool bounded = true, stack = false;
   for (uint32_t i = 0; i < n_chunks; ++i) {
     const iso_chunk_desc& ch = chunks[i];
@@ -1720,6 +1720,7 @@ int iso_batch_upload(iso_ctx* c, const iso_node* nodes, uint64_t n_nodes,
     sign_words += static_cast<uint64_t>(D.n_sign_words) + 3;
     row_words += static_cast<uint64_t>(iso::mc_dims_pitched(L).n_sign_words) + 3;
     tiles += static_cast<uint64_t>(iso::tile_count(L.nx, L.ny, L.nz));
+    samples += static_cast<uint64_t>(D.n_points);
     cells += static_cast<uint64_t>(D.n_cells);
     if (segs >= (1ull << 26))
       return fail(c, ISO_ERR_INVALID_ARGUMENT, "batch has 2^26 or more 64-cell segments");
@@ -1727,9 +1728,11 @@ int iso_batch_upload(iso_ctx* c, const iso_node* nodes, uint64_t n_nodes,
   seg_start[n_chunks] = static_cast<uint32_t>(segs);
   word_start[n_chunks] = words;
   tile_start[n_chunks] = static_cast<uint32_t>(tiles);
-  // Sparse classification unless bounds are not sound somewhere, or the rows
-  // are so narrow that row-aligned words would be mostly padding.
-  const bool sparse = bounded && row_words <= 8 * sign_words && tiles < (1ull << 30);
+  // Sparse classification unless bounds are not sound somewhere, too many tiles
+  // are nearly empty, or the rows are so narrow that row-aligned words would be
+  // mostly padding.
+  const bool sparse = bounded && row_words <= 8 * sign_words &&
+                      iso::sparse_batch(static_cast<int64_t>(tiles), static_cast<int64_t>(samples));
   if (sparse) {
     sign_words = row_words;
     sign_off = row_off;

@@ -44,6 +44,20 @@ inline bool sparse_lattice(const Lattice& L, bool program_is_bounded) {
 // Tiles of a lattice.
 int64_t tile_count(int64_t nx, int64_t ny, int64_t nz);
 
+// Whether a batch is classified sparsely, by the tiles and samples of its
+// chunks (its programs and lattices bounded): a tile costs the bounds of its
+// operations, a chain, however little of it the chunk fills.  Where more tiles
+// than the chip holds at once are nearly empty, the flat pass over the samples
+// does better: whole calls of 8192 chunks of 5^3, flat / sparse, over four
+// primitives with a value stack 130 / 170 us, over two 95 / 113.  Chunks of 9^3
+// fill enough (257 / 254), and 2048 chunks of 3^3 take 106 / 101.
+constexpr int64_t kBatchManyTiles = 4096;
+constexpr int64_t kBatchTileSamples = 256;
+inline bool sparse_batch(int64_t tiles, int64_t samples) {
+  return tiles < (int64_t(1) << 30) &&
+         (tiles <= kBatchManyTiles || samples >= kBatchTileSamples * tiles);
+}
+
 // Program signs like launch_signs_program, from dims of mc_dims_pitched:
 // bounds prove the sign of whole 4^3 bricks of samples, and only the bricks
 // they cannot prove are evaluated (their samples go to `values` when it is

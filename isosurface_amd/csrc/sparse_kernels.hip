@@ -428,7 +428,13 @@ hipError_t launch_batch_signs_sparse(const BatchPlan& P, const McBuffers& B, int
   R.incl = B.incl;
   R.n_blocks = n_blocks;
   R.totals = B.totals;
-  constexpr int64_t kGroup = 4;  // about a row of a chunk's tiles
+  // About a row of a chunk's tiles.  Not a divisor of their usual numbers, 8, 27,
+  // 64, 125: where a chunk of S cells has tiles of one sample at its ends, its
+  // full ones would all go to the same half of the XCDs (1024 chunks of 17^3 over
+  // four primitives with a value stack: signs 214 us by groups of 4, 137 by 8 or
+  // 16, 85 by 7; over 31 without 487 / 350 / 217; of 65^3, 128 chunks, 133 / 133
+  // / 144).
+  constexpr int64_t kGroup = 7;
   if (P.n_tiles >= kManyTiles)
     return P.stack ? launch_tiles(k_signs_sparse<BatchTiles, 1, true, kSigns>, 64, t, P.n_tiles, kGroup, R, s)
                    : launch_tiles(k_signs_sparse<BatchTiles, 1, false, kSigns>, 64, t, P.n_tiles, kGroup, R, s);

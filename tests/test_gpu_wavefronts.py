@@ -1,13 +1,14 @@
 """The sparse kernels' splits of a tile among wavefronts (sparse_kernels.hip)
 against the oracle byte for byte: eight for up to 2048 tiles, four for fewer
 than 16384, one from there on, each side of both lines; signs, dual contouring's
-samples and directed values of a lattice, and a batch's signs (four or one);
-programs without a value stack and with one.  The lattices are long rows of
+samples and directed values of a lattice, and a batch's signs (four or one, or
+the flat pass where many tiles are nearly empty); programs without a value stack
+and with one.  The lattices are long rows of
 tiles, most of them a few samples thick."""
 import numpy as np
 import pytest
 
-from isosurface_amd import BatchedMarchingCubes, _abi as A
+from isosurface_amd import BatchedMarchingCubes, _abi as A, chunk_desc
 from isosurface_amd.sources import Difference, RectangularPrism, Sphere, Torus, Translate, Union, union_all
 from oracle import oracle as O
 
@@ -74,16 +75,27 @@ def test_directed_values(ctx, n, name):
     same(ctx.extract_emc(d, 1e-4), O.extract_emc(src.program(), O.as_desc(d), epsilon=1e-4))
 
 
-@pytest.mark.parametrize("name", sorted(SOURCES))
-@pytest.mark.parametrize("chunks", [511, 512])  # of 32 tiles
-def test_batch_signs(ctx, chunks, name):
-    parts = [(Translate((-0.25 * i, 0.0, 0.0), SOURCES[name]()), desc((512, 3, 3), 4.0))
-             for i in range(chunks)]
+def same_batch(ctx, parts):
     meshes = BatchedMarchingCubes(ctx).extract_meshes(parts)
     found = 0
     for (src, d), m in zip(parts, meshes):
-        ref = O.extract_mc(src.program(), desc=O.as_desc(d))
+        grid = O.sample_lattice_threads(src.program(), O.as_desc(d), threads=8)
+        ref = O.extract_mc(grid=grid, desc=O.as_desc(d))
         assert np.array_equal(m.indices, ref.indices)
         assert m.vertices.tobytes() == ref.vertices.tobytes()
         found += len(ref.indices) > 0
-    assert found > 50
+    assert found > len(parts) // 10
+
+
+@pytest.mark.parametrize("name", sorted(SOURCES))
+@pytest.mark.parametrize("chunks", [64, 512])  # of 32 tiles of 1280 samples
+def test_batch_signs(ctx, chunks, name):
+    same_batch(ctx, [(Translate((-0.25 * i, 0.0, 0.0), SOURCES[name]()), desc((512, 16, 5), 4.0))
+                     for i in range(chunks)])
+
+
+@pytest.mark.parametrize("chunks", [4096, 4097])  # of one tile of 125: the flat pass for more
+def test_batches_of_nearly_empty_tiles(ctx, chunks):
+    ball = Union(Difference(Sphere(0.25), Sphere(0.3)), Difference(Torus(0.2, 0.1), Sphere(0.2)))
+    same_batch(ctx, [(Translate((0.5 + 0.0001 * i, 0.5, 0.5), ball), chunk_desc(4))
+                     for i in range(chunks)])
