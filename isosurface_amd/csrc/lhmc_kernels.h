@@ -2,9 +2,9 @@
 //
 // The octree is built breadth first; its nodes live in one array, depth by
 // depth, families of eight together (in Morton order), the families of a depth
-// in no order.  Primal vertices are listed in ascending key order: for shallow trees by marking a bit lattice at depth max_depth + 1
-// indexed by Morton code and scanning it, for deeper ones by sorting the
-// leaves' (vertex, level) pairs.  Dual cubes are then processed in that order
+// in no order.  Primal vertices are listed in ascending key order: for shallow
+// trees by marking a bit lattice at depth max_depth + 1 indexed by Morton code
+// and scanning it, for deeper ones by sorting the leaves' (vertex, level) pairs.  Dual cubes are then processed in that order
 // with an open-addressing table over their edges.
 //
 // Node, vertex and cube counts pass from launch to launch in device memory
@@ -34,7 +34,6 @@ constexpr int kLhmcDenseDepth = 9;
 enum : unsigned long long {
   kLhmcErrScan = 2ull,        // a look-back gave up (scan::State::err)
   kLhmcErrTable = 8ull,       // edge table full
-  kLhmcErrOverflow = 16ull,   // ids beyond u32
 };
 
 // Words of LhmcTree::ctl.

@@ -31,10 +31,18 @@ ProgramKind program_kind(const DevOp* ops, int n_ops);
 // Whether a program lattice is classified sparsely: sound bounds, rows of at
 // least one tile (narrower ones would leave most of a tile and of a sign word
 // empty), and enough samples.  On a small lattice a tile spans many operands
-// and few tiles run, so the dense pass is the faster one: whole extractions,
-// dense / sparse, of 64 spheres minus a torus take 68 / 94 us at 65^3, 83 / 83
-// at 81^3, 102 / 77 at 97^3 and 158 / 74 at 129^3, and of a torus alone 36 /
-// 38, 39 / 44, 41 / 41 and 46 / 42.
+// and few tiles run, so the dense pass is the faster one.  Whole extractions,
+// dense / sparse, in us at 65^3, 81^3, 97^3 and 129^3:
+//   marching cubes
+//     64 spheres minus a torus         71 / 90    86 / 81   109 / 76   169 / 74
+//     1000 smoothly joined spheres   309 / 1937 345 / 357  405 / 290  652 / 224
+//     a sphere minus a torus           37 / 38    40 / 38    44 / 40    57 / 42
+//   dual contouring, a box             87 / 94    91 / 94    95 / 97   125 / 116
+//     32 boxes                        126 / 151  143 / 149  165 / 153  242 / 183
+//     1000 smoothly joined spheres   464 / 2114 526 / 2112 653 / 624 1035 / 668
+//   extended, a box                  129 / 134  131 / 132  136 / 136  146 / 135
+//     32 boxes                       199 / 242  218 / 244  248 / 249  339 / 259
+//     a torus (never proven)         108 / 118  113 / 121  118 / 127  130 / 144
 constexpr int64_t kSparseMinPoints = 786432;  // 92^3
 inline bool sparse_lattice(const Lattice& L, bool program_is_bounded) {
   return L.nx >= kTileSide && L.nx * L.ny * L.nz >= kSparseMinPoints && program_is_bounded &&
