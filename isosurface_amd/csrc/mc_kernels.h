@@ -73,12 +73,12 @@ struct CellSpace {
   const uint64_t* signs;    // the lattice's sign bits, row (y, z) at bit (z ny + y) sign_pitch
   uint32_t segs_per_row;
   uint32_t seg_off;         // global index of the lattice's first segment
+  int64_t sign_pitch;       // nx (flat), or a multiple of 64 (row-aligned)
   const DevOp* ops;         // program source
   int32_t n_ops;
   int32_t reserved;
   const float* grid;        // dense samples (a batch's stored program samples), or null
   const float* positions;   // per-point vertex positions, or null
-  int64_t sign_pitch;       // nx (flat), or a multiple of 64 (row-aligned)
 };
 
 // Entry i (the same for every lane) of a chunk table, by scalar loads.
