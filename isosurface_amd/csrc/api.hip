@@ -878,6 +878,7 @@ int extract_lattice(iso_ctx* c, const iso::Lattice& L, const float* grid, const 
       k.ops = grid ? nullptr : ops;
       k.values = values;
       k.n_prog = grid ? 0 : c->n_prog;
+      // (n_prog decides the rest)
       k.program_kind = grid ? 0 : (c->prog_kind.bounded ? 1 : 0) + (c->prog_kind.stack ? 2 : 0);
       k.B = b;
       return k;
@@ -1688,7 +1689,7 @@ int iso_batch_upload(iso_ctx* c, const iso_node* nodes, uint64_t n_nodes,
   std::vector<uint32_t> op_off(n_chunks), seg_start(n_chunks + 1), tile_start(n_chunks + 1);
   std::vector<uint64_t> word_start(n_chunks + 1), sign_off(n_chunks), row_off(n_chunks);
   uint64_t segs = 0, words = 0, sign_words = 0, row_words = 0, tiles = 0, samples = 0, cells = 0;
-  bool bounded = true, stack = false;
+  bool bounded = true, stack = false, long_programs = false;
   for (uint32_t i = 0; i < n_chunks; ++i) {
     const iso_chunk_desc& ch = chunks[i];
     iso::Lattice L;
@@ -1709,6 +1710,7 @@ int iso_batch_upload(iso_ctx* c, const iso_node* nodes, uint64_t n_nodes,
     const int n_part = static_cast<int>(part.size());
     bounded = bounded && iso::program_bounded(part.data(), n_part) && iso::lattice_bounded(L);
     stack = stack || iso::program_needs_stack(part.data(), n_part);
+    long_programs = long_programs || n_part > iso::kTileListCap;
     seg_start[i] = static_cast<uint32_t>(segs);
     word_start[i] = words;
     tile_start[i] = static_cast<uint32_t>(tiles);
@@ -1786,6 +1788,7 @@ int iso_batch_upload(iso_ctx* c, const iso_node* nodes, uint64_t n_nodes,
   ISO_HIP(c, hipStreamSynchronize(c->stream));
   c->plan.sparse = sparse;
   c->plan.stack = stack;
+  c->plan.long_programs = long_programs;
   c->plan.tile_start = static_cast<const uint32_t*>(c->b_tilestart.ptr);
   c->plan.n_tiles = static_cast<int64_t>(tiles);
   c->plan.chunks = static_cast<const iso::CellSpace*>(c->b_chunks.ptr);

@@ -198,6 +198,7 @@ struct BatchPlan {
   // words of every sample.
   bool sparse;
   bool stack;                  // a chunk's program needs a value stack
+  bool long_programs;          // a chunk's program is longer than a tile's list
   const uint32_t* tile_start;  // device, n_chunks + 1: first tile of each chunk
   int64_t n_tiles;
 };

@@ -797,6 +797,11 @@ __device__ __forceinline__ void sdf_eval_near(OpsPtr ops, int n, const DevOp& he
   }
 }
 
+// Whether a tile of whose n_ops operations m matter, too many for its list, is
+// better evaluated by sdf_eval_near: where nearly all matter throughout the tile
+// they also do in a wavefront's share of it, and bounding them again is lost.
+__device__ __forceinline__ bool prunes_near(int m, int n_ops) { return m <= n_ops - n_ops / 64; }
+
 // A barrier for what the tile's wavefronts exchange in LDS: __syncthreads
 // would also wait for the samples on their way to memory (two microseconds a
 // tile).

@@ -11,6 +11,7 @@ namespace iso {
 // A tile: 16^3 samples, in 64 bricks of 4^3.
 constexpr int kTileShift = 4;
 constexpr int kTileSide = 1 << kTileShift;
+constexpr int kTileListCap = 512;  // operations of a tile's list; a longer one is not kept
 
 // Whether interval bounds of the program over this lattice are sound: every
 // parameter and coordinate is finite and far from overflowing a square.

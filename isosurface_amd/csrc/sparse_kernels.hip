@@ -38,7 +38,7 @@ namespace {
 using namespace mcd;
 
 constexpr int kBricks = 64;      // bricks of a tile: 4 x 4 x 4
-constexpr int kListCap = 512;    // operations of a tile's list; a longer one is not kept
+constexpr int kListCap = kTileListCap;
 constexpr uint32_t kSparseXcds = 8;
 
 // One lattice: its tiles x fastest.
@@ -88,7 +88,18 @@ struct BatchTiles {
 // value that is read, those of all corners of a mixed cell.
 enum SparseMode : int { kSigns, kSamples, kDirected };
 
-template <class Tiles, int W, bool kStack, int kMode>
+//
+// kLong: the program may be longer than a list.  A tile whose list does not fit
+// is then not bounded brick by brick (a chain as long as the program): all its
+// bricks are evaluated, each wavefront bounding the operations for its own
+// samples, 64 at a time (sdf_eval_near).  Whole extractions at 93^3, the program
+// bounded and evaluated whole / near / the dense pass: 2040 smoothly joined
+// spheres 3.87 / 0.44 / 0.68 ms, 2040 joined by minima 2.36 / 0.31 / 0.62; dual
+// contouring of them 4.31 / 0.85 / 7.79 and 2.68 / 0.54 / 5.46.  Where the bounds
+// of the tile leave nearly all operations in, the program is bounded and
+// evaluated whole: 550 spheres that blend everywhere at 129^3 take 1.17 ms so,
+// near 2.20.
+template <class Tiles, int W, bool kStack, int kMode, bool kLong>
 __global__ __launch_bounds__(64 * W) void k_signs_sparse(Tiles tiles, uint32_t n_tiles,
                                                          uint32_t group, ResetArgs R) {
   constexpr int kMargin = kMode == kSamples ? 2 : 1;  // neighbours in a brick's box
@@ -168,12 +179,14 @@ __global__ __launch_bounds__(64 * W) void k_signs_sparse(Tiles tiles, uint32_t n
       }
       lds_barrier<1>();
       const bool fits = len <= kListCap;
-      const int left = bound_lanes<kStack, kMode == kDirected>(
-          ops, first, fits ? len : n_ops - first, blo, bhi, active, fits ? s_list : nullptr, s_mask,
-          &lo, &hi);
-      if (fits) len = left;
-      outside = lo > kOutside;
-      inside = hi <= 0.0f;
+      if (!kLong || fits || !prunes_near(len, n_ops)) {
+        const int left = bound_lanes<kStack, kMode == kDirected>(
+            ops, first, fits ? len : n_ops - first, blo, bhi, active, fits ? s_list : nullptr,
+            s_mask, &lo, &hi);
+        if (fits) len = left;
+        outside = lo > kOutside;
+        inside = hi <= 0.0f;
+      }
     }
     s_sign[lane] = inside ? ~0ull : 0ull;
     const uint64_t todo = __ballot(active && !outside && !inside);
@@ -205,6 +218,7 @@ __global__ __launch_bounds__(64 * W) void k_signs_sparse(Tiles tiles, uint32_t n
     }
   }
   const uint16_t* list = len <= kListCap ? s_list : nullptr;
+  const bool near = kLong && len > kListCap && prunes_near(len, n_ops);
   const int m = len <= kListCap ? len : n_ops - first;
   const int lx = lane & 3, ly = (lane >> 2) & 3, lz = lane >> 4;
   const bool full = s0[0] + kTileSide <= nx && s0[1] + kTileSide <= ny && s0[2] + kTileSide <= nz;
@@ -243,6 +257,19 @@ __global__ __launch_bounds__(64 * W) void k_signs_sparse(Tiles tiles, uint32_t n
 #pragma unroll
       for (int j = 0; j < kPoints; ++j)  // Directed::is_positive, distance.rs:76-79
         v[j] = d[j][0] > 0.0f || d[j][1] > 0.0f || d[j][2] > 0.0f ? 1.0f : -1.0f;
+    } else if (near) {
+      // (outside the leading scopes, which it enters itself)
+#pragma unroll
+      for (int j = 0; j < kPoints; ++j) {
+        const int b = brick[j];
+        const int32_t at[3] = {s0[0] + 4 * (b & 3) + lx, s0[1] + (b & 12) + ly,
+                               s0[2] + 4 * (b >> 4) + lz};
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+          p[j][a] = C.origin[a] +
+                    static_cast<float>(at[a] < n[a] ? at[a] : n[a] - 1) * C.spacing[a];
+      }
+      sdf_eval_near<kPoints, kStack>(ops, n_ops, lane_ops(ops, 0, n_ops), p, v);
     } else {
       sdf_eval_list<kPoints, kStack>(ops, first, list, s_mask, bricks, m, p, v);
     }
@@ -366,19 +393,43 @@ ProgramKind program_kind(const DevOp* ops, int n_ops) {
 
 namespace {
 
+template <int kMode, bool kStack, bool kLong>
+hipError_t launch_single_as(const SingleTiles& t, const Lattice& L, const ResetArgs& R,
+                            hipStream_t s) {
+  const int64_t n = tile_count(L.nx, L.ny, L.nz);
+  const int64_t group = (L.nx + kTileSide - 1) >> kTileShift;
+  if (n <= kFewTiles)
+    return launch_tiles(k_signs_sparse<SingleTiles, 8, kStack, kMode, kLong>, 512, t, n, group, R, s);
+  if constexpr (!kLong) {
+    if (n >= kManyTiles)
+      return launch_tiles(k_signs_sparse<SingleTiles, 1, kStack, kMode, false>, 64, t, n, group, R, s);
+    return launch_tiles(k_signs_sparse<SingleTiles, 4, kStack, kMode, false>, 256, t, n, group, R, s);
+  }
+  return hipErrorInvalidValue;
+}
+
 template <int kMode>
 hipError_t launch_single(const SingleTiles& t, bool stack, const Lattice& L, const ResetArgs& R,
                          hipStream_t s) {
-  const int64_t n = tile_count(L.nx, L.ny, L.nz);
-  const int64_t group = (L.nx + kTileSide - 1) >> kTileShift;
-  if (n >= kManyTiles)
-    return stack ? launch_tiles(k_signs_sparse<SingleTiles, 1, true, kMode>, 64, t, n, group, R, s)
-                 : launch_tiles(k_signs_sparse<SingleTiles, 1, false, kMode>, 64, t, n, group, R, s);
-  if (n <= kFewTiles)
-    return stack ? launch_tiles(k_signs_sparse<SingleTiles, 8, true, kMode>, 512, t, n, group, R, s)
-                 : launch_tiles(k_signs_sparse<SingleTiles, 8, false, kMode>, 512, t, n, group, R, s);
-  return stack ? launch_tiles(k_signs_sparse<SingleTiles, 4, true, kMode>, 256, t, n, group, R, s)
-               : launch_tiles(k_signs_sparse<SingleTiles, 4, false, kMode>, 256, t, n, group, R, s);
+  // (directed values have no evaluation near a wavefront's samples; tiles of
+  // larger lattices span so little that lists fit)
+  if constexpr (kMode != kDirected) {
+    if (t.C.n_ops > kListCap && tile_count(L.nx, L.ny, L.nz) <= kFewTiles)
+      return stack ? launch_single_as<kMode, true, true>(t, L, R, s)
+                   : launch_single_as<kMode, false, true>(t, L, R, s);
+  }
+  return stack ? launch_single_as<kMode, true, false>(t, L, R, s)
+               : launch_single_as<kMode, false, false>(t, L, R, s);
+}
+
+template <bool kStack, bool kLong>
+hipError_t launch_batch_as(const BatchTiles& t, int64_t n_tiles, int64_t group, const ResetArgs& R,
+                           hipStream_t s) {
+  if (n_tiles >= kManyTiles)
+    return launch_tiles(k_signs_sparse<BatchTiles, 1, kStack, kSigns, kLong>, 64, t, n_tiles, group,
+                        R, s);
+  return launch_tiles(k_signs_sparse<BatchTiles, 4, kStack, kSigns, kLong>, 256, t, n_tiles, group,
+                      R, s);
 }
 
 ResetArgs reset_args(const McDims& D, const McBuffers& B) {
@@ -435,11 +486,11 @@ hipError_t launch_batch_signs_sparse(const BatchPlan& P, const McBuffers& B, int
   // 16, 85 by 7; over 31 without 487 / 350 / 217; of 65^3, 128 chunks, 133 / 133
   // / 144).
   constexpr int64_t kGroup = 7;
-  if (P.n_tiles >= kManyTiles)
-    return P.stack ? launch_tiles(k_signs_sparse<BatchTiles, 1, true, kSigns>, 64, t, P.n_tiles, kGroup, R, s)
-                   : launch_tiles(k_signs_sparse<BatchTiles, 1, false, kSigns>, 64, t, P.n_tiles, kGroup, R, s);
-  return P.stack ? launch_tiles(k_signs_sparse<BatchTiles, 4, true, kSigns>, 256, t, P.n_tiles, kGroup, R, s)
-                 : launch_tiles(k_signs_sparse<BatchTiles, 4, false, kSigns>, 256, t, P.n_tiles, kGroup, R, s);
+  if (P.long_programs)
+    return P.stack ? launch_batch_as<true, true>(t, P.n_tiles, kGroup, R, s)
+                   : launch_batch_as<false, true>(t, P.n_tiles, kGroup, R, s);
+  return P.stack ? launch_batch_as<true, false>(t, P.n_tiles, kGroup, R, s)
+                 : launch_batch_as<false, false>(t, P.n_tiles, kGroup, R, s);
 }
 
 }  // namespace iso

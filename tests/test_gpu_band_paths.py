@@ -31,11 +31,20 @@ def desc(n, origin=(0.0, 0.0, 0.0), spacing=None):
     return d
 
 
-def smooth(n, more=(), k=0.02):
+def cluster(far):
+    """Spheres whose values differ by less than the blend's width everywhere, and
+    some that matter nowhere near them."""
+    r = W.SplitMix64(9)
+    return smooth_union_all([Translate(tuple(r.uniform(-0.02, 0.02) for _ in range(3)),
+                                       Sphere(r.uniform(0.2, 0.25))) for _ in range(550)] +
+                            [Translate((5.0 + i, 0.0, 0.0), Sphere(0.1)) for i in range(far)], 0.15)
+
+
+def smooth(n, more=()):
     r = W.SplitMix64(41)
     return DemoSource(smooth_union_all(
         [Translate(tuple(r.uniform(-0.4, 0.4) for _ in range(3)), Sphere(r.uniform(0.02, 0.06)))
-         for _ in range(n)] + list(more), k))
+         for _ in range(n)] + list(more), 0.02))
 
 
 def tree():
@@ -50,7 +59,10 @@ SOURCES = {
     "tree": tree,
     "unbounded": lambda: DemoSource(Union(Sphere(0.3), Translate((1e30, 0.0, 0.0), Sphere(0.1)))),
     "unbounded100": lambda: smooth(100, [Translate((1e30, 0.0, 0.0), Sphere(0.1))]),
-    "blended600": lambda: smooth(600, k=0.3),
+    "cluster550": lambda: DemoSource(cluster(0)),
+    "cluster650": lambda: DemoSource(cluster(100)),
+    "cluster650_stack": lambda: DemoSource(Union(Difference(Sphere(0.2), cluster(100)),
+                                                 Difference(Sphere(0.1), Torus(0.3, 0.05)))),
 }
 
 

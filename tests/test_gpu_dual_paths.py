@@ -84,6 +84,19 @@ def test_steps_without_sound_bounds(ctx):
     check(ctx, tree(), desc((33, 34, 35)), 1e16)
 
 
+def test_lists_that_do_not_fit(ctx):
+    # spheres whose values differ by less than the blend's width everywhere, and
+    # some that matter nowhere near them
+    r = W.SplitMix64(9)
+    long = smooth_union_all([Translate(tuple(r.uniform(-0.02, 0.02) for _ in range(3)),
+                                       Sphere(r.uniform(0.2, 0.25))) for _ in range(550)] +
+                            [Translate((5.0 + i, 0.0, 0.0), Sphere(0.1)) for i in range(100)], 0.15)
+    d = desc((16384, 7, 7), origin=(0.0, 0.47, 0.47), spacing=(1.0 / 16383, 0.01, 0.01))
+    check(ctx, DemoSource(long), d)
+    check(ctx, DemoSource(Union(Difference(Sphere(0.2), long),
+                                Difference(Sphere(0.1), Torus(0.3, 0.05)))), d)
+
+
 def test_analytic_normals(ctx):
     check(ctx, W.boxes_union(32, seed=4), desc((96, 97, 98)), 0.0)
 

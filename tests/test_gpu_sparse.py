@@ -93,6 +93,39 @@ def test_long_runs(ctx, n_ops, k):
     check(ctx, DemoSource(smooth_union_all(parts, k) if k else union_all(parts)), desc(93, 93, 92))
 
 
+def cluster(n, far=0):
+    """n spheres whose values differ by less than the blend's width everywhere, and
+    some that matter nowhere near them."""
+    r = W.SplitMix64(9)
+    return smooth_union_all([Translate(tuple(r.uniform(-0.02, 0.02) for _ in range(3)),
+                                       Sphere(r.uniform(0.2, 0.25))) for _ in range(n)] +
+                            [Translate((5.0 + i, 0.0, 0.0), Sphere(0.1)) for i in range(far)], 0.15)
+
+
+@pytest.mark.parametrize("name", ["run", "stack", "pruned_run", "pruned_stack"])
+@pytest.mark.parametrize("n", [(93, 93, 92), (33000, 5, 5), (262129, 2, 2)])  # 8, 4, 1 wavefronts
+def test_lists_that_do_not_fit(ctx, n, name):
+    if n[0] > 100 and "pruned" in name:
+        pytest.skip("lattices of more tiles have no other branch")
+    long = cluster(550, 100 if "pruned" in name else 0)
+    src = DemoSource(long) if name.endswith("run") else DemoSource(
+        Union(Difference(Sphere(0.2), long), Difference(Sphere(0.1), Torus(0.3, 0.05))))
+    check(ctx, src, desc(*n) if n[1] > 5 else
+          desc(*n, origin=(0.0, 0.44, 0.46), spacing=(1.0 / (n[0] - 1), 0.03, 0.03)))
+
+
+def test_batch_lists_that_do_not_fit(ctx):
+    from isosurface_amd import BatchedMarchingCubes, chunk_desc
+    for src in (DemoSource(cluster(550)), DemoSource(cluster(550, 100)),
+                DemoSource(Union(Difference(Sphere(0.2), cluster(520, 100)),
+                                 Difference(Sphere(0.1), Torus(0.3, 0.05))))):
+        chunks = [(src, chunk_desc(s)) for s in (16, 33, 48)]
+        for (_, d), m in zip(chunks, BatchedMarchingCubes(ctx).extract_meshes(chunks)):
+            ref = O.extract_mc(src.program(), desc=O.as_desc(d))
+            assert len(ref.indices) > 0 and np.array_equal(m.indices, ref.indices)
+            assert m.vertices.tobytes() == ref.vertices.tobytes()
+
+
 def test_surface_through_lattice_points(ctx):
     # faces on lattice planes: the samples there are exactly 0
     check(ctx, Translate((48.0, 48.0, 48.0), RectangularPrism((20.0, 20.0, 15.0))),
