@@ -4,8 +4,9 @@
 // depth, families of eight together (in Morton order), the families of a depth
 // in no order.  Primal vertices are listed in ascending key order: for shallow
 // trees by marking a bit lattice at depth max_depth + 1 indexed by Morton code
-// and scanning it, for deeper ones by sorting the leaves' (vertex, level) pairs.  Dual cubes are then processed in that order
-// with an open-addressing table over their edges.
+// and scanning it, for deeper ones by sorting the leaves' (vertex, level) pairs.
+// Dual cubes are then processed in that order with an open-addressing table over
+// their edges.
 //
 // Node, vertex and cube counts pass from launch to launch in device memory
 // (LhmcTree::ctl).  A launch whose results outgrow a buffer leaves out the

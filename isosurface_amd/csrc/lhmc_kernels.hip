@@ -21,10 +21,10 @@
 //               scanned into first ids, and their crossings written;
 //   5. emit     every listed cube writes its index triples.
 // All steps are queued together, and one round trip tells the host the sizes.
-// Latency bounds this path (a few thousand to a few hundred thousand nodes): depth 7 of the union of 32 boxes took 917 us in 60
-// launches and copies with 13 round trips, of which 131 us scanned 16.7 M
-// lattice words and 133 us searched sorted keys by bisection; now 249 us in
-// fourteen launches.
+// Latency bounds this path (a few thousand to a few hundred thousand nodes):
+// depth 7 of the union of 32 boxes took 917 us in 60 launches and copies with 13
+// round trips, of which 131 us scanned 16.7 M lattice words and 133 us searched
+// sorted keys by bisection; now 249 us in fourteen launches.
 // The output is the reference's for the primal-vertex order "ascending
 // Morton key" (the reference's own order is a std HashMap's, random per
 // process).  Morton::level() keeps the reference's quirk: the truncated

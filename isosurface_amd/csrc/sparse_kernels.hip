@@ -5,13 +5,13 @@
 // four or eight wavefronts takes a tile of 16^3 samples; its first wavefront, one
 // lane for each of the tile's 64 bricks of 4^3, bounds the program over each
 // brick's samples and their lattice neighbours (the box one sample wider on every
-// side): where the bounds exclude zero, the sign of all of them is proven.  A crossing edge joins two neighbouring
-// samples of different sign, so neither of them lies in a proven brick: the
-// evaluated bricks hold every value that is read.  The same pass lists the
-// operations that can change the program's value anywhere in the tile
-// (sparse_eval.h), and the unproven bricks are evaluated over that list, dealt to
-// the wavefronts, a sample of each of two or four bricks a lane.  Signs and values are the dense evaluation's, bit for
-// bit.
+// side): where the bounds exclude zero, the sign of all of them is proven.  A
+// crossing edge joins two neighbouring samples of different sign, so neither of
+// them lies in a proven brick: the evaluated bricks hold every value that is
+// read.  The same pass lists the operations that can change the program's value
+// anywhere in the tile (sparse_eval.h), and the unproven bricks are evaluated
+// over that list, dealt to the wavefronts, a sample of each of two or four bricks
+// a lane.  Signs and values are the dense evaluation's, bit for bit.
 //
 // The sign words are row-aligned (each sample row starts a new word), so a
 // tile's 16 samples of a row are one 16-bit store and no two tiles share a
